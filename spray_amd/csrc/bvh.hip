@@ -489,6 +489,74 @@ __device__ __forceinline__ float boxArea(const float* b) {
   return dx * dy + dy * dz + dz * dx;
 }
 
+// Writes a node's grid and child planes from the boxes of its first nc
+// children (lo xyz, hi xyz each); child words are the caller's.  Per axis the
+// step is the power of two that covers the children's extent in at most 253
+// steps (at least 2^-20 of the largest coordinate, so that base's rounding
+// stays below an eighth of a step), base lies 1/64 of a step or more below
+// the lowest plane, and planes are rounded outwards with 2^-9 of a step to
+// spare: the distance test's cancellation error (nodeBoxes) is below 2^-15 of
+// a step.  An axis whose extent is not finite, or would need a step of 2^62
+// or more, covers everything.
+__device__ __forceinline__ void quantizeNode(const float (&b)[4][6], int nc, BNode4& nd) {
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    float lo = kInfF, hi = -kInfF;
+    bool finite = true;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (i < nc) {
+        lo = fminf(lo, b[i][k]);
+        hi = fmaxf(hi, b[i][3 + k]);
+        finite = finite && fabsf(b[i][k]) < kInfF && fabsf(b[i][3 + k]) < kInfF;
+      }
+    const double ext = (double)hi - (double)lo;
+    const double big = fmax(fabs((double)lo), fabs((double)hi));
+    int e = -126;
+    if (finite) {
+      // smallest e with 253 * 2^e >= ext and 2^e >= big * 2^-20
+      if (ext > 0.0) {
+        e = max(e, ilogb(ext / 253.0));
+        if (ldexp(253.0, e) < ext) ++e;
+      }
+      if (big > 0.0) e = max(e, ilogb(big) - 19);
+    }
+    uint32_t ql = 0, qh = 0;
+    if (!finite || e >= 62) {
+      nd.base[k] = -3.0e38f;
+      nd.scale[k] = ldexpf(1.f, 121);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        if (i < nc)
+          qh |= 255u << (8 * i);
+        else
+          ql |= 255u << (8 * i);
+      }
+    } else {
+      const double s = ldexp(1.0, e), inv = ldexp(1.0, -e);
+      const double bd = (double)lo - s * 0.015625;
+      float base = (float)bd;
+      if ((double)base > bd) base = nextafterf(base, -kInfF);
+      nd.base[k] = base;
+      nd.scale[k] = (float)s;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        uint32_t l = 255u, h = 0u;
+        if (i < nc) {
+          const double x = floor(((double)b[i][k] - (double)base) * inv - 0.001953125);
+          const double y = ceil(((double)b[i][3 + k] - (double)base) * inv + 0.001953125);
+          l = (uint32_t)fmin(fmax(x, 0.0), 255.0);
+          h = (uint32_t)fmin(fmax(y, 0.0), 255.0);
+        }
+        ql |= l << (8 * i);
+        qh |= h << (8 * i);
+      }
+    }
+    nd.plane[2 * k] = ql;
+    nd.plane[2 * k + 1] = qh;
+  }
+}
+
 // Takes cnt consecutive entries of *ctr per lane, in lane order, with one
 // atomic per wave; every lane of the wave calls it (cnt may be 0).
 __device__ __forceinline__ int waveAlloc(int* ctr, int cnt) {
@@ -558,19 +626,14 @@ __device__ __forceinline__ void collapseLevel(
     int q = waveAlloc(nout, ninner);
     if (!act) continue;
     BNode4 nd;
+    float b[4][6];
+#pragma unroll
     for (int i = 0; i < 4; ++i) {
-      float b[6];
-      int word;
-      if (i >= nc) {
-        for (int k = 0; k < 3; ++k) {
-          b[k] = kInfF;
-          b[3 + k] = -kInfF;
-        }
-        word = (int)0x80000000u;
-      } else {
+      int word = (int)0x80000000u;
+      if (i < nc) {
         int c = ch[i];
         const float* src = c < 0 ? leafbox + (size_t)(~c) * 6 : innerbox + (size_t)c * 6;
-        for (int k = 0; k < 6; ++k) b[k] = src[k];
+        for (int k = 0; k < 6; ++k) b[i][k] = src[k];
         if (c < 0) {
           word = (int)(0x80000000u | (1u << 24) | (uint32_t)(~c));
         } else if (count(c) <= kLeafMax) {
@@ -581,16 +644,12 @@ __device__ __forceinline__ void collapseLevel(
           fout[q++] = FrontierItem{c, slot};
           word = slot++;
         }
+      } else {
+        for (int k = 0; k < 6; ++k) b[i][k] = 0.f;
       }
-      nd.lox[i] = b[0];
-      nd.loy[i] = b[1];
-      nd.loz[i] = b[2];
-      nd.hix[i] = b[3];
-      nd.hiy[i] = b[4];
-      nd.hiz[i] = b[5];
       nd.child[i] = word;
     }
-    nd.pad[0] = nd.pad[1] = nd.pad[2] = nd.pad[3] = 0;
+    quantizeNode(b, nc, nd);
     nodes[f.wnode] = nd;
   }
 }
@@ -646,23 +705,15 @@ __global__ void kCollapseGroupLevel(CollapseGroup G, int l, int blocks_per_dom) 
 // Root for tiny domains (<= kLeafMax triangles): one leaf child.
 __global__ void kTinyRoot(int nf, const float* __restrict__ leafbox, BNode4* nodes) {
   BNode4 nd;
-  float b[6] = {kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF};
+  float b[4][6] = {{kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF}};
   for (int i = 0; i < nf; ++i)
     for (int k = 0; k < 3; ++k) {
-      b[k] = fminf(b[k], leafbox[i * 6 + k]);
-      b[3 + k] = fmaxf(b[3 + k], leafbox[i * 6 + 3 + k]);
+      b[0][k] = fminf(b[0][k], leafbox[i * 6 + k]);
+      b[0][3 + k] = fmaxf(b[0][3 + k], leafbox[i * 6 + 3 + k]);
     }
-  for (int i = 0; i < 4; ++i) {
-    bool used = (i == 0);
-    nd.lox[i] = used ? b[0] : kInfF;
-    nd.loy[i] = used ? b[1] : kInfF;
-    nd.loz[i] = used ? b[2] : kInfF;
-    nd.hix[i] = used ? b[3] : -kInfF;
-    nd.hiy[i] = used ? b[4] : -kInfF;
-    nd.hiz[i] = used ? b[5] : -kInfF;
-    nd.child[i] = used ? (int)(0x80000000u | ((uint32_t)nf << 24)) : (int)0x80000000u;
-    nd.pad[i] = 0;
-  }
+  quantizeNode(b, nf > 0 ? 1 : 0, nd);
+  for (int i = 0; i < 4; ++i)
+    nd.child[i] = i == 0 ? (int)(0x80000000u | ((uint32_t)nf << 24)) : (int)0x80000000u;
   nodes[0] = nd;
 }
 

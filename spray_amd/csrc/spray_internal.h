@@ -98,16 +98,21 @@ int scenegenWrite(const spray_scenegen_params& p, const char* dir, const char* n
 // ---------------------------------------------------------------------------
 // Device layouts (shared by host and kernels)
 
-// One 4-wide BVH node: 128 bytes = one HBM/L2 line.  child[i] >= 0 is an
-// inner node index (relative to the domain's node base); a negative value
-// is a leaf: bit 31 set, bits 24..30 the triangle count, bits 0..23 the
-// first triangle in leaf order.  Unused slots have an empty box.
-struct alignas(128) BNode4 {
-  float lox[4], hix[4], loy[4], hiy[4], loz[4], hiz[4];
+// One 4-wide BVH node in 64 bytes (half an L2 line).  Child boxes are 8-bit
+// plane numbers on the node's own grid: plane q of axis k lies at
+// base[k] + q * scale[k], scale[k] a power of two.  plane[2k] / plane[2k + 1]
+// hold the four children's lower / upper planes, child i in byte i, rounded
+// outwards (quantizeNode).  child[i] >= 0 is an inner node index (relative to the
+// domain's node base); a negative value is a leaf: bit 31 set, bits 24..30
+// the triangle count, bits 0..23 the first triangle in leaf order.  Unused
+// slots have an inverted box (lower plane 255, upper plane 0) and an empty
+// leaf.
+struct alignas(64) BNode4 {
+  float base[3], scale[3];
+  uint32_t plane[6];  // lower x, upper x, lower y, upper y, lower z, upper z
   int32_t child[4];
-  int32_t pad[4];
 };
-static_assert(sizeof(BNode4) == 128, "BNode4 must be 128 bytes");
+static_assert(sizeof(BNode4) == 64, "BNode4 must be 64 bytes");
 
 // Triangle in leaf order: 48 bytes; v0.w holds the primitive id.
 struct alignas(16) LTri {

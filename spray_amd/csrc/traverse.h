@@ -17,8 +17,11 @@ namespace spray {
 constexpr int kRing = 16;
 constexpr int kOverflow = 112;
 constexpr uint32_t kStackEmpty = 0xffffffffu;
-// robust slab test (Ize, "Robust BVH Ray Traversal", JCGT 2013): 1 + 2*gamma(3)
-constexpr float kSlabInflate = 1.0000003576278687f;
+// Slack of the interval test (after Ize, "Robust BVH Ray Traversal", JCGT
+// 2013): nodeBoxes' plane distances are within 2^-22 of exact, relatively
+// (1/dir, base - org, their product and the fma round once each); the exit
+// distance is inflated by 2^-20.
+constexpr float kSlabInflate = 1.00000095367431640625f;
 // a ray visits each node of a tree at most once; the bound only stops a
 // corrupt (cyclic) tree from spinning forever
 constexpr uint32_t kMaxNodeVisits = 1u << 22;
@@ -101,44 +104,67 @@ struct TravCount {
   uint32_t tris = 0;
 };
 
+// Largest |1/dir| of the fused box test: beyond it scale * inv could
+// overflow (quantizeNode keeps scale below 2^62).
+constexpr float kFusedInvMax = 1.8446744073709552e19f;  // 2^64
+__device__ __forceinline__ bool needsSafeBoxes(const float inv[3]) {
+  return !(fabsf(inv[0]) < kFusedInvMax && fabsf(inv[1]) < kFusedInvMax && fabsf(inv[2]) < kFusedInvMax);
+}
+
 // Tests the 4 child boxes of a node against [tnear, tfar]; returns a 4-bit
-// hit mask and the entry distances.  kSafe: a ray parallel to a slab with
-// its origin on one of the slab's planes gives 0 * inf = NaN there; that
-// axis then bounds nothing (only rays with an infinite 1/dir component
-// can produce it, so waves without such rays use the unchecked form).
+// hit mask and the entry distances.  The distance of plane q is
+//   (base + q * scale - org) * inv = fma(q, scale * inv, (base - org) * inv)
+// where scale * inv is exact.  Its error is relative to t plus, where the two
+// terms cancel, at most 2^-15 of a plane step: the boxes are at least 2^-9 of
+// a step too large (quantizeNode), so no box the ray meets is missed, and no
+// absolute pad is needed.  A ray's near planes are the lower ones where inv
+// >= 0 and the upper ones elsewhere, one select per axis for all four
+// children.  kSafe (waves with an axis-parallel ray): the difference first,
+// then the product with a possibly infinite inv; 0 * inf = NaN (the origin on
+// the plane) bounds nothing, as max and min drop NaN operands.
 template <bool kSafe>
 __device__ __forceinline__ int nodeBoxes(const BNode4* __restrict__ nd, const float org[3],
                                          const float inv[3], float tnear, float tfar,
                                          float tmin_o[4], int child_o[4]) {
   const float4* q = (const float4*)nd;
-  float4 lox = q[0], hix = q[1], loy = q[2], hiy = q[3], loz = q[4], hiz = q[5];
-  int4 ch = ((const int4*)nd)[6];
-  float lx[4] = {lox.x, lox.y, lox.z, lox.w}, hx[4] = {hix.x, hix.y, hix.z, hix.w};
-  float ly[4] = {loy.x, loy.y, loy.z, loy.w}, hy[4] = {hiy.x, hiy.y, hiy.z, hiy.w};
-  float lz[4] = {loz.x, loz.y, loz.z, loz.w}, hz[4] = {hiz.x, hiz.y, hiz.z, hiz.w};
+  const float4 w0 = q[0];
+  const uint4 w1 = ((const uint4*)nd)[1], w2 = ((const uint4*)nd)[2];
+  const int4 ch = ((const int4*)nd)[3];
   child_o[0] = ch.x;
   child_o[1] = ch.y;
   child_o[2] = ch.z;
   child_o[3] = ch.w;
+  const float bo[3] = {w0.x - org[0], w0.y - org[1], w0.z - org[2]};
+  const float sc[3] = {w0.w, __uint_as_float(w1.x), __uint_as_float(w1.y)};
+  const uint32_t lo[3] = {w1.z, w2.x, w2.z}, hi[3] = {w1.w, w2.y, w2.w};
+  uint32_t nq[3], fq[3];
+  float m[3], c[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const bool neg = inv[k] < 0.f;
+    nq[k] = neg ? hi[k] : lo[k];
+    fq[k] = neg ? lo[k] : hi[k];
+    m[k] = kSafe ? sc[k] : sc[k] * inv[k];
+    c[k] = kSafe ? bo[k] : bo[k] * inv[k];
+  }
   int mask = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    float ax = (lx[i] - org[0]) * inv[0], bx = (hx[i] - org[0]) * inv[0];
-    float ay = (ly[i] - org[1]) * inv[1], by = (hy[i] - org[1]) * inv[1];
-    float az = (lz[i] - org[2]) * inv[2], bz = (hz[i] - org[2]) * inv[2];
-    float lx0 = fminf(ax, bx), lx1 = fmaxf(ax, bx);
-    float ly0 = fminf(ay, by), ly1 = fmaxf(ay, by);
-    float lz0 = fminf(az, bz), lz1 = fmaxf(az, bz);
-    if (kSafe) {
-      if (ax != ax || bx != bx) lx0 = -kInfF, lx1 = kInfF;
-      if (ay != ay || by != by) ly0 = -kInfF, ly1 = kInfF;
-      if (az != az || bz != bz) lz0 = -kInfF, lz1 = kInfF;
+    float tn[3], tf[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float qn = (float)((nq[k] >> (8 * i)) & 255u), qf = (float)((fq[k] >> (8 * i)) & 255u);
+      tn[k] = __builtin_fmaf(qn, m[k], c[k]);
+      tf[k] = __builtin_fmaf(qf, m[k], c[k]);
+      if (kSafe) {
+        tn[k] *= inv[k];
+        tf[k] *= inv[k];
+      }
     }
-    float t0 = fmaxf(fmaxf(lx0, ly0), fmaxf(lz0, tnear));
-    float t1 = fminf(fminf(lx1, ly1), fminf(lz1, tfar));
-    t1 = t1 * kSlabInflate;
+    const float t0 = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), tnear);
+    const float t1 = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), tfar) * kSlabInflate;
     tmin_o[i] = t0;
-    if (t0 <= t1 && lx[i] <= hx[i]) mask |= 1 << i;
+    if (t0 <= t1) mask |= 1 << i;
   }
   return mask;
 }
@@ -303,12 +329,11 @@ __device__ __forceinline__ void travNodeLoop(TravState& s, LaneStack& st, TravCo
   }
 }
 
-// NaN-checked box tests only in waves with an axis-parallel ray: two copies
-// of the loop, so that the common one carries no NaN handling (whose merges
-// would also cost a canonicalisation before every min/max).
+// The safe box tests only in waves with an axis-parallel (or nearly so) ray:
+// two copies of the loop, so that the common one carries no handling of them.
 __device__ __forceinline__ void travNodePhase(TravState& s, LaneStack& st, TravCount& cnt,
                                               bool active, const BNode4* __restrict__ nodes) {
-  if (__ballot(active && hasInfInv(s.inv)) != 0ull)
+  if (__ballot(active && needsSafeBoxes(s.inv)) != 0ull)
     travNodeLoop<true>(s, st, cnt, active, nodes);
   else
     travNodeLoop<false>(s, st, cnt, active, nodes);
