@@ -1409,7 +1409,8 @@ __global__ void __launch_bounds__(kQBlock) kTraceRays(
     const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,
     long long n, int mode, uint32_t max_nodes, float* t_o, float* u_o, float* v_o, int* prim_o,
     uint32_t* ovf, int* err) {
-  __shared__ uint32_t ring[kRing * kQBlock];
+  __shared__ __align__(16) uint32_t ring[kRing * kQBlock + (kQBlock / 64) * kLeafLdsWords];
+  uint32_t* leaf_lds = ring + kRing * kQBlock + (threadIdx.x >> 6) * kLeafLdsWords;
   LaneStack st;
   st.init(ring, ovf);
   TravCount tc;
@@ -1426,7 +1427,7 @@ __global__ void __launch_bounds__(kQBlock) kTraceRays(
     }
     while (__ballot(active && !travDone(s)) != 0ull) {
       travNodePhase(s, st, tc, active, nodes);
-      travLeafPhase(s, st, tc, active, tris);
+      travLeafPhase(s, st, tc, active, tris, leaf_lds);
     }
     if (active) {
       if (mode == 0) {

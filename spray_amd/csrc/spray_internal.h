@@ -106,7 +106,11 @@ int scenegenWrite(const spray_scenegen_params& p, const char* dir, const char* n
 // domain's node base); a negative value is a leaf: bit 31 set, bits 24..30
 // the triangle count, bits 0..23 the first triangle in leaf order.  Unused
 // slots have an inverted box (lower plane 255, upper plane 0) and an empty
-// leaf.
+// leaf.  Traversal loads a node per lane from a place of the lane's own, which
+// the address units serve about one lane and 16 bytes a cycle: they were busy
+// 68% of the time with float boxes (seven loads in 128 bytes); four loads,
+// and fewer operations on planes, took a 64-domain 1024x1024 8 spp frame from
+// 30.5 to 28.6 ms.
 struct alignas(64) BNode4 {
   float base[3], scale[3];
   uint32_t plane[6];  // lower x, upper x, lower y, upper y, lower z, upper z

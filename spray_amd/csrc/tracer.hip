@@ -1212,6 +1212,7 @@ __global__ void __launch_bounds__(kTravBlock) kTraverse(TraceParams P, int plain
   const uint32_t total = nr + ns + nb;
   LaneStack st;
   st.init(ring, P.ovf);
+  uint32_t* leaf_lds = ring + kRing * blockDim.x + (threadIdx.x >> 6) * kLeafLdsWords;
   TravCount tc;
   TravState s;
   unsigned long long rvis = 0, svis = 0, pruned = 0;  // wave-uniform
@@ -1436,7 +1437,7 @@ __global__ void __launch_bounds__(kTravBlock) kTraverse(TraceParams P, int plain
     }
     const bool live = active && !travDone(s);
     travNodePhase(s, st, tc, live, P.nodes);
-    travLeafPhase(s, st, tc, live, P.tris);
+    travLeafPhase(s, st, tc, live, P.tris, leaf_lds);
   }
   shadeSlotsEmpty(P, sh_cur, sh_end, lane);
   blockFlush<5>({&c->radiance_visits, &c->shadow_visits, &c->pruned, &c->node_visits,
@@ -2096,7 +2097,7 @@ static size_t scatterShmem(int nd) { return (size_t)nd * (8 + 4) * 4; }  // boxe
 
 static void ensureOverflow(TracerState* T, size_t lanes) { need(T, T->ovf, lanes * kOverflow * 4); }
 
-static size_t travShmem(int block) { return (size_t)kRing * block * 4; }
+static size_t travShmem(int block) { return ((size_t)kRing * block + (size_t)(block / 64) * kLeafLdsWords) * 4; }
 
 // Blocks of kTraverse with `block` threads that the GPU holds at once.
 static int travResidentBlocks(Ctx* c, int block) {
