@@ -1,6 +1,6 @@
 // HBM domain pool: vertex normals, BVH build (Morton codes, LDS radix sort,
 // PLOC clustering or a Karras hierarchy whose inner boxes are leaf-range
-// unions, collapse to a 4-wide BVH)
+// unions, collapse to a 8-wide BVH)
 // and the batch ray queries behind spray_trace_rays / spray_domain_list.
 //
 // Replaces the reference's per-domain Embree scene (rtcCommit in
@@ -461,27 +461,29 @@ static long long rangeLevels(int n, RangeLevels* L, int* nlev) {
   return off;
 }
 
-// 4-wide nodes of a domain of nf triangles, at most.  In the collapsed tree
-// every inner node has two or more children and at most nf leaves; a node
-// with fewer than four children has only leaf children, so it covers more
-// than kLeafMax triangles, and those nodes are disjoint.  With N4 nodes of
-// four children and Ns of fewer: 3 N4 + Ns <= nf - 1 and Ns <= nf / (kLeafMax
-// + 1), so N4 + Ns <= (nf - 1) / 3 + 2 nf / (3 (kLeafMax + 1)).
+// 8-wide nodes of a domain of nf triangles, at most.  In the collapsed tree
+// a node with fewer than eight children has only leaf children, so it covers
+// more than kLeafMax triangles, and those nodes are disjoint.  With N8 nodes
+// of eight children and Ns of fewer (two or more): 7 N8 + Ns <= nf - 1 and
+// Ns <= nf / (kLeafMax + 1), so N8 + Ns <= (nf - 1) / 7 + 6 nf / (7 (kLeafMax
+// + 1)).
 __host__ __device__ inline long long nodeCap(long long nf) {
-  return nf / 3 + (2 * nf) / (3 * (kLeafMax + 1)) + 16;
+  return nf / 7 + (6 * nf) / (7 * (kLeafMax + 1)) + 16;
 }
+// leaf lists number a domain's nodes in 23 bits (a domain has fewer than 2^24 faces)
+static_assert((1 << 24) / 7 + (6ll * (1 << 24)) / (7 * (kLeafMax + 1)) + 16 < (1 << 23), "node numbers");
 
-// 4-wide collapse levels launched per host wait, and at most (deeper trees
+// 8-wide collapse levels launched per host wait, and at most (deeper trees
 // do not fit the traversal stack anyway); a level counter block is the node
 // counter, the overflow flag and the item count of every level
 constexpr int kLevelBatch = 16;
 constexpr int kMaxLevels = 48;
 constexpr int kLevelWords = 2 + kMaxLevels + 1;
 
-// Collapse the binary tree into 4-wide nodes, one frontier level per launch.
+// Collapse the binary tree into 8-wide nodes, one frontier level per launch.
 struct FrontierItem {
   int bnode;  // binary inner node
-  int wnode;  // 4-wide node slot
+  int wnode;  // 8-wide node slot
 };
 
 __device__ __forceinline__ float boxArea(const float* b) {
@@ -489,22 +491,24 @@ __device__ __forceinline__ float boxArea(const float* b) {
   return dx * dy + dy * dz + dz * dx;
 }
 
-// Writes a node's grid and child planes from the boxes of its first nc
-// children (lo xyz, hi xyz each); child words are the caller's.  Per axis the
-// step is the power of two that covers the children's extent in at most 253
-// steps (at least 2^-20 of the largest coordinate, so that base's rounding
-// stays below an eighth of a step), base lies 1/64 of a step or more below
-// the lowest plane, and planes are rounded outwards with 2^-9 of a step to
-// spare: the distance test's cancellation error (nodeBoxes) is below 2^-15 of
-// a step.  An axis whose extent is not finite, or would need a step of 2^62
-// or more, covers everything.
-__device__ __forceinline__ void quantizeNode(const float (&b)[4][6], int nc, BNode4& nd) {
+// Writes a node's grid and child planes from the boxes (lo xyz, hi xyz) of
+// its children: child i < nc goes to slot slot(i) (4 bits each in slots).  Per
+// axis the step is the power of two that covers the children's extent in at
+// most 253 steps (at least 2^-20 of the largest coordinate, so that base's
+// rounding stays below an eighth of a step), base lies 1/64 of a step or more
+// below the lowest plane, and planes are rounded outwards with 2^-9 of a step
+// to spare: the distance test's cancellation error (nodeBoxes) is below 2^-15
+// of a step.  An axis whose extent is not finite, or would need a step of
+// 2^62 or more, covers everything.  Returns the exponent bytes of meta.
+__device__ __forceinline__ uint32_t quantizeNode(const float (&b)[8][6], int nc, uint32_t slots,
+                                                 BNode8* nd) {
+  uint32_t meta = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     float lo = kInfF, hi = -kInfF;
-    bool finite = true;
+    bool finite = nc > 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < 8; ++i)
       if (i < nc) {
         lo = fminf(lo, b[i][k]);
         hi = fmaxf(hi, b[i][3 + k]);
@@ -521,40 +525,79 @@ __device__ __forceinline__ void quantizeNode(const float (&b)[4][6], int nc, BNo
       }
       if (big > 0.0) e = max(e, ilogb(big) - 19);
     }
-    uint32_t ql = 0, qh = 0;
-    if (!finite || e >= 62) {
-      nd.base[k] = -3.0e38f;
-      nd.scale[k] = ldexpf(1.f, 121);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        if (i < nc)
-          qh |= 255u << (8 * i);
-        else
-          ql |= 255u << (8 * i);
-      }
+    const bool all = !finite || e >= 62;
+    const double inv = ldexp(1.0, all ? 0 : -e);
+    float base = -3.0e38f;
+    if (all) {
+      e = 121;
     } else {
-      const double s = ldexp(1.0, e), inv = ldexp(1.0, -e);
-      const double bd = (double)lo - s * 0.015625;
-      float base = (float)bd;
+      const double bd = (double)lo - ldexp(1.0, e) * 0.015625;
+      base = (float)bd;
       if ((double)base > bd) base = nextafterf(base, -kInfF);
-      nd.base[k] = base;
-      nd.scale[k] = (float)s;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        uint32_t l = 255u, h = 0u;
-        if (i < nc) {
-          const double x = floor(((double)b[i][k] - (double)base) * inv - 0.001953125);
-          const double y = ceil(((double)b[i][3 + k] - (double)base) * inv + 0.001953125);
-          l = (uint32_t)fmin(fmax(x, 0.0), 255.0);
-          h = (uint32_t)fmin(fmax(y, 0.0), 255.0);
-        }
-        ql |= l << (8 * i);
-        qh |= h << (8 * i);
-      }
     }
-    nd.plane[2 * k] = ql;
-    nd.plane[2 * k + 1] = qh;
+    unsigned long long ql = ~0ull, qh = 0ull;  // unused slots: inverted
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < nc) {
+        uint32_t l = 0u, h = 255u;
+        if (!all) {
+          l = (uint32_t)fmin(fmax(floor(((double)b[i][k] - (double)base) * inv - 0.001953125), 0.0), 255.0);
+          h = (uint32_t)fmin(fmax(ceil(((double)b[i][3 + k] - (double)base) * inv + 0.001953125), 0.0), 255.0);
+        }
+        const int sh = 8 * (int)((slots >> (4 * i)) & 7u);
+        ql = (ql & ~(255ull << sh)) | ((unsigned long long)l << sh);
+        qh |= (unsigned long long)h << sh;
+      }
+    nd->base[k] = base;
+    unsigned long long* w = (unsigned long long*)nd->plane[k];
+    w[0] = ql;
+    w[1] = qh;
+    meta |= (uint32_t)(e + 127) << (8 * k);
   }
+  return meta;
+}
+
+// Slots of a node's nc children, 4 bits each: greedily the (child, slot) pair
+// whose child centre lies farthest to the slot's side of the node (bit k of
+// the slot: the upper side of axis k).
+__device__ __forceinline__ uint32_t assignSlots(const float (&b)[8][6], int nc) {
+  float d[8][3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    float lo = kInfF, hi = -kInfF;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if (i < nc) {
+        lo = fminf(lo, b[i][k]);
+        hi = fmaxf(hi, b[i][3 + k]);
+      }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) d[i][k] = (b[i][k] + b[i][3 + k]) - (lo + hi);
+  }
+  uint32_t slots = 0, freec = nc >= 8 ? 255u : (1u << nc) - 1u, frees = 255u;
+  while (freec) {
+    // a pair exists even where every comparison is false (boxes that are not numbers)
+    float best = -kInfF;
+    uint32_t bi = (uint32_t)__ffs((int)freec) - 1u, bs = (uint32_t)__ffs((int)frees) - 1u;
+#pragma unroll
+    for (int i = 0; i < 8; ++i)
+      if ((freec >> i) & 1u) {
+#pragma unroll
+        for (int s = 0; s < 8; ++s) {
+          const float v = ((s & 1) ? d[i][0] : -d[i][0]) + ((s & 2) ? d[i][1] : -d[i][1]) +
+                          ((s & 4) ? d[i][2] : -d[i][2]);
+          if (((frees >> s) & 1u) && v > best) {
+            best = v;
+            bi = i;
+            bs = s;
+          }
+        }
+      }
+    slots |= bs << (4 * bi);
+    freec &= ~(1u << bi);
+    frees &= ~(1u << bs);
+  }
+  return slots;
 }
 
 // Takes cnt consecutive entries of *ctr per lane, in lane order, with one
@@ -581,76 +624,104 @@ __device__ __forceinline__ void collapseLevel(
     int blk, int nblk, const FrontierItem* __restrict__ fin, const int* __restrict__ nin_ptr,
     FrontierItem* fout, int* nout, int* node_counter, int node_cap, const int* __restrict__ left,
     const int* __restrict__ right, const int* __restrict__ first, const int* __restrict__ last,
-    const float* __restrict__ leafbox, const float* __restrict__ innerbox, BNode4* nodes,
+    const float* __restrict__ leafbox, const float* __restrict__ innerbox, BNode8* nodes,
     int* overflow) {
   const int nin = *nin_ptr;
   for (int base = blk * blockDim.x; base < nin; base += nblk * blockDim.x) {
     const int it = base + threadIdx.x;
     const bool act = it < nin;
     FrontierItem f{0, 0};
-    int ch[4] = {0, 0, 0, 0};
+    int ch[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+    float area[8] = {-1.f, -1.f, -1.f, -1.f, -1.f, -1.f, -1.f, -1.f};  // < 0: a leaf, or unused
     int nc = 0;
     auto count = [&](int c) { return c < 0 ? 1 : last[c] - first[c] + 1; };
+    auto openArea = [&](int c) {
+      return c >= 0 && count(c) > kLeafMax ? boxArea(innerbox + (size_t)c * 6) : -1.f;
+    };
+    float b[8][6];
+    uint32_t slots = 0, im = 0;
     int ninner = 0;
     if (act) {
       f = fin[it];
       nc = 2;
       ch[0] = left[f.bnode];
       ch[1] = right[f.bnode];
-      while (nc < 4) {
-        int best = -1;
+      area[0] = openArea(ch[0]);
+      area[1] = openArea(ch[1]);
+      while (nc < 8) {  // open the inner child of the largest area
+        int best = -1, c = 0;
         float barea = -1.f;
-        for (int i = 0; i < nc; ++i) {
-          if (ch[i] >= 0 && count(ch[i]) > kLeafMax) {
-            float a = boxArea(innerbox + (size_t)ch[i] * 6);
-            if (a > barea) {
-              barea = a;
-              best = i;
-            }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+          if (area[i] > barea) {
+            barea = area[i];
+            best = i;
+            c = ch[i];
+          }
+        if (best < 0) break;
+        const int l = left[c], r = right[c];
+        const float al = openArea(l), ar = openArea(r);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+          if (i == best) {
+            ch[i] = l;
+            area[i] = al;
+          }
+          if (i == nc) {
+            ch[i] = r;
+            area[i] = ar;
           }
         }
-        if (best < 0) break;
-        int c = ch[best];
-        ch[best] = left[c];
-        ch[nc++] = right[c];
+        ++nc;
       }
-      // the inner children of a node take consecutive slots (siblings share
-      // cache lines when a ray enters several of them)
-      for (int i = 0; i < nc; ++i) ninner += (ch[i] >= 0 && count(ch[i]) > kLeafMax) ? 1 : 0;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        if (i < nc) {
+          const float* src = ch[i] < 0 ? leafbox + (size_t)(~ch[i]) * 6 : innerbox + (size_t)ch[i] * 6;
+          for (int k = 0; k < 6; ++k) b[i][k] = src[k];
+        } else {
+          for (int k = 0; k < 6; ++k) b[i][k] = 0.f;
+        }
+      }
+      slots = assignSlots(b, nc);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (i < nc && ch[i] >= 0 && count(ch[i]) > kLeafMax) im |= 1u << ((slots >> (4 * i)) & 7u);
+      ninner = __popc(im);
     }
-    int slot = waveAlloc(node_counter, ninner);
-    if (ninner > 0 && slot + ninner > node_cap) {
+    // the inner children of a node take consecutive indices
+    const int cbase = waveAlloc(node_counter, ninner);
+    if (ninner > 0 && cbase + ninner > node_cap) {
       atomicExch(overflow, 1);
       ninner = 0;
+      im = 0;  // capacity exceeded (reported through overflow)
     }
-    int q = waveAlloc(nout, ninner);
+    const int q = waveAlloc(nout, ninner);
     if (!act) continue;
-    BNode4 nd;
-    float b[4][6];
+    BNode8* nd = nodes + f.wnode;
+    const uint32_t meta = quantizeNode(b, nc, slots, nd);
+    nd->child_base = (uint32_t)cbase;
+    nd->meta = meta | (im << 24);
+    for (int i = 0; i < 7; ++i) nd->pad[i] = 0;
+    uint32_t used = 0;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      int word = (int)0x80000000u;
+    for (int i = 0; i < 8; ++i)
       if (i < nc) {
-        int c = ch[i];
-        const float* src = c < 0 ? leafbox + (size_t)(~c) * 6 : innerbox + (size_t)c * 6;
-        for (int k = 0; k < 6; ++k) b[i][k] = src[k];
-        if (c < 0) {
-          word = (int)(0x80000000u | (1u << 24) | (uint32_t)(~c));
+        const uint32_t s = (slots >> (4 * i)) & 7u;
+        const int c = ch[i];
+        uint32_t word = 0;
+        if ((im >> s) & 1u) {
+          const int rank = __popc(im & ((1u << s) - 1u));
+          fout[q + rank] = FrontierItem{c, cbase + rank};
+        } else if (c < 0) {
+          word = (1u << 24) | (uint32_t)(~c);
         } else if (count(c) <= kLeafMax) {
-          word = (int)(0x80000000u | ((uint32_t)count(c) << 24) | (uint32_t)first[c]);
-        } else if (ninner == 0) {  // capacity exceeded (reported through overflow)
-          word = (int)0x80000000u;
-        } else {
-          fout[q++] = FrontierItem{c, slot};
-          word = slot++;
+          word = ((uint32_t)count(c) << 24) | (uint32_t)first[c];
         }
-      } else {
-        for (int k = 0; k < 6; ++k) b[i][k] = 0.f;
+        nd->leaf[s] = word;
+        used |= 1u << s;
       }
-      nd.child[i] = word;
-    }
-    quantizeNode(b, nc, nd);
-    nodes[f.wnode] = nd;
+    for (uint32_t m = ~used & 255u; m != 0u; m &= m - 1u) nd->leaf[__ffs((int)m) - 1] = 0u;
   }
 }
 
@@ -659,7 +730,7 @@ __global__ void kCollapse(const FrontierItem* __restrict__ fin, const int* __res
                           const int* __restrict__ left, const int* __restrict__ right,
                           const int* __restrict__ first, const int* __restrict__ last,
                           const float* __restrict__ leafbox, const float* __restrict__ innerbox,
-                          BNode4* nodes, int* overflow) {
+                          BNode8* nodes, int* overflow) {
   collapseLevel(blockIdx.x, gridDim.x, fin, nin_ptr, fout, nout, node_counter, node_cap, left, right,
                 first, last, leafbox, innerbox, nodes, overflow);
 }
@@ -673,7 +744,7 @@ struct CollapseDom {
   const int *left, *right, *first, *last;
   const float *leafbox, *innerbox;
   FrontierItem *fa, *fb;
-  BNode4* nodes;
+  BNode8* nodes;
   int* cc;
   int node_cap;
 };
@@ -703,18 +774,17 @@ __global__ void kCollapseGroupLevel(CollapseGroup G, int l, int blocks_per_dom) 
 
 
 // Root for tiny domains (<= kLeafMax triangles): one leaf child.
-__global__ void kTinyRoot(int nf, const float* __restrict__ leafbox, BNode4* nodes) {
-  BNode4 nd;
-  float b[4][6] = {{kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF}};
+__global__ void kTinyRoot(int nf, const float* __restrict__ leafbox, BNode8* nodes) {
+  float b[8][6] = {{kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF}};
   for (int i = 0; i < nf; ++i)
     for (int k = 0; k < 3; ++k) {
       b[0][k] = fminf(b[0][k], leafbox[i * 6 + k]);
       b[0][3 + k] = fmaxf(b[0][3 + k], leafbox[i * 6 + 3 + k]);
     }
-  quantizeNode(b, nf > 0 ? 1 : 0, nd);
-  for (int i = 0; i < 4; ++i)
-    nd.child[i] = i == 0 ? (int)(0x80000000u | ((uint32_t)nf << 24)) : (int)0x80000000u;
-  nodes[0] = nd;
+  nodes->meta = quantizeNode(b, nf > 0 ? 1 : 0, 0u, nodes);
+  nodes->child_base = 0;
+  for (int i = 0; i < 7; ++i) nodes->pad[i] = 0;
+  for (int i = 0; i < 8; ++i) nodes->leaf[i] = i == 0 ? (uint32_t)nf << 24 : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -1015,13 +1085,13 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.nrm.reserve(maxv * 12 + 64);
     P.tris.reserve((size_t)P.capacity * maxf * sizeof(LTri) + 64);
     P.fshade.reserve((size_t)P.capacity * maxf * 48 + 64);
-    P.nodes.reserve((size_t)P.capacity * max_nodes * sizeof(BNode4) + 64);
+    P.nodes.reserve((size_t)P.capacity * max_nodes * sizeof(BNode8) + 64);
     size_t bytes = 0;
     P.h_image_off.resize(nd);
     for (int d = 0; d < nd; ++d) {
       P.h_image_off[d] = (long long)bytes;
       const size_t nf = (size_t)P.desc[d].num_tris;
-      bytes += ((size_t)nodeCap((long long)nf) * sizeof(BNode4) + nf * (sizeof(LTri) + 48) + 255) & ~(size_t)255;
+      bytes += ((size_t)nodeCap((long long)nf) * sizeof(BNode8) + nf * (sizeof(LTri) + 48) + 255) & ~(size_t)255;
     }
     SPRAY_HIP(hipHostMalloc(&P.h_image, bytes, hipHostMallocDefault));
     P.h_nrm.resize(nd);
@@ -1033,7 +1103,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.nrm.reserve(tv * 12);
     P.tris.reserve(tf * sizeof(LTri));
     P.fshade.reserve(tf * 48 + 64);
-    P.nodes.reserve(tn * sizeof(BNode4));
+    P.nodes.reserve(tn * sizeof(BNode8));
   }
   // A whole-scene LBVH build runs up to kBuildStreams domain pipelines side
   // by side, one per free hardware queue (domain d on stream d % K, each
@@ -1115,7 +1185,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       std::swap(va, vb);
     }
     LTri* tris = P.tris.as<LTri>() + D.tri_off;
-    BNode4* nodes = P.nodes.as<BNode4>() + D.node_off;
+    BNode8* nodes = P.nodes.as<BNode8>() + D.node_off;
     float* leafbox = TS.lb.as<float>();
     const int node_cap = (int)nodeCap(nf);
     // paged pool: the finished domain's image goes to pinned host memory
@@ -1123,7 +1193,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     auto pageOut = [&]() {
       if (!paged) return;
       char* dst = (char*)P.h_image + P.h_image_off[d];
-      const size_t nb = (size_t)D.num_nodes * sizeof(BNode4), tb = (size_t)nf * sizeof(LTri);
+      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)nf * sizeof(LTri);
       SPRAY_HIP(hipMemcpyAsync(dst, nodes, nb, hipMemcpyDeviceToHost, s));
       SPRAY_HIP(hipMemcpyAsync(dst + nb, tris, tb, hipMemcpyDeviceToHost, s));
       SPRAY_HIP(hipMemcpyAsync(dst + nb + tb, P.fshade.as<float4>() + D.shade_off * 3,
@@ -1145,8 +1215,8 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     int* F = TS.fst.as<int>();
     int* Lst = TS.lst.as<int>();
     float* inner = TS.ib.as<float>();
-    // Collapse the binary tree under `root` into 4-wide nodes; returns the
-    // number of 4-wide levels.
+    // Collapse the binary tree under `root` into 8-wide nodes; returns the
+    // number of 8-wide levels.
     // Levels are launched kLevelBatch at a time; each reads its item count
     // from the device, so the host waits once per batch (a level past the
     // last finds 0 items).  Returns the number of levels with items
@@ -1182,8 +1252,8 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         }
       }
     };
-    // worst-case stack need: three pushes per 4-wide level
-    auto fitsStack = [](int depth) { return 3 * depth + 1 <= kRing + kOverflow; };
+    // worst-case stack need: three pushes per 8-wide level
+    auto fitsStack = [](int depth) { return depth <= kStackMax; };
     int depth = -1;
     if (c->bvh_builder == 1) {
       // PLOC passes until one cluster is left
@@ -1327,7 +1397,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         X.innerbox = TS.ib.as<float>();
         X.fa = TS.fa.as<FrontierItem>();
         X.fb = TS.fb.as<FrontierItem>();
-        X.nodes = P.nodes.as<BNode4>() + D.node_off;
+        X.nodes = P.nodes.as<BNode8>() + D.node_off;
         X.cc = lvl_all.as<int>() + (size_t)d * kLevelWords;
         X.node_cap = (int)nodeCap(D.num_tris);
         levels = std::max(levels, prev_depth.empty() ? kMaxLevels
@@ -1336,8 +1406,8 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       }
       kCollapseGroupInit<<<CG.n, 64, 0, pipe(k)>>>(CG);
       for (int l = 0; l < levels; ++l) {
-        // level l holds at most 4^l items (one root, at most four children per item)
-        const int b = l < 12 ? std::min(bpd, (int)(((1ll << (2 * l)) + 255) / 256)) : bpd;
+        // level l holds at most 8^l items (one root, at most eight children per item)
+        const int b = l < 8 ? std::min(bpd, (int)(((1ll << (3 * l)) + 255) / 256)) : bpd;
         kCollapseGroupLevel<<<CG.n * b, 256, 0, pipe(k)>>>(CG, l, b);
       }
       SPRAY_HIP(hipGetLastError());
@@ -1372,7 +1442,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       }
       int depth = 0;
       while (depth < launched[d] && cc[2 + depth] > 0) ++depth;
-      if (3 * depth + 1 > kRing + kOverflow)
+      if (depth > kStackMax)
         throw StatusError(SPRAY_ERR_CAPACITY, "BVH too deep for the traversal stack");
       P.desc[d].num_nodes = cc[0];
       P.bvh_depth[d] = depth;
@@ -1405,14 +1475,14 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
 constexpr int kQBlock = 256;
 
 __global__ void __launch_bounds__(kQBlock) kTraceRays(
-    const BNode4* __restrict__ nodes, const LTri* __restrict__ tris, const float* __restrict__ org,
+    const BNode8* __restrict__ nodes, const LTri* __restrict__ tris, const float* __restrict__ org,
     const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,
     long long n, int mode, uint32_t max_nodes, float* t_o, float* u_o, float* v_o, int* prim_o,
     uint32_t* ovf, int* err) {
-  __shared__ __align__(16) uint32_t ring[kRing * kQBlock + (kQBlock / 64) * kLeafLdsWords];
-  uint32_t* leaf_lds = ring + kRing * kQBlock + (threadIdx.x >> 6) * kLeafLdsWords;
+  __shared__ __align__(16) uint32_t lds[(kQBlock / 64) * kTravLdsWords];
+  uint32_t* area = lds + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kTravLdsWords;
   LaneStack st;
-  st.init(ring, ovf);
+  st.init(area, ovf);
   TravCount tc;
   TravState s;
   // the loop bound is uniform per block, so every wave runs the phases whole
@@ -1427,7 +1497,7 @@ __global__ void __launch_bounds__(kQBlock) kTraceRays(
     }
     while (__ballot(active && !travDone(s)) != 0ull) {
       travNodePhase(s, st, tc, active, nodes);
-      travLeafPhase(s, st, tc, active, tris, leaf_lds);
+      travLeafPhase(s, st, tc, active, nodes, tris, area);
     }
     if (active) {
       if (mode == 0) {
@@ -1448,11 +1518,11 @@ void traceRaysDevice(Ctx* c, const float* d_org, const float* d_dir, const float
                      float* d_v, int* d_prim) {
   const DomainDesc& D = c->pool.desc[domain];
   int grid = std::min<long long>(2048, std::max<long long>(1, ((long long)n + kQBlock - 1) / kQBlock));
-  c->q_out.reserve((size_t)grid * kQBlock * kOverflow * 4 + 64);
-  int* err = (int*)((char*)c->q_out.p + (size_t)grid * kQBlock * kOverflow * 4);
+  c->q_out.reserve((size_t)grid * kQBlock * kOverflowWords * 4 + 64);
+  int* err = (int*)((char*)c->q_out.p + (size_t)grid * kQBlock * kOverflowWords * 4);
   SPRAY_HIP(hipMemsetAsync(err, 0, 4, c->stream));
   kTraceRays<<<grid, kQBlock, 0, c->stream>>>(
-      c->pool.nodes.as<BNode4>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
+      c->pool.nodes.as<BNode8>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
       d_tnear, d_tfar, (long long)n, mode, (uint32_t)D.num_nodes, d_t, d_u, d_v, d_prim,
       c->q_out.as<uint32_t>(), err);
   int h = 0;
@@ -1469,7 +1539,7 @@ void traceRaysDevice(Ctx* c, const float* d_org, const float* d_dir, const float
 // code never uses the array's name as an address: scratchInit looks up each
 // device's copy once (hipGetSymbolAddress) and keeps the pointer per device.
 constexpr int kScratchBlocks = 256;
-constexpr size_t kScratchStackBytes = (size_t)kScratchBlocks * kQBlock * kOverflow * 4;
+constexpr size_t kScratchStackBytes = (size_t)kScratchBlocks * kQBlock * kOverflowWords * 4;
 constexpr size_t kScratchBytes = kScratchStackBytes + 256;
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 
@@ -1515,7 +1585,7 @@ void traceRaysNoAlloc(Ctx* c, const float* d_org, const float* d_dir, const floa
   int* err = (int*)((char*)base + kScratchStackBytes);
   kClearWord<<<1, 1, 0, c->stream>>>(err);
   kTraceRays<<<grid, kQBlock, 0, c->stream>>>(
-      c->pool.nodes.as<BNode4>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
+      c->pool.nodes.as<BNode8>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
       d_tnear, d_tfar, (long long)n, mode, (uint32_t)D.num_nodes, d_t, d_u, d_v, d_prim, ovf, err);
   SPRAY_HIP(hipGetLastError());
   int h = 0;

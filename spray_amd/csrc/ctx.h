@@ -68,7 +68,7 @@ struct DomainPool {
   std::vector<long long> nverts; // vertices per domain as loaded
   DevBuf d_desc;                 // DomainDesc[ndomains]
   DevBuf vtx, face, rgb, nrm;    // float3 / uint3 / uint32 / float3
-  DevBuf nodes;                  // BNode4
+  DevBuf nodes;                  // BNode8
   DevBuf tris;                   // LTri (leaf order)
   DevBuf fshade;                 // float4[3] per face: vertex normal xyz + vertex rgb bits
   std::vector<int> bvh_depth;

@@ -42,7 +42,7 @@ void DomainPool::releasePaging() {
 
 // Bytes of domain d's image: nodes, leaf-ordered triangles, shading records.
 static size_t imageBytes(const DomainDesc& D) {
-  return (size_t)D.num_nodes * sizeof(BNode4) + (size_t)D.num_tris * (sizeof(LTri) + 48);
+  return (size_t)D.num_nodes * sizeof(BNode8) + (size_t)D.num_tris * (sizeof(LTri) + 48);
 }
 
 // Points domain d's descriptor at block b (host copy and device copy, the
@@ -94,8 +94,8 @@ static int lruLoad(Ctx* c, int d, int keep) {
   const char* src = (const char*)P.h_image + P.h_image_off[d];
   hipStream_t cs = P.copy_stream;
   SPRAY_HIP(hipStreamWaitEvent(cs, P.block_free[victim], 0));
-  const size_t nb = (size_t)D.num_nodes * sizeof(BNode4), tb = (size_t)D.num_tris * sizeof(LTri);
-  SPRAY_HIP(hipMemcpyAsync(P.nodes.as<BNode4>() + (size_t)victim * P.block_nodes, src, nb,
+  const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)D.num_tris * sizeof(LTri);
+  SPRAY_HIP(hipMemcpyAsync(P.nodes.as<BNode8>() + (size_t)victim * P.block_nodes, src, nb,
                            hipMemcpyHostToDevice, cs));
   SPRAY_HIP(hipMemcpyAsync(P.tris.as<LTri>() + (size_t)victim * P.block_tris, src + nb, tb,
                            hipMemcpyHostToDevice, cs));

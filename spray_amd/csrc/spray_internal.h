@@ -98,25 +98,26 @@ int scenegenWrite(const spray_scenegen_params& p, const char* dir, const char* n
 // ---------------------------------------------------------------------------
 // Device layouts (shared by host and kernels)
 
-// One 4-wide BVH node in 64 bytes (half an L2 line).  Child boxes are 8-bit
+// One 8-wide BVH node in 128 bytes, one L2 line.  Child boxes are 8-bit
 // plane numbers on the node's own grid: plane q of axis k lies at
-// base[k] + q * scale[k], scale[k] a power of two.  plane[2k] / plane[2k + 1]
-// hold the four children's lower / upper planes, child i in byte i, rounded
-// outwards (quantizeNode).  child[i] >= 0 is an inner node index (relative to the
-// domain's node base); a negative value is a leaf: bit 31 set, bits 24..30
-// the triangle count, bits 0..23 the first triangle in leaf order.  Unused
-// slots have an inverted box (lower plane 255, upper plane 0) and an empty
-// leaf.  Traversal loads a node per lane from a place of the lane's own, which
-// the address units serve about one lane and 16 bytes a cycle: they were busy
-// 68% of the time with float boxes (seven loads in 128 bytes); four loads,
-// and fewer operations on planes, took a 64-domain 1024x1024 8 spp frame from
-// 30.5 to 28.6 ms.
-struct alignas(64) BNode4 {
-  float base[3], scale[3];
-  uint32_t plane[6];  // lower x, upper x, lower y, upper y, lower z, upper z
-  int32_t child[4];
+// base[k] + q * 2^e[k].  plane[k][0..7] / plane[k][8..15] are the children's
+// lower / upper planes by slot, rounded outwards (quantizeNode).  meta holds
+// the biased exponents (e[k] + 127 in byte k) and, in byte 3, the slots that
+// are inner nodes; those are numbered consecutively from child_base in slot
+// order.  The other slots are leaves: leaf[slot] has the triangle count in
+// bits 24..30 (0: unused slot, its box inverted) and the first triangle in
+// bits 0..23.  A child's slot says on which side of the node it lies (bit k:
+// the upper side of axis k), so that a ray meets the slots roughly in the
+// order of slot ^ (its direction's signs).
+struct alignas(128) BNode8 {
+  float base[3];
+  uint32_t child_base;
+  uint8_t plane[3][16];
+  uint32_t meta;
+  uint32_t pad[7];
+  uint32_t leaf[8];
 };
-static_assert(sizeof(BNode4) == 64, "BNode4 must be 64 bytes");
+static_assert(sizeof(BNode8) == 128, "BNode8 must be 128 bytes");
 
 // Triangle in leaf order: 48 bytes; v0.w holds the primitive id.
 struct alignas(16) LTri {

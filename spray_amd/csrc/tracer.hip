@@ -1138,7 +1138,7 @@ __device__ __forceinline__ void shadeSlotsEmpty(const TraceParams& P, uint32_t c
     P.sh_rec[(size_t)i * kShadeRec + 4] = make_float4(kInfF, 0.f, 0.f, __int_as_float(-1));
 }
 
-__global__ void __launch_bounds__(kTravBlock) kTraverse(TraceParams P, int plain_dom, int phase) {
+__global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int plain_dom, int phase) {
   extern __shared__ uint32_t ring[];
   DevCounters* c = P.ctr;
   if (!c->active) return;
@@ -1211,8 +1211,8 @@ __global__ void __launch_bounds__(kTravBlock) kTraverse(TraceParams P, int plain
   }
   const uint32_t total = nr + ns + nb;
   LaneStack st;
-  st.init(ring, P.ovf);
-  uint32_t* leaf_lds = ring + kRing * blockDim.x + (threadIdx.x >> 6) * kLeafLdsWords;
+  uint32_t* area = ring + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) * kTravLdsWords;
+  st.init(area, P.ovf);
   TravCount tc;
   TravState s;
   unsigned long long rvis = 0, svis = 0, pruned = 0;  // wave-uniform
@@ -1437,7 +1437,7 @@ __global__ void __launch_bounds__(kTravBlock) kTraverse(TraceParams P, int plain
     }
     const bool live = active && !travDone(s);
     travNodePhase(s, st, tc, live, P.nodes);
-    travLeafPhase(s, st, tc, live, P.tris, leaf_lds);
+    travLeafPhase(s, st, tc, live, P.nodes, P.tris, area);
   }
   shadeSlotsEmpty(P, sh_cur, sh_end, lane);
   blockFlush<5>({&c->radiance_visits, &c->shadow_visits, &c->pruned, &c->node_visits,
@@ -1928,7 +1928,7 @@ static TraceParams makeParams(Ctx* c) {
   const DomainPool& pool = c->pool;
   P.desc = pool.d_desc.as<DomainDesc>();
   P.dbox = c->tracer->dbox.as<float4>();
-  P.nodes = pool.nodes.as<BNode4>();
+  P.nodes = pool.nodes.as<BNode8>();
   P.tris = pool.tris.as<LTri>();
   P.vtx = pool.vtx.as<float>();
   P.face = pool.face.as<uint32_t>();
@@ -2095,9 +2095,9 @@ static void domainBoxesUpload(Ctx* c, hipStream_t s) {
 
 static size_t scatterShmem(int nd) { return (size_t)nd * (8 + 4) * 4; }  // boxes, slots, bases
 
-static void ensureOverflow(TracerState* T, size_t lanes) { need(T, T->ovf, lanes * kOverflow * 4); }
+static void ensureOverflow(TracerState* T, size_t lanes) { need(T, T->ovf, lanes * kOverflowWords * 4); }
 
-static size_t travShmem(int block) { return ((size_t)kRing * block + (size_t)(block / 64) * kLeafLdsWords) * 4; }
+static size_t travShmem(int block) { return (size_t)(block / 64) * kTravLdsWords * 4; }
 
 // Blocks of kTraverse with `block` threads that the GPU holds at once.
 static int travResidentBlocks(Ctx* c, int block) {

@@ -72,7 +72,7 @@ struct TraceParams {
   // cell offsets (uint32, at gridOffBytes) and cell domain ids (uint16, at
   // gridIdsBytes)
   const float4* dbox;
-  const BNode4* nodes;
+  const BNode8* nodes;
   const LTri* tris;
   const float* vtx;
   const uint32_t* face;

@@ -1,12 +1,24 @@
-// Closest-hit and any-hit traversal of one domain's 4-wide BVH.
+// Closest-hit and any-hit traversal of one domain's 8-wide BVH.
 //
-// Per-lane short stack: a 16-entry ring in LDS.  Each wave owns kRing x 64
-// words (slot s of lane l of wave w at lds[(w * kRing + s) * 64 + l], so a
-// wave's pushes hit 64 consecutive banks and the address needs no block
-// size);
-// when the ring is full its bottom entry spills to a per-lane overflow
-// stack in HBM, which is popped only once the ring is empty.  The overflow
-// depth bounds the BVH depth; the build rejects deeper trees.
+// What bounds it: vector instructions (issued 75% of the time on a 64-domain
+// 1024x1024 8 spp frame, two thirds of them in node visits) and L2 misses
+// (a random 128-byte line costs the same as a random 64-byte one, and the
+// card serves about 57 G of them a second; the kernel takes about 30 G).
+// Eight children in one line against four in half a line: 20% fewer node
+// visits, 32% fewer wave steps (a step keeps 68% of the lanes busy, 57%
+// before, as a lane no longer stops at its second leaf).  Trace time of a
+// pass, 4-wide -> 8-wide: 256x192 2 spp plain schedule 9.1 -> 7.8 ms,
+// ambient occlusion 512x512 1.11 -> 1.03 ms, 256 uneven domains 13.9 -> 13.5
+// ms, 64 even domains 17.4 -> 17.6 ms.  Tried on it and left out: choosing
+// the nearest child by its entry distance (as many visits as in slot order,
+// 3% slower); node lines fetched by four lanes each through LDS (5% slower).
+//
+// Per-lane stack of node groups (a group: the children of one node that the
+// ray has still to visit): the first kRing entries in LDS.  Each wave owns
+// kRing x 64 entries of 8 bytes (entry e of lane l at (e * 64 + l) * 8 from
+// the wave's base); entries past kRing go to a per-lane overflow stack in
+// HBM.  A node leaves at most one group behind, so the tree's depth bounds
+// the stack; the build rejects deeper trees.
 #pragma once
 
 #include "dmath.h"
@@ -14,86 +26,74 @@
 
 namespace spray {
 
-constexpr int kRing = 16;
-constexpr int kOverflow = 112;
+constexpr int kRing = 12;           // LDS entries, one of them the sentinel
+constexpr int kOverflow = 40;       // HBM entries (2 words each)
+constexpr int kOverflowWords = 2 * kOverflow;
+constexpr int kStackMax = kRing - 1 + kOverflow;  // groups a traversal may hold
+constexpr int kLeafList = 4;        // nodes with leaves to test that a lane may hold
 constexpr uint32_t kStackEmpty = 0xffffffffu;
 // Slack of the interval test (after Ize, "Robust BVH Ray Traversal", JCGT
 // 2013): nodeBoxes' plane distances are within 2^-22 of exact, relatively
 // (1/dir, base - org, their product and the fma round once each); the exit
 // distance is inflated by 2^-20.
 constexpr float kSlabInflate = 1.00000095367431640625f;
-// a ray visits each node of a tree at most once; the bound only stops a
-// corrupt (cyclic) tree from spinning forever
-constexpr uint32_t kMaxNodeVisits = 1u << 22;
+// A ray visits each node of a tree at most once; the bounds only stop a
+// corrupt (cyclic) tree from spinning forever: steps of one node phase, and
+// of all phases of a ray.
+constexpr uint32_t kMaxPhaseSteps = 1u << 16;
+constexpr uint32_t kMaxNodeVisits = 1u << 24;
 
-// The stack state is one packed word per lane: ring head (bits 0-3), ring
-// fill (4-8), overflow fill (9-15), overflow error (16).  The ring pointer
-// carries the LDS address space, so ring accesses stay ds_read/ds_write and
-// are never merged with the overflow path into flat accesses.
+// The ring pointer carries the LDS address space, so ring accesses stay
+// ds_read/ds_write and are never merged with the overflow path into flat
+// accesses.
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
+// n counts the entries, the sentinel (an empty group) at the bottom included.
+// A group is (index of the node's first inner child, children left to visit
+// by their visiting order in bits 0..7 and the node's inner slots in bits
+// 8..15); only the sentinel has no children left.
 struct LaneStack {
-  lds_u32* lds;        // this block's ring base
-  uint32_t* ovf;       // overflow areas of the grid (kOverflow words per thread)
-  uint32_t w;
-  __device__ void init(uint32_t* lds_base, uint32_t* ovf_base) {
-    lds = (lds_u32*)lds_base;
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  typedef __attribute__((address_space(3))) u32x2 lds_u2;
+  lds_u2* lane;        // this lane's entry 0 (entries 64 apart)
+  lds_u32* list;       // this lane's leaf list (entries 64 words apart)
+  uint32_t* ovf;       // overflow areas of the grid (kOverflowWords per thread)
+  uint32_t n;
+  bool err;
+  // area: the wave's LDS (kTravLdsWords)
+  __device__ void init(uint32_t* area, uint32_t* ovf_base) {
+    lane = (lds_u2*)area + (threadIdx.x & 63);
+    list = (lds_u32*)area + kRing * 128 + (threadIdx.x & 63);
     ovf = ovf_base;
-    w = 0;
+    lane[0] = u32x2{0u, 0u};
+    n = 1;
+    err = false;
   }
-  __device__ void reset() { w &= 1u << 16; }
-  __device__ bool overflowed() const { return (w >> 16) & 1u; }
-  __device__ uint32_t count() const { return (w >> 4) & 31u; }
-  __device__ uint32_t* lane_ovf() const {  // only on the rare spill path
-    return ovf + (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * kOverflow;
+  __device__ void reset() {
+    lane[0] = u32x2{0u, 0u};
+    n = 1;
   }
-  __device__ lds_u32& slot(uint32_t s) const {
-    return lds[(((threadIdx.x >> 6) * kRing + (s & (kRing - 1))) << 6) + (threadIdx.x & 63)];
+  __device__ bool overflowed() const { return err; }
+  __device__ uint32_t* spilled(uint32_t e) const {  // only on the rare spill path
+    return ovf + (blockIdx.x * (size_t)blockDim.x + threadIdx.x) * kOverflowWords + 2 * (e - kRing);
   }
-  __device__ void push(uint32_t x) {
-    uint32_t head = w & 15u, count = (w >> 4) & 31u, spilled = (w >> 9) & 127u, err = w >> 16;
-    if (count == kRing) {
-      uint32_t bottom = slot(head);
-      if (spilled < kOverflow)
-        lane_ovf()[spilled++] = bottom;
-      else
-        err = 1;  // reported to the host; never silently dropped
-      head = (head + 1) & (kRing - 1);
-      --count;
-    }
-    slot(head + count) = x;
-    ++count;
-    w = head | (count << 4) | (spilled << 9) | (err << 16);
+  __device__ u32x2 get(uint32_t e) const {
+    if (e < (uint32_t)kRing) return lane[e << 6];
+    const uint32_t* p = spilled(e);
+    return u32x2{p[0], p[1]};
   }
-  // Pushes the first n (<= 3) of x0, x1, x2 (x0 deepest).  With room for
-  // three entries all three slots above the top are written (the unused
-  // ones hold nothing live), so the common case has no branch; a nearly
-  // full ring takes the spilling path.
-  __device__ void push3(uint32_t x0, uint32_t x1, uint32_t x2, uint32_t n) {
-    uint32_t head = w & 15u, count = (w >> 4) & 31u;
-    if (count + 3u <= (uint32_t)kRing) {
-      slot(head + count) = x0;
-      slot(head + count + 1u) = x1;
-      slot(head + count + 2u) = x2;
-      w += n << 4;
+  __device__ bool put(uint32_t e, u32x2 g) {  // false: no room
+    if (e < (uint32_t)kRing) {
+      lane[e << 6] = g;
+    } else if (e < (uint32_t)(kRing + kOverflow)) {
+      uint32_t* p = spilled(e);
+      p[0] = g.x;
+      p[1] = g.y;
     } else {
-      if (n >= 1u) push(x0);
-      if (n >= 2u) push(x1);
-      if (n >= 3u) push(x2);
+      err = true;  // reported to the host; never silently dropped
+      return false;
     }
-  }
-  __device__ uint32_t pop() {
-    uint32_t head = w & 15u, count = (w >> 4) & 31u, spilled = (w >> 9) & 127u;
-    if (count > 0) {
-      w -= 1u << 4;
-      return slot(head + count - 1u);
-    }
-    if (spilled > 0) {
-      --spilled;
-      w = (w & ~(127u << 9)) | (spilled << 9);
-      return lane_ovf()[spilled];
-    }
-    return kStackEmpty;
+    return true;
   }
 };
 
@@ -111,49 +111,44 @@ __device__ __forceinline__ bool needsSafeBoxes(const float inv[3]) {
   return !(fabsf(inv[0]) < kFusedInvMax && fabsf(inv[1]) < kFusedInvMax && fabsf(inv[2]) < kFusedInvMax);
 }
 
-// Tests the 4 child boxes of a node against [tnear, tfar]; returns a 4-bit
-// hit mask and the entry distances.  The distance of plane q is
+// Tests the 8 child boxes of a node against [tnear, tfar]; returns the mask of
+// the slots hit.  The distance of plane q is
 //   (base + q * scale - org) * inv = fma(q, scale * inv, (base - org) * inv)
 // where scale * inv is exact.  Its error is relative to t plus, where the two
 // terms cancel, at most 2^-15 of a plane step: the boxes are at least 2^-9 of
 // a step too large (quantizeNode), so no box the ray meets is missed, and no
 // absolute pad is needed.  A ray's near planes are the lower ones where inv
-// >= 0 and the upper ones elsewhere, one select per axis for all four
-// children.  kSafe (waves with an axis-parallel ray): the difference first,
-// then the product with a possibly infinite inv; 0 * inf = NaN (the origin on
-// the plane) bounds nothing, as max and min drop NaN operands.
+// >= 0 and the upper ones elsewhere, one select per axis for four children.
+// kSafe (waves with an axis-parallel ray): the difference first, then the
+// product with a possibly infinite inv; 0 * inf = NaN (the origin on the
+// plane) bounds nothing, as max and min drop NaN operands.
 template <bool kSafe>
-__device__ __forceinline__ int nodeBoxes(const BNode4* __restrict__ nd, const float org[3],
-                                         const float inv[3], float tnear, float tfar,
-                                         float tmin_o[4], int child_o[4]) {
-  const float4* q = (const float4*)nd;
-  const float4 w0 = q[0];
-  const uint4 w1 = ((const uint4*)nd)[1], w2 = ((const uint4*)nd)[2];
-  const int4 ch = ((const int4*)nd)[3];
-  child_o[0] = ch.x;
-  child_o[1] = ch.y;
-  child_o[2] = ch.z;
-  child_o[3] = ch.w;
-  const float bo[3] = {w0.x - org[0], w0.y - org[1], w0.z - org[2]};
-  const float sc[3] = {w0.w, __uint_as_float(w1.x), __uint_as_float(w1.y)};
-  const uint32_t lo[3] = {w1.z, w2.x, w2.z}, hi[3] = {w1.w, w2.y, w2.w};
-  uint32_t nq[3], fq[3];
+__device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)[3], uint32_t meta,
+                                              const float org[3], const float inv[3], float tnear,
+                                              float tfar) {
+  const float bo[3] = {__uint_as_float(w0.x) - org[0], __uint_as_float(w0.y) - org[1],
+                       __uint_as_float(w0.z) - org[2]};
+  uint32_t nq[3][2], fq[3][2];
   float m[3], c[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
+    const float scale = __uint_as_float(((meta >> (8 * k)) & 255u) << 23);
     const bool neg = inv[k] < 0.f;
-    nq[k] = neg ? hi[k] : lo[k];
-    fq[k] = neg ? lo[k] : hi[k];
-    m[k] = kSafe ? sc[k] : sc[k] * inv[k];
+    nq[k][0] = neg ? pl[k].z : pl[k].x;
+    nq[k][1] = neg ? pl[k].w : pl[k].y;
+    fq[k][0] = neg ? pl[k].x : pl[k].z;
+    fq[k][1] = neg ? pl[k].y : pl[k].w;
+    m[k] = kSafe ? scale : scale * inv[k];
     c[k] = kSafe ? bo[k] : bo[k] * inv[k];
   }
-  int mask = 0;
+  uint32_t mask = 0;
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
+  for (int i = 7; i >= 0; --i) {
     float tn[3], tf[3];
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-      const float qn = (float)((nq[k] >> (8 * i)) & 255u), qf = (float)((fq[k] >> (8 * i)) & 255u);
+      const float qn = (float)((nq[k][i >> 2] >> (8 * (i & 3))) & 255u);
+      const float qf = (float)((fq[k][i >> 2] >> (8 * (i & 3))) & 255u);
       tn[k] = __builtin_fmaf(qn, m[k], c[k]);
       tf[k] = __builtin_fmaf(qf, m[k], c[k]);
       if (kSafe) {
@@ -163,20 +158,17 @@ __device__ __forceinline__ int nodeBoxes(const BNode4* __restrict__ nd, const fl
     }
     const float t0 = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), tnear);
     const float t1 = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), tfar) * kSlabInflate;
-    tmin_o[i] = t0;
-    if (t0 <= t1) mask |= 1 << i;
+    uint32_t carry;
+    mask = __builtin_addc(mask, mask, t0 <= t1 ? 1u : 0u, &carry);
   }
   return mask;
 }
 
 // Resumable traversal of one ray (closest or any hit) in two wave-wide
-// phases (Aila & Laine 2009, "while-while" with speculative traversal):
-// in the node phase every lane descends inner nodes; a lane that reaches a
-// leaf postpones it (one slot, `pend`) and keeps descending while other
-// lanes of its wave have not found a leaf yet.  In the leaf phase every lane
-// tests its postponed leaf and then the leaves at the top of its stack.
-// Node refs and leaf refs share the stack: a leaf ref is the child word of
-// its parent (bit 31, count << 24, first triangle).
+// phases (after Aila & Laine 2009, "while-while" with speculative traversal):
+// in the node phase every lane visits nodes; leaves met on the way are noted
+// in the lane's leaf list, and the lane goes on.  In the leaf phase the wave
+// tests all noted leaves together.
 //
 // Closest hit: `tlim` is the best t so far (initially the ray's tfar, which
 // is therefore also the reported t of a miss); an exact tie in t goes to the
@@ -184,15 +176,13 @@ __device__ __forceinline__ int nodeBoxes(const BNode4* __restrict__ nd, const fl
 struct TravState {
   float org[3], inv[3];
   float Sx, Sy, Sz;
-  uint32_t kk;          // kx | ky << 2 | kz << 4 | any << 8
+  uint32_t kk;          // kx | ky << 2 | kz << 4 | any << 8 | negative directions << 16
   float tnear, tlim, u, v;
   int prim;
-  uint32_t cur, pend, guard;
+  uint32_t cur, guard;  // node to visit (kStackEmpty: none)
+  uint32_t listed;      // leaf list: entries | leaves << 8
   uint32_t node_base, tri_base;  // the domain's first node / leaf-ordered triangle
 };
-
-__device__ __forceinline__ bool isInnerRef(uint32_t r) { return (int32_t)r >= 0; }
-__device__ __forceinline__ bool isLeafRef(uint32_t r) { return (int32_t)r < 0 && r != kStackEmpty; }
 
 __device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint32_t tri_base,
                                          const float org[3], const float dir[3], float tnear,
@@ -207,13 +197,14 @@ __device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint3
   s.Sx = rp.Sx;
   s.Sy = rp.Sy;
   s.Sz = rp.Sz;
-  s.kk = (uint32_t)rp.kx | ((uint32_t)rp.ky << 2) | ((uint32_t)rp.kz << 4) | (any ? 256u : 0u);
+  s.kk = (uint32_t)rp.kx | ((uint32_t)rp.ky << 2) | ((uint32_t)rp.kz << 4) | (any ? 256u : 0u) |
+         (s.inv[0] < 0.f ? 1u << 16 : 0u) | (s.inv[1] < 0.f ? 2u << 16 : 0u) | (s.inv[2] < 0.f ? 4u << 16 : 0u);
   s.tnear = tnear;
   s.tlim = tfar;
   s.u = s.v = 0.f;
   s.prim = -1;
   s.cur = 0;
-  s.pend = kStackEmpty;
+  s.listed = 0;
   s.guard = 0;
   s.node_base = node_base;
   s.tri_base = tri_base;
@@ -221,117 +212,116 @@ __device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint3
 }
 
 __device__ __forceinline__ bool travDone(const TravState& s) {
-  return s.cur == kStackEmpty && s.pend == kStackEmpty;
+  return s.cur == kStackEmpty && s.listed == 0u;
 }
 
-__device__ __forceinline__ void cswap(float& ka, int& ia, float& kb, int& ib) {
-  bool sw = kb < ka;
-  float tk = sw ? kb : ka;
-  int ti = sw ? ib : ia;
-  kb = sw ? ka : kb;
-  ib = sw ? ia : ib;
-  ka = tk;
-  ia = ti;
+// Bit i of the result is bit i ^ o of m (8 bits).
+__device__ __forceinline__ uint32_t permuteSlots(uint32_t m, uint32_t o) {
+  m = (o & 1u) ? ((m >> 1) & 0x55u) | ((m & 0x55u) << 1) : m;
+  m = (o & 2u) ? ((m >> 2) & 0x33u) | ((m & 0x33u) << 2) : m;
+  return (o & 4u) ? (m >> 4) | ((m & 0x0fu) << 4) : m;
 }
 
-// One inner node: the hit children (inner nodes and leaves) in order of
-// entry distance; the nearest becomes `cur`, the others are pushed.
+// One node: leaves that the ray hits are listed, the inner children become a
+// group, and `cur` the first child of that group, or of the group on top of
+// the stack when there is none.  The top group is read beside the node, so
+// the common path has no branch and no pop that waits for LDS.
 template <bool kSafe>
 __device__ __forceinline__ void travNode(TravState& s, LaneStack& st,
-                                         const BNode4* __restrict__ nodes) {
-  if (++s.guard > kMaxNodeVisits) {
-    st.w |= 1u << 16;
-    s.cur = s.pend = kStackEmpty;
-    return;
-  }
-  float tmin[4];
-  int child[4];
-  const BNode4* nd = &nodes[s.node_base + s.cur];
-  int mask = nodeBoxes<kSafe>(nd, s.org, s.inv, s.tnear, s.tlim, tmin, child);
-  float ks[4];
-  int m = 0;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    bool ok = (mask >> i) & 1;
-    ks[i] = ok ? fminf(tmin[i], 3.0e38f) : kInfF;
-    m += ok ? 1 : 0;
-  }
-  float k0 = ks[0], k1 = ks[1], k2 = ks[2], k3 = ks[3];
-  int i0 = child[0], i1 = child[1], i2 = child[2], i3 = child[3];
-  cswap(k0, i0, k1, i1);
-  cswap(k2, i2, k3, i3);
-  cswap(k0, i0, k2, i2);
-  cswap(k1, i1, k3, i3);
-  cswap(k1, i1, k2, i2);
-  if (m == 0) {
-    s.cur = st.pop();
-    return;
-  }
-  // farther children below nearer ones: i3 (if hit) deepest, i1 on top
-  uint32_t x0 = (uint32_t)(m > 3 ? i3 : (m > 2 ? i2 : i1));
-  uint32_t x1 = (uint32_t)(m > 3 ? i2 : i1);
-  st.push3(x0, x1, (uint32_t)i1, (uint32_t)(m - 1));
-  s.cur = (uint32_t)i0;
+                                         const BNode8* __restrict__ nodes) {
+  typedef LaneStack::u32x2 u32x2;
+  const BNode8* nd = &nodes[s.node_base + s.cur];
+  const uint4 w0 = ((const uint4*)nd)[0];
+  const uint4 pl[3] = {((const uint4*)nd)[1], ((const uint4*)nd)[2], ((const uint4*)nd)[3]};
+  const uint32_t meta = nd->meta;
+  const bool fast = st.n < (uint32_t)kRing;
+  u32x2 top = st.lane[(min(st.n, (uint32_t)kRing) - 1u) << 6];
+  if (!fast) top = st.get(st.n - 1u);
+  const uint32_t mask = nodeBoxes<kSafe>(w0, pl, meta, s.org, s.inv, s.tnear, s.tlim);
+  const uint32_t im = meta >> 24, leaves = mask & ~im;
+  st.list[(s.listed & 255u) << 6] = (s.cur << 8) | leaves;  // kept when it has leaves
+  s.listed += leaves ? 1u + ((uint32_t)__popc(leaves) << 8) : 0u;
+  const uint32_t oct = (s.kk >> 16) & 7u;
+  const uint32_t pm = permuteSlots(mask & im, oct);
+  const bool down = pm != 0u;
+  const uint32_t gb = down ? w0.w : top.x, gm = down ? pm | (im << 8) : top.y;
+  const uint32_t slot = ((uint32_t)__ffs((int)gm) - 1u) ^ oct;
+  // the inner children below `slot` come before it
+  const uint32_t child = gb + (uint32_t)__popc(__builtin_amdgcn_ubfe(gm, 8u, slot));
+  uint32_t rest = gm & (gm - 1u);
+  const uint32_t at = down ? st.n : st.n - 1u;
+  if (at < (uint32_t)kRing)
+    st.lane[at << 6] = u32x2{gb, rest};
+  else if (!st.put(at, u32x2{gb, rest}))
+    rest = 0u;
+  st.n = at + ((rest & 255u) ? 1u : 0u);
+  s.cur = gm ? child : kStackEmpty;
 }
 
-// Node phase over the wave: lanes with an inner `cur` descend until every
-// busy lane holds a postponed leaf, none can descend further, or fewer than
-// half of the wave's rays would take a step.
+// Node phase over the wave: lanes visit nodes until three quarters of the
+// wave's rays have leaves to test, or fewer than half have a node to visit.
+// (1024x1024, 8 spp, 64 domains, trace time of a frame: 16.3 ms; leaving at
+// half or all of the rays with leaves 16.5 and 16.7; at a third or three
+// quarters of the rays still stepping 17.3 and 16.7.)
 template <bool kSafe>
 __device__ __forceinline__ void travNodeLoop(TravState& s, LaneStack& st, TravCount& cnt,
-                                             bool active, const BNode4* __restrict__ nodes) {
-  while (true) {
-    const bool step = active && isInnerRef(s.cur);
-    cnt.nodes += (unsigned long long)__popcll(__ballot(step));
-    if (step) {
-      travNode<kSafe>(s, st, nodes);
-      if (isLeafRef(s.cur) && s.pend == kStackEmpty) {
-        s.pend = s.cur;
-        s.cur = st.pop();
-      }
-    }
-    bool more = active && isInnerRef(s.cur);
-    bool hungry = active && s.pend == kStackEmpty && s.cur != kStackEmpty;
-    // leave when no lane lacks a leaf, or when fewer than half of the
-    // wave's rays would step: the rest go to the leaf phase instead of
-    // idling behind a few deep lanes (they resume in the next round).  On
-    // C2, C3 and C5 half was 1% faster than a third and than two thirds.
-    const int nmore = __popcll(__ballot(more));
-    if (nmore == 0 || __ballot(hungry) == 0ull || nmore * 2 < __popcll(__ballot(active))) break;
+                                             bool active, const BNode8* __restrict__ nodes) {
+  auto steps_on = [&] {
+    return active && s.cur != kStackEmpty && (s.listed & 255u) < (uint32_t)kLeafList;
+  };
+  const int nlive = __popcll(__ballot(active));
+  unsigned long long sm = __ballot(steps_on());
+  uint32_t steps = 0;
+  while (sm != 0ull) {
+    cnt.nodes += (unsigned long long)__popcll(sm);
+    if (steps_on()) travNode<kSafe>(s, st, nodes);
+    sm = __ballot(steps_on());
+    const int nleaf = __popcll(__ballot(active && s.listed != 0u));
+    ++steps;
+    if (__popcll(sm) * 2 < nlive || nleaf * 4 >= nlive * 3 || steps >= kMaxPhaseSteps) break;
+  }
+  s.guard += steps;
+  if (active && s.guard > kMaxNodeVisits) {
+    st.err = true;
+    s.cur = kStackEmpty;
+    s.listed = 0;
   }
 }
 
 // The safe box tests only in waves with an axis-parallel (or nearly so) ray:
 // two copies of the loop, so that the common one carries no handling of them.
 __device__ __forceinline__ void travNodePhase(TravState& s, LaneStack& st, TravCount& cnt,
-                                              bool active, const BNode4* __restrict__ nodes) {
+                                              bool active, const BNode8* __restrict__ nodes) {
   if (__ballot(active && needsSafeBoxes(s.inv)) != 0ull)
     travNodeLoop<true>(s, st, cnt, active, nodes);
   else
     travNodeLoop<false>(s, st, cnt, active, nodes);
 }
 
-// Leaf phase over the wave.  Most lanes hold one or two triangles at this
-// point and a few hold more, so the wave's triangles are pooled: every lane
-// lists its triangles (its postponed leaf, and `cur` when that is a leaf too)
-// in LDS, and the wave tests 64 of the list at a time, each lane one triangle
-// of whichever ray owns it (the owner's ray comes by lane permutes).  A hit
-// goes to its owner by a minimum over (t, primitive id), the order that
-// testing one triangle after another keeps.  One triangle per lane and step
-// of the lane's own ray kept 13-23% of the lanes busy, in five steps a round;
-// pooled, a round takes one or two steps.  Measured: 256 uneven domains,
-// 1279x719, 8 spp 22.2 -> 20.7 ms a frame; plain schedule, 256x192 11.7 ->
-// 10.1 ms; 3 M closest-hit queries on one domain 3.16 -> 2.68 ms.
-constexpr int kLeafItems = 128;                                 // triangles listed at once
-constexpr int kLeafLdsWords = kLeafItems + 64 * 2 + 64 * 4;     // per wave: list, keys, hit records
-static_assert(kLeafMax <= 2, "a lane lists at most 4 triangles (two leaves)");
+// Leaf phase over the wave.  Lanes hold different numbers of leaves, so the
+// wave's leaves are pooled: every lane lists its leaves in LDS, and the wave
+// tests 64 of the list at a time, each lane one leaf of whichever ray owns it
+// (the owner's ray comes by lane permutes).  A hit goes to its owner by a
+// minimum over (t, primitive id), the order that testing one triangle after
+// another keeps.
+constexpr int kLeafItems = 192;  // leaves listed at once
+// per wave: stack, leaf lists, pooled leaves, hit keys, hit records
+constexpr int kTravLdsWords = kRing * 128 + kLeafList * 64 + kLeafItems + 64 * 2 + 64 * 4;
+static_assert(kLeafMax <= 2, "a leaf's triangles are loaded together");
+static_assert(kLeafItems >= 8 * kLeafList, "a lane's leaves fit the list");
 
-// Rank of this lane's first item and the wave's total, for 0..4 items a lane.
+// Sum of n (below 64) over the lanes before this one, and over the wave.
 __device__ __forceinline__ uint32_t rankSmall(uint32_t n, uint32_t* total) {
-  const unsigned long long b0 = __ballot(n & 1u), b1 = __ballot(n & 2u), b2 = __ballot(n & 4u);
-  *total = (uint32_t)(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2));
   const unsigned long long lt = (1ull << __lane_id()) - 1ull;
-  return (uint32_t)(__popcll(b0 & lt) + 2 * __popcll(b1 & lt) + 4 * __popcll(b2 & lt));
+  uint32_t r = 0, sum = 0;
+#pragma unroll
+  for (int b = 0; b < 6; ++b) {
+    const unsigned long long m = __ballot((n >> b) & 1u);
+    r += (uint32_t)__popcll(m & lt) << b;
+    sum += (uint32_t)__popcll(m) << b;
+  }
+  *total = sum;
+  return r;
 }
 __device__ __forceinline__ void ldsWaveSync() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -349,98 +339,106 @@ __device__ __forceinline__ uint32_t orderedT(float t) {  // monotone bits; -0 as
   return u ^ ((uint32_t)((int32_t)u >> 31) | 0x80000000u);
 }
 
-// Every lane of the wave calls it, converged (lds: the wave's leaf area).
+// Every lane of the wave calls it, converged (area: the wave's LDS).
 __device__ __forceinline__ void travLeafPhase(TravState& s, LaneStack& st, TravCount& cnt,
-                                              bool active, const LTri* __restrict__ tris,
-                                              uint32_t* lds) {
+                                              bool active, const BNode8* __restrict__ nodes,
+                                              const LTri* __restrict__ tris, uint32_t* area) {
   typedef __attribute__((address_space(3))) unsigned long long lds_u64;
   typedef __attribute__((address_space(3))) float lds_f;
-  lds_u32* items = (lds_u32*)lds;
+  lds_u32* items = (lds_u32*)area + kRing * 128 + kLeafList * 64;
   lds_u64* keys = (lds_u64*)(items + kLeafItems);
   lds_f* recs = (lds_f*)(items + kLeafItems + 128);
   const int lane = __lane_id();
-  while (true) {
-    const bool has = active && s.pend != kStackEmpty;
-    const bool has2 = active && isLeafRef(s.cur);
-    const uint32_t n1 = has ? (s.pend >> 24) & 0x7fu : 0u, n2 = has2 ? (s.cur >> 24) & 0x7fu : 0u;
-    if (__ballot(has || has2) == 0ull) break;
-    const uint32_t n = n1 + n2;
-    uint32_t total;
-    const uint32_t rank = rankSmall(n, &total);
-    // lanes past the list's end keep their leaves for the next turn
-    const bool take = (has || has2) && rank + n <= (uint32_t)kLeafItems;
-    const uint32_t listed = min(total, (uint32_t)kLeafItems);
-    if (take) {
-      const uint32_t own = (uint32_t)lane << 24;
-      const uint32_t p0 = own | (s.pend & 0x00ffffffu), c0 = own | (s.cur & 0x00ffffffu);
-      for (uint32_t i = 0; i < n1; ++i) items[rank + i] = p0 + i;
-      for (uint32_t i = 0; i < n2; ++i) items[rank + n1 + i] = c0 + i;
-      s.pend = kStackEmpty;
-      if (has2) s.cur = st.pop();
+  const uint32_t entries = active ? s.listed & 255u : 0u, n = active ? s.listed >> 8 : 0u;
+  uint32_t total;
+  const uint32_t rank = rankSmall(n, &total);
+  if (total == 0u) return;
+  // lanes past the list's end keep their leaves for the next turn
+  const bool take = n > 0u && rank + n <= (uint32_t)kLeafItems;
+  if (take) {
+    uint32_t at = rank;
+    for (uint32_t e = 0; e < entries; ++e) {
+      const uint32_t w = st.list[e << 6];
+      const uint32_t item = ((uint32_t)lane << 26) | ((w >> 8) << 3);
+      for (uint32_t m = w & 255u; m != 0u; m &= m - 1u) items[at++] = item | ((uint32_t)__ffs((int)m) - 1u);
     }
-    // the last lane taken may end below `listed`: unlisted slots are skipped
-    const unsigned long long tm = __ballot(take && n > 0u);
-    const uint32_t count = tm == 0ull ? 0u : min(listed, __builtin_amdgcn_readlane(rank + n, 63 - __builtin_clzll(tm)));
-    cnt.tris += take ? n : 0u;
-    if (count == 0u) continue;
-    keys[lane] = ~0ull;
-    const bool any = (s.kk >> 8) & 1u;
-    // closest: t <= tlim counts once a hit exists (ties go to the lower id)
-    const float ub = (any || s.prim < 0) ? s.tlim : __uint_as_float(__float_as_uint(s.tlim) + 1u);
-    ldsWaveSync();
-    for (uint32_t base = 0; base < count; base += 64u) {
-      const bool in = base + (uint32_t)lane < count;
-      const uint32_t it = in ? items[base + lane] : (uint32_t)lane << 24;
-      const int own = (int)(it >> 24);
-      const uint32_t kk = laneGet(s.kk, own);
-      const RayPre rp{(int)(kk & 3u), (int)((kk >> 2) & 3u), (int)((kk >> 4) & 3u),
-                      laneGetF(s.Sx, own), laneGetF(s.Sy, own), laneGetF(s.Sz, own)};
-      const float org[3] = {laneGetF(s.org[0], own), laneGetF(s.org[1], own), laneGetF(s.org[2], own)};
-      const float tn = laneGetF(s.tnear, own), lim = laneGetF(ub, own);
-      const uint32_t tb = laneGet(s.tri_base, own);
-      float t = 0.f, u = 0.f, v = 0.f;
-      int p = 0;
-      bool hit = false;
-      if (in) {
-        const float4* tq = (const float4*)&tris[tb + (it & 0x00ffffffu)];
-        const float4 a = tq[0], b = tq[1], c = tq[2];
-        const float v0[3] = {a.x, a.y, a.z}, v1[3] = {b.x, b.y, b.z}, v2[3] = {c.x, c.y, c.z};
-        p = __float_as_int(a.w);
-        hit = triHit(rp, org, v0, v1, v2, tn, lim, &t, &u, &v);
-      }
-      if (__ballot(hit) == 0ull) continue;
-      const unsigned long long key = ((unsigned long long)orderedT(t) << 32) | (uint32_t)p;
-      if (hit) (void)__hip_atomic_fetch_min(&keys[own], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
-      ldsWaveSync();
-      if (hit && keys[own] == key) {
-        recs[own] = t;
-        recs[64 + own] = u;
-        recs[128 + own] = v;
-        recs[192 + own] = __int_as_float(p);
-      }
-    }
-    ldsWaveSync();
-    if (keys[lane] != ~0ull) {
-      const float t = recs[lane];
-      const int p = __float_as_int(recs[192 + lane]);
-      if (any) {
-        s.prim = 1;
-        s.cur = s.pend = kStackEmpty;
-      } else if (s.prim < 0 || t < s.tlim || p < s.prim) {
-        s.tlim = t;
-        s.u = recs[64 + lane];
-        s.v = recs[128 + lane];
-        s.prim = p;
-      }
-    }
-    ldsWaveSync();
-    break;
+    s.listed = 0;
   }
-  // a leaf left in `cur` is the next postponed leaf
-  if (active && s.pend == kStackEmpty && isLeafRef(s.cur)) {
-    s.pend = s.cur;
-    s.cur = st.pop();
+  const unsigned long long tm = __ballot(take);
+  const uint32_t count = __builtin_amdgcn_readlane(rank + n, 63 - __builtin_clzll(tm));
+  keys[lane] = ~0ull;
+  const bool any = (s.kk >> 8) & 1u;
+  // closest: t <= tlim counts once a hit exists (ties go to the lower id)
+  const float ub = (any || s.prim < 0) ? s.tlim : __uint_as_float(__float_as_uint(s.tlim) + 1u);
+  ldsWaveSync();
+  for (uint32_t base = 0; base < count; base += 64u) {
+    const bool in = base + (uint32_t)lane < count;
+    const uint32_t it = in ? items[base + lane] : (uint32_t)lane << 26;
+    const int own = (int)(it >> 26);
+    const uint32_t nb = laneGet(s.node_base, own), tb = laneGet(s.tri_base, own);
+    const uint32_t word = in ? nodes[nb + ((it >> 3) & 0x7fffffu)].leaf[it & 7u] : 0u;
+    const uint32_t kk = laneGet(s.kk, own);
+    const RayPre rp{(int)(kk & 3u), (int)((kk >> 2) & 3u), (int)((kk >> 4) & 3u),
+                    laneGetF(s.Sx, own), laneGetF(s.Sy, own), laneGetF(s.Sz, own)};
+    const float org[3] = {laneGetF(s.org[0], own), laneGetF(s.org[1], own), laneGetF(s.org[2], own)};
+    const float tn = laneGetF(s.tnear, own);
+    float lim = laneGetF(ub, own);
+    const uint32_t ntri = (word >> 24) & 0x7fu;
+    cnt.tris += ntri;
+    const float4* tq = (const float4*)&tris[tb + (word & 0x00ffffffu)];
+    float4 a[2], b[2], c[2];
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if ((uint32_t)j < ntri) {
+        a[j] = tq[3 * j];
+        b[j] = tq[3 * j + 1];
+        c[j] = tq[3 * j + 2];
+      }
+    float t = 0.f, u = 0.f, v = 0.f;
+    int p = 0;
+    bool hit = false;
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+      if ((uint32_t)j < ntri) {
+        const float v0[3] = {a[j].x, a[j].y, a[j].z}, v1[3] = {b[j].x, b[j].y, b[j].z},
+                    v2[3] = {c[j].x, c[j].y, c[j].z};
+        const int q = __float_as_int(a[j].w);
+        float t1, u1, w1;
+        if (triHit(rp, org, v0, v1, v2, tn, lim, &t1, &u1, &w1) && (!hit || t1 < t || (t1 == t && q < p))) {
+          t = t1;
+          u = u1;
+          v = w1;
+          p = q;
+          hit = true;
+        }
+      }
+    if (__ballot(hit) == 0ull) continue;
+    const unsigned long long key = ((unsigned long long)orderedT(t) << 32) | (uint32_t)p;
+    if (hit) (void)__hip_atomic_fetch_min(&keys[own], key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WAVEFRONT);
+    ldsWaveSync();
+    if (hit && keys[own] == key) {
+      recs[own] = t;
+      recs[64 + own] = u;
+      recs[128 + own] = v;
+      recs[192 + own] = __int_as_float(p);
+    }
   }
+  ldsWaveSync();
+  if (keys[lane] != ~0ull) {
+    const float t = recs[lane];
+    const int p = __float_as_int(recs[192 + lane]);
+    if (any) {
+      s.prim = 1;
+      s.cur = kStackEmpty;
+      s.listed = 0;
+    } else if (s.prim < 0 || t < s.tlim || p < s.prim) {
+      s.tlim = t;
+      s.u = recs[64 + lane];
+      s.v = recs[128 + lane];
+      s.prim = p;
+    }
+  }
+  ldsWaveSync();
 }
 
 }  // namespace spray
