@@ -232,10 +232,10 @@ __global__ void kGenEyes(TraceParams P) {
     } else {
       d = cameraDir(P.cam, (float)x, (float)y);
     }
-    P.R.op[i] = make_float4(P.cam.pos.x, P.cam.pos.y, P.cam.pos.z, __int_as_float(y * P.image_w + x));
-    P.R.ds[i] = make_float4(d.x, d.y, d.z, __int_as_float((int)i));
-    P.R.wd[i] = make_float4(1.f, 1.f, 1.f, __int_as_float(0));
-    P.R.h[i] = make_float4(kInfF, kInfF, kInfF, kInfF);
+    P.R.op(i) = make_float4(P.cam.pos.x, P.cam.pos.y, P.cam.pos.z, __int_as_float(y * P.image_w + x));
+    P.R.ds(i) = make_float4(d.x, d.y, d.z, __int_as_float((int)i));
+    P.R.wd(i) = make_float4(1.f, 1.f, 1.f, __int_as_float(0));
+    P.R.h(i) = make_float4(kInfF, kInfF, kInfF, kInfF);
   }
 }
 
@@ -257,17 +257,17 @@ __global__ void kRestartPending(TraceParams P) {
   for (uint32_t base = blockIdx.x * blockDim.x; base < n; base += gridDim.x * blockDim.x) {
     uint32_t i = base + threadIdx.x;
     bool valid = i < n;
-    float4 hh = valid ? P.Pn.h[i] : make_float4(0, 0, 0, 0);
+    float4 hh = valid ? P.Pn.h(i) : make_float4(0, 0, 0, 0);
     float h[4] = {hh.x, hh.y, hh.z, hh.w};
-    int samid = valid ? __float_as_int(P.Pn.ds[i].w) : 0;
+    int samid = valid ? __float_as_int(P.Pn.ds(i).w) : 0;
     bool ok = valid && vbufCorrect(P.vbuf, samid, h, kHistory);
     const uint32_t idx = app(ok, &c->r_count, P.r_cap, &c->err);
     if (ok && idx != 0xffffffffu) {
-      P.R.op[idx] = P.Pn.op[i];
-      P.R.ds[idx] = P.Pn.ds[i];
-      float4 wd = P.Pn.wd[i];
-      P.R.wd[idx] = make_float4(wd.x, wd.y, wd.z, __int_as_float(0));
-      P.R.h[idx] = make_float4(kInfF, kInfF, kInfF, kInfF);
+      P.R.op(idx) = P.Pn.op(i);
+      P.R.ds(idx) = P.Pn.ds(i);
+      float4 wd = P.Pn.wd(i);
+      P.R.wd(idx) = make_float4(wd.x, wd.y, wd.z, __int_as_float(0));
+      P.R.h(idx) = make_float4(kInfF, kInfF, kInfF, kInfF);
       ++useful;
     }
   }
@@ -559,13 +559,13 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
   __syncthreads();
   const DevCounters* c = P.ctr;
   const long long total = (long long)(c->r_end - c->r_beg) + (c->s_end - c->s_beg);
-  const long long stride = (long long)gridDim.x * blockDim.x;
   // The wave's rays are i = wbase + k * stride + j (j < 64, k = 0, 1, ...),
   // the rays a grid-stride loop would give it, so every block counts the
   // rays kScatter's block places.  Walks differ in length, so a lane takes
   // the wave's next ray as soon as its own is done (once kCountRefill lanes
   // wait), instead of the wave waiting for its longest walk.
   const long long wbase = blockIdx.x * (long long)blockDim.x + (threadIdx.x & ~63);
+  const long long stride = (long long)gridDim.x * blockDim.x;
   const int lane = __lane_id();
   uint32_t seq = 0;  // wave-uniform: rays handed out
   bool more = wbase < total;
@@ -601,10 +601,10 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
         uint32_t r = 0;
         bool valid = ii < total && passRay(P, ii, &kind, &r);
         // shadow rays occluded in their spawning domain are done (procShads2)
-        if (valid && kind == 1 && P.Sx.occluded[r]) valid = false;
+        if (valid && kind == 1 && rayOccluded(P.S.wd(r).w)) valid = false;
         if (valid) {
           const RayPool& pool = kind ? P.S : P.R;
-          const float4 op = pool.op[r], ds = pool.ds[r];
+          const float4 op = pool.op(r), ds = pool.ds(r);
           W.o[0] = op.x;
           W.o[1] = op.y;
           W.o[2] = op.z;
@@ -614,7 +614,7 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
           W.inv[0] = 1.0f / ds.x;
           W.inv[1] = 1.0f / ds.y;
           W.inv[2] = 1.0f / ds.z;
-          W.spawn = kind ? (__float_as_int(pool.wd[r].w) >> 8) : -1;
+          W.spawn = kind ? raySpawn(pool.wd(r).w) : -1;
           W.kind = kind;
           for (int w = 0; w < nw; ++w) lmask[w * blockDim.x] = 0ull;
           // NaN-checked slab tests only in waves with an axis-parallel ray
@@ -667,7 +667,7 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
       const uint32_t a = abase + (uint32_t)__popcll(am & ((1ull << lane) - 1ull));
       if (ask && a < P.ask_region) {
         float4* rec = P.ask + ((size_t)blockIdx.x * P.ask_region + a) * 3;
-        const float4 ds = P.R.ds[r];
+        const float4 ds = P.R.ds(r);
         rec[0] = make_float4(W.o[0], W.o[1], W.o[2], ds.x);
         rec[1] = make_float4(ds.y, ds.z, W.tt[0], W.tt[1]);
         rec[2] = make_float4(__uint_as_float(r), __int_as_float(W.ti[0]), __int_as_float(W.ti[1]),
@@ -840,14 +840,14 @@ __global__ void __launch_bounds__(kBlock) kScatter(TraceParams P) {
     float o[3] = {0, 0, 0}, inv[3] = {1, 1, 1};
     if (valid) {
       const RayPool& pool = kind ? P.S : P.R;
-      float4 op = pool.op[r], ds = pool.ds[r];
+      float4 op = pool.op(r), ds = pool.ds(r);
       o[0] = op.x;
       o[1] = op.y;
       o[2] = op.z;
       inv[0] = 1.0f / ds.x;
       inv[1] = 1.0f / ds.y;
       inv[2] = 1.0f / ds.z;
-      if (kind && P.Sx.occluded[r]) valid = false;  // occluded in its spawning domain
+      if (kind && rayOccluded(pool.wd(r).w)) valid = false;  // occluded in its spawning domain
     }
     // the same wave-uniform slab variant as kCount (same rays per wave)
     const bool safe = __ballot(valid && hasInfInv(inv)) != 0ull;
@@ -874,10 +874,10 @@ __global__ void __launch_bounds__(kBlock) kScatter(TraceParams P) {
 __device__ __forceinline__ void writeRay(const RayPool& pool, uint32_t idx, f3 org, int pixid,
                                          f3 dir, int samid, f3 w, int depth_word,
                                          const float h[4]) {
-  pool.op[idx] = make_float4(org.x, org.y, org.z, __int_as_float(pixid));
-  pool.ds[idx] = make_float4(dir.x, dir.y, dir.z, __int_as_float(samid));
-  pool.wd[idx] = make_float4(w.x, w.y, w.z, __int_as_float(depth_word));
-  pool.h[idx] = make_float4(h[0], h[1], h[2], h[3]);
+  pool.op(idx) = make_float4(org.x, org.y, org.z, __int_as_float(pixid));
+  pool.ds(idx) = make_float4(dir.x, dir.y, dir.z, __int_as_float(samid));
+  pool.wd(idx) = make_float4(w.x, w.y, w.z, __int_as_float(depth_word));
+  pool.h(idx) = make_float4(h[0], h[1], h[2], h[3]);
 }
 
 // Children's history: parent's history[0..depth) then t, the rest infinity.
@@ -894,9 +894,7 @@ __device__ __forceinline__ void spawnShadow(const TraceParams& P, BlockAppend& a
   if (idx == 0xffffffffu) return;
   float h[4];
   childHistory(hist, depth, t, h);
-  writeRay(P.S, idx, pos, pixid, wi, samid, Lr, (depth + 1) | (dom << 8), h);
-  P.Sx.tmax[idx] = tmax;
-  P.Sx.occluded[idx] = 0u;
+  writeRay(P.S, idx, pos, __float_as_int(tmax), wi, samid, Lr, (depth + 1) | (dom << 8), h);
 }
 
 // The hit's bounce rays (reflection b1 along d1, transmission b2 along d2),
@@ -1265,16 +1263,17 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
         active = false;
         if (kind == 0) {
           // the history prefix the buffer update checks is fixed for this pass
-          wd = P.R.wd[ray];
-          hh = P.R.h[ray];
+          wd = P.R.wd(ray);
+          hh = P.R.h(ray);
           const int depth = __float_as_int(wd.w) & 0xff;
-          const int samid = __float_as_int(P.R.ds[ray].w);
+          const int samid = __float_as_int(P.R.ds(ray).w);
           float hist[4] = {hh.x, hh.y, hh.z, hh.w};
           upd = s.prim >= 0 && vbufUpdate(P.vbuf, samid, hist, depth, s.tlim);
           logged = log_live;
-          if (upd) atomicMin((uint32_t*)&P.R.h[ray] + depth, __float_as_uint(s.tlim));
+          if (upd) atomicMin((uint32_t*)&P.R.h(ray) + depth, __float_as_uint(s.tlim));
         } else if (s.prim > 0) {
-          __hip_atomic_store(&P.Sx.occluded[ray], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+          (void)__hip_atomic_fetch_or((uint32_t*)&P.S.wd(ray).w, kOccluded, __ATOMIC_RELAXED,
+                                      __HIP_MEMORY_SCOPE_AGENT);
         }
       }
       // visit log for the predictor, (ray, domain, t) of every finished
@@ -1318,8 +1317,8 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
           // [0, depth) is fixed for the pass and entry `depth` is replaced
           // by the hit's t in the children
           float4* rec = P.sh_rec + (size_t)idx * kShadeRec;
-          rec[0] = P.R.op[ray];
-          rec[1] = P.R.ds[ray];
+          rec[0] = P.R.op(ray);
+          rec[1] = P.R.ds(ray);
           // radiance rays keep only their depth in wd.w: the domain joins it
           rec[2] = make_float4(wd.x, wd.y, wd.z, __int_as_float(__float_as_int(wd.w) | (dom << 8)));
           rec[3] = hh;
@@ -1401,8 +1400,8 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
           }
           ray = qe.ray;
           const RayPool& pool = kind ? P.S : P.R;
-          float4 op = pool.op[ray], ds = pool.ds[ray], wd = pool.wd[ray], hh = pool.h[ray];
-          if (local) dom = __float_as_int(wd.w) >> 8;
+          float4 op = pool.op(ray), ds = pool.ds(ray), wd = pool.wd(ray), hh = pool.h(ray);
+          if (local) dom = raySpawn(wd.w);
           float hist[4] = {hh.x, hh.y, hh.z, hh.w};
           const int depth = __float_as_int(wd.w) & 0xff;
           const int samid = __float_as_int(ds.w);
@@ -1411,12 +1410,10 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
             go = qe.tdom <= pick4(hist, depth) && vbufCorrect(P.vbuf, samid, hist, depth);
           } else if (local) {
             go = true;  // spawned from a final-chain hit in this pass
-            tfar = P.Sx.tmax[ray];
+            tfar = op.w;
           } else {
-            go = !__hip_atomic_load(&P.Sx.occluded[ray], __ATOMIC_RELAXED,
-                                    __HIP_MEMORY_SCOPE_AGENT) &&
-                 vbufCorrect(P.vbuf, samid, hist, depth);
-            tfar = P.Sx.tmax[ray];
+            go = !rayOccluded(wd.w) && vbufCorrect(P.vbuf, samid, hist, depth);
+            tfar = op.w;
           }
           if (go) {
             const DomainDesc& D = P.desc[dom];
@@ -1510,15 +1507,15 @@ __global__ void kRetire(TraceParams P) {
   const uint32_t b = c->s_beg, e = c->s_end;
   unsigned long long useful = 0;
   for (uint32_t i = b + blockIdx.x * blockDim.x + threadIdx.x; i < e; i += gridDim.x * blockDim.x) {
-    float4 hh = P.S.h[i];
+    float4 hh = P.S.h(i);
     float hist[4] = {hh.x, hh.y, hh.z, hh.w};
-    float4 wd = P.S.wd[i];
+    float4 wd = P.S.wd(i);
     int depth = __float_as_int(wd.w) & 0xff;
-    int samid = __float_as_int(P.S.ds[i].w);
+    int samid = __float_as_int(P.S.ds(i).w);
     if (!vbufCorrect(P.vbuf, samid, hist, depth)) continue;
     ++useful;
-    if (P.Sx.occluded[i]) continue;
-    int pixid = __float_as_int(P.S.op[i].w);
+    if (rayOccluded(wd.w)) continue;
+    const int pixid = P.tile_rec[0] * P.image_w + samid / P.spp;
     float* px = P.image + (size_t)pixid * 4;
     atomicAdd(px + 0, (float)(P.inv_spp * (double)wd.x));
     atomicAdd(px + 1, (float)(P.inv_spp * (double)wd.y));
@@ -1534,10 +1531,10 @@ __global__ void kWindowEnd(TraceParams P) {
   const uint32_t rend = min(c->r_count, P.r_cap);
   for (uint32_t i = c->r_init + blockIdx.x * blockDim.x + threadIdx.x; i < rend;
        i += gridDim.x * blockDim.x) {
-    float4 hh = P.R.h[i];
+    float4 hh = P.R.h(i);
     float hist[4] = {hh.x, hh.y, hh.z, hh.w};
-    int depth = __float_as_int(P.R.wd[i].w) & 0xff;
-    if (vbufCorrect(P.vbuf, __float_as_int(P.R.ds[i].w), hist, depth)) ++useful;
+    int depth = __float_as_int(P.R.wd(i).w) & 0xff;
+    if (vbufCorrect(P.vbuf, __float_as_int(P.R.ds(i).w), hist, depth)) ++useful;
   }
   const long long S = (long long)P.tile_rec[1] * P.image_w * P.spp;
   for (long long s = blockIdx.x * (long long)blockDim.x + threadIdx.x; s < S;
@@ -1579,9 +1576,9 @@ __global__ void kLogFinalize(TraceParams P) {
       r = vl[(size_t)i * 3];
       dom = (int)vl[(size_t)i * 3 + 1];
       const float t = __uint_as_float(vl[(size_t)i * 3 + 2]);
-      float4 wd = P.R.wd[r];
+      float4 wd = P.R.wd(r);
       int depth = __float_as_int(wd.w) & 0xff;
-      float4 hh = P.R.h[r];
+      float4 hh = P.R.h(r);
       float best = depth == 0 ? hh.x : depth == 1 ? hh.y : depth == 2 ? hh.z : hh.w;
       label = (t != kInfF && t == best) ? 1.f : 0.f;
     }
@@ -1594,7 +1591,7 @@ __global__ void kLogFinalize(TraceParams P) {
          (unsigned long long)__builtin_amdgcn_readlane((uint32_t)sb, leader);
     const unsigned long long slot = sb + (unsigned long long)__popcll(vm & ((1ull << lane) - 1ull));
     if (!valid || slot >= P.log_cap) continue;
-    float4 op = P.R.op[r], ds = P.R.ds[r];
+    float4 op = P.R.op(r), ds = P.R.ds(r);
     float* o = P.log_buf + slot * 8;
     o[0] = op.x;
     o[1] = op.y;
@@ -1613,7 +1610,7 @@ struct TracerState {
   long long S = 0;  // samples of the largest tile
   uint32_t r_cap = 0, s_cap = 0, p_cap = 0, q_cap[2] = {0, 0}, sh_cap = 0, mask_cap = 0;
   int ndomains = 0;
-  DevBuf R[4], Pn[4], Sh[4], s_tmax, s_occ, vbuf, image, ctr, tile_rec, cnt, off, dbase, bcnt, bbase,
+  DevBuf R, Pn, Sh, vbuf, image, ctr, tile_rec, cnt, off, dbase, bcnt, bbase,
       wctr, wq, score, order, q[2], ask, ask_cnt, rkey, dmask, dfmt, dbox, ovf, vlog, log, sh_rec, qa,
       qb, dflag, acnt;
   unsigned long long log_cap = 0;
@@ -1644,9 +1641,7 @@ struct TracerState {
   std::vector<unsigned long long> slog_scores;
   size_t heldBytes() const {
     size_t b = log_ctr.bytes;
-    for (const DevBuf* x : {R, Pn, Sh})
-      for (int k = 0; k < 4; ++k) b += x[k].bytes;
-    for (const DevBuf* x : {&s_tmax, &s_occ, &vbuf, &image, &ctr, &tile_rec, &cnt, &off, &dbase, &bcnt,
+    for (const DevBuf* x : {&R, &Pn, &Sh, &vbuf, &image, &ctr, &tile_rec, &cnt, &off, &dbase, &bcnt,
                             &bbase, &wctr, &wq, &score, &order, &q[0], &q[1], &ask, &ask_cnt, &rkey,
                             &dmask, &dfmt, &dbox, &ovf, &vlog, &log, &sh_rec, &qa, &qb, &dflag, &acnt})
       b += x->bytes;
@@ -1717,9 +1712,7 @@ void tracerRelease(Ctx* c) {
   }
   for (hipEvent_t e : {T->fork_ev, T->join_ev})
     if (e) (void)hipEventDestroy(e);
-  for (auto* arr : {T->R, T->Pn, T->Sh})
-    for (int k = 0; k < 4; ++k) arr[k].release();
-  for (DevBuf* b : {&T->s_tmax, &T->s_occ, &T->vbuf, &T->image, &T->ctr, &T->tile_rec, &T->cnt,
+  for (DevBuf* b : {&T->R, &T->Pn, &T->Sh, &T->vbuf, &T->image, &T->ctr, &T->tile_rec, &T->cnt,
                     &T->off, &T->dbase, &T->bcnt, &T->bbase, &T->wctr, &T->wq, &T->score, &T->order, &T->q[0],
                     &T->q[1], &T->ask, &T->ask_cnt, &T->rkey, &T->dmask, &T->dfmt, &T->dbox, &T->ovf, &T->vlog, &T->log, &T->sh_rec, &T->log_ctr, &T->qa, &T->qb, &T->dflag, &T->acnt})
     b->release();
@@ -1780,7 +1773,7 @@ static double stateBytesPerSample(const Ctx* c) {
   const double r = 1.0 + spec * depths, s = spv * spec * depths, p = spec;
   const double q0 = spec * per_ray, q1 = spv * spec * per_ray * 0.5, m = spec * (1.0 + spv);
   // radiance queue: entry + phase-list index; shadow queue: entry
-  return r * 64 + s * 72 + p * 64 + q0 * (8 + 8) + std::min(q0, r) * kShadeRec * 16 + q1 * 8 +
+  return r * 64 + s * 64 + p * 64 + q0 * (8 + 8) + std::min(q0, r) * kShadeRec * 16 + q1 * 8 +
          m * (8 * words + 1) + 32 + r;
 }
 
@@ -1834,13 +1827,9 @@ static void ensureState(Ctx* c, double grow) {
   T->q_cap[0] = std::max(T->q_cap[0], q0);
   T->q_cap[1] = std::max(T->q_cap[1], q1);
   T->mask_cap = std::max(T->mask_cap, mask_cap);
-  for (int k = 0; k < 4; ++k) {
-    need(T, T->R[k], (size_t)T->r_cap * 16);
-    need(T, T->Pn[k], (size_t)T->p_cap * 16);
-    need(T, T->Sh[k], (size_t)T->s_cap * 16);
-  }
-  need(T, T->s_tmax, (size_t)T->s_cap * 4);
-  need(T, T->s_occ, (size_t)T->s_cap * 4);
+  need(T, T->R, (size_t)T->r_cap * 64);
+  need(T, T->Pn, (size_t)T->p_cap * 64);
+  need(T, T->Sh, (size_t)T->s_cap * 64);
   need(T, T->vbuf, (size_t)S * kHistory * 8);
   if (cfg.schedule == SPRAY_SCHEDULE_LEARNED) {
     need(T, T->ask, (size_t)kQueueGrid * askRegion(T->r_cap) * 48 + 64);
@@ -1935,19 +1924,14 @@ static TraceParams makeParams(Ctx* c) {
   P.rgb = pool.rgb.as<uint32_t>();
   P.nrm = pool.nrm.as<float>();
   P.fshade = pool.fshade.as<float4>();
-  auto pool4 = [](DevBuf* b) {
+  auto rays = [](const DevBuf& b) {
     RayPool r;
-    r.op = b[0].as<float4>();
-    r.ds = b[1].as<float4>();
-    r.wd = b[2].as<float4>();
-    r.h = b[3].as<float4>();
+    r.r = b.as<float4>();
     return r;
   };
-  P.R = pool4(T->R);
-  P.Pn = pool4(T->Pn);
-  P.S = pool4(T->Sh);
-  P.Sx.tmax = T->s_tmax.as<float>();
-  P.Sx.occluded = T->s_occ.as<uint32_t>();
+  P.R = rays(T->R);
+  P.Pn = rays(T->Pn);
+  P.S = rays(T->Sh);
   P.r_cap = T->r_cap;
   P.s_cap = T->s_cap;
   P.p_cap = T->p_cap;

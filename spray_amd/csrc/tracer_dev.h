@@ -20,16 +20,24 @@ __host__ __device__ inline int maskRowWords(int nd) {
   return nw > kHitListWords ? (nw + 1) & ~1 : nw;
 }
 
-// Ray pools are SoA streams of float4 (16-byte loads per lane):
-//   op = (org.xyz, pixid)  ds = (dir.xyz, samid)
-//   wd = (w.xyz, depth | spawn_domain << 8)  h = history[4]
+// Ray pools: 64 bytes per ray, four float4 side by side,
+//   op = (org.xyz, pixid; shadow rays: tmax)  ds = (dir.xyz, samid)
+//   wd = (w.xyz, depth | spawn domain << 8 | occluded << 31)  h = history[4]
+// The trace kernel reads whole rays, at random places within a domain's
+// queue: a ray is half an L2 line, where four streams took four lines.  (A
+// shadow ray's pixel follows from its sample.)
 struct RayPool {
-  float4 *op, *ds, *wd, *h;
+  float4* r;
+  __device__ __forceinline__ float4& op(size_t i) const { return r[i * 4]; }
+  __device__ __forceinline__ float4& ds(size_t i) const { return r[i * 4 + 1]; }
+  __device__ __forceinline__ float4& wd(size_t i) const { return r[i * 4 + 2]; }
+  __device__ __forceinline__ float4& h(size_t i) const { return r[i * 4 + 3]; }
 };
-struct ShadowExtra {
-  float* tmax;
-  uint32_t* occluded;
-};
+constexpr uint32_t kOccluded = 1u << 31;
+// fields of wd.w
+__device__ __forceinline__ int rayDepth(float w) { return __float_as_int(w) & 0xff; }
+__device__ __forceinline__ int raySpawn(float w) { return (__float_as_int(w) >> 8) & 0x7fffff; }
+__device__ __forceinline__ bool rayOccluded(float w) { return __float_as_int(w) < 0; }
 
 // Queue entry: ray index and the distance at which the ray enters the domain
 struct QEntry {
@@ -82,7 +90,6 @@ struct TraceParams {
   // tracer state
   RayPool R, Pn;  // radiance (window) and pending pools
   RayPool S;
-  ShadowExtra Sx;
   uint32_t r_cap, s_cap, p_cap;
   unsigned long long* vbuf;  // 4 words per sample: t bits << 32 | parent bits
   float* image;              // rgba per pixel
