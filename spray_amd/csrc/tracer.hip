@@ -1225,6 +1225,8 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
   const bool log_live = P.log_on && c->log_live;
   const int lane = __lane_id();
   bool active = false, exhausted = false;
+  bool helping = false;  // this lane works on another lane's ray (once the queue is exhausted)
+  bool shared = false;   // wave-uniform: some lane does
   int kind = 0, dom = 0;
   uint32_t ray = 0;
   // wave-uniform: entries left in this wave's range; shade slots left in its chunk
@@ -1264,7 +1266,8 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
     // waits for, and after almost every round of the two phases some lane of
     // 64 is finished (1024x1024, 8 spp, 64 domains: 4.2 M wave rounds, 2.7 M
     // of them now write results; the frame 28.6 -> 26.4 ms).
-    const bool done = active && travDone(s);
+    bool done = active && travDone(s);
+    if (shared) done = !travHelped(s, helping, area) && done;
     const unsigned long long idle = __ballot(!active || done);
     const int nidle = __popcll(idle);
     const unsigned long long dm = __ballot(done);
@@ -1451,9 +1454,15 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
       if (exhausted) break;
       continue;
     }
-    const bool live = active && !travDone(s);
+    const bool live = (active || helping) && !travDone(s);
     travNodePhase(s, st, tc, live, P.nodes);
     travLeafPhase(s, st, tc, live, P.nodes, P.tris, area);
+    if (shared) travFollow(s, helping);
+    if (exhausted) {
+      helping = helping && !travDone(s);
+      if (travShare(s, st, !active && !helping, (active || helping) && !travDone(s), area)) helping = true;
+      shared = __ballot(helping) != 0ull;
+    }
   }
   shadeSlotsEmpty(P, sh_cur, sh_end, lane);
   blockFlush<5>({&c->radiance_visits, &c->shadow_visits, &c->pruned, &c->node_visits,
