@@ -1483,9 +1483,9 @@ constexpr int kQBlock = 256;
 // wave in step with its longest ray (as many blocks as overflow stacks of the
 // greatest depth fitted the static scratch): 3 M closest hits among 524 k
 // triangles 2275 -> 625 us (4.8 G rays/s), 1 M any hits among 180 k 695 -> 241
-// us, 1500 closest hits 50 -> 34 us.
+// us, 1500 closest hits 50 -> 25 us (8 rays a wave 36, 2 and 1 rays 28).
 constexpr int kQRefill = 16;
-constexpr uint32_t kQMinRange = 8;
+constexpr uint32_t kQMinRange = 4;
 __global__ void __launch_bounds__(kQBlock, 4) kTraceRays(
     const BNode8* __restrict__ nodes, const LTri* __restrict__ tris, const float* __restrict__ org,
     const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,

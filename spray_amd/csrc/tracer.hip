@@ -120,7 +120,7 @@ static_assert(kQueueGrid % kBlock == 0, "kBlockBases splits the grid evenly over
 // block instead of per wave (waves that end together would otherwise queue
 // on the same device-scope atomics).  Every thread of the block calls it.
 template <int N>
-__device__ __forceinline__ void blockFlush(unsigned long long* const (&dst)[N],
+__device__ __forceinline__ void blockFlush(DevCounters* c, const Stat (&id)[N],
                                            const unsigned long long (&v)[N]) {
   __shared__ unsigned long long part[16][N];
   const int w = threadIdx.x >> 6;
@@ -130,7 +130,7 @@ __device__ __forceinline__ void blockFlush(unsigned long long* const (&dst)[N],
   if (threadIdx.x < N) {
     unsigned long long sum = 0;
     for (int i = 0; i < (int)(blockDim.x >> 6); ++i) sum += part[i][threadIdx.x];
-    if (sum) atomicAdd(dst[threadIdx.x], sum);
+    if (sum) atomicAdd(&c->stat[blockIdx.x & (kStatCopies - 1)][id[threadIdx.x]], sum);
   }
 }
 
@@ -217,7 +217,7 @@ __global__ void kTileStart(TraceParams P) {
   c->s_count = 0;
   c->s_mark = 0;
   c->p_count = 0;
-  c->useful += S;  // eye rays
+  c->stat[0][kStatUseful] += S;  // eye rays
 }
 
 __global__ void kGenEyes(TraceParams P) {
@@ -279,7 +279,7 @@ __global__ void kRestartPending(TraceParams P) {
       ++useful;
     }
   }
-  blockFlush<1>({&c->useful}, {waveSumULL(useful)});
+  blockFlush<1>(c, {kStatUseful}, {waveSumULL(useful)});
 }
 __global__ void kRestartDone(TraceParams P) {
   DevCounters* c = P.ctr;
@@ -1465,8 +1465,7 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
     }
   }
   shadeSlotsEmpty(P, sh_cur, sh_end, lane);
-  blockFlush<5>({&c->radiance_visits, &c->shadow_visits, &c->pruned, &c->node_visits,
-                 &c->tri_tests},
+  blockFlush<5>(c, {kStatRadiance, kStatShadow, kStatPruned, kStatNodes, kStatTris},
                 {rvis, svis, pruned, tc.nodes, waveSumULL(tc.tris)});
   if (st.overflowed()) atomicOr(&c->err, 4u);
 }
@@ -1509,7 +1508,7 @@ __global__ void __launch_bounds__(kShadeBlock, 4) kShade(TraceParams P) {
     shades += act ? 1 : 0;
     shadeSpawn(P, app, act, dom, op, ds, wd, hist, depth, t, u, v, prim, ray_depth);
   }
-  blockFlush<1>({&c->shades}, {waveSumULL(shades)});
+  blockFlush<1>(c, {kStatShades}, {waveSumULL(shades)});
 }
 
 // After one domain (or chunk of domains) of a paged pool: its shade records
@@ -1549,7 +1548,7 @@ __global__ void kRetire(TraceParams P) {
     atomicAdd(px + 1, (float)(P.inv_spp * (double)wd.y));
     atomicAdd(px + 2, (float)(P.inv_spp * (double)wd.z));
   }
-  blockFlush<1>({&c->useful}, {waveSumULL(useful)});
+  blockFlush<1>(c, {kStatUseful}, {waveSumULL(useful)});
 }
 
 // Window end: census of non-stale spawned radiance rays and final hits.
@@ -1578,7 +1577,7 @@ __global__ void kWindowEnd(TraceParams P) {
       prev = t;
     }
   }
-  blockFlush<2>({&c->useful, &c->final_hits}, {waveSumULL(useful), waveSumULL(hits)});
+  blockFlush<2>(c, {kStatUseful, kStatHits}, {waveSumULL(useful), waveSumULL(hits)});
 }
 __global__ void kWindowAdvance(TraceParams P) {
   int* rec = (int*)P.tile_rec;
@@ -2471,21 +2470,26 @@ void tracerTraceFrame(Ctx* c, float* rgba_out, spray_stats* st) {
     if (rgba_out)
       SPRAY_HIP(hipMemcpy(rgba_out, P.image, (size_t)cfg.image_w * cfg.image_h * 16,
                           hipMemcpyDeviceToHost));
-    st->useful_rays = h.useful;
+    auto total = [&h](Stat id) {
+      unsigned long long sum = 0;
+      for (int k = 0; k < kStatCopies; ++k) sum += h.stat[k][id];
+      return sum;
+    };
+    st->useful_rays = total(kStatUseful);
     st->eye_rays = (unsigned long long)cfg.image_w * cfg.image_h * cfg.pixel_samples;
-    st->radiance_visits = h.radiance_visits;
-    st->shadow_visits = h.shadow_visits;
-    st->shades = h.shades;
-    st->final_hits = h.final_hits;
+    st->radiance_visits = total(kStatRadiance);
+    st->shadow_visits = total(kStatShadow);
+    st->shades = total(kStatShades);
+    st->final_hits = total(kStatHits);
     st->passes = h.passes;
     st->windows = (unsigned long long)windows * ys.size();
     st->tiles = ys.size();
     st->queue_entries = h.queue_entries;
     st->deferred_entries = h.deferred;
-    st->pruned_entries = h.pruned;
+    st->pruned_entries = total(kStatPruned);
     st->trace_ms = ms;
-    st->node_visits = h.node_visits;
-    st->tri_tests = h.tri_tests;
+    st->node_visits = total(kStatNodes);
+    st->tri_tests = total(kStatTris);
     st->cache_hits = c->pool.hits - hits0;
     st->cache_misses = c->pool.misses - misses0;
     st->cache_bytes = c->pool.bytes_in - bytes0;

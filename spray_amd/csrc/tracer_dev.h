@@ -45,6 +45,9 @@ struct QEntry {
   float tdom;
 };
 
+enum Stat { kStatUseful, kStatRadiance, kStatShadow, kStatShades, kStatHits, kStatPruned, kStatNodes, kStatTris };
+constexpr int kStatCopies = 64;
+
 struct DevCounters {
   uint32_t r_count, s_count, p_count;  // pool fill levels (atomic append)
   uint32_t r_beg, r_end, s_beg, s_end;  // rays to enqueue / trace in this pass
@@ -59,8 +62,12 @@ struct DevCounters {
   uint32_t sh_mark, s_local;            // shade records / spawned shadow rays already processed
                                         // (advanced per domain by the paged domain sweep)
   uint32_t n_phase[2];                  // learned form: radiance entries in phase A / B
-  unsigned long long useful, radiance_visits, shadow_visits, shades, final_hits, queue_entries,
-      pruned, deferred, passes, node_visits, tri_tests, log_count;
+  unsigned long long queue_entries, deferred, passes, log_count;
+  // Totals that every block of a launch adds to, kStatCopies times: block b
+  // adds to copy b mod kStatCopies, the host sums the copies.  Atomics on one
+  // address (or line) are served one at a time, so 1024 blocks adding five
+  // totals to one line held up the end of every launch.
+  alignas(128) unsigned long long stat[kStatCopies][16];
 };
 
 struct TraceParams {
