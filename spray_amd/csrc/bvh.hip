@@ -27,27 +27,60 @@ namespace spray {
 // each vertex, visited in ascending face order, reproduces that float
 // summation order exactly.
 // Face corners are numbered in 32 bits: a domain has fewer than 2^24 faces.
-__global__ void kVertCount(const uint32_t* __restrict__ face, long long nf, uint32_t* cnt) {
-  const uint32_t nc = (uint32_t)nf * 3u;
-  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += gridDim.x * blockDim.x)
-    atomicAdd(&cnt[face[i]], 1u);
+//
+// The build kernels take many domains per launch, domain blockIdx.y of the
+// array G each (blockIdx.x and gridDim.x count that domain's blocks): a
+// domain alone is a launch of a few microseconds that fills a fraction of the
+// GPU, and 47 of them per domain were bound by issuing them.
+struct FrontierItem {
+  int bnode;  // binary inner node
+  int wnode;  // 8-wide node slot
+};
+struct BuildDom {
+  const float* vtx;
+  const uint32_t *face, *rgb;
+  float* nrm;
+  float4* fshade;
+  LTri* tris;
+  BNode8* nodes;
+  // scratch: vertex adjacency, centroid bounds, sort buffers, leaf-range unions
+  uint32_t *cnt, *cur, *off, *adj, *bmm, *keys[2], *vals[2], *hist;
+  float *rpre, *rsuf, *rtab;
+  // binary tree: leaf and inner boxes, children, leaf ranges
+  float *leafbox, *innerbox;
+  int *left, *right, *first, *last;
+  FrontierItem* front[2];  // collapse frontiers
+  int* cc;                 // level counters (kLevelWords)
+  int nf, nv, node_cap;
+};
+
+__global__ void kVertClear(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const uint32_t n = 2u * ((uint32_t)B.nv + 1u);  // cnt and, after it, cur
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) B.cnt[i] = 0u;
 }
-__global__ void kVertFill(const uint32_t* __restrict__ face, long long nf,
-                          const uint32_t* __restrict__ off, uint32_t* cursor, uint32_t* adj) {
-  const uint32_t nc = (uint32_t)nf * 3u;
+__global__ void kVertCount(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const uint32_t nc = (uint32_t)B.nf * 3u;
+  for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += gridDim.x * blockDim.x)
+    atomicAdd(&B.cnt[B.face[i]], 1u);
+}
+__global__ void kVertFill(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const uint32_t nc = (uint32_t)B.nf * 3u;
   for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += gridDim.x * blockDim.x) {
-    const uint32_t v = face[i];
-    const uint32_t slot = atomicAdd(&cursor[v], 1u);
-    adj[off[v] + slot] = i / 3u;
+    const uint32_t v = B.face[i];
+    const uint32_t slot = atomicAdd(&B.cur[v], 1u);
+    B.adj[B.off[v] + slot] = i / 3u;
   }
 }
-__global__ void kVertNormal(const float* __restrict__ vtx, const uint32_t* __restrict__ face,
-                            long long nv, const uint32_t* __restrict__ off,
-                            const uint32_t* __restrict__ cnt, uint32_t* adj, float* nrm) {
-  for (long long v = blockIdx.x * (long long)blockDim.x + threadIdx.x; v < nv;
-       v += (long long)gridDim.x * blockDim.x) {
-    uint32_t b = off[v], n = cnt[v];
-    uint32_t* L = adj + b;
+__global__ void kVertNormal(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const float* __restrict__ vtx = B.vtx;
+  const uint32_t* __restrict__ face = B.face;
+  for (int v = blockIdx.x * blockDim.x + threadIdx.x; v < B.nv; v += gridDim.x * blockDim.x) {
+    uint32_t b = B.off[v], n = B.cnt[v];
+    uint32_t* L = B.adj + b;
     for (uint32_t i = 1; i < n; ++i) {  // insertion sort: lists are short
       uint32_t x = L[i];
       int j = (int)i - 1;
@@ -69,9 +102,9 @@ __global__ void kVertNormal(const float* __restrict__ vtx, const uint32_t* __res
       ay += uz * wx - ux * wz;
       az += ux * wy - uy * wx;
     }
-    nrm[v * 3] = ax;
-    nrm[v * 3 + 1] = ay;
-    nrm[v * 3 + 2] = az;
+    B.nrm[(size_t)v * 3] = ax;
+    B.nrm[(size_t)v * 3 + 1] = ay;
+    B.nrm[(size_t)v * 3 + 2] = az;
   }
 }
 
@@ -80,16 +113,14 @@ __global__ void kVertNormal(const float* __restrict__ vtx, const uint32_t* __res
 // of the face and then six vertex attributes.
 // It also sets the centroid bounds (ordered bits, see kCentroidBounds) to
 // their starting values for the Morton pass that follows it on the stream.
-__global__ void kFaceShade(const uint32_t* __restrict__ face, long long nf,
-                           const float* __restrict__ nrm, const uint32_t* __restrict__ rgb,
-                           float4* out, uint32_t* cbounds) {
-  if (blockIdx.x == 0 && threadIdx.x < 6) cbounds[threadIdx.x] = threadIdx.x < 3 ? 0xffffffffu : 0u;
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < nf;
-       i += (long long)gridDim.x * blockDim.x) {
+__global__ void kFaceShade(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  if (blockIdx.x == 0 && threadIdx.x < 6) B.bmm[threadIdx.x] = threadIdx.x < 3 ? 0xffffffffu : 0u;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < B.nf; i += gridDim.x * blockDim.x) {
     for (int k = 0; k < 3; ++k) {
-      uint32_t v = face[i * 3 + k];
-      out[i * 3 + k] = make_float4(nrm[(size_t)v * 3], nrm[(size_t)v * 3 + 1],
-                                   nrm[(size_t)v * 3 + 2], __uint_as_float(rgb[v]));
+      uint32_t v = B.face[(size_t)i * 3 + k];
+      B.fshade[(size_t)i * 3 + k] = make_float4(B.nrm[(size_t)v * 3], B.nrm[(size_t)v * 3 + 1],
+                                                B.nrm[(size_t)v * 3 + 2], __uint_as_float(B.rgb[v]));
     }
   }
 }
@@ -108,10 +139,13 @@ __device__ __forceinline__ float fromOrdered(uint32_t u) {
 // then one atomic per block and bound, so the six bound words see few
 // same-address atomics.
 constexpr int kBoundsGrid = 256;
-__global__ void __launch_bounds__(256) kCentroidBounds(const float* __restrict__ vtx,
-                                                       const uint32_t* __restrict__ face, int nf,
-                                                       uint32_t* bmin, uint32_t* bmax) {
+__global__ void __launch_bounds__(256) kCentroidBounds(const BuildDom* __restrict__ G) {
   __shared__ float red[6][4];
+  const BuildDom& B = G[blockIdx.y];
+  const float* __restrict__ vtx = B.vtx;
+  const uint32_t* __restrict__ face = B.face;
+  const int nf = B.nf;
+  uint32_t *bmin = B.bmm, *bmax = B.bmm + 3;
   float lo[3] = {kInfF, kInfF, kInfF}, hi[3] = {-kInfF, -kInfF, -kInfF};
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) {
     for (int k = 0; k < 3; ++k) {
@@ -150,9 +184,13 @@ __device__ __forceinline__ uint32_t expandBits10(uint32_t v) {
   return v;
 }
 
-__global__ void kMorton(const float* __restrict__ vtx, const uint32_t* __restrict__ face, int nf,
-                        const uint32_t* bmin, const uint32_t* bmax, uint32_t* keys,
-                        uint32_t* vals) {
+__global__ void kMorton(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const float* __restrict__ vtx = B.vtx;
+  const uint32_t* __restrict__ face = B.face;
+  const int nf = B.nf;
+  const uint32_t *bmin = B.bmm, *bmax = B.bmm + 3;
+  uint32_t *keys = B.keys[0], *vals = B.vals[0];
   float lo[3], ext[3];
   for (int k = 0; k < 3; ++k) {
     lo[k] = fromOrdered(bmin[k]);
@@ -183,8 +221,15 @@ constexpr int kRsBlock = 256;
 constexpr int kRsItems = 8;
 constexpr int kRsTile = kRsBlock * kRsItems;
 
-__global__ void kRsHist(const uint32_t* __restrict__ keys, int n, int shift, uint32_t* hist) {
+__host__ __device__ inline int rsTiles(int n) { return (n + kRsTile - 1) / kRsTile; }
+
+// hist[digit][tile] of pass `pass` (8 bits each, buffers alternating)
+__global__ void kRsHist(const BuildDom* __restrict__ G, int pass) {
   __shared__ uint32_t h[256];
+  const BuildDom& B = G[blockIdx.y];
+  const int n = B.nf, tiles = rsTiles(n), shift = 8 * pass;
+  if ((int)blockIdx.x >= tiles) return;
+  const uint32_t* __restrict__ keys = B.keys[pass & 1];
   h[threadIdx.x] = 0;
   __syncthreads();
   int base = blockIdx.x * kRsTile;
@@ -193,17 +238,22 @@ __global__ void kRsHist(const uint32_t* __restrict__ keys, int n, int shift, uin
     if (idx < n) atomicAdd(&h[(keys[idx] >> shift) & 255u], 1u);
   }
   __syncthreads();
-  hist[threadIdx.x * gridDim.x + blockIdx.x] = h[threadIdx.x];
+  B.hist[threadIdx.x * tiles + blockIdx.x] = h[threadIdx.x];
 }
 
-__global__ void kRsScatter(const uint32_t* __restrict__ kin, const uint32_t* __restrict__ vin,
-                           uint32_t* __restrict__ kout, uint32_t* __restrict__ vout, int n,
-                           int shift, const uint32_t* __restrict__ hist_scanned) {
+__global__ void kRsScatter(const BuildDom* __restrict__ G, int pass) {
   __shared__ uint32_t base[256];
   __shared__ uint32_t run[256];
   __shared__ uint32_t wc[4][256];
+  const BuildDom& B = G[blockIdx.y];
+  const int n = B.nf, tiles = rsTiles(n), shift = 8 * pass;
+  if ((int)blockIdx.x >= tiles) return;
+  const uint32_t* __restrict__ kin = B.keys[pass & 1];
+  const uint32_t* __restrict__ vin = B.vals[pass & 1];
+  uint32_t* __restrict__ kout = B.keys[(pass & 1) ^ 1];
+  uint32_t* __restrict__ vout = B.vals[(pass & 1) ^ 1];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  base[tid] = hist_scanned[tid * gridDim.x + blockIdx.x];
+  base[tid] = B.hist[tid * tiles + blockIdx.x];
   run[tid] = 0;
   const int tile = blockIdx.x * kRsTile;
   for (int j = 0; j < kRsItems; ++j) {
@@ -255,8 +305,10 @@ __device__ __forceinline__ int deltaK(const uint32_t* keys, int n, int i, int j)
 }
 
 // inner node i: children encoded c >= 0 inner, c < 0 leaf ~c (sorted position)
-__global__ void kKarras(const uint32_t* __restrict__ keys, int n, int* left, int* right,
-                        int* first, int* last, int* parent_inner, int* parent_leaf) {
+__global__ void kKarras(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const uint32_t* __restrict__ keys = B.keys[0];
+  const int n = B.nf;
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n - 1; i += gridDim.x * blockDim.x) {
     int d = (deltaK(keys, n, i, i + 1) - deltaK(keys, n, i, i - 1)) >= 0 ? 1 : -1;
     int dmin = deltaK(keys, n, i, i - d);
@@ -277,29 +329,22 @@ __global__ void kKarras(const uint32_t* __restrict__ keys, int n, int* left, int
     int lo = i < j ? i : j, hi = i < j ? j : i;
     int lc = (lo == gamma) ? ~gamma : gamma;
     int rc = (hi == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-    left[i] = lc;
-    right[i] = rc;
-    first[i] = lo;
-    last[i] = hi;
-    if (lc < 0)
-      parent_leaf[~lc] = i;
-    else
-      parent_inner[lc] = i;
-    if (rc < 0)
-      parent_leaf[~rc] = i;
-    else
-      parent_inner[rc] = i;
+    B.left[i] = lc;
+    B.right[i] = rc;
+    B.first[i] = lo;
+    B.last[i] = hi;
   }
 }
 
-// Leaf boxes in sorted order + the leaf-ordered triangle array of the pool.
-// parent_init (may be null): set to -1 for every leaf, the Karras
-// hierarchy's parent array before kKarras fills it (the root keeps -1).
-__global__ void kLeaves(const float* __restrict__ vtx, const uint32_t* __restrict__ face, int nf,
-                        const uint32_t* __restrict__ order, float* leafbox, LTri* out,
-                        int* parent_init = nullptr) {
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x) {
-    if (parent_init) parent_init[i] = -1;
+// Leaf boxes in sorted order + the leaf-ordered triangle array of the pool
+// (order: null for the Morton order).
+__global__ void kLeaves(const BuildDom* __restrict__ G, const uint32_t* order_or_null) {
+  const BuildDom& B = G[blockIdx.y];
+  const float* __restrict__ vtx = B.vtx;
+  const uint32_t* __restrict__ face = B.face;
+  const uint32_t* __restrict__ order = order_or_null ? order_or_null : B.vals[0];
+  float* leafbox = B.leafbox;
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < B.nf; i += gridDim.x * blockDim.x) {
     uint32_t p = order[i];
     const float* a = vtx + (size_t)face[p * 3] * 3;
     const float* b = vtx + (size_t)face[p * 3 + 1] * 3;
@@ -315,7 +360,7 @@ __global__ void kLeaves(const float* __restrict__ vtx, const uint32_t* __restric
     t.v0[3] = __int_as_float((int)p);
     t.v1[3] = 0.f;
     t.v2[3] = 0.f;
-    out[i] = t;
+    B.tris[i] = t;
   }
 }
 
@@ -330,9 +375,17 @@ __global__ void kLeaves(const float* __restrict__ vtx, const uint32_t* __restric
 // no device-scope fences or atomics.
 constexpr int kRangeBlock = 64;
 
-struct RangeLevels {
-  long long off[32];  // float offset of table level j (level 0: block boxes)
-};
+// Floats before table level j (level 0: block boxes; level j: nblk - 2^j + 1
+// entries of 6).
+__host__ __device__ inline long long rangeOff(long long nblk, int j) {
+  return 6 * ((long long)j * (nblk + 1) - ((1ll << j) - 1));
+}
+__host__ __device__ inline long long rangeBlocks(int n) { return (n + kRangeBlock - 1) / kRangeBlock; }
+inline int rangeLevels(int n) {
+  int j = 0;
+  for (long long w = 1; w <= rangeBlocks(n) && j < 32; w <<= 1) ++j;
+  return j;
+}
 
 __device__ __forceinline__ void boxMerge(float lo[3], float hi[3], const float* b) {
   for (int k = 0; k < 3; ++k) {
@@ -341,9 +394,11 @@ __device__ __forceinline__ void boxMerge(float lo[3], float hi[3], const float* 
   }
 }
 
-__global__ void __launch_bounds__(256) kLeafScan(const float* __restrict__ leafbox, int n,
-                                                 float* __restrict__ pre, float* __restrict__ suf,
-                                                 float* __restrict__ blockbox) {
+__global__ void __launch_bounds__(256) kLeafScan(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const float* __restrict__ leafbox = B.leafbox;
+  float *__restrict__ pre = B.rpre, *__restrict__ suf = B.rsuf, *__restrict__ blockbox = B.rtab;
+  const int n = B.nf;
   const int lane = threadIdx.x & 63;
   const long long nblk = (n + kRangeBlock - 1) / kRangeBlock;
   const long long nw = ((long long)gridDim.x * blockDim.x) >> 6;
@@ -383,24 +438,16 @@ __global__ void __launch_bounds__(256) kLeafScan(const float* __restrict__ leafb
   }
 }
 
-// table level j from level j - 1: m entries, each the union of entries i
-// and i + half of the level below
-__global__ void kRangeLevel(const float* __restrict__ src, float* __restrict__ dst, long long m,
-                            long long half) {
-  for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < m;
-       i += (long long)gridDim.x * blockDim.x)
-    for (int k = 0; k < 3; ++k) {
-      dst[i * 6 + k] = fminf(src[i * 6 + k], src[(i + half) * 6 + k]);
-      dst[i * 6 + 3 + k] = fmaxf(src[i * 6 + 3 + k], src[(i + half) * 6 + 3 + k]);
-    }
-}
-
 // Levels j and j + 1 of the sparse table in one launch, from level j - 1
 // (h = 2^(j-1) blocks per entry): level j entry i = union(src[i], src[i + h])
 // for i < mj, and level j + 1 entry i = union(level j [i], level j [i + 2h])
-// for i < mj2, each level-j box formed as the one-level kernel forms it.
-__global__ void kRangeLevel2(const float* __restrict__ src, float* __restrict__ dst,
-                             float* __restrict__ dst2, long long mj, long long mj2, long long h) {
+// for i < mj2 (mj2 <= 0: no such level), each level-j box formed alike.
+__global__ void kRangeLevel2(const BuildDom* __restrict__ G, int j) {
+  const BuildDom& B = G[blockIdx.y];
+  const long long nblk = rangeBlocks(B.nf), h = 1ll << (j - 1);
+  const long long mj = nblk - (1ll << j) + 1, mj2 = nblk - (1ll << (j + 1)) + 1;
+  const float* __restrict__ src = B.rtab + rangeOff(nblk, j - 1);
+  float *__restrict__ dst = B.rtab + rangeOff(nblk, j), *__restrict__ dst2 = B.rtab + rangeOff(nblk, j + 1);
   for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < mj;
        i += (long long)gridDim.x * blockDim.x) {
     float lo[3], hi[3];
@@ -420,10 +467,14 @@ __global__ void kRangeLevel2(const float* __restrict__ src, float* __restrict__ 
   }
 }
 
-__global__ void kRangeBoxes(int ninner, const int* __restrict__ first, const int* __restrict__ last,
-                            const float* __restrict__ leafbox, const float* __restrict__ pre,
-                            const float* __restrict__ suf, const float* __restrict__ table,
-                            RangeLevels L, float* __restrict__ innerbox) {
+__global__ void kRangeBoxes(const BuildDom* __restrict__ G) {
+  const BuildDom& B = G[blockIdx.y];
+  const int ninner = B.nf - 1;
+  const int *__restrict__ first = B.first, *__restrict__ last = B.last;
+  const float *__restrict__ leafbox = B.leafbox, *__restrict__ pre = B.rpre, *__restrict__ suf = B.rsuf,
+              *__restrict__ table = B.rtab;
+  float* __restrict__ innerbox = B.innerbox;
+  const long long nblk = rangeBlocks(B.nf);
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ninner; p += gridDim.x * blockDim.x) {
     const int a = first[p], b = last[p];
     const int ba = a / kRangeBlock, bb = b / kRangeBlock;
@@ -436,7 +487,7 @@ __global__ void kRangeBoxes(int ninner, const int* __restrict__ first, const int
       if (bb - ba >= 2) {
         const int x = ba + 1, y = bb - 1;
         const int j = 31 - __clz(y - x + 1);
-        const float* lv = table + L.off[j];
+        const float* lv = table + rangeOff(nblk, j);
         boxMerge(lo, hi, lv + (size_t)x * 6);
         boxMerge(lo, hi, lv + (size_t)(y - (1 << j) + 1) * 6);
       }
@@ -446,19 +497,6 @@ __global__ void kRangeBoxes(int ninner, const int* __restrict__ first, const int
       innerbox[(size_t)p * 6 + 3 + k] = hi[k];
     }
   }
-}
-
-// Table levels for n leaves: offsets and total floats.
-static long long rangeLevels(int n, RangeLevels* L, int* nlev) {
-  const long long nblk = (n + kRangeBlock - 1) / kRangeBlock;
-  long long off = 0;
-  int j = 0;
-  for (long long w = 1; w <= nblk && j < 32; w <<= 1, ++j) {
-    L->off[j] = off;
-    off += (nblk - w + 1) * 6;
-  }
-  *nlev = j;
-  return off;
 }
 
 // 8-wide nodes of a domain of nf triangles, at most.  In the collapsed tree
@@ -479,12 +517,6 @@ static_assert((1 << 24) / 7 + (6ll * (1 << 24)) / (7 * (kLeafMax + 1)) + 16 < (1
 constexpr int kLevelBatch = 16;
 constexpr int kMaxLevels = 48;
 constexpr int kLevelWords = 2 + kMaxLevels + 1;
-
-// Collapse the binary tree into 8-wide nodes, one frontier level per launch.
-struct FrontierItem {
-  int bnode;  // binary inner node
-  int wnode;  // 8-wide node slot
-};
 
 __device__ __forceinline__ float boxArea(const float* b) {
   float dx = fmaxf(b[3] - b[0], 0.f), dy = fmaxf(b[4] - b[1], 0.f), dz = fmaxf(b[5] - b[2], 0.f);
@@ -616,18 +648,22 @@ __device__ __forceinline__ int waveAlloc(int* ctr, int cnt) {
   return base + incl - cnt;
 }
 
-// One frontier level: *nin items in fin (0: nothing to do), next level's
-// items counted in *nout, on blocks blk of nblk.  Launched level after level
-// without host round trips; the loop bound is uniform per block so whole
-// waves allocate.
-__device__ __forceinline__ void collapseLevel(
-    int blk, int nblk, const FrontierItem* __restrict__ fin, const int* __restrict__ nin_ptr,
-    FrontierItem* fout, int* nout, int* node_counter, int node_cap, const int* __restrict__ left,
-    const int* __restrict__ right, const int* __restrict__ first, const int* __restrict__ last,
-    const float* __restrict__ leafbox, const float* __restrict__ innerbox, BNode8* nodes,
-    int* overflow) {
+// One frontier level l of every domain of the launch: cc[2 + l] items (0:
+// nothing to do), the next level's counted in cc[3 + l]; cc[0] counts nodes,
+// cc[1] is the overflow flag.  Launched level after level without host round
+// trips; the loop bound is uniform per block so whole waves allocate.
+__global__ void __launch_bounds__(256) kCollapseLevel(const BuildDom* __restrict__ G, int l) {
+  const BuildDom& B = G[blockIdx.y];
+  const FrontierItem* __restrict__ fin = B.front[l & 1];
+  FrontierItem* fout = B.front[(l & 1) ^ 1];
+  const int *nin_ptr = B.cc + 2 + l, node_cap = B.node_cap;
+  int *nout = B.cc + 3 + l, *node_counter = B.cc, *overflow = B.cc + 1;
+  const int *__restrict__ left = B.left, *__restrict__ right = B.right, *__restrict__ first = B.first,
+            *__restrict__ last = B.last;
+  const float *__restrict__ leafbox = B.leafbox, *__restrict__ innerbox = B.innerbox;
+  BNode8* nodes = B.nodes;
   const int nin = *nin_ptr;
-  for (int base = blk * blockDim.x; base < nin; base += nblk * blockDim.x) {
+  for (int base = blockIdx.x * blockDim.x; base < nin; base += gridDim.x * blockDim.x) {
     const int it = base + threadIdx.x;
     const bool act = it < nin;
     FrontierItem f{0, 0};
@@ -725,56 +761,21 @@ __device__ __forceinline__ void collapseLevel(
   }
 }
 
-__global__ void kCollapse(const FrontierItem* __restrict__ fin, const int* __restrict__ nin_ptr,
-                          FrontierItem* fout, int* nout, int* node_counter, int node_cap,
-                          const int* __restrict__ left, const int* __restrict__ right,
-                          const int* __restrict__ first, const int* __restrict__ last,
-                          const float* __restrict__ leafbox, const float* __restrict__ innerbox,
-                          BNode8* nodes, int* overflow) {
-  collapseLevel(blockIdx.x, gridDim.x, fin, nin_ptr, fout, nout, node_counter, node_cap, left, right,
-                first, last, leafbox, innerbox, nodes, overflow);
+// Collapse state of each domain: node counter 1 (the 8-wide root), no
+// overflow, one frontier item (binary node `root`) at level 0 (none for a
+// domain of one leaf, whose root kTinyRoot writes), empty later levels.
+__global__ void kCollapseInit(const BuildDom* __restrict__ G, int root) {
+  const BuildDom& B = G[blockIdx.y];
+  for (int i = threadIdx.x; i < kLevelWords; i += blockDim.x)
+    B.cc[i] = i == 0 || (i == 2 && B.nf > kLeafMax) ? 1 : 0;
+  if (threadIdx.x == 0) B.front[0][0] = FrontierItem{root, 0};
 }
-
-// A group of domains collapsed together: one launch per level for all of
-// them, blocksPerDom blocks per domain.  Each domain's binary tree sits in
-// its own tree slot; cc is its level counter block ([0] node counter, [1]
-// overflow, [2 + l] items of level l).
-constexpr int kCollapseGroupMax = 16;
-struct CollapseDom {
-  const int *left, *right, *first, *last;
-  const float *leafbox, *innerbox;
-  FrontierItem *fa, *fb;
-  BNode8* nodes;
-  int* cc;
-  int node_cap;
-};
-struct CollapseGroup {
-  CollapseDom dom[kCollapseGroupMax];
-  int n;
-};
-
-// Collapse state of each domain of the group: node counter 1 (the root),
-// no overflow, one frontier item (the binary root) at level 0, empty later
-// levels.
-__global__ void kCollapseGroupInit(CollapseGroup G) {
-  const CollapseDom& D = G.dom[blockIdx.x];
-  for (int i = threadIdx.x; i < kLevelWords; i += blockDim.x) D.cc[i] = (i == 0 || i == 2) ? 1 : 0;
-  if (threadIdx.x == 0) D.fa[0] = FrontierItem{0, 0};
-}
-
-__global__ void kCollapseGroupLevel(CollapseGroup G, int l, int blocks_per_dom) {
-  const int j = blockIdx.x / blocks_per_dom;  // uniform per block
-  const CollapseDom& D = G.dom[j];
-  const FrontierItem* fin = (l & 1) ? D.fb : D.fa;
-  FrontierItem* fout = (l & 1) ? D.fa : D.fb;
-  collapseLevel(blockIdx.x - j * blocks_per_dom, blocks_per_dom, fin, D.cc + 2 + l, fout,
-                D.cc + 3 + l, D.cc, D.node_cap, D.left, D.right, D.first, D.last, D.leafbox,
-                D.innerbox, D.nodes, D.cc + 1);
-}
-
 
 // Root for tiny domains (<= kLeafMax triangles): one leaf child.
-__global__ void kTinyRoot(int nf, const float* __restrict__ leafbox, BNode8* nodes) {
+__global__ void kTinyRoot(const BuildDom* __restrict__ G) {
+  const int nf = G->nf;
+  const float* leafbox = G->leafbox;
+  BNode8* nodes = G->nodes;
   float b[8][6] = {{kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF}};
   for (int i = 0; i < nf; ++i)
     for (int k = 0; k < 3; ++k) {
@@ -943,79 +944,62 @@ static int gridFor(long long n, int block) {
   return (int)g;
 }
 
-// Scratch of one domain build, sized for the largest domain.
-constexpr int kBuildStreams = 4;  // domain pipelines of a whole-scene LBVH build
-// tree slots of all pipelines together at most this many bytes
-constexpr size_t kTreeSlotBudget = (size_t)3 << 29;  // 1.5 GB
-
-// One domain's binary tree (children, leaf ranges, leaf and inner boxes)
-// and its collapse frontiers: what the collapse reads after the build.
-struct TreeSlot {
-  DevBuf lb, ib, lft, rgt, fst, lst, fa, fb;
-  // a frontier level holds disjoint subtrees of more than kLeafMax triangles
-  static size_t frontierItems(int maxf) { return (size_t)maxf / (kLeafMax + 1) + 64; }
-  static size_t bytesFor(int maxf) {
-    return (size_t)maxf * (24 + 24 + 16) + 2 * frontierItems(maxf) * sizeof(FrontierItem);
+// One domain's build scratch within a pipeline's memory (a slot): byte
+// offsets, sized for the largest domain.
+struct SlotLayout {
+  size_t keys[2], vals[2], hist, cnt, bmm, vsums, hsums, adj, rpre, rsuf, rtab, lb, ib, lft, rgt, fst, lst,
+      front[2], bytes = 0;
+  SlotLayout(int maxf, long long maxv) {
+    auto take = [&](size_t b) {
+      const size_t at = bytes;
+      bytes += (b + 255) & ~(size_t)255;
+      return at;
+    };
+    const size_t f = (size_t)maxf + 1, f4 = f * 4, hist_n = (size_t)256 * rsTiles(maxf);
+    for (size_t* x : {&keys[0], &keys[1], &vals[0], &vals[1], &lft, &rgt, &fst, &lst}) *x = take(f4);
+    hist = take(hist_n * 4);
+    cnt = take((size_t)(maxv + 1) * 12);
+    bmm = take(64);
+    vsums = take((size_t)scanSumsWords(maxv + 1) * 4);
+    hsums = take((size_t)scanSumsWords((long long)hist_n) * 4);
+    adj = take(f * 12);
+    for (size_t* x : {&rpre, &rsuf, &lb, &ib}) *x = take(f * 24);
+    rtab = take((size_t)rangeOff(rangeBlocks(maxf), rangeLevels(maxf)) * 4 + 64);
+    // a frontier level holds disjoint subtrees of more than kLeafMax triangles
+    for (size_t* x : {&front[0], &front[1]}) *x = take(((size_t)maxf / (kLeafMax + 1) + 64) * sizeof(FrontierItem));
   }
+};
+constexpr int kBuildStreams = 4;  // pipelines of a whole-scene LBVH build
+constexpr int kBuildGroup = 16;   // domains per launch, at most
+constexpr size_t kSlotBudget = (size_t)2 << 30;  // slots of all pipelines together
+
+struct PlocScratch {
+  DevBuf pc, pc2, pb, pb2, pnn, pcnt, pmf, pkf, pmp, pkp, pperm, pord;
   void reserve(int maxf) {
     const size_t f4 = (size_t)maxf * 4 + 64;
-    for (DevBuf* b : {&lft, &rgt, &fst, &lst}) b->reserve(f4);
-    lb.reserve((size_t)maxf * 24 + 64);
-    ib.reserve((size_t)maxf * 24 + 64);
-    fa.reserve(frontierItems(maxf) * sizeof(FrontierItem));
-    fb.reserve(frontierItems(maxf) * sizeof(FrontierItem));
+    for (DevBuf* b : {&pc, &pc2, &pnn, &pcnt, &pmf, &pkf, &pmp, &pkp, &pperm, &pord}) b->reserve(f4);
+    pb.reserve((size_t)maxf * 24 + 64);
+    pb2.reserve((size_t)maxf * 24 + 64);
   }
-  ~TreeSlot() {
-    for (DevBuf* b : {&lb, &ib, &lft, &rgt, &fst, &lst, &fa, &fb}) b->release();
+  ~PlocScratch() {
+    for (DevBuf* b : {&pc, &pc2, &pb, &pb2, &pnn, &pcnt, &pmf, &pkf, &pmp, &pkp, &pperm, &pord}) b->release();
   }
 };
 
-struct BuildScratch {
-  DevBuf keys, vals, keys2, vals2, hist, pin, plf, cnts, scal, adj, rpre, rsuf, rtab, lvl, sums;
-  DevBuf pc, pc2, pb, pb2, pnn, pcnt, pmf, pkf, pmp, pkp, pperm, pord;  // PLOC
-  std::vector<TreeSlot> slot;  // trees of the domains a group collapse takes together
-  void reserve(int maxf, long long maxv, bool ploc, int nslots = 1) {
-    const size_t f4 = (size_t)maxf * 4 + 64;
-    for (DevBuf* b : {&keys, &vals, &keys2, &vals2, &pin, &plf}) b->reserve(f4);
-    if (slot.size() != (size_t)std::max(1, nslots)) {  // fresh slots (no live buffer is copied)
-      slot.clear();
-      slot.resize(std::max(1, nslots));
-    }
-    for (TreeSlot& t : slot) t.reserve(maxf);
-    hist.reserve((size_t)256 * ((maxf + kRsTile - 1) / kRsTile) * 4 + 64);
-    cnts.reserve((size_t)(maxv + 1) * 12 + 64);
-    scal.reserve(64);
-    lvl.reserve(kLevelWords * 4 + 64);
-    // tile sums of this set's scans (vertex offsets, radix histograms, PLOC flags)
-    const long long scan_n = std::max<long long>(
-        std::max<long long>(maxv + 1, (long long)maxf + 1), 256ll * ((maxf + kRsTile - 1) / kRsTile));
-    sums.reserve((size_t)scanSumsWords(scan_n) * 4 + 64);
-    adj.reserve((size_t)maxf * 12 + 64);
-    rpre.reserve((size_t)maxf * 24 + 64);
-    rsuf.reserve((size_t)maxf * 24 + 64);
-    RangeLevels L;
-    int nlev;
-    rtab.reserve((size_t)rangeLevels(std::max(maxf, 1), &L, &nlev) * 4 + 64);
-    if (ploc) {
-      for (DevBuf* b : {&pc, &pc2, &pnn, &pcnt, &pmf, &pkf, &pmp, &pkp, &pperm, &pord}) b->reserve(f4);
-      pb.reserve((size_t)maxf * 24 + 64);
-      pb2.reserve((size_t)maxf * 24 + 64);
-    }
-  }
-  ~BuildScratch() {
-    for (DevBuf* b : {&keys, &vals, &keys2, &vals2, &hist, &pin, &plf, &cnts, &scal, &adj, &rpre,
-                      &rsuf, &rtab, &lvl, &sums, &pc, &pc2, &pb, &pb2, &pnn, &pcnt, &pmf, &pkf, &pmp,
-                      &pkp, &pperm, &pord})
-      b->release();
-  }
-};
-
+// Build memory: slots of each pipeline, domain descriptors and scan jobs,
+// level counters of every domain.
 struct BuildCache {
-  std::vector<BuildScratch> S;  // one scratch set per build pipeline
+  std::vector<DevBuf> slots;
+  DevBuf descs, levels;
+  ~BuildCache() {
+    for (DevBuf& b : slots) b.release();
+    descs.release();
+    levels.release();
+  }
 };
 
 void buildCacheRelease(Ctx* c) {
-  delete c->build_cache;  // the scratch sets release their buffers
+  delete c->build_cache;
   c->build_cache = nullptr;
 }
 
@@ -1105,168 +1089,207 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.fshade.reserve(tf * 48 + 64);
     P.nodes.reserve(tn * sizeof(BNode8));
   }
-  // A whole-scene LBVH build runs up to kBuildStreams domain pipelines side
-  // by side, one per free hardware queue (domain d on stream d % K, each
-  // stream with its own scratch set), so the many small per-domain kernels of different domains overlap;
-  // each domain's collapse launches a fixed number of levels with no host
-  // wait, and the level counts of every domain are checked once after the
-  // last.  A source whose fills may run concurrently fills each domain in
-  // its pipeline.  PLOC and paged builds stay in one stream with a host
-  // check per domain.
+  // A whole-scene LBVH build takes the domains in groups, one launch per
+  // build step for a group, up to kBuildStreams groups side by side (one per
+  // free hardware queue, each with its own slots); the collapse launches a
+  // fixed number of levels with no host wait, and the level counts of every
+  // domain are checked once after the last.  PLOC and paged builds take one
+  // domain at a time in one stream with a host check per domain.
   const bool multi = !paged && c->bvh_builder == 0 && nd > 1;
-  const bool pipe_fill = multi && src.pipelined();
-  if (!paged && !pipe_fill) {
-    for (int d = 0; d < nd; ++d) {
-      const DomainDesc& D = P.desc[d];
-      src.fill(c, d, P.vtx.as<float>() + D.vtx_off * 3, P.face.as<uint32_t>() + D.face_off * 3,
-               P.rgb.as<uint32_t>() + D.vtx_off, s);
-    }
+  if (!paged) {
+    if (!src.fillAll(c, P.desc, P.vtx.as<float>(), P.face.as<uint32_t>(), P.rgb.as<uint32_t>(), s))
+      for (int d = 0; d < nd; ++d) {
+        const DomainDesc& D = P.desc[d];
+        src.fill(c, d, P.vtx.as<float>() + D.vtx_off * 3, P.face.as<uint32_t>() + D.face_off * 3,
+                 P.rgb.as<uint32_t>() + D.vtx_off, s);
+      }
     src.check(c);
   }
-  DevBuf lvl_all;
-  std::vector<int> launched(nd, 0);  // collapse levels launched per domain (multi)
   // a remesh of the same domain structure launches the previous depth + 4
   // levels (a domain that needs more is rebuilt with host-checked levels)
   std::vector<int> prev_depth;
   if (keep_buffers && (int)P.bvh_depth.size() == nd) prev_depth = P.bvh_depth;
-  struct ReleaseLvl {
-    DevBuf& lvl;
-    ~ReleaseLvl() { lvl.release(); }
-  } release_lvl{lvl_all};
-  // one domain's normals, shading records and BVH, issued on stream s, its
-  // binary tree in tree slot TS; grouped: the collapse is left to the
-  // domain's group (no host wait), else it is host-checked here
-  auto buildOne = [&](BuildScratch& S, TreeSlot& TS, int d, hipStream_t s, bool grouped) {
+  P.bvh_depth.assign(nd, 0);
+  // a remesh keeps the build memory for the next remesh (it only grows), so
+  // repeated remeshes allocate nothing here; other builds hold none afterwards
+  BuildCache local;
+  BuildCache* M = &local;
+  if (multi && src.rebuilds() && keep_buffers) {
+    if (!c->build_cache) c->build_cache = new BuildCache;
+    M = c->build_cache;
+  } else {
+    buildCacheRelease(c);
+  }
+  const SlotLayout SL(std::max(maxf, 1), maxv);
+  const int K = multi ? std::min(pipelineCount(kBuildStreams), nd) : 1;
+  const int GN = multi ? (int)std::max<size_t>(1, std::min<size_t>({(size_t)kBuildGroup, (size_t)((nd + K - 1) / K),
+                                                                     kSlotBudget / ((size_t)K * SL.bytes)}))
+                       : 1;
+  const int ngroups = (nd + GN - 1) / GN;
+  if ((int)M->slots.size() < K) M->slots.resize(K);
+  for (int k = 0; k < K; ++k) M->slots[k].reserve((size_t)GN * SL.bytes);
+  M->levels.reserve((size_t)nd * kLevelWords * 4 + 64);
+  M->descs.reserve((size_t)nd * (sizeof(BuildDom) + 2 * sizeof(ScanJob)) + 64);
+  const BuildDom* dev = M->descs.as<BuildDom>();
+  const ScanJob* vscan = (const ScanJob*)(dev + nd);
+  const ScanJob* hscan = vscan + nd;
+  {
+    std::vector<char> host((size_t)nd * (sizeof(BuildDom) + 2 * sizeof(ScanJob)));
+    BuildDom* hb = (BuildDom*)host.data();
+    ScanJob* hv = (ScanJob*)(hb + nd);
+    ScanJob* hh = hv + nd;
+    for (int d = 0; d < nd; ++d) {
+      DomainDesc& D = P.desc[d];
+      if (paged) {  // built into block d % capacity from the staged mesh
+        const int b = d % P.capacity;
+        D.node_off = (long long)b * P.block_nodes;
+        D.tri_off = D.shade_off = (long long)b * P.block_tris;
+      }
+      char* slot = M->slots[(d / GN) % K].as<char>() + (size_t)(d % GN) * SL.bytes;
+      BuildDom& B = hb[d];
+      B.vtx = P.vtx.as<float>() + D.vtx_off * 3;
+      B.face = P.face.as<uint32_t>() + D.face_off * 3;
+      B.rgb = P.rgb.as<uint32_t>() + D.vtx_off;
+      B.nrm = P.nrm.as<float>() + D.vtx_off * 3;
+      B.fshade = P.fshade.as<float4>() + D.shade_off * 3;
+      B.tris = P.tris.as<LTri>() + D.tri_off;
+      B.nodes = P.nodes.as<BNode8>() + D.node_off;
+      B.nf = D.num_tris;
+      B.nv = (int)src.numVerts(d);
+      B.node_cap = (int)nodeCap(D.num_tris);
+      B.cnt = (uint32_t*)(slot + SL.cnt);
+      B.cur = B.cnt + (B.nv + 1);  // cleared with cnt
+      B.off = B.cur + (B.nv + 1);
+      B.adj = (uint32_t*)(slot + SL.adj);
+      B.bmm = (uint32_t*)(slot + SL.bmm);
+      for (int k = 0; k < 2; ++k) {
+        B.keys[k] = (uint32_t*)(slot + SL.keys[k]);
+        B.vals[k] = (uint32_t*)(slot + SL.vals[k]);
+        B.front[k] = (FrontierItem*)(slot + SL.front[k]);
+      }
+      B.hist = (uint32_t*)(slot + SL.hist);
+      B.rpre = (float*)(slot + SL.rpre);
+      B.rsuf = (float*)(slot + SL.rsuf);
+      B.rtab = (float*)(slot + SL.rtab);
+      B.leafbox = (float*)(slot + SL.lb);
+      B.innerbox = (float*)(slot + SL.ib);
+      B.left = (int*)(slot + SL.lft);
+      B.right = (int*)(slot + SL.rgt);
+      B.first = (int*)(slot + SL.fst);
+      B.last = (int*)(slot + SL.lst);
+      B.cc = M->levels.as<int>() + (size_t)d * kLevelWords;
+      hv[d] = ScanJob{B.cnt, B.off, (uint32_t*)(slot + SL.vsums), (long long)B.nv + 1};
+      hh[d] = ScanJob{B.hist, B.hist, (uint32_t*)(slot + SL.hsums), 256ll * rsTiles(B.nf)};
+    }
+    SPRAY_HIP(hipMemcpy(M->descs.p, host.data(), host.size(), hipMemcpyHostToDevice));
+  }
+  // domains [a, a + m) on stream st: normals, shading records, Morton order
+  auto sortStage = [&](int a, int m, hipStream_t st) {
+    int f = 0, v = 0;
+    for (int d = a; d < a + m; ++d) {
+      f = std::max(f, P.desc[d].num_tris);
+      v = std::max(v, (int)src.numVerts(d));
+    }
+    const BuildDom* G = dev + a;
+    auto grid = [&](long long n) { return dim3((unsigned)gridFor(n, 256), (unsigned)m); };
+    kVertClear<<<grid(2ll * (v + 1)), 256, 0, st>>>(G);
+    kVertCount<<<grid(3ll * f), 256, 0, st>>>(G);
+    exclusiveScanMany(vscan + a, m, (long long)v + 1, st);
+    kVertFill<<<grid(3ll * f), 256, 0, st>>>(G);
+    kVertNormal<<<grid(v), 256, 0, st>>>(G);
+    // Morton codes (kFaceShade sets the centroid bounds' starting values)
+    kFaceShade<<<grid(f), 256, 0, st>>>(G);
+    kCentroidBounds<<<dim3((unsigned)std::min(gridFor(f, 256), kBoundsGrid), (unsigned)m), 256, 0, st>>>(G);
+    kMorton<<<grid(f), 256, 0, st>>>(G);
+    const dim3 tiles((unsigned)std::max(1, rsTiles(f)), (unsigned)m);
+    for (int pass = 0; pass < 4; ++pass) {
+      kRsHist<<<tiles, kRsBlock, 0, st>>>(G, pass);
+      exclusiveScanMany(hscan + a, m, 256ll * rsTiles(f), st);
+      kRsScatter<<<tiles, kRsBlock, 0, st>>>(G, pass);
+    }
+    return f;
+  };
+  // the same domains' leaves and Karras hierarchies (f: the most triangles),
+  // inner boxes as unions over leaf ranges; one-leaf roots are written
+  auto treeStage = [&](int a, int m, int f, hipStream_t st) {
+    const BuildDom* G = dev + a;
+    auto grid = [&](long long n) { return dim3((unsigned)gridFor(n, 256), (unsigned)m); };
+    kLeaves<<<grid(f), 256, 0, st>>>(G, nullptr);
+    kKarras<<<grid(f), 256, 0, st>>>(G);
+    const long long nblk = rangeBlocks(f);
+    kLeafScan<<<grid(nblk * 64), 256, 0, st>>>(G);
+    for (int j = 1; j < rangeLevels(f); j += 2)  // two levels per launch
+      kRangeLevel2<<<grid(nblk - (1ll << j) + 1), 256, 0, st>>>(G, j);
+    kRangeBoxes<<<grid(f - 1), 256, 0, st>>>(G);
+    for (int d = a; d < a + m; ++d)
+      if (P.desc[d].num_tris <= kLeafMax) {
+        kTinyRoot<<<1, 1, 0, st>>>(dev + d);
+        P.desc[d].num_nodes = 1;
+        P.bvh_depth[d] = 1;
+      }
+  };
+  // level l holds at most 8^l items (one root, at most eight children per item)
+  auto collapseBlocks = [](int f, int l) {
+    const int most = std::min(gridFor(std::max(1, f / 8), 256), 2048);
+    return (unsigned)(l < 8 ? std::min<long long>(most, ((1ll << (3 * l)) + 255) / 256) : most);
+  };
+  // Collapse of domain d's binary tree under `root`, kLevelBatch levels per
+  // host wait (a level past the last finds 0 items); returns the number of
+  // levels with items (kMaxLevels + 1 when deeper than kMaxLevels).
+  auto collapseChecked = [&](int d, int root, hipStream_t st) {
+    const BuildDom* G = dev + d;
+    kCollapseInit<<<1, 64, 0, st>>>(G, root);
+    for (int done = 0;;) {
+      const int upto = std::min(done + kLevelBatch, kMaxLevels);
+      for (int l = done; l < upto; ++l) kCollapseLevel<<<collapseBlocks(P.desc[d].num_tris, l), 256, 0, st>>>(G, l);
+      done = upto;
+      int h[kLevelWords];
+      SPRAY_HIP(hipMemcpyAsync(h, M->levels.as<int>() + (size_t)d * kLevelWords, sizeof(h), hipMemcpyDeviceToHost, st));
+      SPRAY_HIP(hipStreamSynchronize(st));
+      if (h[1]) throw StatusError(SPRAY_ERR_CAPACITY, "BVH node capacity exceeded");
+      P.desc[d].num_nodes = h[0];
+      if (h[2 + done] == 0 || done == kMaxLevels) {
+        int depth = 0;
+        while (depth < done && h[2 + depth] > 0) ++depth;
+        return h[2 + done] > 0 ? kMaxLevels + 1 : depth;
+      }
+    }
+  };
+  auto fitsStack = [](int depth) { return depth <= kStackMax; };
+  PlocScratch PS;
+  if (!multi && c->bvh_builder == 1) PS.reserve(maxf);
+  // one domain with host-checked levels (PLOC, paged pools, single domains,
+  // domains deeper than the levels their group launched)
+  auto buildOne = [&](int d, bool ploc) {
     DomainDesc& D = P.desc[d];
     const int nf = D.num_tris;
     const long long nv = src.numVerts(d);
-    if (paged) {  // build into block d % capacity from the staged mesh
-      const int b = d % P.capacity;
-      D.node_off = (long long)b * P.block_nodes;
-      D.tri_off = D.shade_off = (long long)b * P.block_tris;
+    if (paged) {
       src.fill(c, d, P.vtx.as<float>(), P.face.as<uint32_t>(), P.rgb.as<uint32_t>(), s);
       src.check(c);
     }
-    const float* vtx = P.vtx.as<float>() + D.vtx_off * 3;
-    const uint32_t* face = P.face.as<uint32_t>() + D.face_off * 3;
-    if (pipe_fill)
-      src.fill(c, d, P.vtx.as<float>() + D.vtx_off * 3, P.face.as<uint32_t>() + D.face_off * 3,
-               P.rgb.as<uint32_t>() + D.vtx_off, s);
-    // normals
-    uint32_t* cnt = S.cnts.as<uint32_t>();
-    uint32_t* cur = cnt + (nv + 1);  // cleared with cnt in one fill
-    uint32_t* off = cur + (nv + 1);
-    SPRAY_HIP(hipMemsetAsync(cnt, 0, (size_t)(nv + 1) * 8, s));
-    kVertCount<<<gridFor((long long)nf * 3, 256), 256, 0, s>>>(face, nf, cnt);
-    exclusiveScan(cnt, off, nv + 1, s, S.sums.as<uint32_t>());
-    kVertFill<<<gridFor((long long)nf * 3, 256), 256, 0, s>>>(face, nf, off, cur,
-                                                              S.adj.as<uint32_t>());
-    kVertNormal<<<gridFor(nv, 256), 256, 0, s>>>(vtx, face, nv, off, cnt, S.adj.as<uint32_t>(),
-                                                  P.nrm.as<float>() + D.vtx_off * 3);
-    // Morton codes (kFaceShade sets the centroid bounds' starting values)
-    uint32_t* bmm = S.scal.as<uint32_t>();
-    kFaceShade<<<gridFor(nf, 256), 256, 0, s>>>(face, nf, P.nrm.as<float>() + D.vtx_off * 3,
-                                                 P.rgb.as<uint32_t>() + D.vtx_off,
-                                                 P.fshade.as<float4>() + D.shade_off * 3, bmm);
-    kCentroidBounds<<<std::min(gridFor(nf, 256), kBoundsGrid), 256, 0, s>>>(vtx, face, nf, bmm,
-                                                                            bmm + 3);
-    kMorton<<<gridFor(nf, 256), 256, 0, s>>>(vtx, face, nf, bmm, bmm + 3, S.keys.as<uint32_t>(),
-                                             S.vals.as<uint32_t>());
-    // radix sort, 4 passes of 8 bits
-    int nb = (nf + kRsTile - 1) / kRsTile;
-    uint32_t *ka = S.keys.as<uint32_t>(), *va = S.vals.as<uint32_t>(), *kb = S.keys2.as<uint32_t>(),
-             *vb = S.vals2.as<uint32_t>();
-    for (int pass = 0; pass < 4; ++pass) {
-      kRsHist<<<nb, kRsBlock, 0, s>>>(ka, nf, pass * 8, S.hist.as<uint32_t>());
-      exclusiveScan(S.hist.as<uint32_t>(), S.hist.as<uint32_t>(), (long long)256 * nb, s,
-                    S.sums.as<uint32_t>());
-      kRsScatter<<<nb, kRsBlock, 0, s>>>(ka, va, kb, vb, nf, pass * 8, S.hist.as<uint32_t>());
-      std::swap(ka, kb);
-      std::swap(va, vb);
-    }
-    LTri* tris = P.tris.as<LTri>() + D.tri_off;
-    BNode8* nodes = P.nodes.as<BNode8>() + D.node_off;
-    float* leafbox = TS.lb.as<float>();
-    const int node_cap = (int)nodeCap(nf);
-    // paged pool: the finished domain's image goes to pinned host memory
-    // (and its normals to the host, for the normals query)
-    auto pageOut = [&]() {
-      if (!paged) return;
-      char* dst = (char*)P.h_image + P.h_image_off[d];
-      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)nf * sizeof(LTri);
-      SPRAY_HIP(hipMemcpyAsync(dst, nodes, nb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb, tris, tb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb + tb, P.fshade.as<float4>() + D.shade_off * 3,
-                               (size_t)nf * 48, hipMemcpyDeviceToHost, s));
-      P.h_nrm[d].resize((size_t)nv * 3);
-      SPRAY_HIP(hipMemcpyAsync(P.h_nrm[d].data(), P.nrm.p, (size_t)nv * 12, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipStreamSynchronize(s));
-    };
-    if (nf <= kLeafMax) {
-      kLeaves<<<gridFor(nf, 256), 256, 0, s>>>(vtx, face, nf, va, leafbox, tris);
-      kTinyRoot<<<1, 1, 0, s>>>(nf, leafbox, nodes);
-      D.num_nodes = 1;
-      P.bvh_depth[d] = 1;
-      pageOut();
-      return;
-    }
-    int* L = TS.lft.as<int>();
-    int* R = TS.rgt.as<int>();
-    int* F = TS.fst.as<int>();
-    int* Lst = TS.lst.as<int>();
-    float* inner = TS.ib.as<float>();
-    // Collapse the binary tree under `root` into 8-wide nodes; returns the
-    // number of 8-wide levels.
-    // Levels are launched kLevelBatch at a time; each reads its item count
-    // from the device, so the host waits once per batch (a level past the
-    // last finds 0 items).  Returns the number of levels with items
-    // (kMaxLevels + 1 when deeper than kMaxLevels).
-    auto collapse = [&](int root) {
-      int* cc = S.lvl.as<int>();  // [0] node counter, [1] overflow, [2 + l] items of level l
-      int init[kLevelWords] = {};
-      init[0] = 1;
-      init[2] = 1;
-      SPRAY_HIP(hipMemcpyAsync(cc, init, sizeof(init), hipMemcpyHostToDevice, s));
-      FrontierItem item{root, 0};
-      SPRAY_HIP(hipMemcpyAsync(TS.fa.p, &item, sizeof(item), hipMemcpyHostToDevice, s));
-      const int grid = std::min(gridFor(std::max(1, nf / 8), 256), 2048);
-      int done = 0;
-      for (;;) {
-        const int upto = std::min(done + kLevelBatch, kMaxLevels);
-        for (int l = done; l < upto; ++l) {
-          FrontierItem* fin = (l & 1) ? TS.fb.as<FrontierItem>() : TS.fa.as<FrontierItem>();
-          FrontierItem* fout = (l & 1) ? TS.fa.as<FrontierItem>() : TS.fb.as<FrontierItem>();
-          kCollapse<<<grid, 256, 0, s>>>(fin, cc + 2 + l, fout, cc + 3 + l, cc, node_cap, L, R, F,
-                                         Lst, leafbox, inner, nodes, cc + 1);
-        }
-        done = upto;
-        int h[kLevelWords];
-        SPRAY_HIP(hipMemcpyAsync(h, cc, sizeof(h), hipMemcpyDeviceToHost, s));
-        SPRAY_HIP(hipStreamSynchronize(s));
-        if (h[1]) throw StatusError(SPRAY_ERR_CAPACITY, "BVH node capacity exceeded");
-        D.num_nodes = h[0];
-        if (h[2 + done] == 0 || done == kMaxLevels) {
-          int depth = 0;
-          while (depth < done && h[2 + depth] > 0) ++depth;
-          return h[2 + done] > 0 ? kMaxLevels + 1 : depth;
-        }
-      }
-    };
-    // worst-case stack need: three pushes per 8-wide level
-    auto fitsStack = [](int depth) { return depth <= kStackMax; };
-    int depth = -1;
-    if (c->bvh_builder == 1) {
+    const BuildDom* G = dev + d;
+    sortStage(d, 1, s);
+    int depth = nf <= kLeafMax ? 1 : -1;
+    if (ploc && depth < 0) {
       // PLOC passes until one cluster is left
-      int* cid = S.pc.as<int>();
-      int* cid2 = S.pc2.as<int>();
-      float* cbox = S.pb.as<float>();
-      float* cbox2 = S.pb2.as<float>();
-      int* nn = S.pnn.as<int>();
-      int* icount = S.pcnt.as<int>();
-      uint32_t* mflag = S.pmf.as<uint32_t>();
-      uint32_t* kflag = S.pkf.as<uint32_t>();
-      uint32_t* mpos = S.pmp.as<uint32_t>();
-      uint32_t* kpos = S.pkp.as<uint32_t>();
+      const char* slot = M->slots[0].as<char>();  // one-domain builds use slot 0
+      int *L = (int*)(slot + SL.lft), *R = (int*)(slot + SL.rgt), *F = (int*)(slot + SL.fst),
+          *Lst = (int*)(slot + SL.lst);
+      float* inner = (float*)(slot + SL.ib);
+      const uint32_t* va = (const uint32_t*)(slot + SL.vals[0]);
+      const float* vtx = P.vtx.as<float>() + D.vtx_off * 3;
+      const uint32_t* face = P.face.as<uint32_t>() + D.face_off * 3;
+      int* cid = PS.pc.as<int>();
+      int* cid2 = PS.pc2.as<int>();
+      float* cbox = PS.pb.as<float>();
+      float* cbox2 = PS.pb2.as<float>();
+      int* nn = PS.pnn.as<int>();
+      int* icount = PS.pcnt.as<int>();
+      uint32_t* mflag = PS.pmf.as<uint32_t>();
+      uint32_t* kflag = PS.pkf.as<uint32_t>();
+      uint32_t* mpos = PS.pmp.as<uint32_t>();
+      uint32_t* kpos = PS.pkp.as<uint32_t>();
       kPlocInit<<<gridFor(nf, 256), 256, 0, s>>>(vtx, face, nf, va, cid, cbox);
       std::vector<int> pass_base{0};
       int n = nf, made = 0;
@@ -1274,8 +1297,8 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       while (n > 1) {
         kPlocNearest<<<(n + kPlocBlock - 1) / kPlocBlock, kPlocBlock, 0, s>>>(cbox, n, nn);
         kPlocFlags<<<gridFor(n + 1, 256), 256, 0, s>>>(nn, n, mflag, kflag);
-        exclusiveScan(mflag, mpos, n + 1, s, S.sums.as<uint32_t>());
-        exclusiveScan(kflag, kpos, n + 1, s, S.sums.as<uint32_t>());
+        exclusiveScan(mflag, mpos, n + 1, s);
+        exclusiveScan(kflag, kpos, n + 1, s);
         kPlocMerge<<<gridFor(n, 256), 256, 0, s>>>(nn, n, cid, cbox, mpos, kpos, made, cid2, cbox2,
                                                     L, R, inner, icount);
         uint32_t h[2];
@@ -1295,143 +1318,68 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       if (ok) {
         // depth-first leaf order: roots of later passes first
         const int root = made - 1;
-        uint32_t* perm = S.pperm.as<uint32_t>();
+        uint32_t* perm = PS.pperm.as<uint32_t>();
         SPRAY_HIP(hipMemsetAsync(F + root, 0, 4, s));
         for (int p = (int)pass_base.size() - 1; p > 0; --p) {
           int lo = pass_base[p - 1], hi = pass_base[p];
           kPlocRanges<<<gridFor(hi - lo, 256), 256, 0, s>>>(lo, hi, L, R, icount, F, Lst, perm);
         }
-        uint32_t* order = S.pord.as<uint32_t>();
+        uint32_t* order = PS.pord.as<uint32_t>();
         kComposeOrder<<<gridFor(nf, 256), 256, 0, s>>>(perm, va, nf, order);
-        kLeaves<<<gridFor(nf, 256), 256, 0, s>>>(vtx, face, nf, order, leafbox, tris);
-        depth = collapse(root);
+        kLeaves<<<gridFor(nf, 256), 256, 0, s>>>(G, order);
+        depth = collapseChecked(d, root, s);
         if (!fitsStack(depth)) depth = -1;
       }
     }
-    if (depth < 0) {
-      // Karras LBVH: leaves in Morton order, bottom-up refit
-      int* PI = S.pin.as<int>();
-      int* PL = S.plf.as<int>();
-      kLeaves<<<gridFor(nf, 256), 256, 0, s>>>(vtx, face, nf, va, leafbox, tris, PI);
-      kKarras<<<gridFor(nf, 256), 256, 0, s>>>(ka, nf, L, R, F, Lst, PI, PL);
-      // inner boxes as unions over leaf ranges (replaces a bottom-up refit)
-      RangeLevels RL;
-      int nlev;
-      rangeLevels(nf, &RL, &nlev);
-      const long long nblk = (nf + kRangeBlock - 1) / kRangeBlock;
-      float* tab = S.rtab.as<float>();
-      kLeafScan<<<gridFor(nblk * 64, 256), 256, 0, s>>>(leafbox, nf, S.rpre.as<float>(),
-                                                        S.rsuf.as<float>(), tab);
-      for (int j = 1; j < nlev; j += 2) {  // two levels per launch
-        const long long m = nblk - (1ll << j) + 1;
-        if (j + 1 < nlev)
-          kRangeLevel2<<<gridFor(m, 256), 256, 0, s>>>(tab + RL.off[j - 1], tab + RL.off[j],
-                                                       tab + RL.off[j + 1], m,
-                                                       nblk - (1ll << (j + 1)) + 1, 1ll << (j - 1));
-        else
-          kRangeLevel<<<gridFor(m, 256), 256, 0, s>>>(tab + RL.off[j - 1], tab + RL.off[j], m,
-                                                      1ll << (j - 1));
+    if (depth < 0 || nf <= kLeafMax) {
+      treeStage(d, 1, nf, s);
+      if (nf > kLeafMax) {
+        depth = collapseChecked(d, 0, s);
+        if (!fitsStack(depth))
+          throw StatusError(SPRAY_ERR_CAPACITY, "BVH too deep for the traversal stack");
       }
-      kRangeBoxes<<<gridFor(nf - 1, 256), 256, 0, s>>>(nf - 1, F, Lst, leafbox, S.rpre.as<float>(),
-                                                       S.rsuf.as<float>(), tab, RL, inner);
-      if (grouped) return;  // collapsed with its group
-      depth = collapse(0);
-      if (!fitsStack(depth))
-        throw StatusError(SPRAY_ERR_CAPACITY, "BVH too deep for the traversal stack");
     }
     P.bvh_depth[d] = depth;
-    pageOut();
+    if (paged) {  // the finished image goes to pinned host memory, the normals to the host
+      char* dst = (char*)P.h_image + P.h_image_off[d];
+      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)nf * sizeof(LTri);
+      SPRAY_HIP(hipMemcpyAsync(dst, P.nodes.as<BNode8>() + D.node_off, nb, hipMemcpyDeviceToHost, s));
+      SPRAY_HIP(hipMemcpyAsync(dst + nb, P.tris.as<LTri>() + D.tri_off, tb, hipMemcpyDeviceToHost, s));
+      SPRAY_HIP(hipMemcpyAsync(dst + nb + tb, P.fshade.as<float4>() + D.shade_off * 3,
+                               (size_t)nf * 48, hipMemcpyDeviceToHost, s));
+      P.h_nrm[d].resize((size_t)nv * 3);
+      SPRAY_HIP(hipMemcpyAsync(P.h_nrm[d].data(), P.nrm.p, (size_t)nv * 12, hipMemcpyDeviceToHost, s));
+      SPRAY_HIP(hipStreamSynchronize(s));
+    }
   };
-  P.bvh_depth.assign(nd, 0);
   if (!multi) {
-    BuildScratch S;
-    S.reserve(maxf, maxv, c->bvh_builder == 1);
-    for (int d = 0; d < nd; ++d) buildOne(S, S.slot[0], d, s, false);
+    for (int d = 0; d < nd; ++d) buildOne(d, c->bvh_builder == 1);
   } else {
-    const int K = std::min(pipelineCount(kBuildStreams), nd);
-    // each pipeline keeps the binary trees of up to G domains and collapses
-    // them together, one launch per level for the group
-    const size_t slot_b = std::max<size_t>(TreeSlot::bytesFor(maxf), 1);
-    const int G = (int)std::max<size_t>(
-        1, std::min<size_t>({(size_t)kCollapseGroupMax, (size_t)((nd + K - 1) / K),
-                             kTreeSlotBudget / ((size_t)K * slot_b)}));
-    // a remesh keeps the pipelines' scratch sets for the next remesh (they
-    // only grow), so repeated remeshes allocate nothing here; other builds
-    // hold no scratch afterwards
-    std::vector<BuildScratch> local;
-    std::vector<BuildScratch>* Sv = &local;
-    if (src.rebuilds() && keep_buffers) {
-      if (!c->build_cache) c->build_cache = new BuildCache;
-      Sv = &c->build_cache->S;
-    } else {
-      buildCacheRelease(c);
-    }
-    if ((int)Sv->size() != K) {  // fresh sets (no live buffer is copied)
-      Sv->clear();
-      Sv->resize(K);
-    }
-    std::vector<BuildScratch>& S = *Sv;
-    for (auto& x : S) x.reserve(maxf, maxv, false, G);
-    lvl_all.reserve((size_t)nd * kLevelWords * 4 + 64);
-    // pipeline 0 on s, the others on their own streams (declared after the
-    // scratch sets: joined before they go)
-    StreamSet side(K - 1, s);
-    auto pipe = [&](int k) { return k == 0 ? s : side[k - 1]; };
-    std::vector<std::vector<int>> pending(K);  // domains of each pipeline's open group
-    auto flush = [&](int k) {
-      std::vector<int>& g = pending[k];
-      if (g.empty()) return;
-      CollapseGroup CG{};
-      CG.n = (int)g.size();
-      int levels = 1, bpd = 1;
-      for (int j = 0; j < CG.n; ++j) {
-        const int d = g[j];
-        const DomainDesc& D = P.desc[d];
-        TreeSlot& TS = S[k].slot[j];
-        CollapseDom& X = CG.dom[j];
-        X.left = TS.lft.as<int>();
-        X.right = TS.rgt.as<int>();
-        X.first = TS.fst.as<int>();
-        X.last = TS.lst.as<int>();
-        X.leafbox = TS.lb.as<float>();
-        X.innerbox = TS.ib.as<float>();
-        X.fa = TS.fa.as<FrontierItem>();
-        X.fb = TS.fb.as<FrontierItem>();
-        X.nodes = P.nodes.as<BNode8>() + D.node_off;
-        X.cc = lvl_all.as<int>() + (size_t)d * kLevelWords;
-        X.node_cap = (int)nodeCap(D.num_tris);
-        levels = std::max(levels, prev_depth.empty() ? kMaxLevels
-                                                     : std::min(kMaxLevels, prev_depth[d] + 4));
-        bpd = std::max(bpd, std::min(gridFor(std::max(1, D.num_tris / 8), 256), 2048));
+    std::vector<int> launched(nd, 0);  // collapse levels launched per domain
+    {
+      // pipeline 0 on s, the others on their own streams
+      StreamSet side(std::min(K, ngroups) - 1, s);
+      for (int g = 0; g < ngroups; ++g) {
+        const int a = g * GN, m = std::min(GN, nd - a), k = g % K;
+        hipStream_t st = k == 0 ? s : side[k - 1];
+        const int f = sortStage(a, m, st);
+        treeStage(a, m, f, st);
+        int levels = prev_depth.empty() ? kMaxLevels : 1;
+        if (!prev_depth.empty())
+          for (int d = a; d < a + m; ++d) levels = std::max(levels, std::min(kMaxLevels, prev_depth[d] + 4));
+        kCollapseInit<<<dim3(1, (unsigned)m), 64, 0, st>>>(dev + a, 0);
+        for (int l = 0; l < levels; ++l)
+          kCollapseLevel<<<dim3(collapseBlocks(f, l), (unsigned)m), 256, 0, st>>>(dev + a, l);
+        for (int d = a; d < a + m; ++d) launched[d] = levels;
+        SPRAY_HIP(hipGetLastError());
       }
-      kCollapseGroupInit<<<CG.n, 64, 0, pipe(k)>>>(CG);
-      for (int l = 0; l < levels; ++l) {
-        // level l holds at most 8^l items (one root, at most eight children per item)
-        const int b = l < 8 ? std::min(bpd, (int)(((1ll << (3 * l)) + 255) / 256)) : bpd;
-        kCollapseGroupLevel<<<CG.n * b, 256, 0, pipe(k)>>>(CG, l, b);
-      }
-      SPRAY_HIP(hipGetLastError());
-      for (int d : g) launched[d] = levels;
-      g.clear();
-    };
-    for (int d = 0; d < nd; ++d) {
-      const int k = d % K;
-      const bool grouped = P.desc[d].num_tris > kLeafMax;  // one-leaf roots are built directly
-      buildOne(S[k], S[k].slot[pending[k].size()], d, pipe(k), grouped);
-      if (grouped) {
-        pending[k].push_back(d);
-        if ((int)pending[k].size() == G) flush(k);
-      }
-    }
-    for (int k = 0; k < K; ++k) flush(k);
-    side.release();
+    }  // waits for the side streams
     SPRAY_HIP(hipStreamSynchronize(s));  // pipeline 0
-    if (pipe_fill) src.check(c);
     std::vector<int> h((size_t)nd * kLevelWords);
-    SPRAY_HIP(hipMemcpy(h.data(), lvl_all.p, h.size() * 4, hipMemcpyDeviceToHost));
+    SPRAY_HIP(hipMemcpy(h.data(), M->levels.p, h.size() * 4, hipMemcpyDeviceToHost));
     std::vector<int> redo;
     for (int d = 0; d < nd; ++d) {
-      if (P.desc[d].num_tris <= kLeafMax) continue;  // one-leaf root, built directly
+      if (P.desc[d].num_tris <= kLeafMax) continue;  // one-leaf root, written directly
       const int* cc = &h[(size_t)d * kLevelWords];
       if (cc[1]) throw StatusError(SPRAY_ERR_CAPACITY, "BVH node capacity exceeded");
       if (cc[2 + launched[d]] > 0) {  // items left after the last launched level
@@ -1442,12 +1390,12 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       }
       int depth = 0;
       while (depth < launched[d] && cc[2 + depth] > 0) ++depth;
-      if (depth > kStackMax)
+      if (!fitsStack(depth))
         throw StatusError(SPRAY_ERR_CAPACITY, "BVH too deep for the traversal stack");
       P.desc[d].num_nodes = cc[0];
       P.bvh_depth[d] = depth;
     }
-    for (int d : redo) buildOne(S[0], S[0].slot[0], d, s, false);  // deeper than last time: host-checked
+    for (int d : redo) buildOne(d, false);  // deeper than last time: host-checked
   }
   SPRAY_HIP(hipStreamSynchronize(s));
   long long used = 0;

@@ -41,7 +41,8 @@ __device__ __forceinline__ uint32_t blockExclusive(uint32_t v, uint32_t* lds, ui
   return r;
 }
 
-__global__ void kScanTiles(const uint32_t* in, uint32_t* out, long long n, uint32_t* sums) {
+__device__ __forceinline__ void scanTile(const uint32_t* in, uint32_t* out, long long n,
+                                         uint32_t* sums) {
   __shared__ uint32_t lds[kScanBlock / 64 + 1];
   long long base = (long long)blockIdx.x * kScanTile + (long long)threadIdx.x * kScanItems;
   uint32_t vals[kScanItems];
@@ -61,6 +62,14 @@ __global__ void kScanTiles(const uint32_t* in, uint32_t* out, long long n, uint3
   if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
+__global__ void kScanTiles(const uint32_t* in, uint32_t* out, long long n, uint32_t* sums) {
+  scanTile(in, out, n, sums);
+}
+__global__ void kScanTilesMany(const ScanJob* __restrict__ jobs) {
+  const ScanJob J = jobs[blockIdx.y];
+  if ((long long)blockIdx.x * kScanTile < J.n) scanTile(J.in, J.out, J.n, J.sums);  // uniform per block
+}
+
 __global__ void kScanSums(uint32_t* sums, long long m) {
   __shared__ uint32_t lds[1024 / 64 + 1];
   uint32_t carry = 0;
@@ -78,7 +87,7 @@ __global__ void kScanSums(uint32_t* sums, long long m) {
 // each block forms itself, and the separate tile-sum scan is skipped.
 constexpr long long kScanFuseTiles = 1024;
 
-__global__ void kScanAddSum(uint32_t* out, long long n, const uint32_t* sums) {
+__device__ __forceinline__ void scanAddSum(uint32_t* out, long long n, const uint32_t* sums) {
   __shared__ uint32_t pre;
   if (threadIdx.x < 64) {
     uint32_t x = 0;
@@ -92,6 +101,12 @@ __global__ void kScanAddSum(uint32_t* out, long long n, const uint32_t* sums) {
     const long long i = base + j;
     if (i < n) out[i] += pre;
   }
+}
+
+__global__ void kScanAddSum(uint32_t* out, long long n, const uint32_t* sums) { scanAddSum(out, n, sums); }
+__global__ void kScanAddSumMany(const ScanJob* __restrict__ jobs) {
+  const ScanJob J = jobs[blockIdx.y];
+  if (blockIdx.x > 0 && (long long)blockIdx.x * kScanTile < J.n) scanAddSum(J.out, J.n, J.sums);
 }
 
 __global__ void kScanAdd(uint32_t* out, long long n, const uint32_t* sums) {
@@ -115,6 +130,14 @@ void exclusiveScan(const uint32_t* in, uint32_t* out, long long n, hipStream_t s
     kScanSums<<<1, 1024, 0, s>>>(tile_sums, nb);
     kScanAdd<<<(unsigned)nb, kScanBlock, 0, s>>>(out, n, tile_sums);
   }
+  SPRAY_HIP(hipGetLastError());
+}
+
+void exclusiveScanMany(const ScanJob* jobs, int count, long long max_n, hipStream_t s) {
+  if (max_n <= 0 || count <= 0) return;
+  const dim3 grid((unsigned)((max_n + kScanTile - 1) / kScanTile), (unsigned)count);
+  kScanTilesMany<<<grid, kScanBlock, 0, s>>>(jobs);
+  if (grid.x > 1) kScanAddSumMany<<<grid, kScanBlock, 0, s>>>(jobs);
   SPRAY_HIP(hipGetLastError());
 }
 

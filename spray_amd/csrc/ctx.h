@@ -119,9 +119,13 @@ struct MeshSource {
   virtual void fill(Ctx* c, int d, float* v, uint32_t* f, uint32_t* rgb, hipStream_t s) = 0;
   // After the fills issued so far: throws if one of them found bad input.
   virtual void check(Ctx* c) { (void)c; }
-  // fill() of different domains may run concurrently on several streams,
-  // with no host wait inside.
-  virtual bool pipelined() const { return false; }
+  // Every domain's fill in a few launches on stream s (domain d's vertices at
+  // vtx_off[d], faces at face_off[d]), where the source can; else false.
+  virtual bool fillAll(Ctx* c, const std::vector<DomainDesc>& desc, float* v, uint32_t* f, uint32_t* rgb,
+                       hipStream_t s) {
+    (void)c, (void)desc, (void)v, (void)f, (void)rgb, (void)s;
+    return false;
+  }
   // The scene is rebuilt from this kind of source again and again
   // (remeshing): the build keeps its scratch for the next build.
   virtual bool rebuilds() const { return false; }

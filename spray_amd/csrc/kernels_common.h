@@ -34,5 +34,13 @@ __device__ __forceinline__ unsigned long long waveSumULL(unsigned long long v) {
 void exclusiveScan(const uint32_t* in, uint32_t* out, long long n, hipStream_t s);
 void exclusiveScan(const uint32_t* in, uint32_t* out, long long n, hipStream_t s, uint32_t* tile_sums);
 long long scanSumsWords(long long n);
+// Many scans in one launch: job y of `count` jobs in device memory (sums:
+// scanSumsWords(n) words of its own), the longest of max_n values.
+struct ScanJob {
+  const uint32_t* in;
+  uint32_t *out, *sums;
+  long long n;
+};
+void exclusiveScanMany(const ScanJob* jobs, int count, long long max_n, hipStream_t s);
 
 }  // namespace spray

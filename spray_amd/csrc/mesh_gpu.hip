@@ -64,7 +64,7 @@ long long mcVertsCap(long long cap) {
 constexpr int kBlk = 256;
 constexpr int kBoundBlocks = 1024;
 
-__device__ void blockBounds(float lo[3], float hi[3], float* part) {
+__device__ void blockBounds(float lo[3], float hi[3], float* part, int slot) {
   __shared__ float red[6][kBlk / 64];
   const int w = threadIdx.x >> 6, l = threadIdx.x & 63;
   for (int c = 0; c < 3; ++c) {
@@ -79,18 +79,21 @@ __device__ void blockBounds(float lo[3], float hi[3], float* part) {
     float v = red[threadIdx.x][0];
     for (int i = 1; i < (int)(blockDim.x >> 6); ++i)
       v = threadIdx.x < 3 ? fminf(v, red[threadIdx.x][i]) : fmaxf(v, red[threadIdx.x][i]);
-    part[blockIdx.x * 6 + threadIdx.x] = v;
+    part[slot * 6 + threadIdx.x] = v;
   }
 }
 
-__global__ void __launch_bounds__(kBlk) kBoundsFinal(const float* part, int nparts, float* out) {
+__device__ void boundsFinal(const float* part, int nparts, float* out) {
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   for (int i = threadIdx.x; i < nparts; i += blockDim.x)
     for (int c = 0; c < 3; ++c) {
       lo[c] = fminf(lo[c], part[i * 6 + c]);
       hi[c] = fmaxf(hi[c], part[i * 6 + 3 + c]);
     }
-  blockBounds(lo, hi, out);  // a single block: writes out[0..5]
+  blockBounds(lo, hi, out, 0);  // one block's result: out[0..5]
+}
+__global__ void __launch_bounds__(kBlk) kBoundsFinal(const float* part, int nparts, float* out) {
+  boundsFinal(part, nparts, out);
 }
 
 __global__ void __launch_bounds__(kBlk) kPointBounds(const float* v, long long nv, float* part) {
@@ -101,7 +104,7 @@ __global__ void __launch_bounds__(kBlk) kPointBounds(const float* v, long long n
       lo[c] = fminf(lo[c], v[i * 3 + c]);
       hi[c] = fmaxf(hi[c], v[i * 3 + c]);
     }
-  blockBounds(lo, hi, part);
+  blockBounds(lo, hi, part, blockIdx.x);
 }
 
 // ---------------------------------------------------------------------------
@@ -398,6 +401,21 @@ struct McGrid {
   double a, b, phase;
 };
 
+// One domain of a generator launch: its grid and count buffers, where its
+// bounds and totals go, and (emission) its mesh.  The kernels take domain
+// blockIdx.y of an array of these, blockIdx.x and gridDim.x counting that
+// domain's blocks.
+struct McDom {
+  McGrid g;
+  uint8_t* sgn;              // field signs at the grid points
+  unsigned long long* bits;  // cut edges
+  uint32_t *eoff, *coff;     // counts, then offsets, per block of edges / cells
+  float *part, *bounds;      // vertex bounds: per block, final
+  uint32_t* totals;          // vertices, faces
+  float* v;
+  uint32_t *rgb, *f;
+};
+
 struct McCorners {  // per local edge: corner offset and axis
   int dx[12], dy[12], dz[12], axis[12];
 };
@@ -451,8 +469,10 @@ __device__ __forceinline__ double mcFieldAt(const McGrid& g, const double* tab, 
 // Field signs as bytes (1: inside, f < 0): the cut and case tests read one
 // byte per grid point; field values are evaluated again only at the ends
 // of cut edges.
-__global__ void __launch_bounds__(kBlk) kMcSign(McGrid g, uint8_t* __restrict__ sgn) {
+__global__ void __launch_bounds__(kBlk) kMcSign(const McDom* __restrict__ G) {
   extern __shared__ double tab[];
+  const McGrid g = G[blockIdx.y].g;
+  uint8_t* __restrict__ sgn = G[blockIdx.y].sgn;
   mcAxisTables(g, tab);
   const long long np = (long long)g.N * g.N * g.N;
   for (long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x; t < np;
@@ -479,10 +499,12 @@ __device__ __forceinline__ void mcVertex(const McGrid& g, int axis, int i, int j
 // along edge e; edges go in blocks of 256 (four 64-bit words), bcnt[blk] =
 // cuts in the block (bcnt[nblk] = 0, for the exclusive scan of the block
 // counts).
-__global__ void __launch_bounds__(kBlk) kMcEdgeBits(McGrid g, const uint8_t* __restrict__ sgn,
-                                                    unsigned long long* __restrict__ bits,
-                                                    uint32_t* __restrict__ bcnt) {
+__global__ void __launch_bounds__(kBlk) kMcEdgeBits(const McDom* __restrict__ G) {
   __shared__ uint32_t wsum[kBlk / 64];
+  const McGrid g = G[blockIdx.y].g;
+  const uint8_t* __restrict__ sgn = G[blockIdx.y].sgn;
+  unsigned long long* __restrict__ bits = G[blockIdx.y].bits;
+  uint32_t* __restrict__ bcnt = G[blockIdx.y].eoff;
   const long long ne = 3 * g.E, nblk = (ne + kBlk - 1) / kBlk;
   const int w = threadIdx.x >> 6;
   for (long long blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
@@ -547,17 +569,20 @@ __device__ __forceinline__ int mcNthBit(unsigned long long m, uint32_t k) {
 // (16 blocks of 256 edges), scans their cut counts, and gives each lane one
 // cut (its word found by a binary search of the scan, its bit by a
 // popcount search), so the field is evaluated for 64 cuts at a time and the
-// vertex stores are contiguous.  With v == nullptr only the per-block
-// bounds of the vertices are produced (part, one slot per block).
-__global__ void __launch_bounds__(kBlk) kMcVerts(McGrid g,
-                                                 const unsigned long long* __restrict__ bits,
-                                                 const uint32_t* __restrict__ eoff, uint32_t color,
-                                                 float* __restrict__ v, uint32_t* __restrict__ rgb,
-                                                 float* part) {
+// vertex stores are contiguous.  kEmit: vertices and colours are stored;
+// otherwise only the per-block bounds of the vertices (part, one slot per
+// block of the domain).
+template <bool kEmit>
+__global__ void __launch_bounds__(kBlk) kMcVerts(const McDom* __restrict__ G, uint32_t color) {
   static_assert(kBlk % 256 == 0, "a wave's 64 words are whole blocks of edges");
   __shared__ uint32_t scan[kBlk];
   __shared__ unsigned long long word[kBlk];
   extern __shared__ double tab[];
+  const McGrid g = G[blockIdx.y].g;
+  const unsigned long long* __restrict__ bits = G[blockIdx.y].bits;
+  const uint32_t* __restrict__ eoff = G[blockIdx.y].eoff;
+  float* __restrict__ v = G[blockIdx.y].v;
+  uint32_t* __restrict__ rgb = G[blockIdx.y].rgb;
   mcAxisTables(g, tab);
   float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
   const long long nwords = ((3 * g.E + kBlk - 1) / kBlk) * (kBlk / 64);
@@ -594,7 +619,7 @@ __global__ void __launch_bounds__(kBlk) kMcVerts(McGrid g,
       const double f1 = mcFieldAt(g, tab, i + (axis == 0), j + (axis == 1), k + (axis == 2));
       float p[3];
       mcVertex(g, axis, i, j, k, f0, f1, p);
-      if (v) {
+      if (kEmit) {
         const uint32_t id = base + r;
         for (int q = 0; q < 3; ++q) v[(size_t)id * 3 + q] = p[q];
         rgb[id] = color;
@@ -606,7 +631,7 @@ __global__ void __launch_bounds__(kBlk) kMcVerts(McGrid g,
       }
     }
   }
-  if (part) blockBounds(lo, hi, part);
+  if (!kEmit) blockBounds(lo, hi, G[blockIdx.y].part, blockIdx.x);
 }
 
 __device__ __forceinline__ int mcCase(const McGrid& g, const uint8_t* sgn, int i, int j, int k) {
@@ -623,10 +648,12 @@ __device__ __forceinline__ void mcCellDecode(const McGrid& g, long long t, int* 
 }
 
 // Triangles per block of 256 cells (bcnt[nblk] = 0).
-__global__ void __launch_bounds__(kBlk) kMcCellCount(McGrid g, const uint8_t* __restrict__ sgn,
-                                                     const uint8_t* __restrict__ ntri,
-                                                     uint32_t* __restrict__ bcnt) {
+__global__ void __launch_bounds__(kBlk) kMcCellCount(const McDom* __restrict__ G,
+                                                     const uint8_t* __restrict__ ntri) {
   __shared__ uint32_t wsum[kBlk / 64];
+  const McGrid g = G[blockIdx.y].g;
+  const uint8_t* __restrict__ sgn = G[blockIdx.y].sgn;
+  uint32_t* __restrict__ bcnt = G[blockIdx.y].coff;
   const long long nc = (long long)g.n * g.n * g.n, nblk = (nc + kBlk - 1) / kBlk;
   for (long long blk = blockIdx.x; blk < nblk; blk += gridDim.x) {
     const long long t = blk * kBlk + threadIdx.x;
@@ -649,22 +676,20 @@ __global__ void __launch_bounds__(kBlk) kMcCellCount(McGrid g, const uint8_t* __
   if (blockIdx.x == 0 && threadIdx.x == 0) bcnt[nblk] = 0u;
 }
 
-// Grid cap of kMcSign and kMcCells: eight blocks per CU, each stages its
-// tables into LDS once.
-constexpr long long kMcCellBlocks = 2048;
+// Blocks of the kernels that stage tables into LDS, over all domains of a
+// launch: 32 per CU, but at least 8 for each domain.
+constexpr long long kMcTabBlocks = 8192;
+long long mcTabCap(int domains) { return std::max(8ll, kMcTabBlocks / domains); }
+long long mcFlatCap(int domains) { return std::max(64ll, std::min(65535ll, (1ll << 19) / domains)); }
 
 // Triangles of every cell, in cell order: the block's offset plus an
 // exclusive scan of the per-cell counts inside the block.  The vertices of a
 // wave's triangles are then spread over its lanes, one vertex per lane, its
 // cell found by a binary search of the wave's scan, so the edge-id loads of
 // all of them are in flight together and the index stores are contiguous.
-__global__ void __launch_bounds__(kBlk) kMcCells(McGrid g, const uint8_t* __restrict__ sgn,
+__global__ void __launch_bounds__(kBlk) kMcCells(const McDom* __restrict__ G,
                                                  const int8_t* __restrict__ table,
-                                                 const uint8_t* __restrict__ ntri, McCorners ec,
-                                                 const unsigned long long* __restrict__ bits,
-                                                 const uint32_t* __restrict__ eoff,
-                                                 const uint32_t* __restrict__ coff,
-                                                 uint32_t* __restrict__ out) {
+                                                 const uint8_t* __restrict__ ntri, McCorners ec) {
   static_assert(kBlk == 256, "one case per thread when the tables are staged");
   __shared__ int8_t tab[256 * 24];  // the table's rows without their terminator
   __shared__ uint8_t cnt[256];
@@ -673,6 +698,11 @@ __global__ void __launch_bounds__(kBlk) kMcCells(McGrid g, const uint8_t* __rest
   __shared__ uint32_t excl[kBlk];
   __shared__ int ci[kBlk], cj[kBlk], ck[kBlk];
   __shared__ uint8_t ccase[kBlk];
+  const McGrid g = G[blockIdx.y].g;
+  const uint8_t* __restrict__ sgn = G[blockIdx.y].sgn;
+  const unsigned long long* __restrict__ bits = G[blockIdx.y].bits;
+  const uint32_t *__restrict__ eoff = G[blockIdx.y].eoff, *__restrict__ coff = G[blockIdx.y].coff;
+  uint32_t* __restrict__ out = G[blockIdx.y].f;
   for (int x = threadIdx.x; x < 256 * 24; x += kBlk) tab[x] = table[(x / 24) * 25 + x % 24];
   cnt[threadIdx.x] = ntri[threadIdx.x];
   if (threadIdx.x < 12) {
@@ -724,9 +754,18 @@ __global__ void __launch_bounds__(kBlk) kMcCells(McGrid g, const uint8_t* __rest
   }
 }
 
-__global__ void kMcTotals(const uint32_t* vtotal, const uint32_t* ftotal, uint32_t* out) {
-  out[0] = *vtotal;
-  out[1] = *ftotal;
+__device__ __forceinline__ long long mcEdgeBlocks(const McGrid& g) { return (3 * g.E + kBlk - 1) / kBlk; }
+__device__ __forceinline__ long long mcCellBlocks(const McGrid& g) {
+  return ((long long)g.n * g.n * g.n + kBlk - 1) / kBlk;
+}
+__global__ void kMcTotals(const McDom* __restrict__ G, int n) {
+  const int d = blockIdx.x * blockDim.x + threadIdx.x;
+  if (d >= n) return;
+  G[d].totals[0] = G[d].eoff[mcEdgeBlocks(G[d].g)];
+  G[d].totals[1] = G[d].coff[mcCellBlocks(G[d].g)];
+}
+__global__ void __launch_bounds__(kBlk) kMcBounds(const McDom* __restrict__ G, int nparts) {
+  boundsFinal(G[blockIdx.x].part, nparts, G[blockIdx.x].bounds);
 }
 
 // Per domain, the count pass leaves what the emission needs: sign bytes,
@@ -735,7 +774,7 @@ __global__ void kMcTotals(const uint32_t* vtotal, const uint32_t* ftotal, uint32
 // free HBM), they are kept for none and the emission recomputes them per
 // domain into scratch.
 constexpr size_t kMcKeepBudget = (size_t)16 << 30;
-constexpr int kCountStreams = 4;  // streams of the count pass over the domains
+constexpr int kMcBoundBlocks = 64;  // blocks per domain of the bounds pass, at most
 
 struct McSource : MeshSource {
   struct Parts {  // byte offsets of one domain's buffers
@@ -748,8 +787,12 @@ struct McSource : MeshSource {
   std::vector<Parts> parts;
   std::vector<long long> nv, nf;
   std::vector<float> bounds;  // 6 per domain: lo xyz, hi xyz
-  DevBuf& store;  // the context's generator store (kept between remeshes)
-  DevBuf table, ntri, part, dev_out;
+  DevBuf& store;  // the context's generator store (kept between remeshes): count
+                  // buffers, then (aux) tables, descriptors, scan jobs, partials
+  struct Aux {
+    size_t table, ntri, doms, ejobs, cjobs, esums, csums, part, out;
+  } aux;
+  size_t esum_b = 0, csum_b = 0;  // tile sums of one domain's scans
   McCorners ec;
   static long long edgeBlocks(const McGrid& g) { return (3 * g.E + kBlk - 1) / kBlk; }
   static long long cellBlocks(const McGrid& g) {
@@ -760,36 +803,63 @@ struct McSource : MeshSource {
     return Parts{al((size_t)g.N * g.N * g.N), al((size_t)edgeBlocks(g) * (kBlk / 64) * 8),
                  al((size_t)(edgeBlocks(g) + 1) * 4), al((size_t)(cellBlocks(g) + 1) * 4)};
   }
-  // sign bytes, cut bits and scanned block offsets of domain d; with bnd,
-  // also its vertex bounds (partials in bpart), and with tot its vertex and
-  // face totals.  sums: the scans' tile sums (scanSumsWords of the larger
-  // scan), or null for the calling thread's own buffer.
-  void count(const McGrid& g, const Parts& at, float* bnd, uint32_t* tot, hipStream_t s,
-             float* bpart = nullptr, uint32_t* sums = nullptr) {
-    uint8_t* sgn = store.as<uint8_t>() + at.sgn;
-    unsigned long long* bits = (unsigned long long*)(store.as<char>() + at.bits);
-    uint32_t* eoff = (uint32_t*)(store.as<char>() + at.eoff);
-    uint32_t* coff = (uint32_t*)(store.as<char>() + at.coff);
-    const long long np = (long long)g.N * g.N * g.N, ne = 3 * g.E, nc = (long long)g.n * g.n * g.n;
-    const long long eb = edgeBlocks(g), cb = cellBlocks(g);
-    kMcSign<<<gridOf(np, kBlk, kMcCellBlocks), kBlk, mcTabBytes(g), s>>>(g, sgn);
-    kMcEdgeBits<<<gridOf(ne, kBlk), kBlk, 0, s>>>(g, sgn, bits, eoff);
-    auto scan = [&](uint32_t* x, long long n) {
-      if (sums)
-        exclusiveScan(x, x, n, s, sums);
-      else
-        exclusiveScan(x, x, n, s);
-    };
-    scan(eoff, eb + 1);
-    if (bnd) {
-      float* bp = bpart ? bpart : part.as<float>();
-      const int vgrid = gridOf(eb * (kBlk / 64), kBlk, mcVertsCap(kBoundBlocks));
-      kMcVerts<<<vgrid, kBlk, mcTabBytes(g), s>>>(g, bits, eoff, 0u, nullptr, nullptr, bp);
-      kBoundsFinal<<<1, kBlk, 0, s>>>(bp, vgrid, bnd);
+  template <typename T>
+  T* at(size_t off) const {
+    return (T*)(store.as<char>() + off);
+  }
+  // Sign bytes, cut bits and scanned block offsets of domains [a, a + m);
+  // with `measure` also their vertex bounds and totals.
+  void count(int a, int m, bool measure, hipStream_t s) {
+    long long np = 0, ne = 0, nc = 0, eb = 0, cb = 0;
+    size_t tab = 0;
+    for (int d = a; d < a + m; ++d) {
+      const McGrid& g = grid[d];
+      np = std::max(np, (long long)g.N * g.N * g.N);
+      ne = std::max(ne, 3 * g.E);
+      nc = std::max(nc, (long long)g.n * g.n * g.n);
+      eb = std::max(eb, edgeBlocks(g));
+      cb = std::max(cb, cellBlocks(g));
+      tab = std::max(tab, mcTabBytes(g));
     }
-    kMcCellCount<<<gridOf(nc, kBlk), kBlk, 0, s>>>(g, sgn, ntri.as<uint8_t>(), coff);
-    scan(coff, cb + 1);
-    if (tot) kMcTotals<<<1, 1, 0, s>>>(eoff + eb, coff + cb, tot);
+    const McDom* G = at<McDom>(aux.doms) + a;
+    auto grid2 = [&](int x) { return dim3((unsigned)x, (unsigned)m); };
+    kMcSign<<<grid2(gridOf(np, kBlk, mcTabCap(m))), kBlk, tab, s>>>(G);
+    kMcEdgeBits<<<grid2(gridOf(ne, kBlk, mcFlatCap(m))), kBlk, 0, s>>>(G);
+    exclusiveScanMany(at<ScanJob>(aux.ejobs) + a, m, eb + 1, s);
+    if (measure) {
+      const int vgrid =
+          gridOf(eb * (kBlk / 64), kBlk, mcVertsCap(std::min<long long>(kMcBoundBlocks, mcTabCap(m))));
+      kMcVerts<false><<<grid2(vgrid), kBlk, tab, s>>>(G, 0u);
+      kMcBounds<<<m, kBlk, 0, s>>>(G, vgrid);
+    }
+    kMcCellCount<<<grid2(gridOf(nc, kBlk, mcFlatCap(m))), kBlk, 0, s>>>(G, at<uint8_t>(aux.ntri));
+    exclusiveScanMany(at<ScanJob>(aux.cjobs) + a, m, cb + 1, s);
+    if (measure) kMcTotals<<<(m + 255) / 256, 256, 0, s>>>(G, m);
+    SPRAY_HIP(hipGetLastError());
+  }
+  // Vertices, colours and faces of domains [a, a + m), whose descriptors hold
+  // their places.
+  void emit(int a, int m, hipStream_t s) {
+    long long nc = 0, eb = 0;
+    size_t tab = 0;
+    for (int d = a; d < a + m; ++d) {
+      const McGrid& g = grid[d];
+      nc = std::max(nc, (long long)g.n * g.n * g.n);
+      eb = std::max(eb, edgeBlocks(g));
+      tab = std::max(tab, mcTabBytes(g));
+    }
+    const McDom* G = at<McDom>(aux.doms) + a;
+    kMcVerts<true><<<dim3((unsigned)gridOf(eb * (kBlk / 64), kBlk, mcVertsCap(mcTabCap(m))),
+                          (unsigned)m),
+                     kBlk, tab, s>>>(G, p.rgb);
+    kMcCells<<<dim3((unsigned)gridOf(nc, kBlk, mcTabCap(m)), (unsigned)m), kBlk, 0, s>>>(
+        G, at<int8_t>(aux.table), at<uint8_t>(aux.ntri), ec);
+    SPRAY_HIP(hipGetLastError());
+  }
+  std::vector<McDom> hdoms;
+  void uploadDoms(hipStream_t s) {
+    SPRAY_HIP(hipMemcpyAsync(at<McDom>(aux.doms), hdoms.data(), hdoms.size() * sizeof(McDom),
+                             hipMemcpyHostToDevice, s));
   }
   McSource(Ctx* c, const spray_scenegen_params& prm) : p(prm), store(c->gen_store) {
     nd = p.nx * p.ny * p.nz;
@@ -824,19 +894,40 @@ struct McSource : MeshSource {
     size_t free_b = 0, total_b = 0;
     SPRAY_HIP(hipMemGetInfo(&free_b, &total_b));
     keep = total <= std::min(kMcKeepBudget, free_b / 4);
+    size_t need = 0;
     if (keep) {
-      size_t at = 0;
       for (int d = 0; d < nd; ++d) {
         const Parts z = sizes(grid[d]);
-        parts[d] = Parts{at, at + z.sgn, at + z.sgn + z.bits, at + z.sgn + z.bits + z.eoff};
-        at += z.sgn + z.bits + z.eoff + z.coff;
+        parts[d] = Parts{need, need + z.sgn, need + z.sgn + z.bits, need + z.sgn + z.bits + z.eoff};
+        need += z.sgn + z.bits + z.eoff + z.coff;
       }
-      store.reserve(at + 64);
     } else {  // one scratch set, sized for the largest domain
       const Parts one{0, mx.sgn, mx.sgn + mx.bits, mx.sgn + mx.bits + mx.eoff};
       for (int d = 0; d < nd; ++d) parts[d] = one;
-      store.reserve(mx.sgn + mx.bits + mx.eoff + mx.coff + 64);
+      need = mx.sgn + mx.bits + mx.eoff + mx.coff;
     }
+    long long eb = 0, cb = 0;
+    for (int d = 0; d < nd; ++d) {
+      eb = std::max(eb, edgeBlocks(grid[d]));
+      cb = std::max(cb, cellBlocks(grid[d]));
+    }
+    esum_b = align256((size_t)scanSumsWords(eb + 1) * 4);
+    csum_b = align256((size_t)scanSumsWords(cb + 1) * 4);
+    auto take = [&](size_t b) {
+      const size_t at = need;
+      need += align256(b);
+      return at;
+    };
+    aux.table = take(256 * 25);
+    aux.ntri = take(256);
+    aux.doms = take((size_t)nd * sizeof(McDom));
+    aux.ejobs = take((size_t)nd * sizeof(ScanJob));
+    aux.cjobs = take((size_t)nd * sizeof(ScanJob));
+    aux.esums = take((size_t)nd * esum_b);
+    aux.csums = take((size_t)nd * csum_b);
+    aux.part = take((size_t)nd * kMcBoundBlocks * 24);
+    aux.out = take((size_t)nd * 32);
+    store.reserve(need + 64);
     const int8_t* T = mcTriTable();
     uint8_t counts[256];
     for (int cs = 0; cs < 256; ++cs) {
@@ -845,43 +936,37 @@ struct McSource : MeshSource {
       counts[cs] = (uint8_t)(q / 3);
     }
     for (int e = 0; e < 12; ++e) mcEdgeCorner(e, &ec.dx[e], &ec.dy[e], &ec.dz[e], &ec.axis[e]);
-    table.reserve(256 * 25);
-    ntri.reserve(256);
-    part.reserve((size_t)kBoundBlocks * 6 * 4 + 64);
-    dev_out.reserve((size_t)nd * 8 * 4 + 64);
-    hipStream_t s = c->stream;
-    SPRAY_HIP(hipMemcpyAsync(table.p, T, 256 * 25, hipMemcpyHostToDevice, s));
-    SPRAY_HIP(hipMemcpyAsync(ntri.p, counts, 256, hipMemcpyHostToDevice, s));
-    // count pass: vertex and face totals and vertex bounds of every domain;
-    // with every domain's buffers kept, the domains run on up to
-    // kCountStreams streams (the context's among them), each with its own
-    // bound partials and scan tile sums
-    uint32_t* tot = dev_out.as<uint32_t>();
+    uint32_t* tot = at<uint32_t>(aux.out);
     float* bnd = (float*)(tot + 2 * (size_t)nd);
-    if (keep && nd > 1) {
-      const int K = std::min(pipelineCount(kCountStreams), nd);
-      long long scan_max = 0;
-      for (int d = 0; d < nd; ++d)
-        scan_max = std::max(scan_max, std::max(edgeBlocks(grid[d]), cellBlocks(grid[d])) + 1);
-      const size_t part_b = align256((size_t)kBoundBlocks * 6 * 4);
-      const size_t sums_b = align256((size_t)scanSumsWords(scan_max) * 4);
-      struct Per {  // per stream: bound partials, tile sums
-        DevBuf b;
-        ~Per() { b.release(); }
-      } pb;
-      DevBuf& per = pb.b;
-      per.reserve((part_b + sums_b) * K + 64);
-      {
-        StreamSet st(K - 1, s);  // stream 0 is s itself
-        for (int d = 0; d < nd; ++d) {
-          char* base = per.as<char>() + (part_b + sums_b) * (d % K);
-          count(grid[d], parts[d], bnd + 6 * d, tot + 2 * d, d % K ? st[d % K - 1] : s,
-                (float*)base, (uint32_t*)(base + part_b));
-        }
-        st.join(s);
-      }
+    hdoms.resize(nd);
+    std::vector<ScanJob> jobs(2 * (size_t)nd);
+    for (int d = 0; d < nd; ++d) {
+      McDom& D = hdoms[d];
+      D.g = grid[d];
+      D.sgn = at<uint8_t>(parts[d].sgn);
+      D.bits = at<unsigned long long>(parts[d].bits);
+      D.eoff = at<uint32_t>(parts[d].eoff);
+      D.coff = at<uint32_t>(parts[d].coff);
+      D.part = at<float>(aux.part) + (size_t)d * kMcBoundBlocks * 6;
+      D.bounds = bnd + 6 * (size_t)d;
+      D.totals = tot + 2 * (size_t)d;
+      D.v = nullptr;
+      D.rgb = D.f = nullptr;
+      jobs[d] = ScanJob{D.eoff, D.eoff, at<uint32_t>(aux.esums + (size_t)d * esum_b), edgeBlocks(grid[d]) + 1};
+      jobs[nd + d] = ScanJob{D.coff, D.coff, at<uint32_t>(aux.csums + (size_t)d * csum_b), cellBlocks(grid[d]) + 1};
+    }
+    hipStream_t s = c->stream;
+    SPRAY_HIP(hipMemcpyAsync(at<int8_t>(aux.table), T, 256 * 25, hipMemcpyHostToDevice, s));
+    SPRAY_HIP(hipMemcpyAsync(at<uint8_t>(aux.ntri), counts, 256, hipMemcpyHostToDevice, s));
+    SPRAY_HIP(hipMemcpyAsync(at<ScanJob>(aux.ejobs), jobs.data(), (size_t)nd * sizeof(ScanJob), hipMemcpyHostToDevice, s));
+    SPRAY_HIP(hipMemcpyAsync(at<ScanJob>(aux.cjobs), jobs.data() + nd, (size_t)nd * sizeof(ScanJob), hipMemcpyHostToDevice, s));
+    uploadDoms(s);
+    // count pass: vertex and face totals and vertex bounds of every domain,
+    // all domains in each launch when every domain's buffers are kept
+    if (keep) {
+      count(0, nd, true, s);
     } else {
-      for (int d = 0; d < nd; ++d) count(grid[d], parts[d], bnd + 6 * d, tot + 2 * d, s);
+      for (int d = 0; d < nd; ++d) count(d, 1, true, s);
     }
     SPRAY_HIP(hipGetLastError());
     std::vector<uint32_t> h((size_t)nd * 2);
@@ -896,30 +981,30 @@ struct McSource : MeshSource {
       nf[d] = h[2 * d + 1];
     }
   }
-  ~McSource() override {
-    for (DevBuf* b : {&table, &ntri, &part, &dev_out}) b->release();
-  }
   long long numVerts(int d) const override { return nv[d]; }
   long long numFaces(int d) const override { return nf[d]; }
-  // with every domain's count buffers kept, a fill reads only its own
-  bool pipelined() const override { return keep; }
   bool rebuilds() const override { return true; }
+  bool fillAll(Ctx* c, const std::vector<DomainDesc>& desc, float* v, uint32_t* f, uint32_t* rgb,
+               hipStream_t s) override {
+    (void)c;
+    if (!keep) return false;
+    for (int d = 0; d < nd; ++d) {
+      hdoms[d].v = v + desc[d].vtx_off * 3;
+      hdoms[d].rgb = rgb + desc[d].vtx_off;
+      hdoms[d].f = f + desc[d].face_off * 3;
+    }
+    uploadDoms(s);
+    emit(0, nd, s);
+    return true;
+  }
   void fill(Ctx* c, int d, float* v, uint32_t* f, uint32_t* rgb, hipStream_t s) override {
     (void)c;
-    const McGrid& g = grid[d];
-    const Parts& at = parts[d];
-    if (!keep) count(g, at, nullptr, nullptr, s);
-    const uint8_t* sgn = store.as<uint8_t>() + at.sgn;
-    const unsigned long long* bits = (const unsigned long long*)(store.as<char>() + at.bits);
-    const uint32_t* eoff = (const uint32_t*)(store.as<char>() + at.eoff);
-    const uint32_t* coff = (const uint32_t*)(store.as<char>() + at.coff);
-    const long long ne = 3 * g.E, nc = (long long)g.n * g.n * g.n;
-    kMcVerts<<<gridOf(edgeBlocks(g) * (kBlk / 64), kBlk, mcVertsCap(65535)), kBlk, mcTabBytes(g), s>>>(
-        g, bits, eoff, p.rgb, v, rgb, nullptr);
-    kMcCells<<<gridOf(nc, kBlk, kMcCellBlocks), kBlk, 0, s>>>(g, sgn, table.as<int8_t>(),
-                                                             ntri.as<uint8_t>(), ec, bits, eoff,
-                                                             coff, f);
-    SPRAY_HIP(hipGetLastError());
+    hdoms[d].v = v;
+    hdoms[d].rgb = rgb;
+    hdoms[d].f = f;
+    SPRAY_HIP(hipMemcpyAsync(at<McDom>(aux.doms) + d, &hdoms[d], sizeof(McDom), hipMemcpyHostToDevice, s));
+    if (!keep) count(d, 1, false, s);
+    emit(d, 1, s);
   }
 };
 
