@@ -32,10 +32,6 @@ namespace spray {
 // array G each (blockIdx.x and gridDim.x count that domain's blocks): a
 // domain alone is a launch of a few microseconds that fills a fraction of the
 // GPU, and 47 of them per domain were bound by issuing them.
-struct FrontierItem {
-  int bnode;  // binary inner node
-  int wnode;  // 8-wide node slot
-};
 struct BuildDom {
   const float* vtx;
   const uint32_t *face, *rgb;
@@ -46,10 +42,11 @@ struct BuildDom {
   // scratch: vertex adjacency, centroid bounds, sort buffers, leaf-range unions
   uint32_t *cnt, *cur, *off, *adj, *bmm, *keys[2], *vals[2], *hist;
   float *rpre, *rsuf, *rtab;
-  // binary tree: leaf and inner boxes, children, leaf ranges
+  // binary tree: leaf and inner boxes; per inner node its children (left,
+  // right: c >= 0 inner, c < 0 leaf ~c) and leaf range (first, last)
   float *leafbox, *innerbox;
-  int *left, *right, *first, *last;
-  FrontierItem* front[2];  // collapse frontiers
+  int4* tree;
+  int* front[2];           // collapse frontiers: binary inner nodes
   int* cc;                 // level counters (kLevelWords)
   int nf, nv, node_cap;
 };
@@ -329,10 +326,7 @@ __global__ void kKarras(const BuildDom* __restrict__ G) {
     int lo = i < j ? i : j, hi = i < j ? j : i;
     int lc = (lo == gamma) ? ~gamma : gamma;
     int rc = (hi == gamma + 1) ? ~(gamma + 1) : gamma + 1;
-    B.left[i] = lc;
-    B.right[i] = rc;
-    B.first[i] = lo;
-    B.last[i] = hi;
+    B.tree[i] = make_int4(lc, rc, lo, hi);
   }
 }
 
@@ -470,13 +464,13 @@ __global__ void kRangeLevel2(const BuildDom* __restrict__ G, int j) {
 __global__ void kRangeBoxes(const BuildDom* __restrict__ G) {
   const BuildDom& B = G[blockIdx.y];
   const int ninner = B.nf - 1;
-  const int *__restrict__ first = B.first, *__restrict__ last = B.last;
+  const int4* __restrict__ tree = B.tree;
   const float *__restrict__ leafbox = B.leafbox, *__restrict__ pre = B.rpre, *__restrict__ suf = B.rsuf,
               *__restrict__ table = B.rtab;
   float* __restrict__ innerbox = B.innerbox;
   const long long nblk = rangeBlocks(B.nf);
   for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < ninner; p += gridDim.x * blockDim.x) {
-    const int a = first[p], b = last[p];
+    const int a = tree[p].z, b = tree[p].w;
     const int ba = a / kRangeBlock, bb = b / kRangeBlock;
     float lo[3] = {kInfF, kInfF, kInfF}, hi[3] = {-kInfF, -kInfF, -kInfF};
     if (ba == bb) {
@@ -512,8 +506,8 @@ __host__ __device__ inline long long nodeCap(long long nf) {
 static_assert((1 << 24) / 7 + (6ll * (1 << 24)) / (7 * (kLeafMax + 1)) + 16 < (1 << 23), "node numbers");
 
 // 8-wide collapse levels launched per host wait, and at most (deeper trees
-// do not fit the traversal stack anyway); a level counter block is the node
-// counter, the overflow flag and the item count of every level
+// do not fit the traversal stack anyway); a level counter block is an unused
+// word, the overflow flag and the item count of every level
 constexpr int kLevelBatch = 16;
 constexpr int kMaxLevels = 48;
 constexpr int kLevelWords = 2 + kMaxLevels + 1;
@@ -523,269 +517,287 @@ __device__ __forceinline__ float boxArea(const float* b) {
   return dx * dy + dy * dz + dz * dx;
 }
 
-// Writes a node's grid and child planes from the boxes (lo xyz, hi xyz) of
-// its children: child i < nc goes to slot slot(i) (4 bits each in slots).  Per
+// Reductions over the 8 lanes of a group (lanes 8i .. 8i + 7), the result in
+// every lane: exchanges within pairs, pairs of pairs, and both quads.
+template <int kCtl>
+__device__ __forceinline__ uint32_t dpp8u(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, kCtl, 0xf, 0xf, true);
+}
+template <int kCtl>
+__device__ __forceinline__ float dpp8(float v) {
+  return __uint_as_float(dpp8u<kCtl>(__float_as_uint(v)));
+}
+__device__ __forceinline__ float groupMin(float v) {
+  v = fminf(v, dpp8<0xB1>(v));
+  v = fminf(v, dpp8<0x4E>(v));
+  return fminf(v, dpp8<0x141>(v));
+}
+__device__ __forceinline__ float groupMax(float v) {
+  v = fmaxf(v, dpp8<0xB1>(v));
+  v = fmaxf(v, dpp8<0x4E>(v));
+  return fmaxf(v, dpp8<0x141>(v));
+}
+// the lanes of the group with p set, bit i for its lane i
+__device__ __forceinline__ uint32_t groupBallot(bool p) {
+  return (uint32_t)(__ballot(p) >> (threadIdx.x & 56)) & 255u;
+}
+
+// Writes a node's grid and child planes; called by the 8 lanes of a group,
+// each with the box (lo xyz, hi xyz) and slot of one child (used), the other
+// lanes with a slot of their own among those left.  Per
 // axis the step is the power of two that covers the children's extent in at
 // most 253 steps (at least 2^-20 of the largest coordinate, so that base's
 // rounding stays below an eighth of a step), base lies 1/64 of a step or more
 // below the lowest plane, and planes are rounded outwards with 2^-9 of a step
 // to spare: the distance test's cancellation error (nodeBoxes) is below 2^-15
 // of a step.  An axis whose extent is not finite, or would need a step of
-// 2^62 or more, covers everything.  Returns the exponent bytes of meta.
-__device__ __forceinline__ uint32_t quantizeNode(const float (&b)[8][6], int nc, uint32_t slots,
-                                                 BNode8* nd) {
+// 2^62 or more, covers everything.  Lane k of the group works out axis k's
+// grid.  Returns the exponent bytes of meta.
+__device__ __forceinline__ uint32_t quantizeNode(const float (&b)[6], bool used, uint32_t slot, BNode8* nd) {
+  const int me = threadIdx.x & 7;
+  float lo = 0.f, hi = 0.f;
+  bool finite = false;
+  const bool any = groupBallot(used) != 0u;
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    const float l = groupMin(used ? b[k] : kInfF), h = groupMax(used ? b[3 + k] : -kInfF);
+    const bool f = groupBallot(used && !(fabsf(b[k]) < kInfF && fabsf(b[3 + k]) < kInfF)) == 0u;
+    if (me == k) {
+      lo = l;
+      hi = h;
+      finite = any && f;
+    }
+  }
+  auto exponent = [](double x) { return (int)((__double2hiint(x) >> 20) & 2047) - 1023; };
+  auto power = [](int x) { return __hiloint2double((x + 1023) << 20, 0); };
+  const double ext = (double)hi - (double)lo;  // (of floats: no subnormal double)
+  const double big = fmax(fabs((double)lo), fabs((double)hi));
+  int e = -126;
+  if (finite) {
+    // smallest e with 253 * 2^e >= ext and 2^e >= big * 2^-20
+    if (ext > 0.0) {
+      e = max(e, exponent(ext) - 7);
+      if (253.0 * power(e) < ext) ++e;
+    }
+    if (big > 0.0) e = max(e, exponent(big) - 19);
+  }
+  const bool all = !finite || e >= 62;
+  float base = -3.0e38f;
+  if (all) {
+    e = 121;
+  } else {
+    const double bd = (double)lo - power(e) * 0.015625;
+    base = (float)bd;
+    if ((double)base > bd) base = nextafterf(base, -kInfF);
+  }
+  if (me < 3) nd->base[me] = base;
   uint32_t meta = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    float lo = kInfF, hi = -kInfF;
-    bool finite = nc > 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < nc) {
-        lo = fminf(lo, b[i][k]);
-        hi = fmaxf(hi, b[i][3 + k]);
-        finite = finite && fabsf(b[i][k]) < kInfF && fabsf(b[i][3 + k]) < kInfF;
-      }
-    const double ext = (double)hi - (double)lo;
-    const double big = fmax(fabs((double)lo), fabs((double)hi));
-    int e = -126;
-    if (finite) {
-      // smallest e with 253 * 2^e >= ext and 2^e >= big * 2^-20
-      if (ext > 0.0) {
-        e = max(e, ilogb(ext / 253.0));
-        if (ldexp(253.0, e) < ext) ++e;
-      }
-      if (big > 0.0) e = max(e, ilogb(big) - 19);
+    const int ek = __shfl(e, k, 8);
+    const double bk = (double)__shfl(base, k, 8), inv = power(-ek);
+    const bool allk = ek == 121;
+    uint32_t l = 255u, h = 0u;  // unused slots: inverted
+    if (used) {
+      l = allk ? 0u : (uint32_t)fmin(fmax(floor(((double)b[k] - bk) * inv - 0.001953125), 0.0), 255.0);
+      h = allk ? 255u : (uint32_t)fmin(fmax(ceil(((double)b[3 + k] - bk) * inv + 0.001953125), 0.0), 255.0);
     }
-    const bool all = !finite || e >= 62;
-    const double inv = ldexp(1.0, all ? 0 : -e);
-    float base = -3.0e38f;
-    if (all) {
-      e = 121;
-    } else {
-      const double bd = (double)lo - ldexp(1.0, e) * 0.015625;
-      base = (float)bd;
-      if ((double)base > bd) base = nextafterf(base, -kInfF);
-    }
-    unsigned long long ql = ~0ull, qh = 0ull;  // unused slots: inverted
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < nc) {
-        uint32_t l = 0u, h = 255u;
-        if (!all) {
-          l = (uint32_t)fmin(fmax(floor(((double)b[i][k] - (double)base) * inv - 0.001953125), 0.0), 255.0);
-          h = (uint32_t)fmin(fmax(ceil(((double)b[i][3 + k] - (double)base) * inv + 0.001953125), 0.0), 255.0);
-        }
-        const int sh = 8 * (int)((slots >> (4 * i)) & 7u);
-        ql = (ql & ~(255ull << sh)) | ((unsigned long long)l << sh);
-        qh |= (unsigned long long)h << sh;
-      }
-    nd->base[k] = base;
-    unsigned long long* w = (unsigned long long*)nd->plane[k];
-    w[0] = ql;
-    w[1] = qh;
-    meta |= (uint32_t)(e + 127) << (8 * k);
+    nd->plane[k][slot] = (uint8_t)l;
+    nd->plane[k][8 + slot] = (uint8_t)h;
+    meta |= (uint32_t)(ek + 127) << (8 * k);
   }
   return meta;
 }
 
-// Slots of a node's nc children, 4 bits each: greedily the (child, slot) pair
-// whose child centre lies farthest to the slot's side of the node (bit k of
-// the slot: the upper side of axis k).
-__device__ __forceinline__ uint32_t assignSlots(const float (&b)[8][6], int nc) {
-  float d[8][3];
+// Slot of each lane's child (one child per used lane of the group; the other
+// lanes get the slots left): greedily the (child, slot) pair whose child
+// centre lies farthest to the slot's side of the node (bit k of the slot: the
+// upper side of axis k).  Distances are compared as ordered integers with the
+// pair in their last six bits, so that one maximum over a lane's slots and
+// the group's lanes names the pair; a distance that is not a number comes
+// last.
+__device__ __forceinline__ uint32_t assignSlot(const float (&b)[6], bool used) {
+  const uint32_t me = threadIdx.x & 7;
+  float d[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    float lo = kInfF, hi = -kInfF;
+    const float lo = groupMin(used ? b[k] : kInfF), hi = groupMax(used ? b[3 + k] : -kInfF);
+    d[k] = (b[k] + b[3 + k]) - (lo + hi);
+  }
+  uint32_t key[8];  // > 0 while the slot is free
 #pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < nc) {
-        lo = fminf(lo, b[i][k]);
-        hi = fmaxf(hi, b[i][3 + k]);
+  for (int s = 0; s < 8; ++s) {
+    const float t = ((s & 1) ? d[0] : -d[0]) + ((s & 2) ? d[1] : -d[1]) + ((s & 4) ? d[2] : -d[2]);
+    const uint32_t u = __float_as_uint(t == t ? t : -kInfF);
+    key[s] = ((u ^ ((u >> 31) ? 0xffffffffu : 0x80000000u)) & ~63u) | ((7u - me) << 3) | (7u - s);
+  }
+  uint32_t slot = 0, frees = 255u;
+  bool open = used;
+#pragma unroll
+  for (int n = 0; n < 8; ++n) {
+    uint32_t top = 0;
+#pragma unroll
+    for (int s = 0; s < 8; ++s) top = max(top, key[s]);
+    top = open ? top : 0u;
+    top = max(top, dpp8u<0xB1>(top));
+    top = max(top, dpp8u<0x4E>(top));
+    top = max(top, dpp8u<0x141>(top));
+    if (top != 0u) {  // (0: no child left)
+      const uint32_t bs = 7u - (top & 7u);
+      if (me == 7u - ((top >> 3) & 7u)) {
+        slot = bs;
+        open = false;
       }
+      frees &= ~(1u << bs);
 #pragma unroll
-    for (int i = 0; i < 8; ++i) d[i][k] = (b[i][k] + b[i][3 + k]) - (lo + hi);
+      for (int s = 0; s < 8; ++s) key[s] = bs == (uint32_t)s ? 0u : key[s];
+    }
   }
-  uint32_t slots = 0, freec = nc >= 8 ? 255u : (1u << nc) - 1u, frees = 255u;
-  while (freec) {
-    // a pair exists even where every comparison is false (boxes that are not numbers)
-    float best = -kInfF;
-    uint32_t bi = (uint32_t)__ffs((int)freec) - 1u, bs = (uint32_t)__ffs((int)frees) - 1u;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if ((freec >> i) & 1u) {
-#pragma unroll
-        for (int s = 0; s < 8; ++s) {
-          const float v = ((s & 1) ? d[i][0] : -d[i][0]) + ((s & 2) ? d[i][1] : -d[i][1]) +
-                          ((s & 4) ? d[i][2] : -d[i][2]);
-          if (((frees >> s) & 1u) && v > best) {
-            best = v;
-            bi = i;
-            bs = s;
-          }
-        }
-      }
-    slots |= bs << (4 * bi);
-    freec &= ~(1u << bi);
-    frees &= ~(1u << bs);
+  const uint32_t taken = groupBallot(used);  // (of all the group's lanes)
+  if (!used) {  // the r-th unused lane takes the r-th free slot
+    int r = __popc(~taken & ((1u << me) - 1u));
+    for (; r > 0; --r) frees &= frees - 1u;
+    slot = (uint32_t)__ffs((int)frees) - 1u;
   }
-  return slots;
-}
-
-// Takes cnt consecutive entries of *ctr per lane, in lane order, with one
-// atomic per wave; every lane of the wave calls it (cnt may be 0).
-__device__ __forceinline__ int waveAlloc(int* ctr, int cnt) {
-  const int lane = threadIdx.x & 63;
-  int incl = cnt;
-  for (int o = 1; o < 64; o <<= 1) {
-    const int v = __shfl_up(incl, o, 64);
-    if (lane >= o) incl += v;
-  }
-  const int total = __shfl(incl, 63, 64);
-  int base = 0;
-  if (lane == 63 && total > 0) base = atomicAdd(ctr, total);
-  base = __shfl(base, 63, 64);
-  return base + incl - cnt;
+  return slot;
 }
 
 // One frontier level l of every domain of the launch: cc[2 + l] items (0:
-// nothing to do), the next level's counted in cc[3 + l]; cc[0] counts nodes,
-// cc[1] is the overflow flag.  Launched level after level without host round
-// trips; the loop bound is uniform per block so whole waves allocate.
+// nothing to do), the next level's counted in cc[3 + l]; cc[1] is the
+// overflow flag.  A level's items are its nodes, numbered after those of the
+// levels above.  Launched level after level without host round trips; the
+// loop bound is uniform per block.
+//
+// Eight lanes take an item, one per child: a lane holds its child's box and
+// record, so that opening the largest inner child is one round of loads by
+// the two lanes that get its children, and the node leaves through LDS as one
+// line.  Bound by vector issue (about 1570 instructions per wave of 8 items,
+// 55% of the time) and the chain of six rounds of loads.  One lane per item,
+// all eight boxes in its registers, spilled at 128 registers, took an eighth
+// of the waves and read left, right, first and last of each child from four
+// arrays: the collapse launches of a remesh of 128 domains (8 x 4 x 4, field
+// resolution 72) took 5.8 ms, now 3.4 ms.
 __global__ void __launch_bounds__(256) kCollapseLevel(const BuildDom* __restrict__ G, int l) {
+  __shared__ BNode8 img[32];
+  __shared__ int alloc[32];
   const BuildDom& B = G[blockIdx.y];
-  const FrontierItem* __restrict__ fin = B.front[l & 1];
-  FrontierItem* fout = B.front[(l & 1) ^ 1];
-  const int *nin_ptr = B.cc + 2 + l, node_cap = B.node_cap;
-  int *nout = B.cc + 3 + l, *node_counter = B.cc, *overflow = B.cc + 1;
-  const int *__restrict__ left = B.left, *__restrict__ right = B.right, *__restrict__ first = B.first,
-            *__restrict__ last = B.last;
+  const int nin = B.cc[2 + l];
+  const int over = B.cc[1];  // 1 + the level that overflowed (its blocks all finish)
+  if (nin <= (int)(blockIdx.x * 32) || (over != 0 && over <= l)) return;
+  int start = 0;  // nodes of the levels above
+  for (int j = 0; j < l; ++j) start += B.cc[2 + j];
+  const int* __restrict__ fin = B.front[l & 1];
+  int* fout = B.front[(l & 1) ^ 1];
+  const int4* __restrict__ tree = B.tree;
   const float *__restrict__ leafbox = B.leafbox, *__restrict__ innerbox = B.innerbox;
-  BNode8* nodes = B.nodes;
-  const int nin = *nin_ptr;
-  for (int base = blockIdx.x * blockDim.x; base < nin; base += gridDim.x * blockDim.x) {
-    const int it = base + threadIdx.x;
+  const int me = threadIdx.x & 7, grp = threadIdx.x >> 3;
+  for (int base = blockIdx.x * 32; base < nin; base += gridDim.x * 32) {
+    const int it = base + grp;
     const bool act = it < nin;
-    FrontierItem f{0, 0};
-    int ch[8] = {0, 0, 0, 0, 0, 0, 0, 0};
-    float area[8] = {-1.f, -1.f, -1.f, -1.f, -1.f, -1.f, -1.f, -1.f};  // < 0: a leaf, or unused
-    int nc = 0;
-    auto count = [&](int c) { return c < 0 ? 1 : last[c] - first[c] + 1; };
-    auto openArea = [&](int c) {
-      return c >= 0 && count(c) > kLeafMax ? boxArea(innerbox + (size_t)c * 6) : -1.f;
+    int c = 0;               // this lane's child, its record, box and area when it can be opened
+    int4 rec{0, 0, 0, 0};
+    float b[6] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    float area = -1.f;
+    auto load = [&] {
+      const float2* src = (const float2*)(c < 0 ? leafbox + (size_t)(~c) * 6 : innerbox + (size_t)c * 6);
+      rec = c < 0 ? make_int4(0, 0, ~c, ~c) : tree[c];
+      const float2 x = src[0], y = src[1], z = src[2];
+      b[0] = x.x, b[1] = x.y, b[2] = y.x, b[3] = y.y, b[4] = z.x, b[5] = z.y;
+      area = rec.w - rec.z + 1 > kLeafMax ? boxArea(b) : -1.f;
     };
-    float b[8][6];
-    uint32_t slots = 0, im = 0;
-    int ninner = 0;
+    int nc = 0;
     if (act) {
-      f = fin[it];
+      const int4 root = tree[fin[it]];
       nc = 2;
-      ch[0] = left[f.bnode];
-      ch[1] = right[f.bnode];
-      area[0] = openArea(ch[0]);
-      area[1] = openArea(ch[1]);
-      while (nc < 8) {  // open the inner child of the largest area
-        int best = -1, c = 0;
-        float barea = -1.f;
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-          if (area[i] > barea) {
-            barea = area[i];
-            best = i;
-            c = ch[i];
-          }
-        if (best < 0) break;
-        const int l = left[c], r = right[c];
-        const float al = openArea(l), ar = openArea(r);
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-          if (i == best) {
-            ch[i] = l;
-            area[i] = al;
-          }
-          if (i == nc) {
-            ch[i] = r;
-            area[i] = ar;
-          }
-        }
-        ++nc;
+      if (me < 2) {
+        c = me == 0 ? root.x : root.y;
+        load();
       }
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        if (i < nc) {
-          const float* src = ch[i] < 0 ? leafbox + (size_t)(~ch[i]) * 6 : innerbox + (size_t)ch[i] * 6;
-          for (int k = 0; k < 6; ++k) b[i][k] = src[k];
-        } else {
-          for (int k = 0; k < 6; ++k) b[i][k] = 0.f;
-        }
-      }
-      slots = assignSlots(b, nc);
-#pragma unroll
-      for (int i = 0; i < 8; ++i)
-        if (i < nc && ch[i] >= 0 && count(ch[i]) > kLeafMax) im |= 1u << ((slots >> (4 * i)) & 7u);
-      ninner = __popc(im);
     }
-    // the inner children of a node take consecutive indices
-    const int cbase = waveAlloc(node_counter, ninner);
-    if (ninner > 0 && cbase + ninner > node_cap) {
-      atomicExch(overflow, 1);
-      ninner = 0;
-      im = 0;  // capacity exceeded (reported through overflow)
-    }
-    const int q = waveAlloc(nout, ninner);
-    if (!act) continue;
-    BNode8* nd = nodes + f.wnode;
-    const uint32_t meta = quantizeNode(b, nc, slots, nd);
-    nd->child_base = (uint32_t)cbase;
-    nd->meta = meta | (im << 24);
-    for (int i = 0; i < 7; ++i) nd->pad[i] = 0;
-    uint32_t used = 0;
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-      if (i < nc) {
-        const uint32_t s = (slots >> (4 * i)) & 7u;
-        const int c = ch[i];
-        uint32_t word = 0;
-        if ((im >> s) & 1u) {
-          const int rank = __popc(im & ((1u << s) - 1u));
-          fout[q + rank] = FrontierItem{c, cbase + rank};
-        } else if (c < 0) {
-          word = (1u << 24) | (uint32_t)(~c);
-        } else if (count(c) <= kLeafMax) {
-          word = ((uint32_t)count(c) << 24) | (uint32_t)first[c];
-        }
-        nd->leaf[s] = word;
-        used |= 1u << s;
+    // open the inner child of the largest area, the first such; its lane
+    // takes the left child and the next free lane the right one
+    for (int n = 0; n < 6; ++n) {
+      const float top = groupMax(area);
+      const bool go = top > -1.f;
+      if (__ballot(go) == 0ull) break;
+      const int best = __ffs((int)groupBallot(area == top)) - 1;
+      const int lc = __shfl(rec.x, best, 8), rc = __shfl(rec.y, best, 8);
+      if (go && (me == best || me == nc)) {
+        c = me == best ? lc : rc;
+        load();
       }
-    for (uint32_t m = ~used & 255u; m != 0u; m &= m - 1u) nd->leaf[__ffs((int)m) - 1] = 0u;
+      nc += go ? 1 : 0;
+    }
+    const bool used = me < nc;
+    const int cnt = rec.w - rec.z + 1;
+    const bool inner = used && cnt > kLeafMax;
+    const uint32_t slot = assignSlot(b, used);
+    // children of a node that are inner nodes take consecutive numbers in slot order
+    uint32_t im = inner ? 1u << slot : 0u;
+    for (int o = 1; o < 8; o <<= 1) im |= (uint32_t)__shfl_xor((int)im, o, 8);
+    if (me == 0) alloc[grp] = __popc(im);
+    __syncthreads();
+    if (threadIdx.x < 64) {
+      const int lane = threadIdx.x;
+      const int own = lane < 32 ? alloc[lane] : 0;
+      int incl = own;
+      for (int o = 1; o < 32; o <<= 1) {
+        const int v = __shfl_up(incl, o, 64);
+        if (lane >= o) incl += v;
+      }
+      const int total = __shfl(incl, 31, 64);
+      int first = 0;
+      if (lane == 0 && total > 0) first = atomicAdd(&B.cc[3 + l], total);
+      first = __shfl(first, 0, 64);
+      if (lane < 32) alloc[lane] = first + incl - own;
+    }
+    __syncthreads();
+    const int q = alloc[grp], cbase = start + nin + q;
+    const bool fits = cbase + __popc(im) <= B.node_cap;
+    if (!fits && me == 0) atomicExch(&B.cc[1], l + 1);  // the levels below return at once
+    BNode8* nd = &img[grp];
+    const uint32_t meta = quantizeNode(b, used, slot, nd);
+    if (me == 0) {
+      nd->child_base = (uint32_t)cbase;
+      nd->meta = meta | (im << 24);
+    }
+    if (me < 7) nd->pad[me] = 0u;
+    nd->leaf[slot] = used && !inner ? ((uint32_t)cnt << 24) | (uint32_t)rec.z : 0u;
+    if (inner && fits) fout[q + __popc(im & ((1u << slot) - 1u))] = c;
+    __syncthreads();
+    if (act) ((float4*)(B.nodes + start + it))[me] = ((const float4*)nd)[me];
+    __syncthreads();
   }
 }
 
-// Collapse state of each domain: node counter 1 (the 8-wide root), no
-// overflow, one frontier item (binary node `root`) at level 0 (none for a
-// domain of one leaf, whose root kTinyRoot writes), empty later levels.
+// Collapse state of each domain: no overflow, one frontier item (binary node
+// `root`) at level 0 (none for a domain of one leaf, whose root kTinyRoot
+// writes), empty later levels.
 __global__ void kCollapseInit(const BuildDom* __restrict__ G, int root) {
   const BuildDom& B = G[blockIdx.y];
   for (int i = threadIdx.x; i < kLevelWords; i += blockDim.x)
-    B.cc[i] = i == 0 || (i == 2 && B.nf > kLeafMax) ? 1 : 0;
-  if (threadIdx.x == 0) B.front[0][0] = FrontierItem{root, 0};
+    B.cc[i] = i == 2 && B.nf > kLeafMax ? 1 : 0;
+  if (threadIdx.x == 0) B.front[0][0] = root;
 }
 
-// Root for tiny domains (<= kLeafMax triangles): one leaf child.
+// Root for tiny domains (<= kLeafMax triangles): one leaf child.  One group.
 __global__ void kTinyRoot(const BuildDom* __restrict__ G) {
-  const int nf = G->nf;
+  const int nf = G->nf, me = threadIdx.x;
   const float* leafbox = G->leafbox;
-  BNode8* nodes = G->nodes;
-  float b[8][6] = {{kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF}};
+  BNode8* nd = G->nodes;
+  float b[6] = {kInfF, kInfF, kInfF, -kInfF, -kInfF, -kInfF};
   for (int i = 0; i < nf; ++i)
     for (int k = 0; k < 3; ++k) {
-      b[0][k] = fminf(b[0][k], leafbox[i * 6 + k]);
-      b[0][3 + k] = fmaxf(b[0][3 + k], leafbox[i * 6 + 3 + k]);
+      b[k] = fminf(b[k], leafbox[i * 6 + k]);
+      b[3 + k] = fmaxf(b[3 + k], leafbox[i * 6 + 3 + k]);
     }
-  nodes->meta = quantizeNode(b, nf > 0 ? 1 : 0, 0u, nodes);
-  nodes->child_base = 0;
-  for (int i = 0; i < 7; ++i) nodes->pad[i] = 0;
-  for (int i = 0; i < 8; ++i) nodes->leaf[i] = i == 0 ? (uint32_t)nf << 24 : 0u;
+  const uint32_t meta = quantizeNode(b, me == 0 && nf > 0, (uint32_t)me, nd);
+  if (me == 0) {
+    nd->meta = meta;
+    nd->child_base = 0;
+  }
+  if (me < 7) nd->pad[me] = 0;
+  nd->leaf[me] = me == 0 ? (uint32_t)nf << 24 : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -875,7 +887,7 @@ __global__ void kPlocFlags(const int* __restrict__ nn, int n, uint32_t* mflag, u
 __global__ void kPlocMerge(const int* __restrict__ nn, int n, const int* __restrict__ cid,
                            const float* __restrict__ cbox, const uint32_t* __restrict__ mpos,
                            const uint32_t* __restrict__ kpos, int node_base, int* cid2,
-                           float* cbox2, int* left, int* right, float* innerbox, int* icount) {
+                           float* cbox2, int4* tree, float* innerbox, int* icount) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
     int j = nn[i];
     bool mutual = nn[j] == i;
@@ -884,8 +896,8 @@ __global__ void kPlocMerge(const int* __restrict__ nn, int n, const int* __restr
     if (mutual) {
       int id = node_base + (int)mpos[i];
       int a = cid[i], b = cid[j];
-      left[id] = a;
-      right[id] = b;
+      tree[id].x = a;
+      tree[id].y = b;
       icount[id] = (a < 0 ? 1 : icount[a]) + (b < 0 ? 1 : icount[b]);
       for (int k = 0; k < 3; ++k) {
         float l = fminf(cbox[(size_t)i * 6 + k], cbox[(size_t)j * 6 + k]);
@@ -907,26 +919,26 @@ __global__ void kPlocMerge(const int* __restrict__ nn, int n, const int* __restr
 // parents come from later passes and are already placed).  Leaf children are
 // renumbered to their depth-first position q, and perm[q] keeps the Morton
 // position they came from.
-__global__ void kPlocRanges(int id_lo, int id_hi, int* left, int* right,
-                            const int* __restrict__ icount, int* first, int* last, uint32_t* perm) {
+__global__ void kPlocRanges(int id_lo, int id_hi, int4* tree, const int* __restrict__ icount,
+                            uint32_t* perm) {
   for (int id = id_lo + blockIdx.x * blockDim.x + threadIdx.x; id < id_hi;
        id += gridDim.x * blockDim.x) {
-    int f = first[id];
-    int a = left[id], b = right[id];
+    int f = tree[id].z;
+    int a = tree[id].x, b = tree[id].y;
     int fb = f + (a < 0 ? 1 : icount[a]);
     if (a < 0) {
       perm[f] = (uint32_t)(~a);
-      left[id] = ~f;
+      tree[id].x = ~f;
     } else {
-      first[a] = f;
+      tree[a].z = f;
     }
     if (b < 0) {
       perm[fb] = (uint32_t)(~b);
-      right[id] = ~fb;
+      tree[id].y = ~fb;
     } else {
-      first[b] = fb;
+      tree[b].z = fb;
     }
-    last[id] = f + icount[id] - 1;
+    tree[id].w = f + icount[id] - 1;
   }
 }
 
@@ -947,7 +959,7 @@ static int gridFor(long long n, int block) {
 // One domain's build scratch within a pipeline's memory (a slot): byte
 // offsets, sized for the largest domain.
 struct SlotLayout {
-  size_t keys[2], vals[2], hist, cnt, bmm, vsums, hsums, adj, rpre, rsuf, rtab, lb, ib, lft, rgt, fst, lst,
+  size_t keys[2], vals[2], hist, cnt, bmm, vsums, hsums, adj, rpre, rsuf, rtab, lb, ib, tree,
       front[2], bytes = 0;
   SlotLayout(int maxf, long long maxv) {
     auto take = [&](size_t b) {
@@ -956,17 +968,18 @@ struct SlotLayout {
       return at;
     };
     const size_t f = (size_t)maxf + 1, f4 = f * 4, hist_n = (size_t)256 * rsTiles(maxf);
-    for (size_t* x : {&keys[0], &keys[1], &vals[0], &vals[1], &lft, &rgt, &fst, &lst}) *x = take(f4);
+    for (size_t* x : {&keys[0], &keys[1], &vals[0], &vals[1]}) *x = take(f4);
     hist = take(hist_n * 4);
     cnt = take((size_t)(maxv + 1) * 12);
     bmm = take(64);
     vsums = take((size_t)scanSumsWords(maxv + 1) * 4);
     hsums = take((size_t)scanSumsWords((long long)hist_n) * 4);
     adj = take(f * 12);
+    tree = take(f * sizeof(int4));
     for (size_t* x : {&rpre, &rsuf, &lb, &ib}) *x = take(f * 24);
     rtab = take((size_t)rangeOff(rangeBlocks(maxf), rangeLevels(maxf)) * 4 + 64);
     // a frontier level holds disjoint subtrees of more than kLeafMax triangles
-    for (size_t* x : {&front[0], &front[1]}) *x = take(((size_t)maxf / (kLeafMax + 1) + 64) * sizeof(FrontierItem));
+    for (size_t* x : {&front[0], &front[1]}) *x = take(((size_t)maxf / (kLeafMax + 1) + 64) * 4);
   }
 };
 constexpr int kBuildStreams = 4;  // pipelines of a whole-scene LBVH build
@@ -1165,7 +1178,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       for (int k = 0; k < 2; ++k) {
         B.keys[k] = (uint32_t*)(slot + SL.keys[k]);
         B.vals[k] = (uint32_t*)(slot + SL.vals[k]);
-        B.front[k] = (FrontierItem*)(slot + SL.front[k]);
+        B.front[k] = (int*)(slot + SL.front[k]);
       }
       B.hist = (uint32_t*)(slot + SL.hist);
       B.rpre = (float*)(slot + SL.rpre);
@@ -1173,10 +1186,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       B.rtab = (float*)(slot + SL.rtab);
       B.leafbox = (float*)(slot + SL.lb);
       B.innerbox = (float*)(slot + SL.ib);
-      B.left = (int*)(slot + SL.lft);
-      B.right = (int*)(slot + SL.rgt);
-      B.first = (int*)(slot + SL.fst);
-      B.last = (int*)(slot + SL.lst);
+      B.tree = (int4*)(slot + SL.tree);
       B.cc = M->levels.as<int>() + (size_t)d * kLevelWords;
       hv[d] = ScanJob{B.cnt, B.off, (uint32_t*)(slot + SL.vsums), (long long)B.nv + 1};
       hh[d] = ScanJob{B.hist, B.hist, (uint32_t*)(slot + SL.hsums), 256ll * rsTiles(B.nf)};
@@ -1223,15 +1233,15 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     kRangeBoxes<<<grid(f - 1), 256, 0, st>>>(G);
     for (int d = a; d < a + m; ++d)
       if (P.desc[d].num_tris <= kLeafMax) {
-        kTinyRoot<<<1, 1, 0, st>>>(dev + d);
+        kTinyRoot<<<1, 8, 0, st>>>(dev + d);
         P.desc[d].num_nodes = 1;
         P.bvh_depth[d] = 1;
       }
   };
   // level l holds at most 8^l items (one root, at most eight children per item)
-  auto collapseBlocks = [](int f, int l) {
-    const int most = std::min(gridFor(std::max(1, f / 8), 256), 2048);
-    return (unsigned)(l < 8 ? std::min<long long>(most, ((1ll << (3 * l)) + 255) / 256) : most);
+  auto collapseBlocks = [](int f, int l, int m) {
+    const int most = std::min(gridFor(std::max(1, f / (kLeafMax + 1)), 32), 4096 / m);
+    return (unsigned)(l < 8 ? std::min<long long>(most, ((1ll << (3 * l)) + 31) / 32) : most);
   };
   // Collapse of domain d's binary tree under `root`, kLevelBatch levels per
   // host wait (a level past the last finds 0 items); returns the number of
@@ -1241,16 +1251,16 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     kCollapseInit<<<1, 64, 0, st>>>(G, root);
     for (int done = 0;;) {
       const int upto = std::min(done + kLevelBatch, kMaxLevels);
-      for (int l = done; l < upto; ++l) kCollapseLevel<<<collapseBlocks(P.desc[d].num_tris, l), 256, 0, st>>>(G, l);
+      for (int l = done; l < upto; ++l) kCollapseLevel<<<collapseBlocks(P.desc[d].num_tris, l, 1), 256, 0, st>>>(G, l);
       done = upto;
       int h[kLevelWords];
       SPRAY_HIP(hipMemcpyAsync(h, M->levels.as<int>() + (size_t)d * kLevelWords, sizeof(h), hipMemcpyDeviceToHost, st));
       SPRAY_HIP(hipStreamSynchronize(st));
       if (h[1]) throw StatusError(SPRAY_ERR_CAPACITY, "BVH node capacity exceeded");
-      P.desc[d].num_nodes = h[0];
       if (h[2 + done] == 0 || done == kMaxLevels) {
         int depth = 0;
-        while (depth < done && h[2 + depth] > 0) ++depth;
+        P.desc[d].num_nodes = 0;
+        while (depth < done && h[2 + depth] > 0) P.desc[d].num_nodes += h[2 + depth++];
         return h[2 + done] > 0 ? kMaxLevels + 1 : depth;
       }
     }
@@ -1274,8 +1284,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     if (ploc && depth < 0) {
       // PLOC passes until one cluster is left
       const char* slot = M->slots[0].as<char>();  // one-domain builds use slot 0
-      int *L = (int*)(slot + SL.lft), *R = (int*)(slot + SL.rgt), *F = (int*)(slot + SL.fst),
-          *Lst = (int*)(slot + SL.lst);
+      int4* T = (int4*)(slot + SL.tree);
       float* inner = (float*)(slot + SL.ib);
       const uint32_t* va = (const uint32_t*)(slot + SL.vals[0]);
       const float* vtx = P.vtx.as<float>() + D.vtx_off * 3;
@@ -1300,7 +1309,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         exclusiveScan(mflag, mpos, n + 1, s);
         exclusiveScan(kflag, kpos, n + 1, s);
         kPlocMerge<<<gridFor(n, 256), 256, 0, s>>>(nn, n, cid, cbox, mpos, kpos, made, cid2, cbox2,
-                                                    L, R, inner, icount);
+                                                    T, inner, icount);
         uint32_t h[2];
         SPRAY_HIP(hipMemcpyAsync(&h[0], mpos + n, 4, hipMemcpyDeviceToHost, s));
         SPRAY_HIP(hipMemcpyAsync(&h[1], kpos + n, 4, hipMemcpyDeviceToHost, s));
@@ -1319,10 +1328,10 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         // depth-first leaf order: roots of later passes first
         const int root = made - 1;
         uint32_t* perm = PS.pperm.as<uint32_t>();
-        SPRAY_HIP(hipMemsetAsync(F + root, 0, 4, s));
+        SPRAY_HIP(hipMemsetAsync(&T[root].z, 0, 4, s));
         for (int p = (int)pass_base.size() - 1; p > 0; --p) {
           int lo = pass_base[p - 1], hi = pass_base[p];
-          kPlocRanges<<<gridFor(hi - lo, 256), 256, 0, s>>>(lo, hi, L, R, icount, F, Lst, perm);
+          kPlocRanges<<<gridFor(hi - lo, 256), 256, 0, s>>>(lo, hi, T, icount, perm);
         }
         uint32_t* order = PS.pord.as<uint32_t>();
         kComposeOrder<<<gridFor(nf, 256), 256, 0, s>>>(perm, va, nf, order);
@@ -1369,7 +1378,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
           for (int d = a; d < a + m; ++d) levels = std::max(levels, std::min(kMaxLevels, prev_depth[d] + 4));
         kCollapseInit<<<dim3(1, (unsigned)m), 64, 0, st>>>(dev + a, 0);
         for (int l = 0; l < levels; ++l)
-          kCollapseLevel<<<dim3(collapseBlocks(f, l), (unsigned)m), 256, 0, st>>>(dev + a, l);
+          kCollapseLevel<<<dim3(collapseBlocks(f, l, m), (unsigned)m), 256, 0, st>>>(dev + a, l);
         for (int d = a; d < a + m; ++d) launched[d] = levels;
         SPRAY_HIP(hipGetLastError());
       }
@@ -1388,11 +1397,11 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         redo.push_back(d);
         continue;
       }
-      int depth = 0;
-      while (depth < launched[d] && cc[2 + depth] > 0) ++depth;
+      int depth = 0, nodes = 0;
+      while (depth < launched[d] && cc[2 + depth] > 0) nodes += cc[2 + depth++];
       if (!fitsStack(depth))
         throw StatusError(SPRAY_ERR_CAPACITY, "BVH too deep for the traversal stack");
-      P.desc[d].num_nodes = cc[0];
+      P.desc[d].num_nodes = nodes;
       P.bvh_depth[d] = depth;
     }
     for (int d : redo) buildOne(d, false);  // deeper than last time: host-checked
