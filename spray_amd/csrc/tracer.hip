@@ -39,12 +39,16 @@ namespace spray {
 constexpr int kBlock = 256;
 // grid of kCount and kScatter (they must match: blocks own queue slots)
 constexpr int kQueueGrid = 1024;
+// and their threads per block, a block's entries for one domain and round
+// being one run of the queue: kScatter takes 1.09 / 0.80 / 0.90 ms per frame of
+// 64 even domains with 256 / 512 / 1024, kCount 2.08 / 2.18 / 2.21 ms.
+constexpr int kQueueBlock = 512;
 constexpr int kShadeRec = 5;  // float4s per shade record
-// Ask records per kCount block region: a block takes at most kBlock of
-// every kQueueGrid * kBlock consecutive rays of a pass.
+// Ask records per kCount block region: a block takes at most kQueueBlock of
+// every kQueueGrid * kQueueBlock consecutive rays of a pass.
 inline uint32_t askRegion(uint32_t r_cap) {
-  const uint32_t stride = (uint32_t)kQueueGrid * kBlock;
-  return (uint32_t)kBlock * ((r_cap + stride - 1) / stride);
+  const uint32_t stride = (uint32_t)kQueueGrid * kQueueBlock;
+  return (uint32_t)kQueueBlock * ((r_cap + stride - 1) / stride);
 }
 // Domain grid of the domain-list pass: a uniform grid over the domain boxes
 // (at most kGridCells cells, kGridMaxRes per axis), each cell listing the
@@ -53,11 +57,14 @@ inline uint32_t askRegion(uint32_t r_cap) {
 // axis, so a box that fills a cell is listed once); at most
 // kGridIdsPerDomain list entries per domain on average (the grid is
 // coarsened until that holds).  Contacts on cell faces, edges and corners
-// are the walk's business (kGridTol).
+// are the walk's business (kGridTol).  A cell's word is kCellEmpty, kCellOne
+// + the id of its only domain, or the start of its list, whose last id has
+// kLastId added: most cells take one load.
 constexpr int kGridCells = 32768;
 constexpr int kGridMaxRes = 64;
 constexpr int kGridIdsPerDomain = 32;
 constexpr float kGridTol = 1e-4f;
+constexpr uint32_t kCellEmpty = 0xffffffffu, kCellOne = 0x80000000u, kLastId = 0x8000u;
 // dbox bytes: domain boxes, grid header (4 float4), cell offsets, cell ids
 __host__ __device__ inline size_t gridHeadBytes(int nd) { return (size_t)nd * 32; }
 __host__ __device__ inline size_t gridOffBytes(int nd) { return gridHeadBytes(nd) + 64; }
@@ -69,9 +76,10 @@ __host__ __device__ inline size_t dboxBytes(int nd) {
 }
 
 // kCount's dynamic LDS (byte offsets): domain boxes, counts, scores, the
-// block's hit-mask words ([word][thread]).
+// block's hit-mask words ([word][thread]) and the rays' top lists (ids,
+// [entry][thread]).
 struct CountLds {
-  size_t lc, ls, mask, total;
+  size_t lc, ls, mask, top, total;
 };
 __host__ __device__ inline CountLds countLds(int nd, int block) {
   const int nw = (nd + 63) / 64;
@@ -79,7 +87,8 @@ __host__ __device__ inline CountLds countLds(int nd, int block) {
   L.lc = (size_t)nd * 32;
   L.ls = L.lc + (size_t)nd * 8;
   L.mask = (L.ls + (size_t)nd * 4 + 7) & ~(size_t)7;
-  L.total = L.mask + (size_t)nw * block * 8;
+  L.top = L.mask + (size_t)nw * block * 8;
+  L.total = L.top + (size_t)kTopDepths * block * 2;
   return L;
 }
 
@@ -361,8 +370,8 @@ __device__ __forceinline__ bool passRay(const TraceParams& P, long long i, int* 
 }
 
 // One ray's domain list, a walk that a lane resumes one cell step at a
-// time: per-domain counts (lc), the 16 nearest (t, id) entries sorted
-// (registers), the domains hit as a bit mask (one word per 64 domains, this
+// time: per-domain counts (lc), the 16 nearest domains sorted by (t, id)
+// (LDS), the domains hit as a bit mask (one word per 64 domains, this
 // lane's words at mask[w * stride]) so that the scatter re-tests only those,
 // and the number of domains hit.  Candidates come from
 // a 3D-DDA walk of the domain grid over the ray's t range inside the grid
@@ -389,11 +398,19 @@ struct DomEnv {
 };
 
 struct DomWalk {
-  // the ray and its list
+  // the ray and its list: the ids of the first kTopDepths domains it hits,
+  // sorted by (t, id), in LDS (this lane's entries at top[k * stride]), and
+  // the last entry's t.  The walk meets domains nearly in order, so most go to
+  // the end; where one does not, the t of the entries it passes are worked out
+  // again (the same arithmetic, so the same value).  A list of (t, id) in
+  // registers, every insertion passing all of it, and two dependent loads for a
+  // cell's range took 2.52 ms of a frame of 64 even domains; now 2.18 ms, bound
+  // by issue (vector instructions half the time, at 32 of 64 lanes, and the
+  // scalar ones of its branches; twice the waves do not help).
   float o[3], d[3], inv[3];
   int spawn, kind;
-  float tt[kTopDepths];
-  int ti[kTopDepths];
+  uint16_t* top;
+  float tlast;
   int kept, hits;
   // the walk: current cell (8 bits per axis, kGridMaxRes <= 256), step per
   // axis (2 bits each, -1..1 stored + 1), exit t, steps left (0: done)
@@ -401,47 +418,57 @@ struct DomWalk {
   float t1;
   int left;
 
+  __device__ __forceinline__ float entry(const DomEnv& E, int dd, bool safe) const {
+    float t;
+    (void)slabBox4(E.box[2 * dd], E.box[2 * dd + 1], o, inv, safe, &t);
+    return t;
+  }
+  __device__ __forceinline__ void insert(const DomEnv& E, float ct, int ci, bool safe) {
+    const int s = E.stride;
+    if (kept == kTopDepths && !(ct < tlast)) return;
+    if (kept == 0 || ct > tlast || (ct == tlast && ci > (int)top[(kept - 1) * s])) {
+      top[kept++ * s] = (uint16_t)ci;
+      tlast = ct;
+      return;
+    }
+    const bool full = kept == kTopDepths;
+    int j = kept - 1;  // (ahead of the last entry, which moves on or, in a full list, drops out)
+    if (!full) {
+      top[kept * s] = top[j * s];
+      ++kept;
+    }
+    for (; j > 0; --j) {
+      const int pi = top[(j - 1) * s];
+      const float pt = entry(E, pi, safe);
+      if (!(ct < pt || (ct == pt && ci < pi))) break;
+      top[j * s] = (uint16_t)pi;
+    }
+    top[j * s] = (uint16_t)ci;
+    if (full) tlast = j == kTopDepths - 1 ? ct : entry(E, top[(kTopDepths - 1) * s], safe);
+  }
+
   // candidates of one cell (cells outside the grid have none)
   __device__ __forceinline__ void visit(const DomEnv& E, int x, int y, int z, bool safe) {
     const DomGrid& G = E.G;
     if (x < 0 || y < 0 || z < 0 || x >= G.r[0] || y >= G.r[1] || z >= G.r[2]) return;
     const int cl = (z * G.r[1] + y) * G.r[0] + x;
-    const uint32_t q1 = E.coff[cl + 1];
-    for (uint32_t q = E.coff[cl]; q < q1; ++q) {
-      const int dd = E.cids[q];
+    const uint32_t word = E.coff[cl];
+    if (word == kCellEmpty) return;
+    uint32_t id = word >= kCellOne ? word | kLastId : E.cids[word];
+    for (uint32_t q = word;; id = E.cids[++q]) {
+      const int dd = (int)(id & (kLastId - 1u));
       unsigned long long* mw = &E.mask[(dd >> 6) * E.stride];
-      if ((*mw >> (dd & 63)) & 1ull) continue;  // already a hit
       float tmin;
       // isectWithoutCurrentDomain (ooc_isector.h:147-174): a shadow ray's
       // spawning domain was tested right after shading
-      if (!slabBox4(E.box[2 * dd], E.box[2 * dd + 1], o, inv, safe, &tmin) || dd == spawn) continue;
-      ++hits;
-      atomicAdd(&E.lc[kind * E.nd + dd], 1u);
-      *mw |= 1ull << (dd & 63);
-      // insertion into the (t, id)-sorted top list (unrolled: stays in
-      // registers); steps past every active lane's list end are skipped
-      if (kept < kTopDepths || tmin < tt[kTopDepths - 1]) {
-        float ct = tmin;
-        int ci = dd;
-#pragma unroll
-        for (int j = 0; j < kTopDepths; ++j) {
-          if (__ballot(j <= kept) == 0ull) break;
-          if (j < kept) {
-            if (ct < tt[j] || (ct == tt[j] && ci < ti[j])) {
-              float xt = tt[j];
-              int xi = ti[j];
-              tt[j] = ct;
-              ti[j] = ci;
-              ct = xt;
-              ci = xi;
-            }
-          } else if (j == kept) {
-            tt[j] = ct;
-            ti[j] = ci;
-          }
-        }
-        if (kept < kTopDepths) ++kept;
+      if (!((*mw >> (dd & 63)) & 1ull) &&  // not yet a hit
+          slabBox4(E.box[2 * dd], E.box[2 * dd + 1], o, inv, safe, &tmin) && dd != spawn) {
+        ++hits;
+        atomicAdd(&E.lc[kind * E.nd + dd], 1u);
+        *mw |= 1ull << (dd & 63);
+        insert(E, tmin, dd, safe);
       }
+      if (id & kLastId) break;
     }
   }
 
@@ -479,10 +506,11 @@ struct DomWalk {
       nb[k] = (fr < kGridTol && c[k] > 0) ? -1 : (fr > 1.f - kGridTol && c[k] < G.r[k] - 1) ? 1 : 0;
     }
     const int nbm = (nb[0] != 0 ? 1 : 0) | (nb[1] != 0 ? 2 : 0) | (nb[2] != 0 ? 4 : 0);
-    for (int sub = 1; sub < 8; ++sub)
-      if ((sub & ~nbm) == 0)
-        visit(E, c[0] + ((sub & 1) ? nb[0] : 0), c[1] + ((sub & 2) ? nb[1] : 0),
-              c[2] + ((sub & 4) ? nb[2] : 0), safe);
+    if (nbm != 0)
+      for (int sub = 1; sub < 8; ++sub)
+        if ((sub & ~nbm) == 0)
+          visit(E, c[0] + ((sub & 1) ? nb[0] : 0), c[1] + ((sub & 2) ? nb[1] : 0),
+                c[2] + ((sub & 4) ? nb[2] : 0), safe);
     cell = (uint32_t)c[0] | ((uint32_t)c[1] << 8) | ((uint32_t)c[2] << 16);
     steps = (uint32_t)(st[0] + 1) | ((uint32_t)(st[1] + 1) << 2) | ((uint32_t)(st[2] + 1) << 4);
     left = G.r[0] + G.r[1] + G.r[2] + 3;
@@ -511,10 +539,11 @@ struct DomWalk {
     const int tm = (st[0] != 0 && tn[0] <= lim ? 1 : 0) | (st[1] != 0 && tn[1] <= lim ? 2 : 0) |
                    (st[2] != 0 && tn[2] <= lim ? 4 : 0);
     // crossings at (nearly) the same t: the cells of the partial steps too
-    for (int sub = 1; sub < 7; ++sub)
-      if ((sub & ~tm) == 0 && sub != tm)
-        visit(E, c[0] + ((sub & 1) ? st[0] : 0), c[1] + ((sub & 2) ? st[1] : 0),
-              c[2] + ((sub & 4) ? st[2] : 0), safe);
+    if ((tm & (tm - 1)) != 0)
+      for (int sub = 1; sub < 7; ++sub)
+        if ((sub & ~tm) == 0 && sub != tm)
+          visit(E, c[0] + ((sub & 1) ? st[0] : 0), c[1] + ((sub & 2) ? st[1] : 0),
+                c[2] + ((sub & 4) ? st[2] : 0), safe);
 #pragma unroll
     for (int k = 0; k < 3; ++k)
       if (tm & (1 << k)) {
@@ -534,7 +563,7 @@ struct DomWalk {
 // write the packed list instead of the mask (an instantiation of its own, so
 // scenes with fewer domains keep the mask-only register set).
 template <bool kLearned, bool kList>
-__global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
+__global__ void __launch_bounds__(kQueueBlock) kCount(TraceParams P) {
   extern __shared__ uint32_t sm[];
   if (!P.ctr->active) return;
   const int nd = P.ndomains, nw = (nd + 63) >> 6;
@@ -589,6 +618,8 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
   E.stride = blockDim.x;
   E.nd = nd;
   DomWalk W;
+  W.top = (uint16_t*)(smc + L.top) + threadIdx.x;
+  W.tlast = 0.f;
   W.kind = 0;
   W.left = 0;
   W.kept = W.hits = 0;
@@ -644,8 +675,8 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
         uint32_t pk[kTopDepths / 2];
 #pragma unroll
         for (int j = 0; j < kTopDepths / 2; ++j)
-          pk[j] = (2 * j < W.hits ? (uint32_t)W.ti[2 * j] : 0xffffu) |
-                  ((2 * j + 1 < W.hits ? (uint32_t)W.ti[2 * j + 1] : 0xffffu) << 16);
+          pk[j] = (2 * j < W.hits ? (uint32_t)W.top[2 * j * E.stride] : 0xffffu) |
+                  ((2 * j + 1 < W.hits ? (uint32_t)W.top[(2 * j + 1) * E.stride] : 0xffffu) << 16);
         uint4* r4 = (uint4*)row;
         r4[0] = make_uint4(pk[0], pk[1], pk[2], pk[3]);
         r4[1] = make_uint4(pk[4], pk[5], pk[6], pk[7]);
@@ -654,10 +685,9 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
         for (int w = 0; w < nw; ++w) row[w] = lmask[w * blockDim.x];
         if (kList) P.dfmt[i] = 0;
       }
-#pragma unroll
-      for (int k = 0; k < kTopDepths; ++k)
-        if (k < W.kept) atomicAdd(&ls[W.ti[k]], (uint32_t)(kTopDepths - k));
     }
+    for (int k = 0; __ballot(fin && k < W.kept) != 0ull; ++k)
+      if (fin && k < W.kept) atomicAdd(&ls[W.top[k * E.stride]], (uint32_t)(kTopDepths - k));
     // learned form: a radiance ray with two or more candidate domains writes
     // an ask record for the predictor into this block's region (one LDS
     // atomic per wave); the others have no phase-A bound
@@ -676,9 +706,10 @@ __global__ void __launch_bounds__(kBlock, 4) kCount(TraceParams P) {
       if (ask && a < P.ask_region) {
         float4* rec = P.ask + ((size_t)blockIdx.x * P.ask_region + a) * 3;
         const float4 ds = P.R.ds(r);
+        const int d0 = W.top[0], d1 = W.top[E.stride];
         rec[0] = make_float4(W.o[0], W.o[1], W.o[2], ds.x);
-        rec[1] = make_float4(ds.y, ds.z, W.tt[0], W.tt[1]);
-        rec[2] = make_float4(__uint_as_float(r), __int_as_float(W.ti[0]), __int_as_float(W.ti[1]),
+        rec[1] = make_float4(ds.y, ds.z, W.entry(E, d0, true), W.entry(E, d1, true));
+        rec[2] = make_float4(__uint_as_float(r), __int_as_float(d0), __int_as_float(d1),
                              __int_as_float(min(W.hits, 255)));
       } else if (rad) {
         P.rkey[r] = kNoBound;
@@ -824,7 +855,7 @@ __global__ void __launch_bounds__(kBlock) kBlockBases(TraceParams P) {
 // kCount, so each block owns the slots kBlockBases reserved for it.
 // kList: the rays kCount gave a packed hit list (as kCount's kList).
 template <bool kList>
-__global__ void __launch_bounds__(kBlock) kScatter(TraceParams P) {
+__global__ void __launch_bounds__(kQueueBlock) kScatter(TraceParams P) {
   extern __shared__ uint32_t sm[];
   if (!P.ctr->active) return;
   const int nd = P.ndomains;
@@ -2006,10 +2037,10 @@ static TraceParams makeParams(Ctx* c) {
   return P;
 }
 
-static size_t countShmem(int nd) { return countLds(nd, kBlock).total; }
+static size_t countShmem(int nd) { return countLds(nd, kQueueBlock).total; }
 
 // Domain boxes for the ray/domain slab tests, plus kCount's domain grid:
-// header, cell offsets and the cells' domain ids (ascending).
+// header, cell words and the cells' domain ids (ascending).
 static void domainBoxesUpload(Ctx* c, hipStream_t s) {
   TracerState* T = c->tracer;
   const int nd = c->pool.ndomains;
@@ -2079,6 +2110,11 @@ static void domainBoxesUpload(Ctx* c, hipStream_t s) {
         for (int y = a[1]; y <= b[1]; ++y)
           for (int x = a[0]; x <= b[0]; ++x) ids[cur[(z * r[1] + y) * r[0] + x]++] = (uint16_t)d;
     }
+    for (int i = 0; i < ncell; ++i) {  // the cell words
+      const uint32_t at = off[i];
+      if (cnt[i] > 0) ids[at + cnt[i] - 1] |= (uint16_t)kLastId;
+      off[i] = cnt[i] == 0 ? kCellEmpty : cnt[i] == 1 ? kCellOne | (ids[at] & (kLastId - 1u)) : at;
+    }
     break;
   }
   const size_t bytes = gridIdsBytes(nd) + ids.size() * 2;
@@ -2131,13 +2167,13 @@ static void passQueues(Ctx* c, const TraceParams& P) {
   const bool list = (nd + 63) / 64 > kHitListWords;  // packed hit lists (kScatter agrees)
   const size_t sh = countShmem(nd);
   if (P.learned && list)
-    kCount<true, true><<<kQueueGrid, kBlock, sh, s>>>(P);
+    kCount<true, true><<<kQueueGrid, kQueueBlock, sh, s>>>(P);
   else if (P.learned)
-    kCount<true, false><<<kQueueGrid, kBlock, sh, s>>>(P);
+    kCount<true, false><<<kQueueGrid, kQueueBlock, sh, s>>>(P);
   else if (list)
-    kCount<false, true><<<kQueueGrid, kBlock, sh, s>>>(P);
+    kCount<false, true><<<kQueueGrid, kQueueBlock, sh, s>>>(P);
   else
-    kCount<false, false><<<kQueueGrid, kBlock, sh, s>>>(P);
+    kCount<false, false><<<kQueueGrid, kQueueBlock, sh, s>>>(P);
   // learned form: the predictor needs only kCount's ask records, so it runs
   // on the second stream beside the schedule and the scatter
   if (P.learned) {
@@ -2149,9 +2185,9 @@ static void passQueues(Ctx* c, const TraceParams& P) {
   kSchedule<<<1, 1024, 0, s>>>(P);
   kBlockBases<<<2 * nd, kBlock, 0, s>>>(P);
   if (list)
-    kScatter<true><<<kQueueGrid, kBlock, scatterShmem(nd), s>>>(P);
+    kScatter<true><<<kQueueGrid, kQueueBlock, scatterShmem(nd), s>>>(P);
   else
-    kScatter<false><<<kQueueGrid, kBlock, scatterShmem(nd), s>>>(P);
+    kScatter<false><<<kQueueGrid, kQueueBlock, scatterShmem(nd), s>>>(P);
   if (P.learned) {
     SPRAY_HIP(hipStreamWaitEvent(s, T->join_ev, 0));
     predictorAssign(c, P);

@@ -84,7 +84,7 @@ struct TraceParams {
   // pool
   const DomainDesc* desc;
   // per domain (lo, 0), (hi, 0); then the domain grid: header (4 float4),
-  // cell offsets (uint32, at gridOffBytes) and cell domain ids (uint16, at
+  // cell words (uint32, at gridOffBytes) and cell domain ids (uint16, at
   // gridIdsBytes)
   const float4* dbox;
   const BNode8* nodes;
