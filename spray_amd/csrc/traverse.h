@@ -113,6 +113,11 @@ __device__ __forceinline__ bool needsSafeBoxes(const float inv[3]) {
   return !(fabsf(inv[0]) < kFusedInvMax && fabsf(inv[1]) < kFusedInvMax && fabsf(inv[2]) < kFusedInvMax);
 }
 
+// The bits of a where m is set, those of b elsewhere.
+__device__ __forceinline__ uint32_t pickBits(uint32_t m, uint32_t a, uint32_t b) {
+  return __builtin_amdgcn_bitop3_b32(m, a, b, 0xca);
+}
+
 // Tests the 8 child boxes of a node against [tnear, tfar]; returns the mask of
 // the slots hit.  The distance of plane q is
 //   (base + q * scale - org) * inv = fma(q, scale * inv, (base - org) * inv)
@@ -121,6 +126,10 @@ __device__ __forceinline__ bool needsSafeBoxes(const float inv[3]) {
 // a step too large (quantizeNode), so no box the ray meets is missed, and no
 // absolute pad is needed.  A ray's near planes are the lower ones where inv
 // >= 0 and the upper ones elsewhere, one select per axis for four children.
+// fma, add, mul and the three-operand bit operation issue in 2 cycles a wave,
+// byte conversions, min, max, compares, selects and shifts in 4: so planes are
+// picked by bits and a miss is a sign bit shifted in (1% of the trace time
+// against selects, compares and carries).
 // kSafe (waves with an axis-parallel ray): the difference first, then the
 // product with a possibly infinite inv; 0 * inf = NaN (the origin on the
 // plane) bounds nothing, as max and min drop NaN operands.
@@ -135,15 +144,15 @@ __device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const float scale = __uint_as_float(((meta >> (8 * k)) & 255u) << 23);
-    const bool neg = inv[k] < 0.f;
-    nq[k][0] = neg ? pl[k].z : pl[k].x;
-    nq[k][1] = neg ? pl[k].w : pl[k].y;
-    fq[k][0] = neg ? pl[k].x : pl[k].z;
-    fq[k][1] = neg ? pl[k].y : pl[k].w;
+    const uint32_t neg = (uint32_t)((int32_t)__float_as_uint(inv[k]) >> 31);
+    nq[k][0] = pickBits(neg, pl[k].z, pl[k].x);
+    nq[k][1] = pickBits(neg, pl[k].w, pl[k].y);
+    fq[k][0] = pickBits(neg, pl[k].x, pl[k].z);
+    fq[k][1] = pickBits(neg, pl[k].y, pl[k].w);
     m[k] = kSafe ? scale : scale * inv[k];
     c[k] = kSafe ? bo[k] : bo[k] * inv[k];
   }
-  uint32_t mask = 0;
+  uint32_t miss = 0;
 #pragma unroll
   for (int i = 7; i >= 0; --i) {
     float tn[3], tf[3];
@@ -159,11 +168,12 @@ __device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)
       }
     }
     const float t0 = fmaxf(fmaxf(fmaxf(tn[0], tn[1]), tn[2]), tnear);
-    const float t1 = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), tfar) * kSlabInflate;
-    uint32_t carry;
-    mask = __builtin_addc(mask, mask, t0 <= t1 ? 1u : 0u, &carry);
+    const float t1 = fminf(fminf(fminf(tf[0], tf[1]), tf[2]), tfar);
+    // a miss is the sign of the inflated t1 - t0, shifted in
+    const float d = __builtin_fmaf(t1, kSlabInflate, -t0);
+    miss = __builtin_amdgcn_alignbit(miss, __float_as_uint(d), 31u);
   }
-  return mask;
+  return ~miss & 255u;
 }
 
 // Resumable traversal of one ray (closest or any hit) in two wave-wide
