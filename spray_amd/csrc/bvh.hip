@@ -39,6 +39,7 @@ struct BuildDom {
   float4* fshade;
   LTri* tris;
   BNode8* nodes;
+  NodeLeaves* leaves;
   // scratch: vertex adjacency, centroid bounds, sort buffers, leaf-range unions
   uint32_t *cnt, *cur, *off, *adj, *bmm, *keys[2], *vals[2], *hist;
   float *rpre, *rsuf, *rtab;
@@ -542,18 +543,34 @@ __device__ __forceinline__ uint32_t groupBallot(bool p) {
   return (uint32_t)(__ballot(p) >> (threadIdx.x & 56)) & 255u;
 }
 
+// The largest float at least 1/64 of a step (2^e) below lo whose last byte is
+// e + 127.
+__device__ __forceinline__ float gridBase(float lo, int e, double step) {
+  const double bd = (double)lo - step * 0.015625;
+  float f = (float)bd;
+  if ((double)f > bd) f = nextafterf(f, -kInfF);
+  const uint32_t u = __float_as_uint(f), byte = (uint32_t)(e + 127);
+  uint32_t w = (u & ~255u) | byte;
+  if (u >> 31) {
+    if (w < u) w += 256u;
+  } else if (w > u) {
+    w = u >= 256u ? w - 256u : 0x80000000u | byte;
+  }
+  return __uint_as_float(w);
+}
+
 // Writes a node's grid and child planes; called by the 8 lanes of a group,
 // each with the box (lo xyz, hi xyz) and slot of one child (used), the other
 // lanes with a slot of their own among those left.  Per
 // axis the step is the power of two that covers the children's extent in at
-// most 253 steps (at least 2^-20 of the largest coordinate, so that base's
-// rounding stays below an eighth of a step), base lies 1/64 of a step or more
-// below the lowest plane, and planes are rounded outwards with 2^-9 of a step
-// to spare: the distance test's cancellation error (nodeBoxes) is below 2^-15
-// of a step.  An axis whose extent is not finite, or would need a step of
-// 2^62 or more, covers everything.  Lane k of the group works out axis k's
-// grid.  Returns the exponent bytes of meta.
-__device__ __forceinline__ uint32_t quantizeNode(const float (&b)[6], bool used, uint32_t slot, BNode8* nd) {
+// most 253 steps (at least 2^-20 of the largest coordinate), or the next one:
+// base, whose last byte is the step's exponent, lies 1/64 of a step to 33
+// steps below the lowest plane, and the highest has to be within 255 steps of
+// it.  Planes are rounded outwards with 2^-9 of a step to spare: the distance
+// test's cancellation error (nodeBoxes) is below 2^-15 of a step.  An axis
+// whose extent is not finite, or would need a step of 2^62 or more, covers
+// everything.  Lane k of the group works out axis k's grid.
+__device__ __forceinline__ void quantizeNode(const float (&b)[6], bool used, uint32_t slot, BNode8* nd) {
   const int me = threadIdx.x & 7;
   float lo = 0.f, hi = 0.f;
   bool finite = false;
@@ -581,17 +598,19 @@ __device__ __forceinline__ uint32_t quantizeNode(const float (&b)[6], bool used,
     }
     if (big > 0.0) e = max(e, exponent(big) - 19);
   }
-  const bool all = !finite || e >= 62;
-  float base = -3.0e38f;
+  const bool all = !finite || e >= 61;
+  float base = __uint_as_float(0xff61b1f8u);  // -3e38, with the exponent of `all`
   if (all) {
     e = 121;
   } else {
-    const double bd = (double)lo - power(e) * 0.015625;
-    base = (float)bd;
-    if ((double)base > bd) base = nextafterf(base, -kInfF);
+    base = gridBase(lo, e, power(e));
+    // at twice the step the extent is below 127 steps, and base's distance halves
+    if (((double)hi - (double)base) * power(-e) + 0.001953125 > 255.0) {
+      ++e;
+      base = gridBase(lo, e, power(e));
+    }
   }
   if (me < 3) nd->base[me] = base;
-  uint32_t meta = 0;
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int ek = __shfl(e, k, 8);
@@ -604,9 +623,7 @@ __device__ __forceinline__ uint32_t quantizeNode(const float (&b)[6], bool used,
     }
     nd->plane[k][slot] = (uint8_t)l;
     nd->plane[k][8 + slot] = (uint8_t)h;
-    meta |= (uint32_t)(ek + 127) << (8 * k);
   }
-  return meta;
 }
 
 // Slot of each lane's child (one child per used lane of the group; the other
@@ -679,6 +696,7 @@ __device__ __forceinline__ uint32_t assignSlot(const float (&b)[6], bool used) {
 // resolution 72) took 5.8 ms, now 3.4 ms.
 __global__ void __launch_bounds__(256) kCollapseLevel(const BuildDom* __restrict__ G, int l) {
   __shared__ BNode8 img[32];
+  __shared__ NodeLeaves limg[32];
   __shared__ int alloc[32];
   const BuildDom& B = G[blockIdx.y];
   const int nin = B.cc[2 + l];
@@ -755,17 +773,15 @@ __global__ void __launch_bounds__(256) kCollapseLevel(const BuildDom* __restrict
     const int q = alloc[grp], cbase = start + nin + q;
     const bool fits = cbase + __popc(im) <= B.node_cap;
     if (!fits && me == 0) atomicExch(&B.cc[1], l + 1);  // the levels below return at once
-    BNode8* nd = &img[grp];
-    const uint32_t meta = quantizeNode(b, used, slot, nd);
-    if (me == 0) {
-      nd->child_base = (uint32_t)cbase;
-      nd->meta = meta | (im << 24);
-    }
-    if (me < 7) nd->pad[me] = 0u;
-    nd->leaf[slot] = used && !inner ? ((uint32_t)cnt << 24) | (uint32_t)rec.z : 0u;
+    quantizeNode(b, used, slot, &img[grp]);
+    if (me == 0) img[grp].kids = ((uint32_t)cbase & 0xffffffu) | (im << 24);
+    limg[grp].leaf[slot] = used && !inner ? ((uint32_t)cnt << 24) | (uint32_t)rec.z : 0u;
     if (inner && fits) fout[q + __popc(im & ((1u << slot) - 1u))] = c;
     __syncthreads();
-    if (act) ((float4*)(B.nodes + start + it))[me] = ((const float4*)nd)[me];
+    if (act && me < 4)
+      ((float4*)(B.nodes + start + it))[me] = ((const float4*)&img[grp])[me];
+    else if (act && me < 6)
+      ((float4*)(B.leaves + start + it))[me - 4] = ((const float4*)&limg[grp])[me - 4];
     __syncthreads();
   }
 }
@@ -791,13 +807,9 @@ __global__ void kTinyRoot(const BuildDom* __restrict__ G) {
       b[k] = fminf(b[k], leafbox[i * 6 + k]);
       b[3 + k] = fmaxf(b[3 + k], leafbox[i * 6 + 3 + k]);
     }
-  const uint32_t meta = quantizeNode(b, me == 0 && nf > 0, (uint32_t)me, nd);
-  if (me == 0) {
-    nd->meta = meta;
-    nd->child_base = 0;
-  }
-  if (me < 7) nd->pad[me] = 0;
-  nd->leaf[me] = me == 0 ? (uint32_t)nf << 24 : 0u;
+  quantizeNode(b, me == 0 && nf > 0, (uint32_t)me, nd);
+  if (me == 0) nd->kids = 0;
+  G->leaves->leaf[me] = me == 0 ? (uint32_t)nf << 24 : 0u;
 }
 
 // ---------------------------------------------------------------------------
@@ -1083,12 +1095,13 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.tris.reserve((size_t)P.capacity * maxf * sizeof(LTri) + 64);
     P.fshade.reserve((size_t)P.capacity * maxf * 48 + 64);
     P.nodes.reserve((size_t)P.capacity * max_nodes * sizeof(BNode8) + 64);
+    P.leaves.reserve((size_t)P.capacity * max_nodes * sizeof(NodeLeaves) + 64);
     size_t bytes = 0;
     P.h_image_off.resize(nd);
     for (int d = 0; d < nd; ++d) {
       P.h_image_off[d] = (long long)bytes;
       const size_t nf = (size_t)P.desc[d].num_tris;
-      bytes += ((size_t)nodeCap((long long)nf) * sizeof(BNode8) + nf * (sizeof(LTri) + 48) + 255) & ~(size_t)255;
+      bytes += ((size_t)nodeCap((long long)nf) * (sizeof(BNode8) + sizeof(NodeLeaves)) + nf * (sizeof(LTri) + 48) + 255) & ~(size_t)255;
     }
     SPRAY_HIP(hipHostMalloc(&P.h_image, bytes, hipHostMallocDefault));
     P.h_nrm.resize(nd);
@@ -1101,6 +1114,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.tris.reserve(tf * sizeof(LTri));
     P.fshade.reserve(tf * 48 + 64);
     P.nodes.reserve(tn * sizeof(BNode8));
+    P.leaves.reserve(tn * sizeof(NodeLeaves));
   }
   // A whole-scene LBVH build takes the domains in groups, one launch per
   // build step for a group, up to kBuildStreams groups side by side (one per
@@ -1167,6 +1181,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
       B.fshade = P.fshade.as<float4>() + D.shade_off * 3;
       B.tris = P.tris.as<LTri>() + D.tri_off;
       B.nodes = P.nodes.as<BNode8>() + D.node_off;
+      B.leaves = P.leaves.as<NodeLeaves>() + D.node_off;
       B.nf = D.num_tris;
       B.nv = (int)src.numVerts(d);
       B.node_cap = (int)nodeCap(D.num_tris);
@@ -1351,10 +1366,12 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.bvh_depth[d] = depth;
     if (paged) {  // the finished image goes to pinned host memory, the normals to the host
       char* dst = (char*)P.h_image + P.h_image_off[d];
-      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)nf * sizeof(LTri);
+      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), lb = (size_t)D.num_nodes * sizeof(NodeLeaves),
+                   tb = (size_t)nf * sizeof(LTri);
       SPRAY_HIP(hipMemcpyAsync(dst, P.nodes.as<BNode8>() + D.node_off, nb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb, P.tris.as<LTri>() + D.tri_off, tb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb + tb, P.fshade.as<float4>() + D.shade_off * 3,
+      SPRAY_HIP(hipMemcpyAsync(dst + nb, P.leaves.as<NodeLeaves>() + D.node_off, lb, hipMemcpyDeviceToHost, s));
+      SPRAY_HIP(hipMemcpyAsync(dst + nb + lb, P.tris.as<LTri>() + D.tri_off, tb, hipMemcpyDeviceToHost, s));
+      SPRAY_HIP(hipMemcpyAsync(dst + nb + lb + tb, P.fshade.as<float4>() + D.shade_off * 3,
                                (size_t)nf * 48, hipMemcpyDeviceToHost, s));
       P.h_nrm[d].resize((size_t)nv * 3);
       SPRAY_HIP(hipMemcpyAsync(P.h_nrm[d].data(), P.nrm.p, (size_t)nv * 12, hipMemcpyDeviceToHost, s));
@@ -1444,8 +1461,8 @@ constexpr int kQBlock = 256;
 constexpr int kQRefill = 16;
 constexpr uint32_t kQMinRange = 4;
 __global__ void __launch_bounds__(kQBlock, 4) kTraceRays(
-    const BNode8* __restrict__ nodes, const LTri* __restrict__ tris, const float* __restrict__ org,
-    const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,
+    const BNode8* __restrict__ nodes, const NodeLeaves* __restrict__ leaves,
+    const LTri* __restrict__ tris, const float* __restrict__ org, const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,
     uint32_t n, uint32_t range, int mode, float* t_o, float* u_o, float* v_o, int* prim_o,
     uint32_t* ovf, uint32_t ovf_words, uint32_t* ctr, int* err) {
   __shared__ __align__(16) uint32_t lds[(kQBlock / 64) * kTravLdsWords];
@@ -1510,7 +1527,7 @@ __global__ void __launch_bounds__(kQBlock, 4) kTraceRays(
     }
     const bool live = (active || helping) && !travDone(s);
     travNodePhase(s, st, tc, live, nodes);
-    travLeafPhase(s, st, tc, live, nodes, tris, area);
+    travLeafPhase(s, st, tc, live, leaves, tris, area);
     if (shared) travFollow(s, helping);
     if (exhausted) {
       helping = helping && !travDone(s);
@@ -1564,8 +1581,8 @@ void traceRaysDevice(Ctx* c, const float* d_org, const float* d_dir, const float
     uint32_t* ctr = (uint32_t*)((char*)c->q_out.p + ovf_bytes);  // work counter, error word
     kClearWords<<<1, 2, 0, c->stream>>>(ctr);
     kTraceRays<<<q.grid, kQBlock, 0, c->stream>>>(
-        c->pool.nodes.as<BNode8>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org + at * 3,
-        d_dir + at * 3, d_tnear + at, d_tfar + at, (uint32_t)m, q.range, mode, d_t + at, d_u + at,
+        c->pool.nodes.as<BNode8>() + D.node_off, c->pool.leaves.as<NodeLeaves>() + D.node_off,
+        c->pool.tris.as<LTri>() + D.tri_off, d_org + at * 3, d_dir + at * 3, d_tnear + at, d_tfar + at, (uint32_t)m, q.range, mode, d_t + at, d_u + at,
         d_v + at, d_prim + at, c->q_out.as<uint32_t>(), q.words, ctr, (int*)(ctr + 1));
     int h = 0;
     SPRAY_HIP(hipMemcpyAsync(&h, ctr + 1, 4, hipMemcpyDeviceToHost, c->stream));
@@ -1625,7 +1642,8 @@ void traceRaysNoAlloc(Ctx* c, const float* d_org, const float* d_dir, const floa
   int* err = (int*)(ctr + 1);
   kClearWords<<<1, 2, 0, c->stream>>>(ctr);
   kTraceRays<<<q.grid, kQBlock, 0, c->stream>>>(
-      c->pool.nodes.as<BNode8>() + D.node_off, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
+      c->pool.nodes.as<BNode8>() + D.node_off, c->pool.leaves.as<NodeLeaves>() + D.node_off,
+      c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir,
       d_tnear, d_tfar, (uint32_t)n, q.range, mode, d_t, d_u, d_v, d_prim, ovf, q.words, ctr, err);
   SPRAY_HIP(hipGetLastError());
   int h = 0;

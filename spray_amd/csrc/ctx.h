@@ -68,7 +68,7 @@ struct DomainPool {
   std::vector<long long> nverts; // vertices per domain as loaded
   DevBuf d_desc;                 // DomainDesc[ndomains]
   DevBuf vtx, face, rgb, nrm;    // float3 / uint3 / uint32 / float3
-  DevBuf nodes;                  // BNode8
+  DevBuf nodes, leaves;          // BNode8, NodeLeaves
   DevBuf tris;                   // LTri (leaf order)
   DevBuf fshade;                 // float4[3] per face: vertex normal xyz + vertex rgb bits
   std::vector<int> bvh_depth;
@@ -80,7 +80,7 @@ struct DomainPool {
   bool paged = false;
   int capacity = 0;
   long long block_nodes = 0, block_tris = 0;
-  void* h_image = nullptr;                // pinned: per domain nodes, tris, shading records
+  void* h_image = nullptr;                // pinned: per domain nodes, their leaves, tris, shading records
   std::vector<long long> h_image_off;     // byte offset of each domain's image
   std::vector<std::vector<float>> h_nrm;  // per-domain vertex normals (query API)
   DomainDesc* h_desc_pinned = nullptr;    // staging for descriptor uploads
@@ -99,6 +99,7 @@ struct DomainPool {
     rgb.release();
     nrm.release();
     nodes.release();
+    leaves.release();
     tris.release();
     fshade.release();
     releasePaging();

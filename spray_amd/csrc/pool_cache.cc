@@ -40,9 +40,9 @@ void DomainPool::releasePaging() {
   tick = hits = misses = bytes_in = 0;
 }
 
-// Bytes of domain d's image: nodes, leaf-ordered triangles, shading records.
+// Bytes of domain d's image: nodes, their leaves, leaf-ordered triangles, shading records.
 static size_t imageBytes(const DomainDesc& D) {
-  return (size_t)D.num_nodes * sizeof(BNode8) + (size_t)D.num_tris * (sizeof(LTri) + 48);
+  return (size_t)D.num_nodes * (sizeof(BNode8) + sizeof(NodeLeaves)) + (size_t)D.num_tris * (sizeof(LTri) + 48);
 }
 
 // Points domain d's descriptor at block b (host copy and device copy, the
@@ -94,12 +94,15 @@ static int lruLoad(Ctx* c, int d, int keep) {
   const char* src = (const char*)P.h_image + P.h_image_off[d];
   hipStream_t cs = P.copy_stream;
   SPRAY_HIP(hipStreamWaitEvent(cs, P.block_free[victim], 0));
-  const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), tb = (size_t)D.num_tris * sizeof(LTri);
+  const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), lb = (size_t)D.num_nodes * sizeof(NodeLeaves),
+               tb = (size_t)D.num_tris * sizeof(LTri);
   SPRAY_HIP(hipMemcpyAsync(P.nodes.as<BNode8>() + (size_t)victim * P.block_nodes, src, nb,
                            hipMemcpyHostToDevice, cs));
-  SPRAY_HIP(hipMemcpyAsync(P.tris.as<LTri>() + (size_t)victim * P.block_tris, src + nb, tb,
+  SPRAY_HIP(hipMemcpyAsync(P.leaves.as<NodeLeaves>() + (size_t)victim * P.block_nodes, src + nb, lb,
                            hipMemcpyHostToDevice, cs));
-  SPRAY_HIP(hipMemcpyAsync(P.fshade.as<float4>() + (size_t)victim * P.block_tris * 3, src + nb + tb,
+  SPRAY_HIP(hipMemcpyAsync(P.tris.as<LTri>() + (size_t)victim * P.block_tris, src + nb + lb, tb,
+                           hipMemcpyHostToDevice, cs));
+  SPRAY_HIP(hipMemcpyAsync(P.fshade.as<float4>() + (size_t)victim * P.block_tris * 3, src + nb + lb + tb,
                            (size_t)D.num_tris * 48, hipMemcpyHostToDevice, cs));
   bindBlock(P, d, victim, cs);
   SPRAY_HIP(hipEventRecord(P.block_ready[victim], cs));

@@ -98,26 +98,29 @@ int scenegenWrite(const spray_scenegen_params& p, const char* dir, const char* n
 // ---------------------------------------------------------------------------
 // Device layouts (shared by host and kernels)
 
-// One 8-wide BVH node in 128 bytes, one L2 line.  Child boxes are 8-bit
+// One 8-wide BVH node: the 64 bytes that a visit reads.  Child boxes are 8-bit
 // plane numbers on the node's own grid: plane q of axis k lies at
-// base[k] + q * 2^e[k].  plane[k][0..7] / plane[k][8..15] are the children's
-// lower / upper planes by slot, rounded outwards (quantizeNode).  meta holds
-// the biased exponents (e[k] + 127 in byte k) and, in byte 3, the slots that
-// are inner nodes; those are numbered consecutively from child_base in slot
-// order.  The other slots are leaves: leaf[slot] has the triangle count in
-// bits 24..30 (0: unused slot, its box inverted) and the first triangle in
-// bits 0..23.  A child's slot says on which side of the node it lies (bit k:
-// the upper side of axis k), so that a ray meets the slots roughly in the
-// order of slot ^ (its direction's signs).
-struct alignas(128) BNode8 {
+// base[k] + q * 2^e[k], and the last byte of base[k], part of its value, is
+// e[k] + 127.  plane[k][0..7] / plane[k][8..15] are the children's lower /
+// upper planes by slot, rounded outwards (quantizeNode).  kids has the slots
+// that are inner nodes in bits 24..31; those are numbered consecutively in
+// slot order from bits 0..23.  The other slots are leaves, described beside
+// the nodes (NodeLeaves).  A child's slot says on which side of the node it
+// lies (bit k: the upper side of axis k), so that a ray meets the slots
+// roughly in the order of slot ^ (its direction's signs).
+struct alignas(64) BNode8 {
   float base[3];
-  uint32_t child_base;
+  uint32_t kids;
   uint8_t plane[3][16];
-  uint32_t meta;
-  uint32_t pad[7];
+};
+static_assert(sizeof(BNode8) == 64, "BNode8 must be 64 bytes");
+
+// A node's leaves by slot: the triangle count in bits 24..30 (0: an inner
+// node, or an unused slot, its box inverted) and the first triangle in bits
+// 0..23.
+struct alignas(32) NodeLeaves {
   uint32_t leaf[8];
 };
-static_assert(sizeof(BNode8) == 128, "BNode8 must be 128 bytes");
 
 // Triangle in leaf order: 48 bytes; v0.w holds the primitive id.
 struct alignas(16) LTri {

@@ -1487,7 +1487,7 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
     }
     const bool live = (active || helping) && !travDone(s);
     travNodePhase(s, st, tc, live, P.nodes);
-    travLeafPhase(s, st, tc, live, P.nodes, P.tris, area);
+    travLeafPhase(s, st, tc, live, P.leaves, P.tris, area);
     if (shared) travFollow(s, helping);
     if (exhausted) {
       helping = helping && !travDone(s);
@@ -1976,6 +1976,7 @@ static TraceParams makeParams(Ctx* c) {
   P.desc = pool.d_desc.as<DomainDesc>();
   P.dbox = c->tracer->dbox.as<float4>();
   P.nodes = pool.nodes.as<BNode8>();
+  P.leaves = pool.leaves.as<NodeLeaves>();
   P.tris = pool.tris.as<LTri>();
   P.vtx = pool.vtx.as<float>();
   P.face = pool.face.as<uint32_t>();

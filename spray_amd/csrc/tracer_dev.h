@@ -88,6 +88,7 @@ struct TraceParams {
   // gridIdsBytes)
   const float4* dbox;
   const BNode8* nodes;
+  const NodeLeaves* leaves;
   const LTri* tris;
   const float* vtx;
   const uint32_t* face;

@@ -1,17 +1,21 @@
 // Closest-hit and any-hit traversal of one domain's 8-wide BVH.
 //
-// What bounds it: vector instructions (issued 75% of the time on a 64-domain
-// 1024x1024 8 spp frame, two thirds of them in node visits) and L2 misses
-// (a random 128-byte line costs the same as a random 64-byte one, and the
-// card serves about 57 G of them a second; the kernel takes about 30 G).
-// Eight children in one line against four in half a line: 20% fewer node
-// visits, 32% fewer wave steps (a step keeps 68% of the lanes busy, 57%
-// before, as a lane no longer stops at its second leaf).  Trace time of a
-// pass, 4-wide -> 8-wide: 256x192 2 spp plain schedule 9.1 -> 7.8 ms,
-// ambient occlusion 512x512 1.11 -> 1.03 ms, 256 uneven domains 13.9 -> 13.5
-// ms, 64 even domains 17.4 -> 17.6 ms.  Tried on it and left out: choosing
-// the nearest child by its entry distance (as many visits as in slot order,
-// 3% slower); node lines fetched by four lanes each through LDS (5% slower).
+// What bounds it: vector instructions (issued 70% of the time on a 64-domain
+// 1024x1024 8 spp frame, two thirds of them in node visits), the address unit
+// (60%: one lane a cycle and load) and, behind them, L2 misses.  So a visit
+// reads 64 bytes in four loads, and what only leaves need lies elsewhere: one
+// more dword load a visit costs 3%, and a node of 128 bytes in five loads took
+// 16.07 ms where this takes 15.54 (256 uneven domains 10.5 -> 10.2, ambient
+// occlusion 0.89 -> 0.86).
+// Eight children against four: 20% fewer node visits, 32% fewer wave steps (a
+// step keeps 68% of the lanes busy, 57% before, as a lane no longer stops at
+// its second leaf).  Trace time of a pass, 4-wide -> 8-wide: 256x192 2 spp
+// plain schedule 9.1 -> 7.8 ms, ambient occlusion 512x512 1.11 -> 1.03 ms, 256
+// uneven domains 13.9 -> 13.5 ms, 64 even domains 17.4 -> 17.6 ms.  Tried on
+// it and left out: choosing the nearest child by its entry distance (as many
+// visits as in slot order, 3% slower); node lines fetched by four lanes each
+// through LDS (5% slower); leaves of 3 or 4 triangles (3 and 5% slower); five
+// waves a SIMD with half the LDS stack and triangles one at a time (a wash).
 //
 // Per-lane stack of node groups (a group: the children of one node that the
 // ray has still to visit): the first kRing entries in LDS.  Each wave owns
@@ -49,9 +53,8 @@ constexpr uint32_t kMaxNodeVisits = 1u << 24;
 typedef __attribute__((address_space(3))) uint32_t lds_u32;
 
 // n counts the entries, the sentinel (an empty group) at the bottom included.
-// A group is (index of the node's first inner child, children left to visit
-// by their visiting order in bits 0..7 and the node's inner slots in bits
-// 8..15); only the sentinel has no children left.
+// A group is (the node's kids word, children left to visit by their visiting
+// order in bits 0..7); only the sentinel has no children left.
 struct LaneStack {
   typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
   typedef __attribute__((address_space(3))) u32x2 lds_u2;
@@ -134,16 +137,16 @@ __device__ __forceinline__ uint32_t pickBits(uint32_t m, uint32_t a, uint32_t b)
 // product with a possibly infinite inv; 0 * inf = NaN (the origin on the
 // plane) bounds nothing, as max and min drop NaN operands.
 template <bool kSafe>
-__device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)[3], uint32_t meta,
-                                              const float org[3], const float inv[3], float tnear,
-                                              float tfar) {
+__device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)[3], const float org[3],
+                                              const float inv[3], float tnear, float tfar) {
   const float bo[3] = {__uint_as_float(w0.x) - org[0], __uint_as_float(w0.y) - org[1],
                        __uint_as_float(w0.z) - org[2]};
+  const uint32_t wb[3] = {w0.x, w0.y, w0.z};
   uint32_t nq[3][2], fq[3][2];
   float m[3], c[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const float scale = __uint_as_float(((meta >> (8 * k)) & 255u) << 23);
+    const float scale = __uint_as_float((wb[k] << 23) & 0x7f800000u);
     const uint32_t neg = (uint32_t)((int32_t)__float_as_uint(inv[k]) >> 31);
     nq[k][0] = pickBits(neg, pl[k].z, pl[k].x);
     nq[k][1] = pickBits(neg, pl[k].w, pl[k].y);
@@ -236,6 +239,11 @@ __device__ __forceinline__ uint32_t permuteSlots(uint32_t m, uint32_t o) {
   return (o & 4u) ? (m >> 4) | ((m & 0x0fu) << 4) : m;
 }
 
+// The child in `slot` of a node with this kids word.
+__device__ __forceinline__ uint32_t groupChild(uint32_t kids, uint32_t slot) {
+  return (kids & 0xffffffu) + (uint32_t)__popc(__builtin_amdgcn_ubfe(kids, 24u, slot));
+}
+
 // One node: leaves that the ray hits are listed, the inner children become a
 // group, and `cur` the first child of that group, or of the group on top of
 // the stack when there is none.  The top group is read beside the node, so
@@ -247,28 +255,27 @@ __device__ __forceinline__ void travNode(TravState& s, LaneStack& st,
   const BNode8* nd = &nodes[s.node_base + s.cur];
   const uint4 w0 = ((const uint4*)nd)[0];
   const uint4 pl[3] = {((const uint4*)nd)[1], ((const uint4*)nd)[2], ((const uint4*)nd)[3]};
-  const uint32_t meta = nd->meta;
   const bool fast = st.n < (uint32_t)kRing;
   u32x2 top = st.lane[(min(st.n, (uint32_t)kRing) - 1u) << 6];
   if (!fast) top = st.get(st.n - 1u);
-  const uint32_t mask = nodeBoxes<kSafe>(w0, pl, meta, s.org, s.inv, s.tnear, s.tlim);
-  const uint32_t im = meta >> 24, leaves = mask & ~im;
+  const uint32_t mask = nodeBoxes<kSafe>(w0, pl, s.org, s.inv, s.tnear, s.tlim);
+  const uint32_t im = w0.w >> 24, leaves = mask & ~im;
   st.list[(s.listed & 255u) << 6] = (s.cur << 8) | leaves;  // kept when it has leaves
   s.listed += leaves ? 1u + ((uint32_t)__popc(leaves) << 8) : 0u;
   const uint32_t oct = (s.kk >> 16) & 7u;
   const uint32_t pm = permuteSlots(mask & im, oct);
   const bool down = pm != 0u;
-  const uint32_t gb = down ? w0.w : top.x, gm = down ? pm | (im << 8) : top.y;
+  const uint32_t gb = down ? w0.w : top.x, gm = down ? pm : top.y;
   const uint32_t slot = ((uint32_t)__ffs((int)gm) - 1u) ^ oct;
   // the inner children below `slot` come before it
-  const uint32_t child = gb + (uint32_t)__popc(__builtin_amdgcn_ubfe(gm, 8u, slot));
+  const uint32_t child = groupChild(gb, slot);
   uint32_t rest = gm & (gm - 1u);
   const uint32_t at = down ? st.n : st.n - 1u;
   if (at < (uint32_t)kRing)
     st.lane[at << 6] = u32x2{gb, rest};
   else if (!st.put(at, u32x2{gb, rest}))
     rest = 0u;
-  st.n = at + ((rest & 255u) ? 1u : 0u);
+  st.n = at + (rest ? 1u : 0u);
   s.cur = gm ? child : kStackEmpty;
 }
 
@@ -357,7 +364,7 @@ __device__ __forceinline__ uint32_t orderedT(float t) {  // monotone bits; -0 as
 
 // Every lane of the wave calls it, converged (area: the wave's LDS).
 __device__ __forceinline__ void travLeafPhase(TravState& s, LaneStack& st, TravCount& cnt,
-                                              bool active, const BNode8* __restrict__ nodes,
+                                              bool active, const NodeLeaves* __restrict__ leaves,
                                               const LTri* __restrict__ tris, uint32_t* area) {
   typedef __attribute__((address_space(3))) unsigned long long lds_u64;
   typedef __attribute__((address_space(3))) float lds_f;
@@ -392,7 +399,7 @@ __device__ __forceinline__ void travLeafPhase(TravState& s, LaneStack& st, TravC
     const uint32_t it = in ? items[base + lane] : (uint32_t)lane << 26;
     const int own = (int)(it >> 26);
     const uint32_t nb = laneGet(s.node_base, own), tb = laneGet(s.tri_base, own);
-    const uint32_t word = in ? nodes[nb + ((it >> 3) & 0x7fffffu)].leaf[it & 7u] : 0u;
+    const uint32_t word = in ? leaves[nb + ((it >> 3) & 0x7fffffu)].leaf[it & 7u] : 0u;
     const uint32_t kk = laneGet(s.kk, own);
     const RayPre rp{(int)(kk & 3u), (int)((kk >> 2) & 3u), (int)((kk >> 4) & 3u),
                     laneGetF(s.Sx, own), laneGetF(s.Sy, own), laneGetF(s.Sz, own)};
@@ -513,11 +520,11 @@ __device__ __forceinline__ bool travShare(TravState& s, LaneStack& st, bool idle
     s.guard = 0;
     s.share = (uint32_t)own | (1u << 8);
     const uint32_t slot = ((uint32_t)__ffs((int)gm) - 1u) ^ ((kk >> 16) & 7u);
-    s.cur = gb + (uint32_t)__popc(__builtin_amdgcn_ubfe(gm, 8u, slot));
+    s.cur = groupChild(gb, slot);
     const uint32_t rest = gm & (gm - 1u);
     st.lane[0] = u32x2{0u, 0u};
     st.lane[64] = u32x2{gb, rest};
-    st.n = (rest & 255u) ? 2u : 1u;
+    st.n = rest ? 2u : 1u;
   }
   ldsWaveSync();
   return take;
