@@ -1014,10 +1014,10 @@ struct PlocScratch {
 // Build memory: slots of each pipeline, domain descriptors and scan jobs,
 // level counters of every domain.
 struct BuildCache {
-  std::vector<DevBuf> slots;
+  DevBuf slots;
   DevBuf descs, levels;
   ~BuildCache() {
-    for (DevBuf& b : slots) b.release();
+    slots.release();
     descs.release();
     levels.release();
   }
@@ -1046,8 +1046,9 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
   if (keep_buffers && !paged && !P.paged) {
     P.desc.clear();  // device buffers stay; they grow when too small
   } else {
-    P.release();
+    P.release(!paged);
   }
+  if (paged && !c->tracer) c->frame_mem.release();
   P.ndomains = nd;
   P.desc.resize(nd);
   P.nverts.resize(nd);
@@ -1107,14 +1108,24 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.h_nrm.resize(nd);
     SPRAY_HIP(hipStreamCreate(&P.copy_stream));
   } else {
-    P.vtx.reserve(tv * 12);
-    P.face.reserve(tf * 12);
-    P.rgb.reserve(tv * 4);
-    P.nrm.reserve(tv * 12);
-    P.tris.reserve(tf * sizeof(LTri));
-    P.fshade.reserve(tf * 48 + 64);
-    P.nodes.reserve(tn * sizeof(BNode8));
-    P.leaves.reserve(tn * sizeof(NodeLeaves));
+    BufPlan plan;
+    plan.want(P.vtx, tv * 12);
+    plan.want(P.face, tf * 12);
+    plan.want(P.rgb, tv * 4);
+    plan.want(P.nrm, tv * 12);
+    plan.want(P.tris, tf * sizeof(LTri));
+    plan.want(P.fshade, tf * 48 + 64);
+    plan.want(P.nodes, tn * sizeof(BNode8));
+    plan.want(P.leaves, tn * sizeof(NodeLeaves));
+    if (!plan.fits()) {
+      try {
+        plan.place(P.mem);
+      } catch (const StatusError&) {
+        if (c->tracer || !c->frame_mem.p) throw;
+        c->frame_mem.release();  // the last scene's frame memory makes room
+        plan.place(P.mem);
+      }
+    }
   }
   // A whole-scene LBVH build takes the domains in groups, one launch per
   // build step for a group, up to kBuildStreams groups side by side (one per
@@ -1153,8 +1164,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
                                                                      kSlotBudget / ((size_t)K * SL.bytes)}))
                        : 1;
   const int ngroups = (nd + GN - 1) / GN;
-  if ((int)M->slots.size() < K) M->slots.resize(K);
-  for (int k = 0; k < K; ++k) M->slots[k].reserve((size_t)GN * SL.bytes);
+  M->slots.reserve((size_t)K * GN * SL.bytes);
   M->levels.reserve((size_t)nd * kLevelWords * 4 + 64);
   M->descs.reserve((size_t)nd * (sizeof(BuildDom) + 2 * sizeof(ScanJob)) + 64);
   const BuildDom* dev = M->descs.as<BuildDom>();
@@ -1172,7 +1182,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
         D.node_off = (long long)b * P.block_nodes;
         D.tri_off = D.shade_off = (long long)b * P.block_tris;
       }
-      char* slot = M->slots[(d / GN) % K].as<char>() + (size_t)(d % GN) * SL.bytes;
+      char* slot = M->slots.as<char>() + ((size_t)((d / GN) % K) * GN + d % GN) * SL.bytes;
       BuildDom& B = hb[d];
       B.vtx = P.vtx.as<float>() + D.vtx_off * 3;
       B.face = P.face.as<uint32_t>() + D.face_off * 3;
@@ -1298,7 +1308,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     int depth = nf <= kLeafMax ? 1 : -1;
     if (ploc && depth < 0) {
       // PLOC passes until one cluster is left
-      const char* slot = M->slots[0].as<char>();  // one-domain builds use slot 0
+      const char* slot = M->slots.as<char>();  // one-domain builds use slot 0
       int4* T = (int4*)(slot + SL.tree);
       float* inner = (float*)(slot + SL.ib);
       const uint32_t* va = (const uint32_t*)(slot + SL.vals[0]);

@@ -175,6 +175,7 @@ void spray_destroy(spray_ctx* ctx) {
   tracerRelease(&ctx->c);
   predictorRelease(&ctx->c);
   ctx->c.pool.release();
+  ctx->c.frame_mem.release();
   ctx->c.q_in.release();
   ctx->c.q_out.release();
   ctx->c.gen_store.release();

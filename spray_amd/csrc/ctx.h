@@ -37,11 +37,13 @@ struct StatusError {
 struct DevBuf {
   void* p = nullptr;
   size_t bytes = 0;
+  bool piece = false;  // of an allocation that another buffer owns (BufPlan)
   void reserve(size_t b) {
     if (b <= bytes) return;
-    if (p) SPRAY_HIP(hipFree(p));
+    if (p && !piece) SPRAY_HIP(hipFree(p));
     p = nullptr;
     bytes = 0;
+    piece = false;
     if (hipMalloc(&p, b) != hipSuccess) {
       p = nullptr;
       (void)hipGetLastError();
@@ -54,9 +56,45 @@ struct DevBuf {
     return (T*)p;
   }
   void release() {
-    if (p) (void)hipFree(p);
+    if (p && !piece) (void)hipFree(p);
     p = nullptr;
     bytes = 0;
+    piece = false;
+  }
+};
+
+// Buffers that are sized together lie in one allocation, kept for the next
+// scene unless that needs less than a quarter of it: freed and allocated one
+// by one (a free waits for the device and unmaps, 0.25 to 0.7 ms for a large
+// buffer), the 33 buffers of a frame, the 9 of a scene and the 4 of a build took
+// 6 of the 12 ms from loading 27 domains to their first image, and a new
+// context's first 96x72 frame 1.6 ms (now 0.9).  Buffers only grow; none keeps
+// its contents when any of them does.
+struct BufPlan {
+  std::vector<std::pair<DevBuf*, size_t>> items;
+  void want(DevBuf& b, size_t bytes) { items.push_back({&b, std::max(bytes, b.bytes)}); }
+  bool fits() const {
+    for (const auto& w : items)
+      if (w.second > w.first->bytes) return false;
+    return true;
+  }
+  void place(DevBuf& mem) {
+    size_t total = 0;
+    for (const auto& w : items) {
+      w.first->release();
+      total += (w.second + 255) & ~(size_t)255;
+    }
+    if (mem.bytes < total || mem.bytes / 4 > total + ((size_t)64 << 20)) {
+      mem.release();
+      mem.reserve(total);
+    }
+    char* at = mem.as<char>();
+    for (const auto& w : items) {
+      w.first->p = at;
+      w.first->bytes = w.second;
+      w.first->piece = true;
+      at += (w.second + 255) & ~(size_t)255;
+    }
   }
 };
 
@@ -66,6 +104,7 @@ struct DomainPool {
   long long total_tris = 0, total_verts = 0, total_nodes = 0;
   std::vector<DomainDesc> desc;  // host copy
   std::vector<long long> nverts; // vertices per domain as loaded
+  DevBuf mem;                    // holds the buffers below of a scene resident as a whole
   DevBuf d_desc;                 // DomainDesc[ndomains]
   DevBuf vtx, face, rgb, nrm;    // float3 / uint3 / uint32 / float3
   DevBuf nodes, leaves;          // BNode8, NodeLeaves
@@ -92,7 +131,7 @@ struct DomainPool {
   unsigned long long tick = 0, hits = 0, misses = 0, bytes_in = 0;
   hipStream_t copy_stream = nullptr;
   void releasePaging();
-  void release() {
+  void release(bool keep_mem = false) {
     d_desc.release();
     vtx.release();
     face.release();
@@ -102,6 +141,7 @@ struct DomainPool {
     leaves.release();
     tris.release();
     fshade.release();
+    if (!keep_mem) mem.release();
     releasePaging();
     desc.clear();
     ndomains = 0;
@@ -208,6 +248,7 @@ struct Predictor;    // mlp.hip
 // Smallest sample budget of a batch of blocking tiles (the budget grows with
 // the HBM left after the scene is loaded).
 constexpr long long kBatchSamples = 8ll << 20;
+constexpr size_t kKeepFrameMem = (size_t)4 << 30;
 
 struct BuildCache;  // bvh.hip: build scratch kept between remeshes
 
@@ -221,6 +262,7 @@ struct Ctx {
   CameraDev cam;
   bool camera_set = false;
   TracerState* tracer = nullptr;
+  DevBuf frame_mem;  // holds the tracer's buffers; kept when the scene changes (up to kKeepFrameMem)
   Predictor* pred = nullptr;
   int batch_chunk = 16;  // refill threshold of the trace kernel (idle lanes per wave)
   int tiles_in_flight = 0;  // blocking tiles traced together (batched forms); 0 = automatic

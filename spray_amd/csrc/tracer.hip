@@ -1610,6 +1610,21 @@ __global__ void kWindowEnd(TraceParams P) {
   }
   blockFlush<2>(c, {kStatUseful, kStatHits}, {waveSumULL(useful), waveSumULL(hits)});
 }
+// A frame's start: an empty image and counters; a batch's: its rows.  One
+// launch for two fills and one for a copy, the domain boxes uploaded only when
+// the configuration changed, and no query of the free HBM where one tile is
+// all there is: a 96x72 frame without its image 432 -> 360 us.
+__global__ void kFrameClear(float4* image, long long pixels, DevCounters* c) {
+  const long long i0 = blockIdx.x * (long long)blockDim.x + threadIdx.x, n = (long long)gridDim.x * blockDim.x;
+  for (long long i = i0; i < pixels; i += n) image[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  for (long long i = i0; i < (long long)(sizeof(DevCounters) / 4); i += n) ((uint32_t*)c)[i] = 0u;
+}
+__global__ void kTileRec(int* rec, int row, int rows) {
+  rec[0] = row;
+  rec[1] = rows;
+  rec[2] = rec[3] = 0;
+}
+
 __global__ void kWindowAdvance(TraceParams P) {
   int* rec = (int*)P.tile_rec;
   rec[2] += kHistory;
@@ -1665,6 +1680,7 @@ __global__ void kLogFinalize(TraceParams P) {
 // ---------------------------------------------------------------------------
 // Host side
 struct TracerState {
+  int box_version = -1;  // configuration version of the uploaded domain boxes
   long long S = 0;  // samples of the largest tile
   uint32_t r_cap = 0, s_cap = 0, p_cap = 0, q_cap[2] = {0, 0}, sh_cap = 0, mask_cap = 0;
   int ndomains = 0;
@@ -1697,14 +1713,7 @@ struct TracerState {
   int slog_max = 0;
   std::vector<int> slog_meta, slog_order;
   std::vector<unsigned long long> slog_scores;
-  size_t heldBytes() const {
-    size_t b = log_ctr.bytes;
-    for (const DevBuf* x : {&R, &Pn, &Sh, &vbuf, &image, &ctr, &tile_rec, &cnt, &off, &dbase, &bcnt,
-                            &bbase, &wctr, &wq, &score, &order, &q[0], &q[1], &ask, &ask_cnt, &rkey,
-                            &dmask, &dfmt, &dbox, &ovf, &vlog, &log, &sh_rec, &qa, &qb, &dflag, &acnt})
-      b += x->bytes;
-    return b;
-  }
+  size_t heldBytes() const { return ovf.bytes + vlog.bytes + log.bytes + log_ctr.bytes; }  // beside frame_mem
   // learned form: the predictor's stream beside the schedule and scatter
   // (forked from and joined back to the tracer's stream, graph capture included)
   hipStream_t aux = nullptr;
@@ -1770,10 +1779,8 @@ void tracerRelease(Ctx* c) {
   }
   for (hipEvent_t e : {T->fork_ev, T->join_ev})
     if (e) (void)hipEventDestroy(e);
-  for (DevBuf* b : {&T->R, &T->Pn, &T->Sh, &T->vbuf, &T->image, &T->ctr, &T->tile_rec, &T->cnt,
-                    &T->off, &T->dbase, &T->bcnt, &T->bbase, &T->wctr, &T->wq, &T->score, &T->order, &T->q[0],
-                    &T->q[1], &T->ask, &T->ask_cnt, &T->rkey, &T->dmask, &T->dfmt, &T->dbox, &T->ovf, &T->vlog, &T->log, &T->sh_rec, &T->log_ctr, &T->qa, &T->qb, &T->dflag, &T->acnt})
-    b->release();
+  for (DevBuf* b : {&T->ovf, &T->vlog, &T->log, &T->log_ctr}) b->release();
+  if (c->frame_mem.bytes > kKeepFrameMem) c->frame_mem.release();
   delete T;
   c->tracer = nullptr;
 }
@@ -1839,12 +1846,14 @@ static void ensureState(Ctx* c, double grow) {
   const spray_config& cfg = c->cfg;
   std::vector<int> ys, hs;
   tileList(cfg, &ys, &hs);
-  {  // automatic batches: samples whose state takes at most 40% of the HBM the
+  // (one tile is one batch whatever the HBM holds)
+  if (hs.size() > 1 && cfg.schedule != SPRAY_SCHEDULE_PLAIN && c->tiles_in_flight <= 0) {
+    // automatic batches: samples whose state takes at most 40% of the HBM the
      // tracer can use (free plus what it already holds), so that one grown
      // retry still fits
     size_t free_b = 0, total_b = 0;
     SPRAY_HIP(hipMemGetInfo(&free_b, &total_b));
-    const double held = c->tracer ? (double)c->tracer->heldBytes() : 0.0;
+    const double held = (double)c->frame_mem.bytes + (c->tracer ? (double)c->tracer->heldBytes() : 0.0);
     c->batch_samples = (long long)(0.40 * ((double)free_b + held) / stateBytesPerSample(c));
   }
   const int per_batch = cfg.schedule != SPRAY_SCHEDULE_PLAIN ? tilesPerBatch(c, hs) : 1;
@@ -1885,44 +1894,49 @@ static void ensureState(Ctx* c, double grow) {
   T->q_cap[0] = std::max(T->q_cap[0], q0);
   T->q_cap[1] = std::max(T->q_cap[1], q1);
   T->mask_cap = std::max(T->mask_cap, mask_cap);
-  need(T, T->R, (size_t)T->r_cap * 64);
-  need(T, T->Pn, (size_t)T->p_cap * 64);
-  need(T, T->Sh, (size_t)T->s_cap * 64);
-  need(T, T->vbuf, (size_t)S * kHistory * 8);
-  if (cfg.schedule == SPRAY_SCHEDULE_LEARNED) {
-    need(T, T->ask, (size_t)kQueueGrid * askRegion(T->r_cap) * 48 + 64);
-    need(T, T->ask_cnt, (size_t)kQueueGrid * 4 + 64);
-    need(T, T->rkey, (size_t)T->r_cap * 4 + 64);
-  }
-  need(T, T->dmask, (size_t)T->mask_cap * maskRowWords(nd) * 8 + 64);
-  need(T, T->dfmt, (size_t)T->mask_cap + 64);
-  need(T, T->dbox, dboxBytes(nd));
-  need(T, T->ctr, sizeof(DevCounters));
-  need(T, T->tile_rec, 64);
-  need(T, T->cnt, (size_t)2 * nd * 4 + 64);
-  need(T, T->off, (size_t)2 * (nd + 1) * 4 + 64);
-  need(T, T->dbase, (size_t)2 * nd * 4 + 64);
-  need(T, T->bcnt, (size_t)2 * nd * kQueueGrid * 4 + 64);
-  need(T, T->bbase, (size_t)2 * nd * kQueueGrid * 4 + 64);
-  need(T, T->wctr, (size_t)(nd + 3) * 4 + 64);
-  need(T, T->wq, (size_t)3 * kWorkCounters * kWorkStride * 4);
-  need(T, T->qa, (size_t)T->q_cap[0] * 4);
-  need(T, T->qb, (size_t)T->q_cap[0] * 4);
-  if (cfg.schedule == SPRAY_SCHEDULE_LEARNED) {
-    need(T, T->dflag, ((size_t)T->q_cap[0] / 64 + 2) * 8);
-    need(T, T->acnt, (size_t)2 * kAssignWaves * 4 + 64);
-  }
+  // every buffer is planned, so that one which this frame does not use moves with the others
+  BufPlan plan;
+  auto want = [&](DevBuf& b, size_t bytes) { plan.want(b, bytes); };
+  want(T->R, (size_t)T->r_cap * 64);
+  want(T->Pn, (size_t)T->p_cap * 64);
+  want(T->Sh, (size_t)T->s_cap * 64);
+  want(T->vbuf, (size_t)S * kHistory * 8);
+  const size_t learned = cfg.schedule == SPRAY_SCHEDULE_LEARNED ? 1 : 0;
+  want(T->ask, learned * ((size_t)kQueueGrid * askRegion(T->r_cap) * 48 + 64));
+  want(T->ask_cnt, learned * ((size_t)kQueueGrid * 4 + 64));
+  want(T->rkey, learned * ((size_t)T->r_cap * 4 + 64));
+  want(T->dmask, (size_t)T->mask_cap * maskRowWords(nd) * 8 + 64);
+  want(T->dfmt, (size_t)T->mask_cap + 64);
+  want(T->dbox, dboxBytes(nd));
+  want(T->ctr, sizeof(DevCounters));
+  want(T->tile_rec, 64);
+  want(T->cnt, (size_t)2 * nd * 4 + 64);
+  want(T->off, (size_t)2 * (nd + 1) * 4 + 64);
+  want(T->dbase, (size_t)2 * nd * 4 + 64);
+  want(T->bcnt, (size_t)2 * nd * kQueueGrid * 4 + 64);
+  want(T->bbase, (size_t)2 * nd * kQueueGrid * 4 + 64);
+  want(T->wctr, (size_t)(nd + 3) * 4 + 64);
+  want(T->wq, (size_t)3 * kWorkCounters * kWorkStride * 4);
+  want(T->qa, (size_t)T->q_cap[0] * 4);
+  want(T->qb, (size_t)T->q_cap[0] * 4);
+  want(T->dflag, learned * (((size_t)T->q_cap[0] / 64 + 2) * 8));
+  want(T->acnt, learned * ((size_t)2 * kAssignWaves * 4 + 64));
   // shade records: one per accepted hit of a pass, far fewer than queue
   // entries (an overflow grows and re-renders like any other pool)
   T->sh_cap = std::min(T->q_cap[0], T->r_cap);
-  need(T, T->sh_rec, (size_t)T->sh_cap * kShadeRec * 16);
-  need(T, T->score, (size_t)nd * 8 + 64);
-  need(T, T->order, (size_t)nd * 4 + 64);
-  need(T, T->q[0], (size_t)T->q_cap[0] * sizeof(QEntry));
-  need(T, T->q[1], (size_t)T->q_cap[1] * sizeof(QEntry));
+  want(T->sh_rec, (size_t)T->sh_cap * kShadeRec * 16);
+  want(T->score, (size_t)nd * 8 + 64);
+  want(T->order, (size_t)nd * 4 + 64);
+  want(T->q[0], (size_t)T->q_cap[0] * sizeof(QEntry));
+  want(T->q[1], (size_t)T->q_cap[1] * sizeof(QEntry));
   T->h_cnt.resize(2 * nd);
   T->h_order.resize(nd);
-  need(T, T->image, (size_t)cfg.image_w * cfg.image_h * 16);
+  want(T->image, (size_t)cfg.image_w * cfg.image_h * 16);
+  if (!plan.fits()) {
+    T->releaseGraph();
+    T->box_version = -1;
+    plan.place(c->frame_mem);
+  }
   hipDeviceProp_t prop;
   SPRAY_HIP(hipGetDeviceProperties(&prop, c->device));
   // resident blocks: enough waves per CU to hide traversal latency
@@ -2442,9 +2456,11 @@ void tracerTraceFrame(Ctx* c, float* rgba_out, spray_stats* st) {
     }
     TraceParams P = makeParams(c);
     P.ovf = T->ovf.as<uint32_t>();
-    domainBoxesUpload(c, s);
-    SPRAY_HIP(hipMemsetAsync(P.image, 0, (size_t)cfg.image_w * cfg.image_h * 16, s));
-    SPRAY_HIP(hipMemsetAsync(P.ctr, 0, sizeof(DevCounters), s));
+    if (T->box_version != c->param_version) {
+      domainBoxesUpload(c, s);
+      T->box_version = c->param_version;
+    }
+    kFrameClear<<<T->num_cu, 256, 0, s>>>((float4*)P.image, (long long)cfg.image_w * cfg.image_h, P.ctr);
     int windows = (cfg.bounces + kHistory - 1) / kHistory;
     hipEvent_t e0, e1;
     SPRAY_HIP(hipEventCreate(&e0));
@@ -2481,9 +2497,8 @@ void tracerTraceFrame(Ctx* c, float* rgba_out, spray_stats* st) {
     for (size_t b0 = 0; b0 < ys.size(); b0 += per_batch) {
       int rows = 0;
       for (size_t ti = b0; ti < std::min(ys.size(), b0 + (size_t)per_batch); ++ti) rows += hs[ti];
-      int rec[4] = {ys[b0], rows, 0, 0};
       T->cur_tile = (int)b0;
-      SPRAY_HIP(hipMemcpyAsync(T->tile_rec.p, rec, sizeof(rec), hipMemcpyHostToDevice, s));
+      kTileRec<<<1, 1, 0, s>>>(T->tile_rec.as<int>(), ys[b0], rows);
       if (use_graph)
         SPRAY_HIP(hipGraphLaunch(exec, s));
       else
