@@ -796,6 +796,12 @@ __global__ void kCollapseInit(const BuildDom* __restrict__ G, int root) {
   if (threadIdx.x == 0) B.front[0][0] = root;
 }
 
+// Primitive ids in leaf order.
+__global__ void kPrimIds(const LTri* __restrict__ tris, int nf, uint32_t* order) {
+  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nf; i += gridDim.x * blockDim.x)
+    order[i] = __float_as_uint(tris[i].v0[3]);
+}
+
 // Root for tiny domains (<= kLeafMax triangles): one leaf child.  One group.
 __global__ void kTinyRoot(const BuildDom* __restrict__ G) {
   const int nf = G->nf, me = threadIdx.x;
@@ -1102,11 +1108,10 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     for (int d = 0; d < nd; ++d) {
       P.h_image_off[d] = (long long)bytes;
       const size_t nf = (size_t)P.desc[d].num_tris;
-      bytes += ((size_t)nodeCap((long long)nf) * (sizeof(BNode8) + sizeof(NodeLeaves)) + nf * (sizeof(LTri) + 48) + 255) & ~(size_t)255;
+      bytes += (ImageLayout(nodeCap((long long)nf), (long long)nf, P.nverts[d]).bytes + 255) & ~(size_t)255;
     }
     SPRAY_HIP(hipHostMalloc(&P.h_image, bytes, hipHostMallocDefault));
     P.h_nrm.resize(nd);
-    SPRAY_HIP(hipStreamCreate(&P.copy_stream));
   } else {
     BufPlan plan;
     plan.want(P.vtx, tv * 12);
@@ -1376,13 +1381,24 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     P.bvh_depth[d] = depth;
     if (paged) {  // the finished image goes to pinned host memory, the normals to the host
       char* dst = (char*)P.h_image + P.h_image_off[d];
-      const size_t nb = (size_t)D.num_nodes * sizeof(BNode8), lb = (size_t)D.num_nodes * sizeof(NodeLeaves),
-                   tb = (size_t)nf * sizeof(LTri);
-      SPRAY_HIP(hipMemcpyAsync(dst, P.nodes.as<BNode8>() + D.node_off, nb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb, P.leaves.as<NodeLeaves>() + D.node_off, lb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb + lb, P.tris.as<LTri>() + D.tri_off, tb, hipMemcpyDeviceToHost, s));
-      SPRAY_HIP(hipMemcpyAsync(dst + nb + lb + tb, P.fshade.as<float4>() + D.shade_off * 3,
-                               (size_t)nf * 48, hipMemcpyDeviceToHost, s));
+      const ImageLayout L(D.num_nodes, nf, nv);
+      auto put = [&](size_t off, const void* src, size_t n) {
+        SPRAY_HIP(hipMemcpyAsync(dst + off, src, n, hipMemcpyDeviceToHost, s));
+      };
+      put(0, P.nodes.as<BNode8>() + D.node_off, (size_t)D.num_nodes * sizeof(BNode8));
+      put(L.leaves, P.leaves.as<NodeLeaves>() + D.node_off, (size_t)D.num_nodes * sizeof(NodeLeaves));
+      if (L.indexed) {
+        uint32_t* order = (uint32_t*)(M->slots.as<char>() + SL.keys[1]);  // (the sort is done with it)
+        kPrimIds<<<gridFor(nf, 256), 256, 0, s>>>(P.tris.as<LTri>() + D.tri_off, nf, order);
+        put(L.order, order, (size_t)nf * 4);
+        put(L.face, P.face.p, (size_t)nf * 12);
+        put(L.vtx, P.vtx.p, (size_t)nv * 12);
+        put(L.nrm, P.nrm.p, (size_t)nv * 12);
+        put(L.rgb, P.rgb.p, (size_t)nv * 4);
+      } else {
+        put(L.tris, P.tris.as<LTri>() + D.tri_off, (size_t)nf * sizeof(LTri));
+        put(L.shade, P.fshade.as<float4>() + D.shade_off * 3, (size_t)nf * 48);
+      }
       P.h_nrm[d].resize((size_t)nv * 3);
       SPRAY_HIP(hipMemcpyAsync(P.h_nrm[d].data(), P.nrm.p, (size_t)nv * 12, hipMemcpyDeviceToHost, s));
       SPRAY_HIP(hipStreamSynchronize(s));

@@ -98,6 +98,35 @@ struct BufPlan {
   }
 };
 
+// A domain's image in pinned host memory, as byte offsets of its pieces: what
+// a miss copies into HBM.  Triangles and shading records of 96 bytes a
+// triangle are unpacked on the GPU from the mesh (vertices, normals, colours,
+// faces) and the leaf order, unless the mesh shares so few vertices that this
+// would be more.
+struct ImageLayout {
+  size_t leaves, order, face, vtx, nrm, rgb, tris, shade, bytes;  // (the nodes at 0)
+  bool indexed;
+  ImageLayout(long long nodes, long long nf, long long nv) {
+    indexed = 16 * nf + 28 * nv < 96 * nf;
+    size_t at = 0;
+    auto take = [&](long long n) {
+      const size_t o = at;
+      at += ((size_t)n + 15) & ~(size_t)15;
+      return o;
+    };
+    take(nodes * (long long)sizeof(BNode8));
+    leaves = take(nodes * (long long)sizeof(NodeLeaves));
+    order = take(indexed ? nf * 4 : 0);
+    face = take(indexed ? nf * 12 : 0);
+    vtx = take(indexed ? nv * 12 : 0);
+    nrm = take(indexed ? nv * 12 : 0);
+    rgb = take(indexed ? nv * 4 : 0);
+    tris = take(indexed ? 0 : nf * (long long)sizeof(LTri));
+    shade = take(indexed ? 0 : nf * 48);
+    bytes = at;
+  }
+};
+
 // HBM-resident domain pool (replaces the domain cache + Embree scenes)
 struct DomainPool {
   int ndomains = 0;
@@ -114,12 +143,12 @@ struct DomainPool {
   double build_ms = 0;
   // LRU paging (lru_cache.cc:41-171): with a cache smaller than the scene,
   // HBM holds `capacity` blocks of block_nodes nodes and block_tris
-  // triangles + shading records, and every domain's image (nodes, leaf-ordered
-  // triangles, shading records) stays in pinned host memory.
+  // triangles + shading records, and every domain's image (ImageLayout) stays
+  // in pinned host memory.
   bool paged = false;
   int capacity = 0;
   long long block_nodes = 0, block_tris = 0;
-  void* h_image = nullptr;                // pinned: per domain nodes, their leaves, tris, shading records
+  void* h_image = nullptr;                // pinned: the images
   std::vector<long long> h_image_off;     // byte offset of each domain's image
   std::vector<std::vector<float>> h_nrm;  // per-domain vertex normals (query API)
   DomainDesc* h_desc_pinned = nullptr;    // staging for descriptor uploads
@@ -129,7 +158,12 @@ struct DomainPool {
   std::vector<char> pending;              // prefetched, access not yet made
   std::vector<char> pinned;               // in use by the chunk being traced: never evicted
   unsigned long long tick = 0, hits = 0, misses = 0, bytes_in = 0;
-  hipStream_t copy_stream = nullptr;
+  // a missing domain's image is copied to a stage (copy_stream) and unpacked
+  // into its block (unpack_stream); the stages alternate
+  hipStream_t copy_stream = nullptr, unpack_stream = nullptr;
+  DevBuf stage[2];
+  hipEvent_t stage_full[2] = {}, stage_free[2] = {};
+  int next_stage = 0;
   void releasePaging();
   void release(bool keep_mem = false) {
     d_desc.release();
