@@ -151,9 +151,8 @@ int spray_trace_rays(spray_ctx* ctx, const spray_rays_soa* rays, size_t n,
  * DEVICE arrays: org[n*3], dir[n*3] (xyz per ray), tnear[n], tfar[n] in;
  * prim[n] out, and t/u/v[n] out for SPRAY_QUERY_CLOSEST (may be NULL for
  * SPRAY_QUERY_ANY).  It calls no hipMalloc/hipFree and no allocating
- * library routine: the traversal's scratch (overflow stacks, a work counter
- * and an error word, 29.4 MB) is a static device array of the
- * library, one per GPU, held until the process ends.  Every call on a GPU
+ * library routine: the traversal's scratch (overflow stacks, 29.4 MB) is a
+ * static device array of the library, one per GPU, held until the process ends.  Every call on a GPU
  * shares that GPU's array, so calls that overlap on one GPU race; the call
  * returns after its work on the context's stream has finished.  At most
  * 2^31 - 1 rays per call; the scene must be wholly resident (no partial

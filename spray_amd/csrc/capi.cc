@@ -157,6 +157,8 @@ int spray_create(const spray_config* cfg, spray_ctx** out) {
     ctx->c.device = cfg->device;
     SPRAY_HIP(hipSetDevice(cfg->device));
     SPRAY_HIP(hipStreamCreateWithFlags(&ctx->c.stream, hipStreamNonBlocking));
+    SPRAY_HIP(hipHostMalloc((void**)&ctx->c.q_err, 64, hipHostMallocDefault));
+    ctx->c.q_ctr.reserve(64);
     scratchInit(cfg->device);  // this device's copy of the no-allocation entry point's scratch
   });
   if (rc != SPRAY_OK) {
@@ -178,6 +180,8 @@ void spray_destroy(spray_ctx* ctx) {
   ctx->c.frame_mem.release();
   ctx->c.q_in.release();
   ctx->c.q_out.release();
+  ctx->c.q_ctr.release();
+  if (ctx->c.q_err) (void)hipHostFree(ctx->c.q_err);
   ctx->c.gen_store.release();
   buildCacheRelease(&ctx->c);
   if (ctx->c.stream) (void)hipStreamDestroy(ctx->c.stream);

@@ -310,6 +310,11 @@ struct Ctx {
   std::string err;
   // scratch for spray_trace_rays / spray_domain_list
   DevBuf q_in, q_out;
+  // a ray query's work counter, and its error flag in pinned host memory,
+  // which the kernel sets itself
+  DevBuf q_ctr;
+  int* q_err = nullptr;
+  int q_resident = 0;  // query blocks the GPU holds at once
   // a scene made by the GPU generator (spray_scenegen_load) can be remeshed;
   // the generator's per-domain buffers stay allocated between remeshes
   bool generated = false;
