@@ -36,7 +36,6 @@
 
 namespace spray {
 
-constexpr int kBlock = 256;
 // grid of kCount and kScatter (they must match: blocks own queue slots)
 constexpr int kQueueGrid = 1024;
 // and their threads per block, a block's entries for one domain and round
@@ -123,7 +122,6 @@ static_assert((kWorkCounters & (kWorkCounters - 1)) == 0, "a wave steps through 
 constexpr int kCountRefill = 16;
 // Shade slots are taken kShadeChunk at a time per wave.
 constexpr uint32_t kShadeChunk = 64;
-static_assert(kQueueGrid % kBlock == 0, "kBlockBases splits the grid evenly over its threads");
 
 // Block-wide flush of N wave-uniform counts: one atomic per counter and
 // block instead of per wave (waves that end together would otherwise queue
@@ -304,8 +302,9 @@ __global__ void kVbufReset(TraceParams P) {
     P.vbuf[i] = inf;
 }
 
-__global__ void kPassBegin(TraceParams P) {
-  DevCounters* c = P.ctr;
+// A pass's start, in one block: its ray ranges, then its domain counts, scores
+// and work counters at zero.
+__device__ __forceinline__ void passRanges(const TraceParams& P, DevCounters* c) {
   // pool levels past capacity (an overflow, reported to the host) are clamped
   // so that no kernel reads beyond a pool
   c->r_beg = c->r_mark;
@@ -335,19 +334,22 @@ __global__ void kPassBegin(TraceParams P) {
   c->n_phase[0] = 0;
   c->n_phase[1] = 0;
 }
-
-__global__ void kClearQ(TraceParams P) {
-  if (!P.ctr->active) return;
-  int nd = P.ndomains;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nd; i += gridDim.x * blockDim.x) {
+__global__ void __launch_bounds__(256) kPassBegin(TraceParams P) {
+  __shared__ uint32_t active;
+  if (threadIdx.x == 0) {
+    passRanges(P, P.ctr);
+    active = P.ctr->active;
+  }
+  __syncthreads();
+  if (!active) return;
+  const int nd = P.ndomains;
+  for (int i = threadIdx.x; i < nd; i += blockDim.x) {
     P.cnt[i] = 0;
     P.cnt[nd + i] = 0;
     P.score[i] = 0;
   }
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nd + 3; i += gridDim.x * blockDim.x)
-    P.wctr[i] = 0;
-  for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < 3 * kWorkCounters; i += gridDim.x * blockDim.x)
-    P.wq[i * kWorkStride] = 0;
+  for (int i = threadIdx.x; i < nd + 3; i += blockDim.x) P.wctr[i] = 0;
+  for (int i = threadIdx.x; i < 3 * kWorkCounters; i += blockDim.x) P.wq[i * kWorkStride] = 0;
 }
 
 // Ray of the current pass: index into the radiance range, then the shadow range.
@@ -758,18 +760,30 @@ __device__ __forceinline__ uint32_t blockScanExcl(uint32_t v, uint32_t* wsum, ui
   return r;
 }
 
+// Blocks 1 .. 2 * nd: the first queue slot of every (kind, domain, block of
+// kCount/kScatter) within the domain's entries, one block per (kind, domain).
+// (Both in one launch: a launch costs 4 us, a 96x72 frame has 5 passes.  The
+// scores in LDS: ranking 256 domains out of HBM took 18 of 23 us.)
+static_assert(kQueueGrid == 1024, "one thread of kSchedule per block of kCount");
 __global__ void __launch_bounds__(1024) kSchedule(TraceParams P) {
   DevCounters* c = P.ctr;
   if (!c->active) return;
   const int nd = P.ndomains;
   __shared__ uint32_t wsum[16 + 1];
+  __shared__ unsigned long long score[1024];
+  if (blockIdx.x > 0) {
+    const size_t at = (size_t)(blockIdx.x - 1) * kQueueGrid + threadIdx.x;
+    uint32_t total;
+    P.bbase[at] = blockScanExcl(P.bcnt[at], wsum, &total);
+    return;
+  }
+  for (int d = threadIdx.x; d < nd; d += blockDim.x) score[d] = P.score[d];
+  __syncthreads();
   for (int d = threadIdx.x; d < nd; d += blockDim.x) {
-    unsigned long long sd = P.score[d];
+    const unsigned long long sd = score[d];
     int rank = 0;
-    for (int e = 0; e < nd; ++e) {
-      unsigned long long se = P.score[e];
-      rank += (se > sd) || (se == sd && e < d);
-    }
+#pragma unroll 8
+    for (int e = 0; e < nd; ++e) rank += (score[e] > sd) || (score[e] == sd && e < d);
     P.order[rank] = d;
   }
   __syncthreads();
@@ -826,33 +840,8 @@ __device__ __forceinline__ void scatterDomains(const float4* box, int nd, const 
   }
 }
 
-// Queue base of every (kind, domain, block of kCount/kScatter): the
-// domain's base in schedule order plus the entries of the lower blocks.
-// One block per (kind, domain).
-__global__ void __launch_bounds__(kBlock) kBlockBases(TraceParams P) {
-  __shared__ uint32_t wsum[16 + 1];
-  if (!P.ctr->active) return;
-  const int j = blockIdx.x;  // kind * nd + domain
-  constexpr int kPer = kQueueGrid / kBlock;
-  const uint32_t* src = P.bcnt + (size_t)j * kQueueGrid + threadIdx.x * kPer;
-  uint32_t v[kPer], sum = 0;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    v[k] = src[k];
-    sum += v[k];
-  }
-  uint32_t total;
-  uint32_t pre = P.dbase[j] + blockScanExcl(sum, wsum, &total);
-  uint32_t* dst = P.bbase + (size_t)j * kQueueGrid + threadIdx.x * kPer;
-#pragma unroll
-  for (int k = 0; k < kPer; ++k) {
-    dst[k] = pre;
-    pre += v[k];
-  }
-}
-
 // Scatter the queue entries: the same grid and ray-to-block mapping as
-// kCount, so each block owns the slots kBlockBases reserved for it.
+// kCount, so each block owns the slots kSchedule reserved for it.
 // kList: the rays kCount gave a packed hit list (as kCount's kList).
 template <bool kList>
 __global__ void __launch_bounds__(kQueueBlock) kScatter(TraceParams P) {
@@ -865,7 +854,7 @@ __global__ void __launch_bounds__(kQueueBlock) kScatter(TraceParams P) {
   for (int i = threadIdx.x; i < 2 * nd; i += blockDim.x) {
     box[i] = P.dbox[i];
     lc[i] = 0;
-    lb[i] = P.bbase[(size_t)i * kQueueGrid + blockIdx.x];
+    lb[i] = P.dbase[i] + P.bbase[(size_t)i * kQueueGrid + blockIdx.x];
   }
   __syncthreads();
   const DevCounters* c = P.ctr;
@@ -2177,8 +2166,7 @@ static void passQueues(Ctx* c, const TraceParams& P) {
   hipStream_t s = c->stream;
   TracerState* T = c->tracer;
   int nd = P.ndomains;
-  kPassBegin<<<1, 1, 0, s>>>(P);
-  kClearQ<<<(nd + 255) / 256, 256, 0, s>>>(P);
+  kPassBegin<<<1, 256, 0, s>>>(P);
   const bool list = (nd + 63) / 64 > kHitListWords;  // packed hit lists (kScatter agrees)
   const size_t sh = countShmem(nd);
   if (P.learned && list)
@@ -2197,8 +2185,7 @@ static void passQueues(Ctx* c, const TraceParams& P) {
     predictorInfer(c, P, T->aux);
     SPRAY_HIP(hipEventRecord(T->join_ev, T->aux));
   }
-  kSchedule<<<1, 1024, 0, s>>>(P);
-  kBlockBases<<<2 * nd, kBlock, 0, s>>>(P);
+  kSchedule<<<1 + 2 * nd, 1024, 0, s>>>(P);
   if (list)
     kScatter<true><<<kQueueGrid, kQueueBlock, scatterShmem(nd), s>>>(P);
   else
