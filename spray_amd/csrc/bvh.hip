@@ -599,7 +599,9 @@ __device__ __forceinline__ void quantizeNode(const float (&b)[6], bool used, uin
     if (big > 0.0) e = max(e, exponent(big) - 19);
   }
   const bool all = !finite || e >= 61;
-  float base = __uint_as_float(0xff61b1f8u);  // -3e38, with the exponent of `all`
+  // all: not a number, so every plane distance is not a number and bounds
+  // nothing (a finite base as low as that would overflow against 1/dir)
+  float base = __uint_as_float(0x7fc000f8u);
   if (all) {
     e = 121;
   } else {

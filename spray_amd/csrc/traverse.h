@@ -109,9 +109,10 @@ struct TravCount {
   uint32_t tris = 0;
 };
 
-// Largest |1/dir| of the fused box test: beyond it scale * inv could
-// overflow (quantizeNode keeps scale below 2^62).
-constexpr float kFusedInvMax = 1.8446744073709552e19f;  // 2^64
+// Largest |1/dir| of the fused box test: a plane's 255 * scale * inv stays
+// below 2^126 (quantizeNode keeps scale below 2^62), so where the other term
+// overflows, it alone decides.
+constexpr float kFusedInvMax = 1.4411518807585587e17f;  // 2^57
 __device__ __forceinline__ bool needsSafeBoxes(const float inv[3]) {
   return !(fabsf(inv[0]) < kFusedInvMax && fabsf(inv[1]) < kFusedInvMax && fabsf(inv[2]) < kFusedInvMax);
 }
@@ -135,7 +136,8 @@ __device__ __forceinline__ uint32_t pickBits(uint32_t m, uint32_t a, uint32_t b)
 // against selects, compares and carries).
 // kSafe (waves with an axis-parallel ray): the difference first, then the
 // product with a possibly infinite inv; 0 * inf = NaN (the origin on the
-// plane) bounds nothing, as max and min drop NaN operands.
+// plane) bounds nothing, as max and min drop NaN operands.  An axis that
+// covers everything has a base that is not a number.
 template <bool kSafe>
 __device__ __forceinline__ uint32_t nodeBoxes(const uint4& w0, const uint4 (&pl)[3], const float org[3],
                                               const float inv[3], float tnear, float tfar) {
