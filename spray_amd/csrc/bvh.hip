@@ -616,12 +616,13 @@ __device__ __forceinline__ void quantizeNode(const float (&b)[6], bool used, uin
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
     const int ek = __shfl(e, k, 8);
-    const double bk = (double)__shfl(base, k, 8), inv = power(-ek);
+    const float bk = __shfl(base, k, 8), inv = __uint_as_float((uint32_t)(127 - ek) << 23);
     const bool allk = ek == 121;
     uint32_t l = 255u, h = 0u;  // unused slots: inverted
     if (used) {
-      l = allk ? 0u : (uint32_t)fmin(fmax(floor(((double)b[k] - bk) * inv - 0.001953125), 0.0), 255.0);
-      h = allk ? 255u : (uint32_t)fmin(fmax(ceil(((double)b[3 + k] - bk) * inv + 0.001953125), 0.0), 255.0);
+      // (rounding b - base is below 2^-16 of a step, far less than is to spare)
+      l = allk ? 0u : (uint32_t)fminf(fmaxf(floorf((b[k] - bk) * inv - 0.001953125f), 0.f), 255.f);
+      h = allk ? 255u : (uint32_t)fminf(fmaxf(ceilf((b[3 + k] - bk) * inv + 0.001953125f), 0.f), 255.f);
     }
     nd->plane[k][slot] = (uint8_t)l;
     nd->plane[k][8 + slot] = (uint8_t)h;
@@ -669,7 +670,7 @@ __device__ __forceinline__ uint32_t assignSlot(const float (&b)[6], bool used) {
       }
       frees &= ~(1u << bs);
 #pragma unroll
-      for (int s = 0; s < 8; ++s) key[s] = bs == (uint32_t)s ? 0u : key[s];
+      for (int s = 0; s < 8; ++s) key[s] &= (uint32_t)__builtin_amdgcn_sbfe((int)frees, s, 1);
     }
   }
   const uint32_t taken = groupBallot(used);  // (of all the group's lanes)
@@ -1004,7 +1005,12 @@ struct SlotLayout {
 };
 constexpr int kBuildStreams = 4;  // pipelines of a whole-scene LBVH build
 constexpr int kBuildGroup = 16;   // domains per launch, at most
-constexpr size_t kSlotBudget = (size_t)2 << 30;  // slots of all pipelines together
+// Slots of all pipelines together: this, or a sixteenth of the free HBM if that
+// is less.  Domains alone in their launches (a small budget) leave the narrow
+// levels of their trees waiting for memory: remeshes of 128 domains of 563k
+// triangles take 61.4 / 54.3 / 49.2 / 47.6 / 47.6 ms with 0.5 / 1 / 2 / 4 / 8 GB,
+// of 32 of 1.06 M 28.2 / 28.2 / 25.4 / 25.1 / 24.4 ms.
+constexpr size_t kSlotBudget = (size_t)8 << 30;
 
 struct PlocScratch {
   DevBuf pc, pc2, pb, pb2, pnn, pcnt, pmf, pkf, pmp, pkp, pperm, pord;
@@ -1167,9 +1173,14 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
   }
   const SlotLayout SL(std::max(maxf, 1), maxv);
   const int K = multi ? std::min(pipelineCount(kBuildStreams), nd) : 1;
-  const int GN = multi ? (int)std::max<size_t>(1, std::min<size_t>({(size_t)kBuildGroup, (size_t)((nd + K - 1) / K),
-                                                                     kSlotBudget / ((size_t)K * SL.bytes)}))
-                       : 1;
+  int GN = 1;
+  if (multi) {
+    size_t free_b = 0, total_b = 0;
+    SPRAY_HIP(hipMemGetInfo(&free_b, &total_b));
+    const size_t budget = std::min(kSlotBudget, (free_b + M->slots.bytes) / 16);
+    GN = (int)std::max<size_t>(1, std::min<size_t>({(size_t)kBuildGroup, (size_t)((nd + K - 1) / K),
+                                                    budget / ((size_t)K * SL.bytes)}));
+  }
   const int ngroups = (nd + GN - 1) / GN;
   M->slots.reserve((size_t)K * GN * SL.bytes);
   M->levels.reserve((size_t)nd * kLevelWords * 4 + 64);
