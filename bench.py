@@ -116,10 +116,10 @@ def copy_calibration():
 def algorithmic_bytes(st):
     """Bytes one frame's trace kernels must move: per (ray, domain) visit a
     32 B ray record, 16 B hit record and 8 B queue entry; per BVH node fetch
-    128 B; per triangle test 48 B; per accepted shading vertex 80 B ray write
+    64 B; per triangle test 48 B; per accepted shading vertex 80 B ray write
     + 16 B queue + 16 B history."""
     visits = st["radiance_visits"] + st["shadow_visits"]
-    return 56 * visits + 128 * st["node_visits"] + 48 * st["tri_tests"] + 112 * st["shades"]
+    return 56 * visits + 64 * st["node_visits"] + 48 * st["tri_tests"] + 112 * st["shades"]
 
 
 def main():
