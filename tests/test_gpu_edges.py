@@ -185,6 +185,19 @@ def test_small_frames(lattices, size, schedule):
         _frame_ok(ctx, ref["g27"], **kw)
 
 
+@pytest.mark.parametrize("schedule", [0, 1])
+@pytest.mark.parametrize("ao,bounces", [(1, 1), (1, 3), (0, 1), (0, 2), (0, 4), (0, 5), (0, 9)])
+def test_passes_of_a_window(lattices, ao, bounces, schedule):
+    """Paths that end within, at and beyond a window of four depths."""
+    import spray_amd as sa
+    d, ref = lattices
+    kw = dict(image_w=24, image_h=20, pixel_samples=2, ao_mode=ao, ao_samples=2, bounces=bounces, rr_start=6,
+              ao_max_dist=0.5)
+    with sa.Context(_cfg(schedule=schedule, **kw)) as ctx:
+        ctx.load_scene(os.path.join(d, "g27.spray"), d)
+        _frame_ok(ctx, ref["g27"], **kw)
+
+
 def test_context_changes_scene_and_size(lattices):
     """One context's memory serves other scenes and sizes: larger, smaller and
     larger again, each frame as the oracle's."""
