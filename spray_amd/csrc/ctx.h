@@ -158,12 +158,12 @@ struct DomainPool {
   std::vector<char> pending;              // prefetched, access not yet made
   std::vector<char> pinned;               // in use by the chunk being traced: never evicted
   unsigned long long tick = 0, hits = 0, misses = 0, bytes_in = 0;
-  // a missing domain's image is copied to a stage (copy_stream) and unpacked
-  // into its block (unpack_stream); the stages alternate
-  hipStream_t copy_stream = nullptr, unpack_stream = nullptr;
+  // a missing domain's image is copied to a stage and unpacked from there
+  // into its block; the stages alternate, each with a stream of its own
+  hipStream_t load_stream[2] = {};
   DevBuf stage[2];
-  hipEvent_t stage_full[2] = {}, stage_free[2] = {};
   int next_stage = 0;
+  int last_load = -1;  // block of the load before
   void releasePaging();
   void release(bool keep_mem = false) {
     d_desc.release();

@@ -24,18 +24,13 @@ void DomainPool::releasePaging() {
   block_ready.clear();
   if (h_image) (void)hipHostFree(h_image);
   if (h_desc_pinned) (void)hipHostFree(h_desc_pinned);
-  for (hipStream_t* s : {&copy_stream, &unpack_stream}) {
-    if (*s) (void)hipStreamDestroy(*s);
-    *s = nullptr;
-  }
   for (int k = 0; k < 2; ++k) {
+    if (load_stream[k]) (void)hipStreamDestroy(load_stream[k]);
+    load_stream[k] = nullptr;
     stage[k].release();
-    for (hipEvent_t* e : {&stage_full[k], &stage_free[k]}) {
-      if (*e) (void)hipEventDestroy(*e);
-      *e = nullptr;
-    }
   }
   next_stage = 0;
+  last_load = -1;
   h_image = nullptr;
   h_desc_pinned = nullptr;
   h_image_off.clear();
@@ -134,28 +129,33 @@ static int lruLoad(Ctx* c, int d, int keep) {
   P.block_domain[victim] = d;
   P.domain_block[d] = victim;
   P.block_tick[victim] = ++P.tick;
-  // The copy waits for its stage, the unpacking for the copy and the block's
-  // last users; then the descriptor follows.  (The domain's own last users
-  // are done by then: its old block was unpacked into, or is this one.)
+  // Copy, unpacking and descriptor follow one another on the stage's stream;
+  // the unpacking waits for the block's last users and its last filling, the
+  // descriptor for the descriptor before it, so descriptors change in the
+  // order of the loads.  (The domain's own last users are done by then: its
+  // old block was unpacked into, or is this one.)  A stream per stage, not one
+  // for the copies and one for the unpacking: the next image's copy starts
+  // when its own stage is free and no unpacking waits for an event of the
+  // copies (400x300 path trace of 4 samples, 48 domains, 12 blocks: 13.3 ->
+  // 11.1 ms; 1920x1080, 256 domains, 128 blocks: 877 -> 785 ms).
   const DomainDesc& D = P.desc[d];
   const char* src = (const char*)P.h_image + P.h_image_off[d];
   const ImageLayout L(D.num_nodes, D.num_tris, P.nverts[d]);
   const int k = P.next_stage;
   P.next_stage ^= 1;
-  hipStream_t cs = P.copy_stream, us = P.unpack_stream;
-  SPRAY_HIP(hipStreamWaitEvent(cs, P.stage_free[k], 0));
-  SPRAY_HIP(hipMemcpyAsync(P.stage[k].p, src, L.bytes, hipMemcpyHostToDevice, cs));
-  SPRAY_HIP(hipEventRecord(P.stage_full[k], cs));
-  SPRAY_HIP(hipStreamWaitEvent(us, P.stage_full[k], 0));
+  hipStream_t us = P.load_stream[k];
+  SPRAY_HIP(hipMemcpyAsync(P.stage[k].p, src, L.bytes, hipMemcpyHostToDevice, us));
   SPRAY_HIP(hipStreamWaitEvent(us, P.block_free[victim], 0));
+  SPRAY_HIP(hipStreamWaitEvent(us, P.block_ready[victim], 0));
   kUnpack<<<std::max(1, std::min((D.num_tris + 255) / 256, 2048)), 256, 0, us>>>(
       P.stage[k].as<char>(), L, D.num_nodes, D.num_tris, P.nodes.as<BNode8>() + (size_t)victim * P.block_nodes,
       P.leaves.as<NodeLeaves>() + (size_t)victim * P.block_nodes, P.tris.as<LTri>() + (size_t)victim * P.block_tris,
       P.fshade.as<float4>() + (size_t)victim * P.block_tris * 3);
   SPRAY_HIP(hipGetLastError());
-  SPRAY_HIP(hipEventRecord(P.stage_free[k], us));
+  if (P.last_load >= 0) SPRAY_HIP(hipStreamWaitEvent(us, P.block_ready[P.last_load], 0));
   bindBlock(P, d, victim, us);
   SPRAY_HIP(hipEventRecord(P.block_ready[victim], us));
+  P.last_load = victim;
   P.bytes_in += L.bytes;
   return victim;
 }
@@ -191,15 +191,12 @@ void poolInitPaging(Ctx* c, const std::vector<std::pair<int, int>>& resident) {
   P.block_tick.assign(P.capacity, 0);
   P.pending.assign(nd, 0);
   P.pinned.assign(nd, 0);
-  SPRAY_HIP(hipStreamCreate(&P.copy_stream));
-  SPRAY_HIP(hipStreamCreate(&P.unpack_stream));
   size_t most = 0;
   for (int d = 0; d < nd; ++d)
     most = std::max(most, ImageLayout(P.desc[d].num_nodes, P.desc[d].num_tris, P.nverts[d]).bytes);
   for (int k = 0; k < 2; ++k) {
     P.stage[k].reserve(most + 64);
-    SPRAY_HIP(hipEventCreateWithFlags(&P.stage_full[k], hipEventDisableTiming));
-    SPRAY_HIP(hipEventCreateWithFlags(&P.stage_free[k], hipEventDisableTiming));
+    SPRAY_HIP(hipStreamCreate(&P.load_stream[k]));
   }
   P.block_free.resize(P.capacity);
   P.block_ready.resize(P.capacity);
