@@ -1700,6 +1700,7 @@ struct TracerState {
   int grid_persistent = 0;
   int num_cu = 0;
   int trav_res_block = 0, trav_res_blocks = 0;  // block size -> resident kTraverse blocks
+  DevBuf learned_mem;  // holds ask, ask_cnt, rkey, dflag and acnt
   // captured tile graphs by key (schedule, windows, batch parameters,
   // logging, configuration version).  A graph whose buffers were reallocated
   // is retired, never launched again, and destroyed only when the tracer is
@@ -1720,7 +1721,9 @@ struct TracerState {
   int slog_max = 0;
   std::vector<int> slog_meta, slog_order;
   std::vector<unsigned long long> slog_scores;
-  size_t heldBytes() const { return ovf.bytes + vlog.bytes + log.bytes + log_ctr.bytes; }  // beside frame_mem
+  size_t heldBytes() const {  // beside frame_mem
+    return ovf.bytes + vlog.bytes + log.bytes + log_ctr.bytes + learned_mem.bytes;
+  }
   // learned form: the predictor's stream beside the schedule and scatter
   // (forked from and joined back to the tracer's stream, graph capture included)
   hipStream_t aux = nullptr;
@@ -1786,7 +1789,7 @@ void tracerRelease(Ctx* c) {
   }
   for (hipEvent_t e : {T->fork_ev, T->join_ev})
     if (e) (void)hipEventDestroy(e);
-  for (DevBuf* b : {&T->ovf, &T->vlog, &T->log, &T->log_ctr}) b->release();
+  for (DevBuf* b : {&T->ovf, &T->vlog, &T->log, &T->log_ctr, &T->learned_mem}) b->release();
   if (c->frame_mem.bytes > kKeepFrameMem) c->frame_mem.release();
   delete T;
   c->tracer = nullptr;
@@ -1901,17 +1904,13 @@ static void ensureState(Ctx* c, double grow) {
   T->q_cap[0] = std::max(T->q_cap[0], q0);
   T->q_cap[1] = std::max(T->q_cap[1], q1);
   T->mask_cap = std::max(T->mask_cap, mask_cap);
-  // every buffer is planned, so that one which this frame does not use moves with the others
+  // what every frame uses, in one allocation
   BufPlan plan;
   auto want = [&](DevBuf& b, size_t bytes) { plan.want(b, bytes); };
   want(T->R, (size_t)T->r_cap * 64);
   want(T->Pn, (size_t)T->p_cap * 64);
   want(T->Sh, (size_t)T->s_cap * 64);
   want(T->vbuf, (size_t)S * kHistory * 8);
-  const size_t learned = cfg.schedule == SPRAY_SCHEDULE_LEARNED ? 1 : 0;
-  want(T->ask, learned * ((size_t)kQueueGrid * askRegion(T->r_cap) * 48 + 64));
-  want(T->ask_cnt, learned * ((size_t)kQueueGrid * 4 + 64));
-  want(T->rkey, learned * ((size_t)T->r_cap * 4 + 64));
   want(T->dmask, (size_t)T->mask_cap * maskRowWords(nd) * 8 + 64);
   want(T->dfmt, (size_t)T->mask_cap + 64);
   want(T->dbox, dboxBytes(nd));
@@ -1926,8 +1925,6 @@ static void ensureState(Ctx* c, double grow) {
   want(T->wq, (size_t)3 * kWorkCounters * kWorkStride * 4);
   want(T->qa, (size_t)T->q_cap[0] * 4);
   want(T->qb, (size_t)T->q_cap[0] * 4);
-  want(T->dflag, learned * (((size_t)T->q_cap[0] / 64 + 2) * 8));
-  want(T->acnt, learned * ((size_t)2 * kAssignWaves * 4 + 64));
   // shade records: one per accepted hit of a pass, far fewer than queue
   // entries (an overflow grows and re-renders like any other pool)
   T->sh_cap = std::min(T->q_cap[0], T->r_cap);
@@ -1943,6 +1940,24 @@ static void ensureState(Ctx* c, double grow) {
     T->releaseGraph();
     T->box_version = -1;
     plan.place(c->frame_mem);
+  }
+  // What only the learned form uses lies in an allocation of its own, so that
+  // the first learned frame of a context adds it and leaves the others' memory
+  // alone: giving that back and taking a larger allocation waits until the
+  // driver has cleared what other contexts gave back before (960x540, 4 spp,
+  // 256 domains, contexts made and closed in turn: 131-147 ms for the first
+  // learned frame, 8 ms with this; 7 ms the next).
+  if (cfg.schedule == SPRAY_SCHEDULE_LEARNED) {
+    BufPlan lp;
+    lp.want(T->ask, (size_t)kQueueGrid * askRegion(T->r_cap) * 48 + 64);
+    lp.want(T->ask_cnt, (size_t)kQueueGrid * 4 + 64);
+    lp.want(T->rkey, (size_t)T->r_cap * 4 + 64);
+    lp.want(T->dflag, ((size_t)T->q_cap[0] / 64 + 2) * 8);
+    lp.want(T->acnt, (size_t)2 * kAssignWaves * 4 + 64);
+    if (!lp.fits()) {
+      T->releaseGraph();
+      lp.place(T->learned_mem);
+    }
   }
   hipDeviceProp_t prop;
   SPRAY_HIP(hipGetDeviceProperties(&prop, c->device));
