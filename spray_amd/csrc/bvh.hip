@@ -1047,6 +1047,8 @@ constexpr int kBuildGroup = 16;   // domains per launch, at most
 // levels of their trees waiting for memory: remeshes of 128 domains of 563k
 // triangles take 61.4 / 54.3 / 49.2 / 47.6 / 47.6 ms with 0.5 / 1 / 2 / 4 / 8 GB,
 // of 32 of 1.06 M 28.2 / 28.2 / 25.4 / 25.1 / 24.4 ms.
+// Domains too large for that still go one to a launch in as many pipelines as
+// half of the free HBM holds, and in one where it holds none.
 constexpr size_t kSlotBudget = (size_t)8 << 30;
 
 struct PlocScratch {
@@ -1209,12 +1211,13 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     buildCacheRelease(c);
   }
   const SlotLayout SL(std::max(maxf, 1), maxv);
-  const int K = multi ? std::min(pipelineCount(kBuildStreams), nd) : 1;
-  int GN = 1;
+  int K = 1, GN = 1;
   if (multi) {
     size_t free_b = 0, total_b = 0;
     SPRAY_HIP(hipMemGetInfo(&free_b, &total_b));
-    const size_t budget = std::min(kSlotBudget, (free_b + M->slots.bytes) / 16);
+    const size_t avail = free_b + M->slots.bytes, budget = std::min(kSlotBudget, avail / 16);
+    K = (int)std::max<size_t>(1, std::min<size_t>({(size_t)pipelineCount(kBuildStreams), (size_t)nd,
+                                                   avail / 2 / SL.bytes}));
     GN = (int)std::max<size_t>(1, std::min<size_t>({(size_t)kBuildGroup, (size_t)((nd + K - 1) / K),
                                                     budget / ((size_t)K * SL.bytes)}));
   }

@@ -1,7 +1,10 @@
 """What a context keeps in HBM between calls, and what it gives back: the
-frame's buffers while the schedule changes."""
+frame's buffers while the schedule changes, and scenes that leave little of
+the HBM free."""
+import ctypes as C
 import os
 
+import numpy as np
 import pytest
 
 from test_gpu_edges import _cfg, _frame_ok, lattices  # noqa: F401 (lattices: a fixture)
@@ -41,3 +44,65 @@ def test_learned_frames_beside_batched_ones(lattices):  # noqa: F811
             if not held:
                 pytest.skip("this driver does not show device allocations as mappings")
             assert held <= _hbm_blocks(32 << 20), schedule
+
+
+class _Filler:
+    """Device memory taken until only so much is free, from the HIP runtime the
+    library itself links."""
+
+    def __init__(self):
+        self.rt = C.CDLL("libamdhip64.so.7")
+        self.rt.hipMalloc.argtypes = [C.POINTER(C.c_void_p), C.c_size_t]
+        self.rt.hipFree.argtypes = [C.c_void_p]
+        self.bufs = []
+
+    def free_bytes(self):
+        a, b = C.c_size_t(), C.c_size_t()
+        assert self.rt.hipMemGetInfo(C.byref(a), C.byref(b)) == 0
+        return a.value
+
+    def leave(self, want):
+        for step in (64 << 30, 4 << 30, 256 << 20, 32 << 20):
+            while self.free_bytes() - want > step:
+                p = C.c_void_p()
+                if self.rt.hipMalloc(C.byref(p), step) != 0:
+                    break
+                self.bufs.append(p)
+        left = self.free_bytes() - want
+        assert 0 <= left < 96 << 20, left
+
+    def __enter__(self):
+        return self
+
+    def __exit__(self, *a):
+        for p in self.bufs:
+            self.rt.hipFree(p)
+        self.bufs = []
+
+
+def _retained(filler, scene):
+    """HBM that a context holds once this scene is loaded."""
+    import spray_amd as sa
+    before = filler.free_bytes()
+    with sa.Context(_cfg(image_w=16, image_h=12)) as ctx:
+        ctx.scenegen_load("s", **scene)
+        return before - filler.free_bytes()
+
+
+def test_build_in_little_memory(lattices):  # noqa: F811
+    """Four domains of 2 M triangles where the build's memory for one domain is
+    free (0.34 GB), but not for four side by side."""
+    import spray_amd as sa
+    scene = dict(nx=4, ny=1, nz=1, res=300)
+    with _Filler() as filler:
+        need = _retained(filler, scene)
+        with sa.Context(_cfg(image_w=16, image_h=12)) as ctx:
+            filler.leave(need + (640 << 20))
+            ctx.scenegen_load("s", **scene)
+            rng = np.random.default_rng(1)
+            d = rng.normal(size=(1000, 3)).astype(np.float32)
+            org = (rng.uniform(0.2, 0.8, (1000, 3)) + [2.0, 0.0, 0.0]).astype(np.float32)
+            _, _, _, few = ctx.trace_rays(org, d, 2)
+    with sa.Context(_cfg(image_w=16, image_h=12)) as ctx:
+        ctx.scenegen_load("s", **scene)
+        assert np.array_equal(ctx.trace_rays(org, d, 2)[3], few) and (few >= 0).any()
