@@ -1169,15 +1169,7 @@ void buildPool(Ctx* c, MeshSource& src, bool keep_buffers) {
     plan.want(P.fshade, tf * 48 + 64);
     plan.want(P.nodes, tn * sizeof(BNode8));
     plan.want(P.leaves, tn * sizeof(NodeLeaves));
-    if (!plan.fits()) {
-      try {
-        plan.place(P.mem);
-      } catch (const StatusError&) {
-        if (c->tracer || !c->frame_mem.p) throw;
-        c->frame_mem.release();  // the last scene's frame memory makes room
-        plan.place(P.mem);
-      }
-    }
+    if (!plan.fits()) plan.place(P.mem);
   }
   // A whole-scene LBVH build takes the domains in groups, one launch per
   // build step for a group, up to kBuildStreams groups side by side (one per

@@ -18,10 +18,18 @@ namespace {
 thread_local std::string g_create_err;
 constexpr long long kTraceRaysDeviceMax = 2147483647LL;
 
+// Runs f; a call that finds too little HBM while the last scene's frame memory
+// lies idle (kept for the next frames) gives that back and runs again.
 template <typename F>
 int guarded(spray_ctx* ctx, F&& f) {
   try {
-    f();
+    try {
+      f();
+    } catch (const StatusError& e) {
+      if (e.code != SPRAY_ERR_OOM || !ctx || ctx->c.tracer || !ctx->c.frame_mem.p) throw;
+      ctx->c.frame_mem.release();
+      f();
+    }
     if (ctx) ctx->c.err.clear();
     return SPRAY_OK;
   } catch (const StatusError& e) {
@@ -235,9 +243,10 @@ int spray_scenegen_load(spray_ctx* ctx, const spray_scenegen_params* p, const ch
 
 int spray_remesh(spray_ctx* ctx, double phase) {
   if (!ctx) return SPRAY_ERR_INVALID;
+  const bool made = ctx->c.loaded && ctx->c.generated;
   return guarded(ctx, [&] {
     Ctx* c = &ctx->c;
-    if (!c->loaded || !c->generated)
+    if (!made)
       throw StatusError(SPRAY_ERR_STATE, "remeshing needs a scene made by spray_scenegen_load");
     SPRAY_HIP(hipSetDevice(c->device));
     spray_scenegen_params p = c->gen;

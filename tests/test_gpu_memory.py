@@ -106,3 +106,22 @@ def test_build_in_little_memory(lattices):  # noqa: F811
     with sa.Context(_cfg(image_w=16, image_h=12)) as ctx:
         ctx.scenegen_load("s", **scene)
         assert np.array_equal(ctx.trace_rays(org, d, 2)[3], few) and (few >= 0).any()
+
+
+def test_load_gets_idle_frame_memory(lattices):  # noqa: F811
+    """The last scene's frame memory, kept for the next frames, makes room for
+    what the next scene's build needs."""
+    import spray_amd as sa
+    d, _ = lattices
+    scene = dict(nx=1, ny=1, nz=1, res=500)  # 5.5 M triangles, 0.9 GB of build memory
+    with _Filler() as filler:
+        need = _retained(filler, scene)
+        with sa.Context(_cfg(schedule=1, image_w=1024, image_h=1024, pixel_samples=2, ao_samples=1, bounces=4)) as ctx:
+            ctx.load_scene(os.path.join(d, "g2.spray"), d)
+            before = filler.free_bytes()
+            ctx.trace_frame(want_image=False)
+            assert (2 << 30) < before - filler.free_bytes() < (4 << 30)  # (what a context keeps at most)
+            ctx.load_scene(os.path.join(d, "g2.spray"), d)
+            filler.leave(need + (320 << 20))
+            ctx.scenegen_load("s", **scene)
+            assert ctx.num_domains == 1
