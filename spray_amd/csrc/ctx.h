@@ -64,12 +64,13 @@ struct DevBuf {
 };
 
 // Buffers that are sized together lie in one allocation, kept for the next
-// scene unless that needs less than a quarter of it: freed and allocated one
+// scene where that leaves at most kSpareMem of it unused: freed and allocated one
 // by one (a free waits for the device and unmaps, 0.25 to 0.7 ms for a large
 // buffer), the 33 buffers of a frame, the 9 of a scene and the 4 of a build took
 // 6 of the 12 ms from loading 27 domains to their first image, and a new
 // context's first 96x72 frame 1.6 ms (now 0.9).  Buffers only grow; none keeps
 // its contents when any of them does.
+constexpr size_t kSpareMem = (size_t)64 << 20;
 struct BufPlan {
   std::vector<std::pair<DevBuf*, size_t>> items;
   void want(DevBuf& b, size_t bytes) { items.push_back({&b, std::max(bytes, b.bytes)}); }
@@ -84,7 +85,7 @@ struct BufPlan {
       w.first->release();
       total += (w.second + 255) & ~(size_t)255;
     }
-    if (mem.bytes < total || mem.bytes / 4 > total + ((size_t)64 << 20)) {
+    if (mem.bytes < total || mem.bytes > total + kSpareMem) {
       mem.release();
       mem.reserve(total);
     }

@@ -1,6 +1,6 @@
 """What a context keeps in HBM between calls, and what it gives back: the
 frame's buffers while the schedule changes, and scenes that leave little of
-the HBM free."""
+the HBM free or replace one another."""
 import ctypes as C
 import os
 
@@ -125,3 +125,19 @@ def test_load_gets_idle_frame_memory(lattices):  # noqa: F811
             filler.leave(need + (320 << 20))
             ctx.scenegen_load("s", **scene)
             assert ctx.num_domains == 1
+
+
+def test_smaller_scene_gives_memory_back(tmp_path, lattices):  # noqa: F811
+    """After a scene of 0.4 GB, one of 0.15 GB holds what it needs alone."""
+    import spray_amd as sa
+    for name, res in (("large", 330), ("small", 200)):
+        sa.scenegen_write(str(tmp_path), name, 1, 1, 1, res)
+    with _Filler() as filler:
+        held = []
+        for names in (["small"], ["large", "small"]):
+            before = filler.free_bytes()
+            with sa.Context(_cfg(image_w=16, image_h=12)) as ctx:
+                for name in names:
+                    ctx.load_scene(os.path.join(str(tmp_path), name + ".spray"), str(tmp_path))
+                held.append(before - filler.free_bytes())
+        assert held[1] <= held[0] + (80 << 20), held
