@@ -1533,7 +1533,7 @@ constexpr int kQBlock = 256;
 constexpr int kQRefill = 16;
 constexpr uint32_t kQMinRange = 4;
 __global__ void __launch_bounds__(kQBlock, 4) kTraceRays(
-    const BNode8* __restrict__ nodes, const NodeLeaves* __restrict__ leaves,
+    const BNode8* __restrict__ nodes, const NodeLeaves* __restrict__ leaves, int num_nodes,
     const LTri* __restrict__ tris, const float* __restrict__ org, const float* __restrict__ dir, const float* __restrict__ tnear, const float* __restrict__ tfar,
     uint32_t n, uint32_t range, int mode, float* t_o, float* u_o, float* v_o, int* prim_o,
     uint32_t* ovf, uint32_t ovf_words, uint32_t* ctr, int* err) {
@@ -1587,7 +1587,7 @@ __global__ void __launch_bounds__(kQBlock, 4) kTraceRays(
           const size_t q = (size_t)ray * 3;
           float o[3] = {org[q], org[q + 1], org[q + 2]};
           float d[3] = {dir[q], dir[q + 1], dir[q + 2]};
-          travInit(s, 0u, 0u, o, d, tnear[ray], tfar[ray], mode != 0, st);
+          travInit(s, 0u, 0u, num_nodes, o, d, tnear[ray], tfar[ray], mode != 0, st);
           active = true;
         }
         cur = min(cur + (unsigned long long)__popcll(idle), end);
@@ -1653,7 +1653,7 @@ static void runQuery(Ctx* c, const QueryLaunch& q, const DomainDesc& D, const fl
   *c->q_err = 0;
   kTraceRays<<<q.grid, kQBlock, 0, c->stream>>>(
       c->pool.nodes.as<BNode8>() + D.node_off, c->pool.leaves.as<NodeLeaves>() + D.node_off,
-      c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir, d_tnear, d_tfar, n, q.range, mode, d_t, d_u, d_v, d_prim,
+      D.num_nodes, c->pool.tris.as<LTri>() + D.tri_off, d_org, d_dir, d_tnear, d_tfar, n, q.range, mode, d_t, d_u, d_v, d_prim,
       ovf, q.words, ctr, c->q_err);
   SPRAY_HIP(hipGetLastError());
   SPRAY_HIP(hipStreamSynchronize(c->stream));

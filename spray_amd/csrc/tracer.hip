@@ -1460,8 +1460,8 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
           if (go) {
             const DomainDesc& D = P.desc[dom];
             float o[3] = {op.x, op.y, op.z}, d[3] = {ds.x, ds.y, ds.z};
-            travInit(s, (uint32_t)D.node_off, (uint32_t)D.tri_off, o, d, kRayEps, tfar, kind == 1,
-                     st);
+            travInit(s, (uint32_t)D.node_off, (uint32_t)D.tri_off, D.num_nodes, o, d, kRayEps, tfar,
+                     kind == 1, st);
             active = true;
           }
         }

@@ -41,11 +41,10 @@ constexpr uint32_t kStackEmpty = 0xffffffffu;
 // (1/dir, base - org, their product and the fma round once each); the exit
 // distance is inflated by 2^-20.
 constexpr float kSlabInflate = 1.00000095367431640625f;
-// A ray visits each node of a tree at most once; the bounds only stop a
-// corrupt (cyclic) tree from spinning forever: steps of one node phase, and
-// of all phases of a ray.
+// A ray visits each node of a tree at most once, so it has as many visits as
+// the tree has nodes (TravState::guard); that, and a bound on the steps of one
+// node phase, stop a corrupt (cyclic) tree from spinning forever.
 constexpr uint32_t kMaxPhaseSteps = 1u << 16;
-constexpr uint32_t kMaxNodeVisits = 1u << 24;
 
 // The ring pointer carries the LDS address space, so ring accesses stay
 // ds_read/ds_write and are never merged with the overflow path into flat
@@ -201,13 +200,14 @@ struct TravState {
   uint32_t kk;          // kx | ky << 2 | kz << 4 | any << 8 | negative directions << 16
   float tnear, tlim, u, v;
   int prim;
-  uint32_t cur, guard;  // node to visit (kStackEmpty: none)
+  uint32_t cur;         // node to visit (kStackEmpty: none)
+  int guard;            // visits left: a lane's own, not the steps it waits through
   uint32_t listed;      // leaf list: entries | leaves << 8
   uint32_t share;       // lane that owns the ray | lowest stack entry not given away << 8
   uint32_t node_base, tri_base;  // the domain's first node / leaf-ordered triangle
 };
 
-__device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint32_t tri_base,
+__device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint32_t tri_base, int num_nodes,
                                          const float org[3], const float dir[3], float tnear,
                                          float tfar, bool any, LaneStack& st) {
   s.org[0] = org[0];
@@ -229,7 +229,7 @@ __device__ __forceinline__ void travInit(TravState& s, uint32_t node_base, uint3
   s.cur = 0;
   s.listed = 0;
   s.share = (threadIdx.x & 63u) | (1u << 8);
-  s.guard = 0;
+  s.guard = num_nodes;
   s.node_base = node_base;
   s.tri_base = tri_base;
   st.reset();
@@ -302,14 +302,16 @@ __device__ __forceinline__ void travNodeLoop(TravState& s, LaneStack& st, TravCo
   uint32_t steps = 0;
   while (sm != 0ull) {
     cnt.nodes += (unsigned long long)__popcll(sm);
-    if (steps_on()) travNode<kSafe>(s, st, nodes);
+    if (steps_on()) {
+      travNode<kSafe>(s, st, nodes);
+      --s.guard;
+    }
     sm = __ballot(steps_on());
     const int nleaf = __popcll(__ballot(active && s.listed != 0u));
     ++steps;
     if (__popcll(sm) * 2 < nlive || nleaf * 4 >= nlive * 3 || steps >= kMaxPhaseSteps) break;
   }
-  s.guard += steps;
-  if (active && s.guard > kMaxNodeVisits) {
+  if (active && s.guard < 0) {
     st.err = true;
     s.cur = kStackEmpty;
     s.listed = 0;
@@ -515,6 +517,7 @@ __device__ __forceinline__ bool travShare(TravState& s, LaneStack& st, bool idle
   const float i0 = laneGetF(s.inv[0], own), i1 = laneGetF(s.inv[1], own), i2 = laneGetF(s.inv[2], own);
   const float tn = laneGetF(s.tnear, own), tl = laneGetF(s.tlim, own);
   const uint32_t kk = laneGet(s.kk, own), nb = laneGet(s.node_base, own);
+  const int left = (int)laneGet((uint32_t)s.guard, own);  // (owner and helper visit different nodes)
   if (take) {
     s.org[0] = o0;
     s.org[1] = o1;
@@ -527,7 +530,7 @@ __device__ __forceinline__ bool travShare(TravState& s, LaneStack& st, bool idle
     s.kk = kk;
     s.node_base = nb;
     s.listed = 0;
-    s.guard = 0;
+    s.guard = left;
     s.share = (uint32_t)own | (1u << 8);
     const uint32_t slot = ((uint32_t)__ffs((int)gm) - 1u) ^ ((kk >> 16) & 7u);
     s.cur = groupChild(gb, slot);
