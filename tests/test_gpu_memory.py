@@ -1,13 +1,16 @@
 """What a context keeps in HBM between calls, and what it gives back: the
-frame's buffers while the schedule changes, and scenes that leave little of
-the HBM free or replace one another."""
+frame's buffers while the schedule changes, scenes that leave little of the
+HBM free or replace one another, meshes that grow from step to step, and the
+images of paged domains."""
 import ctypes as C
 import os
 
 import numpy as np
 import pytest
 
-from test_gpu_edges import _cfg, _frame_ok, lattices  # noqa: F401 (lattices: a fixture)
+import orc
+import scenes
+from test_gpu_edges import LIGHT, _cfg, _frame_ok, _sheet, _soup, lattices  # noqa: F401 (lattices: a fixture)
 
 pytestmark = pytest.mark.gpu
 
@@ -141,3 +144,51 @@ def test_smaller_scene_gives_memory_back(tmp_path, lattices):  # noqa: F811
                     ctx.load_scene(os.path.join(str(tmp_path), name + ".spray"), str(tmp_path))
                 held.append(before - filler.free_bytes())
         assert held[1] <= held[0] + (80 << 20), held
+
+
+@pytest.mark.parametrize("schedule", [0, 1])
+def test_growing_remeshes(schedule):
+    """Remeshes whose pool outgrows its allocation again and again: every frame
+    is that of a context that generated the step's mesh alone."""
+    import spray_amd as sa
+    kw = dict(image_w=48, image_h=36, pixel_samples=2, ao_mode=0, ao_samples=1, bounces=3, rr_start=3)
+    scene = dict(nx=2, ny=2, nz=1, res=20, rgb=0xB3B3B3, extra_lines=LIGHT)
+    most, grown = 0, 0
+    with sa.Context(_cfg(schedule=schedule, **kw)) as ctx:
+        ctx.scenegen_load("s", **scene)
+        for phase in (0.0, 0.25, 0.5, 0.75, 1.0, 0.25, 2.25):
+            ctx.remesh(phase)
+            tris = sum(ctx.mesh_size(d)[1] for d in range(4))
+            grown += tris > most
+            most = max(most, tris)
+            img, st = ctx.trace_frame()
+            with sa.Context(_cfg(schedule=schedule, **kw)) as alone:
+                alone.scenegen_load("s", phase=phase, **scene)
+                want, wst = alone.trace_frame()
+                assert all(np.array_equal(ctx.normals(d), alone.normals(d)) for d in range(4)), phase
+            assert all(st[k] == wst[k] for k in ("useful_rays", "final_hits", "shades")), phase
+            assert np.abs(img - want).max() <= 1e-5, phase
+    assert grown >= 5
+
+
+@pytest.mark.parametrize("schedule", [0, 1])
+@pytest.mark.parametrize("cache", [2, 5])
+def test_paged_shading_of_both_forms(tmp_path, cache, schedule):
+    """Domains with shared vertices, whose mesh crosses the host link, and
+    without, whose shading records do, every vertex of a colour of its own."""
+    import spray_amd as sa
+    rng = np.random.default_rng(4)
+    doms = []
+    for d in range(6):
+        v, f = _sheet(rng, 13) if d % 2 else _soup(rng, 1 if d == 4 else 211, 0.2)
+        doms.append(dict(verts=v + [d % 3, d // 3, 1.0], faces=f,
+                         rgb=rng.integers(0, 256, (len(v), 3)).astype(np.uint8)))
+    path = scenes.write_scene(str(tmp_path), "s", doms, [LIGHT])
+    kw = dict(image_w=90, image_h=70, pixel_samples=2, ao_mode=0, ao_samples=1, bounces=3, rr_start=3)
+    with sa.Context(_cfg(schedule=schedule, **kw)) as ctx:
+        ctx.set_cache_size(cache)
+        ctx.load_scene(path, str(tmp_path))
+        ref = orc.Scene(path, str(tmp_path))
+        for _ in range(2):
+            _frame_ok(ctx, ref, **kw)
+        assert ctx.cache_state()[3] > 6  # (misses)
