@@ -224,22 +224,18 @@ inline int pipelineCount(int want) {
 }
 
 // Non-blocking streams that start after the work issued so far on `after`;
-// join() makes `after` wait for everything issued on them, and the
-// destructor waits for them and destroys them.
+// the destructor waits for them and destroys them.
 struct StreamSet {
   std::vector<hipStream_t> st;
-  std::vector<hipEvent_t> ev;
+  hipEvent_t ev = nullptr;
   StreamSet(int k, hipStream_t after) {
     if (k <= 0) return;
     st.assign(k, nullptr);
-    ev.assign(k, nullptr);
     try {
-      for (int i = 0; i < k; ++i) {
-        SPRAY_HIP(hipStreamCreateWithFlags(&st[i], hipStreamNonBlocking));
-        SPRAY_HIP(hipEventCreateWithFlags(&ev[i], hipEventDisableTiming));
-      }
-      SPRAY_HIP(hipEventRecord(ev[0], after));
-      for (int i = 0; i < k; ++i) SPRAY_HIP(hipStreamWaitEvent(st[i], ev[0], 0));
+      for (int i = 0; i < k; ++i) SPRAY_HIP(hipStreamCreateWithFlags(&st[i], hipStreamNonBlocking));
+      SPRAY_HIP(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+      SPRAY_HIP(hipEventRecord(ev, after));
+      for (int i = 0; i < k; ++i) SPRAY_HIP(hipStreamWaitEvent(st[i], ev, 0));
     } catch (...) {
       release();
       throw;
@@ -247,24 +243,16 @@ struct StreamSet {
   }
   StreamSet(const StreamSet&) = delete;
   StreamSet& operator=(const StreamSet&) = delete;
-  int size() const { return (int)st.size(); }
   hipStream_t operator[](int i) const { return st[i]; }
-  void join(hipStream_t after) {
-    for (size_t i = 0; i < st.size(); ++i) {
-      SPRAY_HIP(hipEventRecord(ev[i], st[i]));
-      SPRAY_HIP(hipStreamWaitEvent(after, ev[i], 0));
-    }
-  }
   void release() {
     for (hipStream_t x : st)
       if (x) {
         (void)hipStreamSynchronize(x);
         (void)hipStreamDestroy(x);
       }
-    for (hipEvent_t e : ev)
-      if (e) (void)hipEventDestroy(e);
+    if (ev) (void)hipEventDestroy(ev);
+    ev = nullptr;
     st.clear();
-    ev.clear();
   }
   ~StreamSet() { release(); }
 };

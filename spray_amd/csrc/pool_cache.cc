@@ -5,10 +5,13 @@
 // TriMeshBuffer::load (render/trimesh_buffer.cc:117-169): the reference
 // reads a missing domain's PLY file and builds its Embree scene; here every
 // domain is built once at load time and its image (BVH nodes, mesh, leaf
-// order) is kept in pinned host memory, so a miss is one host-to-HBM copy and
-// one launch that unpacks it into the evicted block.  Copies run on the
-// pool's copy stream, unpacking on another; the trace stream waits for a
-// block's unpacking, which waits for the last kernels that used the block.
+// order) is kept in pinned host memory, so a miss is one host-to-HBM copy into
+// a stage and one launch that unpacks it into the evicted block.  There are two
+// stages, taken in turn, each with a stream on which its copy, its unpacking
+// and the domain's descriptor follow one another.  The unpacking also waits for
+// the last kernels that used the block (block_free) and for the block's last
+// filling (block_ready), the descriptor for the load before; the trace stream
+// waits for the block's own load.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>

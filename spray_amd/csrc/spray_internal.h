@@ -98,7 +98,9 @@ int scenegenWrite(const spray_scenegen_params& p, const char* dir, const char* n
 // ---------------------------------------------------------------------------
 // Device layouts (shared by host and kernels)
 
-// One 8-wide BVH node: the 64 bytes that a visit reads.  Child boxes are 8-bit
+// One 8-wide BVH node (after Ylitie, Karras and Laine, HPG 2017, whose grid,
+// octant slots and consecutive inner children it shares; the layout is this
+// one's own): the 64 bytes that a visit reads.  Child boxes are 8-bit
 // plane numbers on the node's own grid: plane q of axis k lies at
 // base[k] + q * 2^e[k], and the last byte of base[k], part of its value, is
 // e[k] + 127.  plane[k][0..7] / plane[k][8..15] are the children's lower /

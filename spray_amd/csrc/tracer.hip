@@ -1175,8 +1175,9 @@ __global__ void __launch_bounds__(kTravBlock, 4) kTraverse(TraceParams P, int pl
   //   plain_dom == -1: every queue of the pass (batched); with the learned
   //     form the phase-A list first and the deferred list last, so that the
   //     deferred entries meet the histories phase A has updated.  When phase
-  //     A and the shadow queues hold fewer than 4 entries per lane of the
-  //     grid, every wave would start on deferred entries at once: then phase
+  //     A and the shadow queues hold fewer than 4 entries per launched lane (6
+  //     per resident one), waves would reach the deferred entries beside
+  //     phase A: then phase
   //     0 stops after the shadow queues and phase 1 (a second launch) takes
   //     the deferred list; otherwise phase 1 has nothing to do
   //   plain_dom == -2: shadow rays spawned in this pass, in their spawning
@@ -1961,7 +1962,8 @@ static void ensureState(Ctx* c, double grow) {
   }
   hipDeviceProp_t prop;
   SPRAY_HIP(hipGetDeviceProperties(&prop, c->device));
-  // resident blocks: enough waves per CU to hide traversal latency
+  // 24 waves per CU are launched.  LDS and registers hold 16 of them at once
+  // (travResidentBlocks); the other blocks start as those end
   int block = 64 * std::max(1, c->batch_tile);
   int per_cu = std::max(1, 1536 / block);
   T->grid_persistent = prop.multiProcessorCount * per_cu;
@@ -2290,8 +2292,8 @@ static bool passPlain(Ctx* c, const TraceParams& P) {
     int d = T->h_order[k];
     if (T->h_cnt[d] + T->h_cnt[nd + d] > 0) doms.push_back(d);
   }
-  // with a paged pool every domain is loaded in turn (the next one ahead, on
-  // the copy stream), and its hits are shaded and its new shadow rays tested
+  // with a paged pool every domain is loaded in turn (the next one ahead, on a
+  // load stream), and its hits are shaded and its new shadow rays tested
   // while it is resident
   const bool paged = c->pool.paged;
   for (size_t j = 0; j < doms.size(); ++j) {
@@ -2321,7 +2323,7 @@ static bool passPlain(Ctx* c, const TraceParams& P) {
 // Batched pass over a paged pool.  The queues are laid out in schedule
 // order, so consecutive scheduled domains own contiguous entry ranges: the
 // pass traces them in chunks of half the cache, one persistent launch per
-// chunk, while the next chunk's domains load on the copy stream.  Each
+// chunk, while the next chunk's domains load on the load streams.  Each
 // chunk's hits are shaded and its new shadow rays tested while it is
 // resident.  Chunks run forward and backward in alternate passes, so the
 // last chunk of a pass is still resident for the first of the next.

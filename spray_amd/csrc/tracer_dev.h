@@ -34,8 +34,7 @@ struct RayPool {
   __device__ __forceinline__ float4& h(size_t i) const { return r[i * 4 + 3]; }
 };
 constexpr uint32_t kOccluded = 1u << 31;
-// fields of wd.w
-__device__ __forceinline__ int rayDepth(float w) { return __float_as_int(w) & 0xff; }
+// fields of wd.w (the depth: its last 8 bits)
 __device__ __forceinline__ int raySpawn(float w) { return (__float_as_int(w) >> 8) & 0x7fffff; }
 __device__ __forceinline__ bool rayOccluded(float w) { return __float_as_int(w) < 0; }
 

@@ -16,6 +16,10 @@
 // visits as in slot order, 3% slower); node lines fetched by four lanes each
 // through LDS (5% slower); leaves of 3 or 4 triangles (3 and 5% slower); five
 // waves a SIMD with half the LDS stack and triangles one at a time (a wash).
+// Nodes of eight children on a grid of the node's own, slots by octant and
+// groups of children on the stack are the method of Ylitie, Karras and Laine,
+// "Efficient Incoherent Ray Traversal on GPUs Through Compressed Wide BVHs"
+// (HPG 2017).
 //
 // Per-lane stack of node groups (a group: the children of one node that the
 // ray has still to visit): the first kRing entries in LDS.  Each wave owns
