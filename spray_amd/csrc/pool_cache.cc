@@ -140,7 +140,9 @@ static int lruLoad(Ctx* c, int d, int keep) {
   // for the copies and one for the unpacking: the next image's copy starts
   // when its own stage is free and no unpacking waits for an event of the
   // copies (400x300 path trace of 4 samples, 48 domains, 12 blocks: 13.3 ->
-  // 11.1 ms; 1920x1080, 256 domains, 128 blocks: 877 -> 785 ms).
+  // 11.0 ms, and 17.0 -> 14.3 to 15.9 in a process whose other streams leave
+  // the trace stream to share a hardware queue with a stage's; 1920x1080, 256
+  // domains, 128 blocks: 877 -> 785 ms).
   const DomainDesc& D = P.desc[d];
   const char* src = (const char*)P.h_image + P.h_image_off[d];
   const ImageLayout L(D.num_nodes, D.num_tris, P.nverts[d]);
